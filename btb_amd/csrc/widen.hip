@@ -153,24 +153,24 @@ __global__ void __launch_bounds__(256) p12_pairs_kernel(const uint8_t* __restric
 
 extern "C" {
 
-// a row's first 8 or 16 escapes as words of the row's own (FmtP12::row_escapes reads them, FmtP12::tail uses them)
+// a row's first 8 or 16 escapes as words of the row's own (FmtP12::row_escapes reads them, FmtP12::tail uses them), a
+// thread a word: a row's words are neighbours in memory and so are the threads that write them
 __global__ void __launch_bounds__(256) p12_row_esc_kernel(const uint8_t* __restrict__ lo, const int32_t* __restrict__ esc_idx,
                                                           const uint8_t* __restrict__ esc_val,
                                                           const int32_t* __restrict__ row_ptr, int rows, int cols,
                                                           uint32_t* __restrict__ out) {
-    const int r = blockIdx.x * 256 + threadIdx.x;
-    if (r >= rows) return;
-    const int e0 = row_ptr[r], e1 = row_ptr[r + 1];
     const int slots = FmtP12::row_esc_slots(cols);
-    const uint32_t more = e1 - e0 > slots ? 0x80000000u : 0u;
-    for (int k = 0; k < slots; ++k) {
-        uint32_t w = FmtP12::ROW_ESC_NONE << 16;
-        if (e0 + k < e1) {
-            const size_t i = (size_t)esc_idx[e0 + k];
-            w = (uint32_t)lo[i] | ((uint32_t)esc_val[e0 + k] << 8) | ((uint32_t)(i - (size_t)r * cols) << 16);
-        }
-        out[(size_t)r * slots + k] = w | more;
+    const size_t at = (size_t)blockIdx.x * 256 + threadIdx.x;
+    const size_t r = at / slots;  // slots: a power of two
+    const int k = (int)(at - r * slots);
+    if (r >= (size_t)rows) return;
+    const int e0 = row_ptr[r], e1 = row_ptr[r + 1];
+    uint32_t w = FmtP12::ROW_ESC_NONE << 16;
+    if (e0 + k < e1) {
+        const size_t i = (size_t)esc_idx[e0 + k];
+        w = (uint32_t)lo[i] | ((uint32_t)esc_val[e0 + k] << 8) | ((uint32_t)(i - r * cols) << 16);
     }
+    out[at] = w | (e1 - e0 > slots ? 0x80000000u : 0u);
 }
 
 int32_t btb_hip_p12_row_esc(const void* lo, const void* esc_idx, const void* esc_val, size_t n_esc, const void* row_ptr,
@@ -179,7 +179,8 @@ int32_t btb_hip_p12_row_esc(const void* lo, const void* esc_idx, const void* esc
     if (n_esc > 0 && (esc_idx == nullptr || esc_val == nullptr)) return ERR_NULL;
     if (rows == 0 || cols == 0 || cols > FmtP12::ROW_ESC_NONE || rows * cols > 0x7FFFFFFFull) return ERR_DOMAIN;
     if (!al(esc_idx, 4) || !al(row_ptr, 4) || !al(row_esc, 4)) return ERR_DOMAIN;
-    hipLaunchKernelGGL(p12_row_esc_kernel, dim3((unsigned)((rows + 255) / 256)), dim3(256), 0,
+    const size_t words = rows * (size_t)FmtP12::row_esc_slots((int)cols);
+    hipLaunchKernelGGL(p12_row_esc_kernel, dim3((unsigned)((words + 255) / 256)), dim3(256), 0,
                        static_cast<hipStream_t>(stream), static_cast<const uint8_t*>(lo),
                        static_cast<const int32_t*>(esc_idx), static_cast<const uint8_t*>(esc_val),
                        static_cast<const int32_t*>(row_ptr), (int)rows, (int)cols, static_cast<uint32_t*>(row_esc));

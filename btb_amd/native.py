@@ -45,6 +45,9 @@ SIGNATURES: dict[str, tuple[Any, list[Any]]] = {
     "btb_hip_gemv_p12_norm": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp, _vp, _vp, _vp, _vp, ctypes.c_float, _i32, _vp,
                                      _vp, _sz, _sz, _sz, _i32, _vp]),
     "btb_hip_gemv_p12": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp, _vp, _vp, _vp, _sz, _sz, _sz, _vp]),
+    "btb_hip_p12_pack_words": (_sz, [_sz]),
+    "btb_hip_p12_pack": (_i32, [_vp, _sz, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "btb_hip_p12_emit": (_i32, [_vp, _vp, _sz, _vp, _sz, _vp, _vp, _sz, _sz, _vp, _vp]),
     "btb_hip_p12_pairs": (_i32, [_vp, _vp, _vp]),
     "btb_hip_p12_row_esc": (_i32, [_vp, _vp, _vp, _sz, _vp, _sz, _sz, _vp, _vp]),
     "btb_hip_p12_row_ptr": (_i32, [_vp, _sz, _sz, _sz, _vp, _vp]),
@@ -365,6 +368,29 @@ class HipCard(CardLaunch):
         if y.numel() != M * R:
             raise ValueError(f"[hip] {what}: y holds {y.numel()} elements, the product has {M * R}")
         return y
+
+    def p12_pack(self, t: torch.Tensor):
+        """(lo, hi4, table, pairs, esc_idx, esc_val, row_ptr) of a bf16 matrix on the GPU: `pack12.pack_bf16`'s bytes, the
+        pair table and the rows' first entries in the escape list, made by the card"""
+        self._need(t, torch.bfloat16, "t")
+        if t.dim() != 2 or t.numel() == 0:
+            raise ValueError(f"[hip] p12_pack takes a matrix, got {tuple(t.shape)}")
+        if t.data_ptr() % 16:
+            t = t.clone()
+        (rows, cols), n, dev = (int(s) for s in t.shape), int(t.numel()), t.device
+        u8 = dict(dtype=torch.uint8, device=dev)
+        lo, hi4, table = torch.empty(n, **u8), torch.empty((n + 1) // 2, **u8), torch.empty(16, **u8)
+        pairs = torch.empty(256, dtype=torch.int16, device=dev)
+        work = torch.empty(int(self.lib.btb_hip_p12_pack_words(n)), dtype=torch.int32, device=dev)
+        total = torch.empty(1, dtype=torch.int32, pin_memory=True)
+        st = _stream()
+        self._call("btb_hip_p12_pack", _p(t), n, _p(lo), _p(hi4), _p(table), _p(pairs), _p(work), _p(total), st)
+        ne = int(total)
+        esc_idx, esc_val = torch.empty(ne, dtype=torch.int32, device=dev), torch.empty(ne, **u8)
+        row_ptr = torch.empty(rows + 1, dtype=torch.int32, device=dev)
+        self._call("btb_hip_p12_emit", _p(t), _p(hi4), n, _p(work), ne, _p(esc_idx) if ne else None,
+                   _p(esc_val) if ne else None, rows, cols, _p(row_ptr), st)
+        return lo, hi4, table, pairs, esc_idx, esc_val, row_ptr
 
     def p12_check(self, esc_idx: torch.Tensor, n: int) -> None:
         """ValueError unless the escape list is strictly ascending inside [0, n): checked on the GPU, once, at upload"""

@@ -4,8 +4,8 @@ Same interface and byte layout as the reference's `btb/pack12.py` (:48-67 `pack_
 :100-110 `blob`, :113-133 `entry`): a bf16 tensor is a low byte per element (`lo`), a 4-bit code per element into a
 15-entry table of high bytes (`hi4`, the earlier element in the low nibble) and an escape list (ascending int32
 indices and their high bytes) for the elements whose high byte is not in the table. The table lists high bytes by
-frequency, ties by byte value, so a tensor packs to the same bytes every time. Everything here runs in torch on
-whatever device the tensor is on, so a whole model packs on the GPU in seconds.
+frequency, ties by byte value, so a tensor packs to the same bytes every time. The codec runs in torch on whatever
+device the tensor is on; `P12Weight.pack` makes the same bytes by the card's own kernels.
 
 `P12Weight` is a packed matrix as the kernels read it: the five arrays on the GPU plus the per-row escape offsets
 (`row_ptr`, built once at upload by `btb_hip_p12_row_ptr`) that let a wave find its row's escapes without a search.
@@ -187,7 +187,8 @@ class P12Weight:
         self.esc_val = esc_val.to(torch.uint8).contiguous()
         self.shape = (int(rows), int(cols))
         # the kernels index the low bytes and x with these: a list from a damaged store must never reach them
-        check_escapes(self.esc_idx, self.esc_val, n)
+        if self.esc_idx.numel() != self.esc_val.numel():
+            raise ValueError(f"[pack12] {self.esc_idx.numel()} escape indices but {self.esc_val.numel()} escape values")
         card.p12_check(self.esc_idx, n)
         self.row_ptr = card.p12_row_ptr(self.esc_idx, rows, cols)
         self.pairs = card.p12_pairs(self.table)
@@ -195,8 +196,20 @@ class P12Weight:
 
     @classmethod
     def pack(cls, w: torch.Tensor, card: Any) -> "P12Weight":
+        """a bf16 matrix on the GPU packed by the card's kernels: `pack_bf16`'s bytes. The list is theirs, so it needs no
+        check; the table's slot 15 is 0."""
         rows, cols = (int(s) for s in w.shape)
-        return cls(*pack_bf16(w), rows, cols, card)
+        if w.dtype != torch.bfloat16:
+            raise ValueError(f"[pack12] only bf16 tensors pack, this one is {w.dtype}")
+        if w.device.type != "cuda":
+            raise ValueError("[pack12] a P12Weight lives on the GPU")
+        check_size(w.numel())
+        self = cls.__new__(cls)
+        self.shape = (rows, cols)
+        (self.lo, self.hi4, self.table, self.pairs, self.esc_idx, self.esc_val,
+         self.row_ptr) = card.p12_pack(w.detach().contiguous())
+        self.row_esc = card.p12_row_esc(self.lo, self.esc_idx, self.esc_val, self.row_ptr, rows, cols)
+        return self
 
     @property
     def nbytes(self) -> int:

@@ -126,6 +126,19 @@ int32_t btb_hip_gemv_p12_embed_norm(const void* lo, const void* hi4, const void*
                                     const void* norm_w, float eps, int32_t centered, void* h_out, void* out, size_t R,
                                     size_t C, size_t M, void* stream);
 
+/* A bf16 tensor t u16[n] into its 12-bit form: lo u8[n], hi4 u8[(n + 1) / 2] (an odd tail's high nibble 0), table u8[16]
+ * and its pairs u16[256], with the number of escapes in *host_total - pinned host memory the device writes - when the
+ * call returns: it waits for that number, not for the encoding queued behind it, so that the caller can allocate the
+ * list. `work`: btb_hip_p12_pack_words(n) u32 words, kept for btb_hip_p12_emit, which then writes the list (esc_idx
+ * i32[n_esc] ascending, esc_val u8[n_esc]) and, where row_ptr i32[rows + 1] is given, rows * cols = n, what
+ * btb_hip_p12_row_ptr makes of it. The bytes of pack12.pack_bf16 (btb/pack12.py:48-67). t 16-byte aligned, n below 2^31.
+ * Waits on the stream's work, so neither is recorded into a capture. */
+size_t btb_hip_p12_pack_words(size_t n);
+int32_t btb_hip_p12_pack(const void* t, size_t n, void* lo, void* hi4, void* table, void* pairs, void* work,
+                         int32_t* host_total, void* stream);
+int32_t btb_hip_p12_emit(const void* t, const void* hi4, size_t n, const void* work, size_t n_esc, void* esc_idx,
+                         void* esc_val, size_t rows, size_t cols, void* row_ptr, void* stream);
+
 /* pairs[b] = table[b & 15] | table[b >> 4] << 8 for every byte b of codes, the escape code's slot 15 taken as 0: the
  * high bytes of the two weights a byte of codes stands for, so that the matvec turns a byte of codes into two high
  * bytes with one 2-byte read of its copy of these 512 bytes in LDS. Made once at upload, beside row_ptr; an escaped

@@ -1,0 +1,50 @@
+"""The 12-bit packer on the card (`HipCard.p12_pack`, `P12Weight.pack`) against the oracle's packer, byte for byte, at the
+sizes where its pieces meet: a lane's 8 weights, a chunk of 2048, a workgroup's 32768, rows that begin inside a chunk, odd
+tails; and on values with no escapes, with few and with most weights escaped."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from btb_amd.pack12 import P12Weight, pack_bf16
+from oracle import codecs
+
+from .helpers import bits16
+
+pytestmark = pytest.mark.gpu
+
+
+def values(kind: str, n: int) -> torch.Tensor:
+    g = torch.Generator().manual_seed(0x0B7B + n)
+    if kind == "normal":
+        return (torch.randn(n, generator=g) * 0.02).to(torch.bfloat16)
+    if kind == "bits":  # every bit pattern: 15 high bytes of 256 have a code
+        return torch.randint(-(2**15), 2**15, (n,), generator=g).to(torch.int16).view(torch.bfloat16)
+    return torch.full((n,), -1.5, dtype=torch.bfloat16)
+
+
+@pytest.mark.parametrize("kind", ["normal", "bits", "one"])
+@pytest.mark.parametrize("rows,cols", [(1, 1), (1, 7), (3, 5), (2, 8), (7, 33), (16, 128), (17, 121), (1, 2047), (1, 32768),
+                                       (3, 10923), (257, 130), (40, 2560), (5, 9728), (300, 1000)])
+def test_packed_on_the_card(card, kind, rows, cols):
+    w = values(kind, rows * cols).reshape(rows, cols)
+    pw = P12Weight.pack(w.cuda(), card)
+    lo, hi4, table, idx, val = codecs.pack12_pack(bits16(w))
+    for got, want in ((pw.lo, lo), (pw.hi4, hi4), (pw.table, table), (pw.esc_idx, idx), (pw.esc_val, val)):
+        assert np.array_equal(got.cpu().numpy(), want)
+    # what the constructor makes at upload of a stored matrix's arrays
+    up = P12Weight(*(t.cuda() for t in pack_bf16(w)), rows, cols, card)
+    for name in ("pairs", "row_ptr", "row_esc"):
+        a, b = getattr(pw, name), getattr(up, name)
+        assert (a is None and b is None and cols > 32767) or torch.equal(a, b), name
+    assert np.array_equal(pw.row_ptr.cpu().numpy(), np.searchsorted(idx, np.arange(rows + 1) * cols))
+
+
+def test_a_view_that_is_not_16_byte_aligned(card):
+    w = values("normal", 4096 + 3)
+    pw = P12Weight.pack(w.cuda()[3:].reshape(64, 64), card)
+    lo, hi4, _, idx, _ = codecs.pack12_pack(bits16(w[3:]))
+    assert np.array_equal(pw.lo.cpu().numpy(), lo) and np.array_equal(pw.hi4.cpu().numpy(), hi4)
+    assert np.array_equal(pw.esc_idx.cpu().numpy(), idx)
