@@ -232,6 +232,11 @@ int32_t attn_decode_mfma(const void* q, const void* K, const void* V, const int3
                          size_t Hq, size_t Hk, long long hs, long long rs, float scale_log2, float* part_m,
                          float* part_l, float* part_acc, size_t S, size_t cap, int win, const int32_t* tbl,
                          hipStream_t st);
+// ... in spans of any number of whole batches, walked with an online softmax (attn_span.hip)
+bool attn_span_fits(size_t T, size_t G);
+int32_t attn_decode_span(const void* q, const void* K, const void* V, const int32_t* n0, const int32_t* par, size_t T,
+                         size_t Hq, size_t Hk, long long hs, long long rs, float scale_log2, float* part_m, float* part_l,
+                         float* part_acc, size_t S, int span, int win, const int32_t* tbl, hipStream_t st);
 bool attn_mfma_qkv_fits(size_t T, size_t G, int span);
 int32_t attn_decode_mfma_qkv(const void* qkv, const void* wq, const void* wk, float eps, int centered, const void* cos_t,
                              const void* sin_t, const int32_t* n0, const int32_t* depth, const int32_t* par, void* K,
@@ -817,6 +822,18 @@ static int32_t attn_decode_any(const void* q, const void* K, const void* V, void
         if (rc != OK) return rc;
         if (G == 4) launch_merge<4>(st, att, T, Hq, Hk, S, part_m, part_l, part_acc, nullptr);
         else launch_merge<2>(st, att, T, Hq, Hk, S, part_m, part_l, part_acc, nullptr);
+        return hip_status(hipGetLastError(), "attn_decode launch");
+    }
+    if (parts == nullptr && attn_span_fits(T, G)) {
+        const int32_t rc = attn_decode_span(q, K, V, n0, par, T, Hq, Hk, (long long)hs, (long long)rs, scale_log2, part_m,
+                                            part_l, part_acc, S, span, (int)win, tbl, st);
+        if (rc != OK) return rc;
+        switch (G) {
+            case 1: launch_merge<1>(st, att, T, Hq, Hk, S, part_m, part_l, part_acc, nullptr); break;
+            case 2: launch_merge<2>(st, att, T, Hq, Hk, S, part_m, part_l, part_acc, nullptr); break;
+            case 4: launch_merge<4>(st, att, T, Hq, Hk, S, part_m, part_l, part_acc, nullptr); break;
+            default: launch_merge<8>(st, att, T, Hq, Hk, S, part_m, part_l, part_acc, nullptr); break;
+        }
         return hip_status(hipGetLastError(), "attn_decode launch");
     }
     if (parts == nullptr && T >= 2 && (span == 128 || span == 256) && (G == 2 || G == 4)) {

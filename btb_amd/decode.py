@@ -82,6 +82,24 @@ def rope_tables(cfg: StackConfig, positions: int, device: Any) -> tuple[torch.Te
     return emb.cos().to(torch.bfloat16).contiguous(), emb.sin().to(torch.bfloat16).contiguous()
 
 
+def pass_spans(cus: int, T: int, Hq: int, Hk: int, cap: int) -> int:
+    """how many spans the attention of a pass of T rows cuts a cache of `cap` slots into. Its workgroup walks a span in
+    batches of 128 keys for up to 64 (row, head) pairs of a kv head, so: a workgroup a CU, spans whole batches. Where a
+    kv head's pairs take several workgroups, which read the same keys, and spans stay at 512 keys or more, two a CU.
+    Measured on MI355X with the fold, us a layer: 8 rows x 32 / 8 heads, 4096 keys: 18 spans 11.9, 9 15.8, 36 15.1; 2
+    rows, 32000 keys: 31 spans 30.8, 16 46.5, 56 32.7; 13 rows x 32 / 4, 6125 keys: 27 spans 19.9, 53 22.6; two a CU: 26
+    rows x 32 / 8, 23367 keys: 29 spans 54.5, 16 61.4, 51 64.8; 32 rows x 64 / 8, 8000 keys: 14 spans 42.6, 8 47.7."""
+    G = Hq // Hk
+    z = -(-T * G // 64)
+    most = 1024 // G  # the fold's limit
+
+    def keys(per_cu: int) -> int:
+        return max(1, -(-cap // max(1, min(most, per_cu * cus // (Hk * z)) * 128))) * 128
+
+    span = keys(2) if z > 1 and keys(2) >= 512 else keys(1)
+    return -(-cap // span)
+
+
 class Linear:
     """one linear's weight on the GPU in its stored form, multiplied as stored: a bf16 tensor or a `P12Weight`"""
 
@@ -160,6 +178,8 @@ class DecodeStep:
                 # against the best span count of the general kernel: 2 rows 2.95 / 3.12, 4 rows 3.51 / 3.68, 8 rows
                 # 3.67 / 3.83, 16 rows 4.64 / 4.83)
                 attn_spans = -(-self.cap // 128)
+            elif self.T > 1 and D == 128 and Hq // Hk in (1, 2, 4, 8):
+                attn_spans = pass_spans(card.sms, self.T, Hq, Hk, self.cap)
         self.S = int(attn_spans)
         self.scratch = card.attn_scratch(T, Hq, Hk, D, self.S, dev)
         # Which sequence: up to three rows the fused launches win (fewer launches, every matvec on the streaming
