@@ -181,6 +181,7 @@ __global__ void __launch_bounds__(256) attn_decode_mfma_kernel(
     const int c = lane & 15, a = lane >> 4;
     const int k_begin = sp * AM_SPAN;
     const float ninf = bits_f32(0xff800000u);
+    const int parent = tree_parent(par, T);
 
     // Everything the workgroup reads from memory is asked for before anything is waited for. Without a row map the
     // addresses do not depend on *n0: a slot at or past the cache's capacity reads the last slot again, and which keys
@@ -251,6 +252,7 @@ __global__ void __launch_bounds__(256) attn_decode_mfma_kernel(
     // the keys any of the workgroup's rows may see end at n_max (a chain's last row, or the whole pass for a tree)
     const int n_max = par != nullptr ? n0 + T : n0 + t_end;
     const int k_lim = min(n_max, k_begin + AM_SPAN);
+    const uint32_t rows = tree_rows(parent, T);
     if constexpr (QKV) {
         auto tables = [&](int id, HeadTile& h) {
             const int t = min(task_row(id), T - 1);
@@ -343,7 +345,7 @@ __global__ void __launch_bounds__(256) attn_decode_mfma_kernel(
     for (int qt = 0; qt < NQT; ++qt) {
         const int r = qt * 16 + c, t = t_base + r / G;
         const bool row_ok = t < T;
-        const RowView rv = row_view(par, min(t, T - 1), T, n0, win);
+        const RowView rv = row_view_of(rows, par, min(t, T - 1), T, n0, win);
         // branch-free: this runs once a workgroup, and a path that short is bound by how fast its code arrives
         const int k_end = row_ok ? min(rv.n, k_lim) : 0;
         const int tb = rv.tree_base >= 0 ? rv.tree_base : 0x7FFFFFFF;  // the first of the pass's own slots, if a tree

@@ -58,6 +58,7 @@ __global__ void __launch_bounds__(256, 2) attn_span_kernel(
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int c = lane & 15, a = lane >> 4;
     const float ninf = bits_f32(0xff800000u);
+    const int parent = tree_parent(par, T);
     const int n0 = *n0p;
     const int k_begin = sp * span;
     // the keys any of the workgroup's rows may see end at n_max (a chain's last row, or the whole pass for a tree)
@@ -106,6 +107,7 @@ __global__ void __launch_bounds__(256, 2) attn_span_kernel(
         request_k(k_begin);
         request_v(k_begin);
     }
+    const uint32_t rows = tree_rows(parent, T);  // while the first batch travels
     for (int kb = k_begin; kb < k_lim; kb += AS_KEYS) {
         // scores: S^T tile [h][qt], lane: pair c of tile qt against keys kb + 32 wv + 16 h + 4 a .. + 3
         f32x4 st[2][NQT];
@@ -134,7 +136,7 @@ __global__ void __launch_bounds__(256, 2) attn_span_kernel(
 #pragma unroll
             for (int qt = 0; qt < NQT; ++qt) {
                 const int t = t_base + ((qt * 16 + c) >> gs);
-                const RowView rv = row_view(par, min(t, T - 1), T, n0, win);
+                const RowView rv = row_view_of(rows, par, min(t, T - 1), T, n0, win);
                 const int k_end = t < T ? min(rv.n, k_lim) : 0;
                 const int tb = rv.tree_base >= 0 ? rv.tree_base : 0x7FFFFFFF;  // the first of the pass's own slots, if a tree
 #pragma unroll

@@ -553,4 +553,37 @@ __device__ __forceinline__ RowView row_view(const int32_t* __restrict__ par, int
     return v;
 }
 
+// The same for many (row, head) pairs a wave without a window: every row's ancestors at once, lane l holding those of row
+// l % 32. Walking par hop by hop is a chain of dependent loads per pair - a chunk of a prompt is a chain of 32 rows, 64
+// hops a tile of pairs: 24 of the 36.8 us of its attention (32 rows x 32 / 8 heads over 1536 keys). Here each lane loads
+// its row's parent once and the sets double in five exchanges: after k of them a lane knows its first 2^k ancestors.
+// A parent outside 0 .. T - 1 is none; T <= 32. All 64 lanes call.
+__device__ __forceinline__ int tree_parent(const int32_t* __restrict__ par, int T) {  // ask early, use in tree_rows
+    const int r = (int)(threadIdx.x & 31);
+    return par != nullptr ? par[min(r, T - 1)] : -1;
+}
+__device__ __forceinline__ uint32_t tree_rows(int parent, int T) {
+    const int r = (int)(threadIdx.x & 31);
+    int up = r < T && parent >= 0 && parent < T ? parent : -1;  // the ancestor 2^k hops up
+    uint32_t mask = 1u << r;
+#pragma unroll
+    for (int k = 0; k < 5; ++k) {
+        const uint32_t theirs = (uint32_t)__builtin_amdgcn_ds_bpermute(max(up, 0) << 2, (int)mask);
+        const int next = __builtin_amdgcn_ds_bpermute(max(up, 0) << 2, up);
+        mask |= up >= 0 ? theirs : 0u;
+        up = up >= 0 ? next : -1;
+    }
+    return mask;
+}
+// row t's view given tree_rows' sets (`rows`: this lane's); all 64 lanes call
+__device__ __forceinline__ RowView row_view_of(uint32_t rows, const int32_t* __restrict__ par, int t, int T, int n0, int win) {
+    if (win > 0) return row_view(par, t, T, n0, win);  // uniform
+    RowView v;
+    v.tree_base = par != nullptr ? n0 : -1;
+    v.n = par != nullptr ? n0 + T : n0 + t + 1;
+    v.tree_mask = (uint32_t)__builtin_amdgcn_ds_bpermute((t & 31) << 2, (int)rows);
+    v.k_first = 0;
+    return v;
+}
+
 }  // namespace btb
