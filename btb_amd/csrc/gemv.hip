@@ -394,7 +394,7 @@ static int32_t launch_stream(const typename F::Params& p, const XArgs& xa, void*
         }
     } else if constexpr (WIDENS) {
         if constexpr (F::TWO_ROWS) {
-            if constexpr (M == 1 && XMODE == X_PLAIN) {
+            if constexpr (M == 1) {
                 // One row of x over FP8: a lane's 5 to 8 units of a row asked for at once, one row a wave - one trip to
                 // memory for the row instead of three or four spans of two units ([18432 x 7168], 7 units a lane:
                 // 26.3 -> 24.4 us; two rows by four units 25.1, by three 25.4, one row by four 27.2).
@@ -571,6 +571,19 @@ static bool norm_on_mfma(const XArgs& xa, size_t R, size_t C, size_t M, bool glu
     auto al8 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 7u) == 0; };
     return tuning("gemv_no_mfma") <= 0 && tuning("mfma_lds") != 0 && C % 32 == 0 && (!glu || (R / 2) % 16 == 0) &&
            mfma_lds_norm_fits((int)R, (int)C, (int)M) && al8(xa.x) && al8(xa.y) && al8(xa.norm_w) && al8(xa.h_out);
+}
+
+static int32_t fp8_dims(const void* w, const void* scales, size_t sr, size_t sc, size_t R, size_t C, size_t M) {
+    if (sr == 0 || sc == 0) return ERR_DOMAIN;
+    const int32_t rc = check_dims(R, C, M, FmtF8::UW);
+    if (rc != OK) return rc;
+    if (R % sr != 0 || C % sc != 0 || (C / sc) % FmtF8::UW != 0) return ERR_DOMAIN;
+    return aligned16(w) && (reinterpret_cast<uintptr_t>(scales) & 3u) == 0 ? OK : ERR_DOMAIN;
+}
+static FmtF8::Params fp8_params(const void* w, const void* scales, size_t sr, size_t sc, size_t R, size_t C) {
+    const uint32_t upb = (uint32_t)(C / sc / FmtF8::UW);
+    return FmtF8::Params{static_cast<const uint8_t*>(w), static_cast<const float*>(scales), (int)sc, (int)(R / sr),
+                         (int)upb, upb > 1 ? (uint32_t)(0x100000000ull / upb + 1) : 0u};
 }
 
 static int32_t p12_params(const void* lo, const void* hi4, const void* table, const void* pairs, const void* esc_idx,
@@ -783,11 +796,9 @@ int32_t btb_hip_gemv_p12_embed_norm(const void* lo, const void* hi4, const void*
 int32_t btb_hip_gemv_fp8(const void* w, const void* scales, size_t sr, size_t sc, const void* x, void* y, size_t R,
                          size_t C, size_t M, void* stream) {
     if (w == nullptr || scales == nullptr || x == nullptr || y == nullptr) return ERR_NULL;
-    if (sr == 0 || sc == 0) return ERR_DOMAIN;
-    int32_t rc = check_dims(R, C, M, FmtF8::UW);
+    int32_t rc = fp8_dims(w, scales, sr, sc, R, C, M);
     if (rc != OK) return rc;
-    if (R % sr != 0 || C % sc != 0 || (C / sc) % FmtF8::UW != 0) return ERR_DOMAIN;
-    if (!aligned16(w) || !aligned16(x) || (reinterpret_cast<uintptr_t>(scales) & 3u) || !aligned2(y)) return ERR_DOMAIN;
+    if (!aligned16(x) || !aligned2(y)) return ERR_DOMAIN;
     const size_t from = fp8_matrix_from(R, C);
     if (wide_pass(M, R, C, true, from) && mfma_dl_fits_fp8((int)R, (int)C, 16, (int)(R / sr), (int)(C / sc))) {
         const uint16_t* xp = static_cast<const uint16_t*>(x);  // the long rows: weights straight into LDS, 16 rows a pass
@@ -811,10 +822,38 @@ int32_t btb_hip_gemv_fp8(const void* w, const void* scales, size_t sr, size_t sc
         }
         return OK;
     }
-    const uint32_t upb = (uint32_t)(C / sc / FmtF8::UW);
-    FmtF8::Params p{static_cast<const uint8_t*>(w), static_cast<const float*>(scales), (int)sc, (int)(R / sr),
-                    (int)upb, upb > 1 ? (uint32_t)(0x100000000ull / upb + 1) : 0u};
-    return run_rows<FmtF8, X_PLAIN, E_PLAIN>(p, plain_x(x), y, R, C, M, static_cast<hipStream_t>(stream));
+    return run_rows<FmtF8, X_PLAIN, E_PLAIN>(fp8_params(w, scales, sr, sc, R, C), plain_x(x), y, R, C, M,
+                                             static_cast<hipStream_t>(stream));
+}
+
+int32_t btb_hip_gemv_fp8_norm(const void* w, const void* scales, size_t sr, size_t sc, const void* h_in, const void* y,
+                              const void* norm_w, float eps, int32_t centered, void* h_out, void* out, size_t R, size_t C,
+                              size_t M, int32_t glu, void* stream) {
+    if (w == nullptr || scales == nullptr || out == nullptr) return ERR_NULL;
+    XArgs xa;
+    int32_t rc = norm_args(h_in, y, norm_w, eps, centered, h_out, &xa);
+    if (rc != OK) return rc;
+    rc = fp8_dims(w, scales, sr, sc, R, C, M);
+    if (rc != OK) return rc;
+    if (!aligned2(out) || (glu && R % 2 != 0)) return ERR_DOMAIN;
+    const FmtF8::Params p = fp8_params(w, scales, sr, sc, R, C);
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    return glu ? run_rows<FmtF8, X_ADDNORM, E_GLU>(p, xa, out, R, C, M, st)
+               : run_rows<FmtF8, X_ADDNORM, E_PLAIN>(p, xa, out, R, C, M, st);
+}
+
+int32_t btb_hip_gemv_fp8_embed_norm(const void* w, const void* scales, size_t sr, size_t sc, const void* table,
+                                    const int32_t* ids, size_t vocab, const void* norm_w, float eps, int32_t centered,
+                                    void* h_out, void* out, size_t R, size_t C, size_t M, void* stream) {
+    if (w == nullptr || scales == nullptr || out == nullptr) return ERR_NULL;
+    XArgs xa;
+    int32_t rc = embed_args(table, ids, vocab, norm_w, eps, centered, h_out, &xa);
+    if (rc != OK) return rc;
+    rc = fp8_dims(w, scales, sr, sc, R, C, M);
+    if (rc != OK) return rc;
+    if (!aligned2(out)) return ERR_DOMAIN;
+    return run_rows<FmtF8, X_ADDNORM, E_PLAIN>(fp8_params(w, scales, sr, sc, R, C), xa, out, R, C, M,
+                                               static_cast<hipStream_t>(stream));
 }
 
 int32_t btb_hip_gemv_mxfp4(const void* blocks, const void* scales, const void* x, void* y, size_t R, size_t C, size_t M,

@@ -18,6 +18,7 @@ from typing import Any, Sequence
 import torch
 
 from .card_launch import CardLaunch
+from .fp8 import F8Weight
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libbtb_hip.so")
@@ -44,6 +45,10 @@ SIGNATURES: dict[str, tuple[Any, list[Any]]] = {
                                            _i32, _vp, _vp, _sz, _sz, _sz, _vp]),
     "btb_hip_gemv_p12_norm": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp, _vp, _vp, _vp, _vp, ctypes.c_float, _i32, _vp,
                                      _vp, _sz, _sz, _sz, _i32, _vp]),
+    "btb_hip_gemv_fp8_norm": (_i32, [_vp, _vp, _sz, _sz, _vp, _vp, _vp, ctypes.c_float, _i32, _vp, _vp, _sz, _sz, _sz,
+                                     _i32, _vp]),
+    "btb_hip_gemv_fp8_embed_norm": (_i32, [_vp, _vp, _sz, _sz, _vp, _vp, _sz, _vp, ctypes.c_float, _i32, _vp, _vp, _sz, _sz,
+                                           _sz, _vp]),
     "btb_hip_gemv_p12": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp, _vp, _vp, _vp, _sz, _sz, _sz, _vp]),
     "btb_hip_p12_pack_words": (_sz, [_sz]),
     "btb_hip_p12_pack": (_i32, [_vp, _sz, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
@@ -306,7 +311,7 @@ class HipCard(CardLaunch):
     def gemv_norm(self, w: Any, h_in: torch.Tensor, y: torch.Tensor | None, norm_w: torch.Tensor, eps: float,
                   h_out: torch.Tensor | None, out: torch.Tensor, glu: bool = False, centered: bool = False) -> torch.Tensor:
         """out = W . rmsnorm(h_in + y) with the add and the norm folded into the matvec's x load; the new residual
-        goes to `h_out` (a different tensor than `h_in`). `w` is a bf16 matrix or a `P12Weight`; `glu` folds the
+        goes to `h_out` (a different tensor than `h_in`). `w` is a bf16 matrix, a `P12Weight` or an `F8Weight`; `glu` folds the
         SwiGLU activation into the epilogue (out is then [M, R / 2])."""
         for t, what in ((h_in, "h_in"), (norm_w, "norm_w"), (out, "out")):
             self._need(t, torch.bfloat16, what)
@@ -324,6 +329,10 @@ class HipCard(CardLaunch):
         if isinstance(w, torch.Tensor):
             self._need(w, torch.bfloat16, "w")
             self._call("btb_hip_gemv_bf16_norm", _p(w), _p(h_in), p(y), _p(norm_w), float(eps),
+                       int(centered), p(h_out), _p(out), R, C, M, int(glu), _stream())
+        elif isinstance(w, F8Weight):
+            sr, sc = w.grid
+            self._call("btb_hip_gemv_fp8_norm", _p(w.w), _p(w.scales), sr, sc, _p(h_in), p(y), _p(norm_w), float(eps),
                        int(centered), p(h_out), _p(out), R, C, M, int(glu), _stream())
         else:
             ne = int(w.esc_idx.numel())
@@ -350,6 +359,10 @@ class HipCard(CardLaunch):
         if isinstance(w, torch.Tensor):
             self._need(w, torch.bfloat16, "w")
             self._call("btb_hip_gemv_bf16_embed_norm", _p(w), _p(table), _p(ids), vocab,
+                       _p(norm_w), float(eps), int(centered), p(h_out), _p(out), R, C, M, _stream())
+        elif isinstance(w, F8Weight):
+            sr, sc = w.grid
+            self._call("btb_hip_gemv_fp8_embed_norm", _p(w.w), _p(w.scales), sr, sc, _p(table), _p(ids), vocab,
                        _p(norm_w), float(eps), int(centered), p(h_out), _p(out), R, C, M, _stream())
         else:
             ne = int(w.esc_idx.numel())

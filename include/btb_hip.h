@@ -178,6 +178,16 @@ int32_t btb_hip_p12_widen(const void* lo, const void* hi4, const void* table, co
 int32_t btb_hip_gemv_fp8(const void* w, const void* scales, size_t sr, size_t sc, const void* x, void* y, size_t R,
                          size_t C, size_t M, void* stream);
 
+/* btb_hip_gemv_bf16_norm and btb_hip_gemv_bf16_embed_norm over a block-scaled FP8 matrix (the arrays and limits of
+ * btb_hip_gemv_fp8): the bits of btb_hip_add_rmsnorm (btb_hip_embed ahead of it), btb_hip_gemv_fp8 at one row a pass and,
+ * with glu, btb_hip_silu_mul. */
+int32_t btb_hip_gemv_fp8_norm(const void* w, const void* scales, size_t sr, size_t sc, const void* h_in, const void* y,
+                              const void* norm_w, float eps, int32_t centered, void* h_out, void* out, size_t R, size_t C,
+                              size_t M, int32_t glu, void* stream);
+int32_t btb_hip_gemv_fp8_embed_norm(const void* w, const void* scales, size_t sr, size_t sc, const void* table,
+                                    const int32_t* ids, size_t vocab, const void* norm_w, float eps, int32_t centered,
+                                    void* h_out, void* out, size_t R, size_t C, size_t M, void* stream);
+
 /* out u16[n] = the stored bf16 nearest to x f32[n], ties to even, a NaN the quiet NaN with its sign and upper payload -
  * the crate's round_bf16 (native/src/gemv.rs:3003-3007) over an array, with the NaN rule of a torch cast; the rounding
  * every bf16 output of this library goes through. */

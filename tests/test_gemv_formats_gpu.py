@@ -18,7 +18,7 @@ from btb_amd import fp8, mxfp4, pack12
 from btb_amd.pack12 import P12Weight
 from oracle import codecs
 
-from .helpers import acts_bf16, bits16, weights_bf16
+from .helpers import acts_bf16, bits16, gen, weights_bf16
 
 pytestmark = pytest.mark.gpu
 
@@ -587,3 +587,40 @@ def test_plain_packed_matvec_with_and_without_the_pair_table(card, R, C, M):
         pw.table[15] = 0xFF
         yr = card.gemv_p12(pw, x)
         assert torch.equal(yr.view(torch.int16), y.view(torch.int16))
+
+
+# rows of 5 units a lane and fewer (one trip), of two spans and a remainder; lanes 16, 32 and 64 a row; odd row counts;
+# blocks of several shapes; one and two rows (the step's widths) and a pass of four and two
+@pytest.mark.parametrize("R,C,block,M", [(384, 512, (128, 128), 1), (130, 896, (2, 128), 1), (768, 2560, (128, 128), 2),
+                                         (256, 4096, (128, 128), 1), (256, 12288, (64, 256), 2), (6, 1664, (2, 16), 6)])
+@pytest.mark.parametrize("glu", [False, True])
+@pytest.mark.parametrize("with_y", [False, True])
+def test_fp8_add_norm_and_activation_in_the_matvec(card, R, C, block, M, glu, with_y):
+    """`gemv_norm` and `gemv_embed_norm` over FP8 against the launches they replace, the same bits"""
+    g = gen(60 + R + C + M)
+    q, s = fp8.quantize(torch.randn(R, C, generator=g) * 0.02, block)
+    w = fp8.F8Weight(q.view(torch.uint8).cuda(), s.cuda(), R, C)
+    h, y = (torch.randn(M, C, generator=g).to(torch.bfloat16).cuda() for _ in range(2))
+    nw = (1.0 + 0.1 * torch.randn(C, generator=g)).to(torch.bfloat16).cuda()
+    y = y if with_y else None
+    h1, x1 = h.clone(), torch.empty_like(h)
+    card.add_rmsnorm(h1, y, nw, 1e-6, x1)
+    card.set_tuning("gemv_no_mfma", 1)  # the plain matvec on the streaming kernel, whose sums the folded one makes
+    try:
+        want = card.gemv_fp8(w, x1)
+    finally:
+        card.set_tuning("gemv_no_mfma", -1)
+    if glu:
+        m = torch.empty(M, R // 2, dtype=torch.bfloat16, device="cuda")
+        card.silu_mul(want, m)
+        want = m
+    h2, out = torch.empty_like(h), torch.empty_like(want)
+    card.gemv_norm(w, h, y, nw, 1e-6, h2, out, glu=glu)
+    assert torch.equal(out.view(torch.int16), want.view(torch.int16))
+    assert torch.equal(h2.view(torch.int16), h1.view(torch.int16))
+    if not with_y and not glu:
+        ids = torch.arange(M, dtype=torch.int32, device="cuda")
+        h3, out3 = torch.empty_like(h), torch.empty_like(want)
+        card.gemv_embed_norm(w, h, ids, nw, 1e-6, h3, out3)
+        assert torch.equal(out3.view(torch.int16), want.view(torch.int16))
+        assert torch.equal(h3.view(torch.int16), h1.view(torch.int16))
