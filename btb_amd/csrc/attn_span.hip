@@ -19,81 +19,151 @@
 
 #include "btb_attn.hpp"
 #include "btb_common.hpp"
+#include "btb_head_tile.hpp"
 #include "btb_tuning.hpp"
 
 #include "../../include/btb_hip.h"
 
 namespace btb {
 
-constexpr int AS_D = 128;
 constexpr int AS_KEYS = 128;  // keys a batch
 constexpr int AS_VROW = 272;  // bytes a V row takes in LDS: 256 + 16, so the eight rows a fragment read touches differ in bank
 constexpr int AS_PROW = 80;   // bytes a pair's 32 weights of a step take: 64 + 16, sixteen pairs in sixteen bank groups
 
-__host__ __device__ constexpr size_t as_lds_bytes(int NQT) {
-    const size_t NQ = 16 * (size_t)NQT;
-    return (size_t)AS_KEYS * AS_VROW + 4 * NQ * sizeof(float) + 4 * NQ * AS_PROW;
-}
+constexpr int AS_HROW = 272;  // bytes a prepared q, k or v row takes in LDS: as a V row
 
-__device__ __forceinline__ float as_xor16(float v) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(((int)(threadIdx.x & 63) ^ 16) << 2, __builtin_bit_cast(int, v)));
+// own: the pass's own rows kept in LDS (their k, then their v), none where q is given
+__host__ __device__ constexpr size_t as_lds_bytes(int NQT, int own) {
+    const size_t NQ = 16 * (size_t)NQT;
+    return (size_t)AS_KEYS * AS_VROW + 4 * NQ * sizeof(float) + 4 * NQ * AS_PROW + 2 * (size_t)own * AS_HROW;
 }
 
 // NQT tiles of 16 (row, head) pairs a workgroup: pair r is row t_base + r / G, head r % G, G = 1 << gs. TBL: the cache
 // has a row map. Every load stays on a slot one of the workgroup's rows may see, so the cache's capacity need not be
 // known and what lies past the rows is never read.
-template <int NQT, bool TBL>
+// QKV: the rows come as the fused qkv rows, before the q / k norm and rope. A workgroup prepares the q heads of its own
+// rows, a tile of 16 a wave and turn, while the first batch's K travels (its addresses then wait for nothing: they stay
+// within the cache's capacity); where its span holds some of the pass's own slots *n0 .. *n0 + T - 1 it prepares the
+// pass's k heads too, takes those keys and values from LDS, and the last of the z axis - whose rows see all of them -
+// writes them into the cache. T <= 32. The arithmetic is norm_rope_kv_kernel's, then this kernel's.
+template <int NQT, bool TBL, bool QKV>
 __global__ void __launch_bounds__(256, 2) attn_span_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ K, const uint16_t* __restrict__ V,
     const int32_t* __restrict__ n0p, const int32_t* __restrict__ par, int T, int Hq, int Hk, int gs, long long hs,
     long long rs, float scale_log2, float* __restrict__ part_m, float* __restrict__ part_l, float* __restrict__ part_acc,
-    int span, int win, const int32_t* __restrict__ tbl) {
-    constexpr int D = AS_D, NQ = 16 * NQT;
+    int span, int win, const int32_t* __restrict__ tbl, int cap, AmQkv x) {
+    constexpr int D = AD, NQ = 16 * NQT;
+    static_assert(!(QKV && TBL), "the fused rows go with a cache without a row map");
     extern __shared__ __align__(16) uint8_t lds[];
     uint8_t* v_lds = lds;                                             // [128 keys][AS_VROW]
     float* red = reinterpret_cast<float*>(lds + AS_KEYS * AS_VROW);   // [4 waves][NQ]: maxima, at the end the sums
     uint8_t* p_lds = reinterpret_cast<uint8_t*>(red + 4 * NQ);        // [4 steps of 32 keys][NQ pairs][AS_PROW]
+    uint8_t* q_lds = p_lds;                                           // QKV, before the first weights: [NQ][AS_HROW]
+    uint8_t* kn_lds = p_lds + 4 * NQ * AS_PROW;                       // QKV: the pass's own k rows, then their v rows
+    uint8_t* vn_lds = kn_lds + T * AS_HROW;
+    static_assert(NQ * AS_HROW <= 4 * NQ * AS_PROW, "the prepared q rows lie where the weights will");
     const int g = blockIdx.x, sp = blockIdx.y, S = gridDim.y, G = 1 << gs;
     const int TPW = NQ >> gs, t_base = blockIdx.z * TPW;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c = lane & 15, a = lane >> 4;
     const float ninf = bits_f32(0xff800000u);
     const int parent = tree_parent(par, T);
-    const int n0 = *n0p;
     const int k_begin = sp * span;
-    // the keys any of the workgroup's rows may see end at n_max (a chain's last row, or the whole pass for a tree)
-    const int n_max = par != nullptr ? n0 + T : n0 + min(T, t_base + TPW);
-    const int k_lim = min(n_max, k_begin + span);
-    const int last = max(k_lim - 1, 0);
-
-    uint4 qreg[NQT][4];
-#pragma unroll
-    for (int qt = 0; qt < NQT; ++qt) {
-        const int r = qt * 16 + c, t = min(t_base + (r >> gs), T - 1), j = r & (G - 1);
-        const uint16_t* qr = q + ((size_t)t * Hq + (size_t)g * G + j) * D + a * 8;
-#pragma unroll
-        for (int ds = 0; ds < 4; ++ds) qreg[qt][ds] = *reinterpret_cast<const uint4*>(qr + ds * 32);
-    }
     const uint16_t* Kg = K + (size_t)g * hs + a * 8;
     const uint16_t* Vg = V + (size_t)g * hs + (tid & 15) * 8;
-    auto slot_of = [&](int key) {
-        const int s = min(key, last);  // past the end: the last key again, not used
-        return TBL ? tbl[s] : s;
-    };
     uint4 kreg[2][4], vreg[8];
-    auto request_k = [&](int kb) {
+    // keys past `last` are the last again, not used
+    auto request_k = [&](int kb, int last) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            const uint16_t* kr = Kg + (size_t)slot_of(kb + 32 * wv + 16 * h + c) * rs;
+            const int s = min(kb + 32 * wv + 16 * h + c, last);
+            const uint16_t* kr = Kg + (size_t)(TBL ? tbl[s] : s) * rs;
 #pragma unroll
             for (int ds = 0; ds < 4; ++ds) kreg[h][ds] = *reinterpret_cast<const uint4*>(kr + ds * 32);
         }
     };
-    auto request_v = [&](int kb) {
+    auto request_v = [&](int kb, int last) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i)
-            vreg[i] = *reinterpret_cast<const uint4*>(Vg + (size_t)slot_of(kb + (tid >> 4) + 16 * i) * rs);
+        for (int i = 0; i < 8; ++i) {
+            const int s = min(kb + (tid >> 4) + 16 * i, last);
+            vreg[i] = *reinterpret_cast<const uint4*>(Vg + (size_t)(TBL ? tbl[s] : s) * rs);
+        }
     };
+    const int in_cap = min(k_begin + span, cap) - 1;
+    if constexpr (QKV) request_k(k_begin, in_cap);
+    const int n0 = *n0p;
+    // the keys any of the workgroup's rows may see end at n_max (a chain's last row, or the whole pass for a tree)
+    const int n_max = par != nullptr ? n0 + T : n0 + min(T, t_base + TPW);
+    const int k_lim = min(n_max, k_begin + span);
+    const int last = max(QKV ? min(k_lim - 1, cap - 1) : k_lim - 1, 0);
+    const bool own_here = QKV && k_begin < n0 + T && n0 < k_begin + span;  // some of the pass's own slots lie in this span
+    const bool any = k_begin < k_lim;
+
+    uint4 qreg[NQT][4];
+    if constexpr (QKV) {
+        if (any) {
+            const size_t width = (size_t)(Hq + 2 * Hk) * D;
+            const int ntask = NQT + (own_here ? (T + 15) / 16 : 0);
+            for (int id = wv; id < ntask; id += 4) {  // uniform in the wave
+                const bool is_k = id >= NQT;
+                const int tr = is_k ? (id - NQT) * 16 + c : t_base + ((id * 16 + c) >> gs), t = min(tr, T - 1);
+                const uint16_t* row = x.qkv + (size_t)t * width;
+                const uint16_t* src = row + (size_t)(is_k ? Hq + g : g * G + ((id * 16 + c) & (G - 1))) * D;
+                const uint16_t* wn = is_k ? x.wk : x.wq;
+                HeadTile h;
+                tile_request(h, src, wn, a);
+                cs_sn_request(h, x.cos_t, x.sin_t, n0 + (x.depth != nullptr ? x.depth[t] : t), a);
+                const uint16_t* vsrc = is_k ? row + (size_t)(Hq + Hk + g) * D : src;
+#pragma unroll
+                for (int ds = 0; ds < 4; ++ds) h.vrow[ds] = *reinterpret_cast<const uint4*>(vsrc + ds * 32 + a * 8);
+                float v[4][8];
+                tile_norm(h, wn != nullptr, x.eps, x.centered, v);
+                uint4 out[4];
+                tile_rope(v, h, out);
+                if (!is_k) {
+#pragma unroll
+                    for (int ds = 0; ds < 4; ++ds)
+                        *reinterpret_cast<uint4*>(q_lds + (id * 16 + c) * AS_HROW + ds * 64 + a * 16) = out[ds];
+                } else if (tr < T) {
+                    const int slot = n0 + tr;
+#pragma unroll
+                    for (int ds = 0; ds < 4; ++ds) {
+                        *reinterpret_cast<uint4*>(kn_lds + tr * AS_HROW + ds * 64 + a * 16) = out[ds];
+                        *reinterpret_cast<uint4*>(vn_lds + tr * AS_HROW + ds * 64 + a * 16) = h.vrow[ds];
+                    }
+                    // (a slot at or past the cache's capacity is not written: the caller has let the cache overflow)
+                    if (blockIdx.z == gridDim.z - 1 && slot >= k_begin && slot < min(k_begin + span, cap)) {
+                        uint16_t* kc = x.Kw + (size_t)g * hs + (size_t)slot * rs + a * 8;
+                        uint16_t* vc = x.Vw + (size_t)g * hs + (size_t)slot * rs + a * 8;
+#pragma unroll
+                        for (int ds = 0; ds < 4; ++ds) {
+                            *reinterpret_cast<uint4*>(kc + ds * 32) = out[ds];
+                            *reinterpret_cast<uint4*>(vc + ds * 32) = h.vrow[ds];
+                        }
+                    }
+                }
+            }
+            request_v(k_begin, last);
+            __syncthreads();
+#pragma unroll
+            for (int qt = 0; qt < NQT; ++qt)
+#pragma unroll
+                for (int ds = 0; ds < 4; ++ds)
+                    qreg[qt][ds] = *reinterpret_cast<const uint4*>(q_lds + (qt * 16 + c) * AS_HROW + ds * 64 + a * 16);
+        }
+    } else {
+#pragma unroll
+        for (int qt = 0; qt < NQT; ++qt) {
+            const int r = qt * 16 + c, t = min(t_base + (r >> gs), T - 1), j = r & (G - 1);
+            const uint16_t* qr = q + ((size_t)t * Hq + (size_t)g * G + j) * D + a * 8;
+#pragma unroll
+            for (int ds = 0; ds < 4; ++ds) qreg[qt][ds] = *reinterpret_cast<const uint4*>(qr + ds * 32);
+        }
+        if (any) {
+            request_k(k_begin, last);
+            request_v(k_begin, last);
+        }
+    }
 
     f32x4 ot[2][NQT];      // O^T tile [dt][qt], lane: pair c of tile qt, dims 32 wv + 16 dt + 4 a .. + 3
     float m[NQT], l[NQT];  // pair c's running maximum (the same in its lanes of every wave), the lane's share of its sum
@@ -103,12 +173,23 @@ __global__ void __launch_bounds__(256, 2) attn_span_kernel(
         l[qt] = 0.f;
         ot[0][qt] = ot[1][qt] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
-    if (k_begin < k_lim) {
-        request_k(k_begin);
-        request_v(k_begin);
-    }
     const uint32_t rows = tree_rows(parent, T);  // while the first batch travels
     for (int kb = k_begin; kb < k_lim; kb += AS_KEYS) {
+        const bool own = own_here && kb < n0 + T && n0 < kb + AS_KEYS;
+        if constexpr (QKV) {
+            if (own) {
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const int tr = kb + 32 * wv + 16 * h + c - n0;  // which of the pass's rows this key is, if any
+                    const uint8_t* kn = kn_lds + min(max(tr, 0), T - 1) * AS_HROW + a * 16;
+#pragma unroll
+                    for (int ds = 0; ds < 4; ++ds) {
+                        const uint4 v = *reinterpret_cast<const uint4*>(kn + ds * 64);
+                        if (tr >= 0 && tr < T) kreg[h][ds] = v;
+                    }
+                }
+            }
+        }
         // scores: S^T tile [h][qt], lane: pair c of tile qt against keys kb + 32 wv + 16 h + 4 a .. + 3
         f32x4 st[2][NQT];
 #pragma unroll
@@ -123,7 +204,7 @@ __global__ void __launch_bounds__(256, 2) attn_span_kernel(
                 st[h][qt] = acc;
             }
         const bool more = kb + AS_KEYS < k_lim;
-        if (more) request_k(kb + AS_KEYS);
+        if (more) request_k(kb + AS_KEYS, last);
         // scaled, masked where a row may not see a key (a batch wholly in the cache, without a window, needs no mask)
         if (kb + AS_KEYS <= n0 && win == 0) {
 #pragma unroll
@@ -158,7 +239,7 @@ __global__ void __launch_bounds__(256, 2) attn_span_kernel(
             for (int h = 0; h < 2; ++h)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) b = fmaxf(b, st[h][qt][i]);
-            b = fmaxf(b, as_xor16(b));
+            b = fmaxf(b, xor_lanes16(b));
             b = fmaxf(b, xor32(b));
             if (a == 0) red[wv * NQ + qt * 16 + c] = b;
         }
@@ -170,7 +251,18 @@ __global__ void __launch_bounds__(256, 2) attn_span_kernel(
             *reinterpret_cast<uint4*>(v_lds + kl * AS_VROW + (tid & 15) * 16) =
                 kb + kl < k_lim ? vreg[i] : make_uint4(0u, 0u, 0u, 0u);
         }
-        if (more) request_v(kb + AS_KEYS);
+        if constexpr (QKV) {
+            if (own) {  // the rows of the pass among them, by the threads that have just written their places
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const int key = kb + (tid >> 4) + 16 * i, tr = key - n0;
+                    if (tr >= 0 && tr < T && key < k_lim)
+                        *reinterpret_cast<uint4*>(v_lds + (key - kb) * AS_VROW + (tid & 15) * 16) =
+                            *reinterpret_cast<const uint4*>(vn_lds + tr * AS_HROW + (tid & 15) * 16);
+                }
+            }
+        }
+        if (more) request_v(kb + AS_KEYS, last);
         // the pairs' maxima move; weights, rounded to bf16, P^T into LDS
 #pragma unroll
         for (int qt = 0; qt < NQT; ++qt) {
@@ -232,7 +324,7 @@ __global__ void __launch_bounds__(256, 2) attn_span_kernel(
 #pragma unroll
     for (int qt = 0; qt < NQT; ++qt) {
         float s = l[qt];
-        s += as_xor16(s);
+        s += xor_lanes16(s);
         s += xor32(s);
         if (a == 0) red[wv * NQ + qt * 16 + c] = s;
     }
@@ -255,42 +347,64 @@ __global__ void __launch_bounds__(256, 2) attn_span_kernel(
     }
 }
 
-template <int NQT>
-static void launch_span(const void* q, const void* K, const void* V, const int32_t* n0, const int32_t* par, int T, int Hq,
-                        int Hk, int gs, long long hs, long long rs, float scale_log2, float* part_m, float* part_l,
-                        float* part_acc, int S, int span, int win, const int32_t* tbl, hipStream_t st) {
-    const int TPW = (16 * NQT) >> gs;
+template <int NQT, bool TBL, bool QKV>
+static int32_t launch_span(const void* q, const void* K, const void* V, const int32_t* n0, const int32_t* par, size_t T,
+                           size_t Hq, size_t Hk, int gs, long long hs, long long rs, float scale_log2, float* part_m,
+                           float* part_l, float* part_acc, size_t S, int span, int win, const int32_t* tbl, int cap,
+                           const AmQkv& x, hipStream_t st) {
+    const size_t TPW = (16 * NQT) >> gs;
     const dim3 grid((unsigned)Hk, (unsigned)S, (unsigned)((T + TPW - 1) / TPW));
-    static_assert(as_lds_bytes(NQT) <= 64 * 1024, "within what a workgroup gets without asking for more");
-#define SPAN(TBL)                                                                                                   \
-    hipLaunchKernelGGL((attn_span_kernel<NQT, TBL>), grid, dim3(256), as_lds_bytes(NQT), st,                        \
-                       static_cast<const uint16_t*>(q), static_cast<const uint16_t*>(K),                            \
-                       static_cast<const uint16_t*>(V), n0, par, T, Hq, Hk, gs, hs, rs, scale_log2, part_m, part_l, \
-                       part_acc, span, win, tbl)
-    if (tbl != nullptr) SPAN(true);
-    else SPAN(false);
-#undef SPAN
+    auto kern = attn_span_kernel<NQT, TBL, QKV>;
+    const size_t lds = as_lds_bytes(NQT, QKV ? (int)T : 0);
+    if (lds > 64 * 1024) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return hip_status(e, "hipFuncSetAttribute");
+    }
+    hipLaunchKernelGGL(kern, grid, dim3(256), lds, st, static_cast<const uint16_t*>(q), static_cast<const uint16_t*>(K),
+                       static_cast<const uint16_t*>(V), n0, par, (int)T, (int)Hq, (int)Hk, gs, hs, rs, scale_log2, part_m,
+                       part_l, part_acc, span, win, tbl, cap, x);
+    return hip_status(hipGetLastError(), "attn_span launch");
 }
 
+static int group_shift(size_t G) { return G == 1 ? 0 : G == 2 ? 1 : G == 4 ? 2 : G == 8 ? 3 : -1; }
+
 // whether a pass takes this kernel: several rows, 1, 2, 4 or 8 query heads a kv head
-bool attn_span_fits(size_t T, size_t G) {
-    return T >= 2 && (G == 1 || G == 2 || G == 4 || G == 8) && tuning("attn_mfma") != 0;
-}
+bool attn_span_fits(size_t T, size_t G) { return T >= 2 && group_shift(G) >= 0 && tuning("attn_mfma") != 0; }
 
 // the partial states of every (row, head, span), for the merge
 int32_t attn_decode_span(const void* q, const void* K, const void* V, const int32_t* n0, const int32_t* par, size_t T,
                          size_t Hq, size_t Hk, long long hs, long long rs, float scale_log2, float* part_m, float* part_l,
                          float* part_acc, size_t S, int span, int win, const int32_t* tbl, hipStream_t st) {
-    const size_t G = Hq / Hk, pairs = T * G;  // pairs of one kv head
-    const int gs = G == 1 ? 0 : G == 2 ? 1 : G == 4 ? 2 : 3;
-#define AS(NN) \
-    launch_span<NN>(q, K, V, n0, par, (int)T, (int)Hq, (int)Hk, gs, hs, rs, scale_log2, part_m, part_l, part_acc, (int)S, \
-                    span, win, tbl, st)
-    if (pairs <= 16) AS(1);
-    else if (pairs <= 32) AS(2);
-    else AS(4);
+    const size_t pairs = T * (Hq / Hk);  // of one kv head
+    const int gs = group_shift(Hq / Hk);
+#define AS(NN, TBL)                                                                                                      \
+    return launch_span<NN, TBL, false>(q, K, V, n0, par, T, Hq, Hk, gs, hs, rs, scale_log2, part_m, part_l, part_acc, S, \
+                                       span, win, tbl, 0, AmQkv{}, st)
+    if (tbl != nullptr) {
+        if (pairs <= 16) AS(1, true);
+        if (pairs <= 32) AS(2, true);
+        AS(4, true);
+    }
+    if (pairs <= 16) AS(1, false);
+    if (pairs <= 32) AS(2, false);
+    AS(4, false);
 #undef AS
-    return hip_status(hipGetLastError(), "attn_decode_span launch");
+}
+
+// the same states from the fused qkv rows; the new K / V rows land in the cache on the way. T <= 32
+int32_t attn_decode_span_qkv(const AmQkv& x, const int32_t* n0, const int32_t* par, size_t T, size_t Hq, size_t Hk,
+                             long long hs, long long rs, float scale_log2, float* part_m, float* part_l, float* part_acc,
+                             size_t S, int span, size_t cap, hipStream_t st) {
+    const size_t pairs = T * (Hq / Hk);
+    const int gs = group_shift(Hq / Hk), capi = (int)(cap < 0x7FFFFFFFu ? cap : 0x7FFFFFFFu);
+#define AS(NN)                                                                                                          \
+    return launch_span<NN, false, true>(nullptr, x.Kw, x.Vw, n0, par, T, Hq, Hk, gs, hs, rs, scale_log2, part_m, part_l, \
+                                        part_acc, S, span, 0, nullptr, capi, x, st)
+    if (pairs <= 16) AS(1);
+    if (pairs <= 32) AS(2);
+    AS(4);
+#undef AS
 }
 
 }  // namespace btb

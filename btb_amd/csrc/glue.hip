@@ -16,6 +16,7 @@
 
 #include "btb_attn.hpp"
 #include "btb_common.hpp"
+#include "btb_head_tile.hpp"
 #include "btb_stream.hpp"
 #include "btb_tuning.hpp"
 
@@ -237,6 +238,9 @@ bool attn_span_fits(size_t T, size_t G);
 int32_t attn_decode_span(const void* q, const void* K, const void* V, const int32_t* n0, const int32_t* par, size_t T,
                          size_t Hq, size_t Hk, long long hs, long long rs, float scale_log2, float* part_m, float* part_l,
                          float* part_acc, size_t S, int span, int win, const int32_t* tbl, hipStream_t st);
+int32_t attn_decode_span_qkv(const AmQkv& x, const int32_t* n0, const int32_t* par, size_t T, size_t Hq, size_t Hk,
+                             long long hs, long long rs, float scale_log2, float* part_m, float* part_l, float* part_acc,
+                             size_t S, int span, size_t cap, hipStream_t st);
 bool attn_mfma_qkv_fits(size_t T, size_t G, int span);
 int32_t attn_decode_mfma_qkv(const void* qkv, const void* wq, const void* wk, float eps, int centered, const void* cos_t,
                              const void* sin_t, const int32_t* n0, const int32_t* depth, const int32_t* par, void* K,
@@ -824,7 +828,7 @@ static int32_t attn_decode_any(const void* q, const void* K, const void* V, void
         else launch_merge<2>(st, att, T, Hq, Hk, S, part_m, part_l, part_acc, nullptr);
         return hip_status(hipGetLastError(), "attn_decode launch");
     }
-    if (parts == nullptr && attn_span_fits(T, G)) {
+    if (parts == nullptr && attn_span_fits(T, G) && al(part_acc, 16)) {
         const int32_t rc = attn_decode_span(q, K, V, n0, par, T, Hq, Hk, (long long)hs, (long long)rs, scale_log2, part_m,
                                             part_l, part_acc, S, span, (int)win, tbl, st);
         if (rc != OK) return rc;
@@ -1018,6 +1022,57 @@ int32_t btb_hip_attn_decode_qkv_rows(const void* qkv, const void* wq, const void
     if (G == 4) launch_merge<4>(st, att, T, Hq, Hk, S, part_m, part_l, part_acc, nullptr);
     else launch_merge<2>(st, att, T, Hq, Hk, S, part_m, part_l, part_acc, nullptr);
     return hip_status(hipGetLastError(), "attn_decode_qkv_rows launch");
+}
+
+int32_t btb_hip_attn_decode_qkv_span(const void* qkv, const void* wq, const void* wk, float eps, int32_t centered,
+                                     const void* cos_t, const void* sin_t, const int32_t* n0, const int32_t* depth,
+                                     const int32_t* par, void* K, void* V, void* att, size_t T, size_t Hq, size_t Hk,
+                                     size_t D, int64_t hs, int64_t rs, float scale, size_t cap, size_t S,
+                                     float* workspace, void* stream) {
+    if (qkv == nullptr || cos_t == nullptr || sin_t == nullptr || n0 == nullptr || K == nullptr || V == nullptr ||
+        att == nullptr || workspace == nullptr)
+        return ERR_NULL;
+    if (T == 0 || T > 32 || Hq == 0 || Hk == 0 || S == 0 || cap == 0 || cap > 0x7FFFFFFFull - 256 || S > 1024 ||
+        Hq % Hk != 0 || hs <= 0 || rs <= 0 || !(scale == scale) || !(eps >= 0.f))
+        return ERR_DOMAIN;
+    const size_t G = Hq / Hk;
+    if (D != (size_t)ATT_D || (G != 1 && G != 2 && G != 4 && G != 8)) {
+        set_error("attn_decode_qkv_span: head_dim 128 and 1, 2, 4 or 8 query heads per kv head");
+        return ERR_DOMAIN;
+    }
+    if (!al(qkv, 16) || !al(wq, 16) || !al(wk, 16) || !al(cos_t, 16) || !al(sin_t, 16) || !al(K, 16) || !al(V, 16) ||
+        !al(par, 4) || !al(depth, 4) || !al(workspace, 16) || (rs % 8) != 0 || (hs % 8) != 0 || (T * Hq * S * 2) % 4 != 0)
+        return ERR_DOMAIN;
+    if (S * G > (size_t)ATT_MAX_STATES) {
+        set_error("attn_decode_qkv_span: spans * (query heads per kv head) is at most 1024");
+        return ERR_DOMAIN;
+    }
+    const int span = (int)(((cap + S - 1) / S + 127) / 128 * 128);
+    float* part_m = workspace;
+    float* part_l = workspace + T * Hq * S;
+    float* part_acc = workspace + 2 * T * Hq * S;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    AmQkv x;
+    x.qkv = static_cast<const uint16_t*>(qkv);
+    x.wq = static_cast<const uint16_t*>(wq);
+    x.wk = static_cast<const uint16_t*>(wk);
+    x.cos_t = static_cast<const uint16_t*>(cos_t);
+    x.sin_t = static_cast<const uint16_t*>(sin_t);
+    x.depth = depth;
+    x.Kw = static_cast<uint16_t*>(K);
+    x.Vw = static_cast<uint16_t*>(V);
+    x.eps = eps;
+    x.centered = centered ? 1 : 0;
+    const int32_t rc = attn_decode_span_qkv(x, n0, par, T, Hq, Hk, (long long)hs, (long long)rs,
+                                            scale * 1.4426950408889634f, part_m, part_l, part_acc, S, span, cap, st);
+    if (rc != OK) return rc;
+    switch (G) {
+        case 1: launch_merge<1>(st, att, T, Hq, Hk, S, part_m, part_l, part_acc, nullptr); break;
+        case 2: launch_merge<2>(st, att, T, Hq, Hk, S, part_m, part_l, part_acc, nullptr); break;
+        case 4: launch_merge<4>(st, att, T, Hq, Hk, S, part_m, part_l, part_acc, nullptr); break;
+        default: launch_merge<8>(st, att, T, Hq, Hk, S, part_m, part_l, part_acc, nullptr); break;
+    }
+    return hip_status(hipGetLastError(), "attn_decode_qkv_span launch");
 }
 
 int32_t btb_hip_silu_mul(const void* gu, void* m, size_t T, size_t I, void* stream) {

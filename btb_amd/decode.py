@@ -100,6 +100,23 @@ def pass_spans(cus: int, T: int, Hq: int, Hk: int, cap: int) -> int:
     return -(-cap // span)
 
 
+def step_on_spans(cus: int, Hq: int, Hk: int, cap: int) -> int:
+    """the span count with which a one-row step's attention over a cache of `cap` slots walks its spans on the matrix
+    cores, 0 where it stays with the kernel that holds a span's keys in registers. One workgroup a CU takes all query
+    heads of a kv head, 64 spans at most (more take the fold's slow form). Its launch has a longer start, so it pays from
+    8192 slots on - with one or two heads a kv head, whose vector arithmetic is less, from 16384, or where the other
+    kernel's spans would be more than 64. Measured on MI355X, us a step, register kernel / this: 20 layers [2048 / 6144],
+    32 / 8 heads, 6000 keys 871 / 865, 12000 990 / 958, 24000 1209 / 1100; 32 / 4: 4000 keys 792 / 800, 8000 892 / 846, 16000
+    1030 / 916; 8 / 2: 4000 685 / 738, 8000 852 / 763; 16 / 8: 8000 851 / 855, 16000 964 / 957; 36 layers [2560 / 9728], 32 / 8,
+    32000 keys 3022 / 2715."""
+    G = Hq // Hk
+    if G not in (1, 2, 4, 8) or cap < 8192 or (G <= 2 and cap < 16384 and Hk > cus // 64):
+        return 0
+    spans = max(1, min(64, cus // Hk))
+    spans = -(-cap // (-(-cap // (spans * 128)) * 128))
+    return spans if Hq * spans % 2 == 0 else 0  # the states' alignment
+
+
 class Linear:
     """one linear's weight on the GPU in its stored form, multiplied as stored: a bf16 tensor or a `P12Weight`"""
 
@@ -165,6 +182,10 @@ class DecodeStep:
         # key spans: enough workgroups (kv heads x spans) to cover the CUs once, a span at least 64 keys; a pass of T
         # rows launches T times the workgroups, so it takes longer spans - two workgroups a CU in all (measured on
         # the [2560 / 9728] stack at 4096 keys: 8 rows 4.32 ms a pass with 32 spans, 3.83 with 8; 16 rows 5.6 / 4.7)
+        default_spans = attn_spans is None
+        one_row_spans = step_on_spans(card.sms, Hq, Hk, self.cap) if self.T == 1 and D == 128 else 0
+        if one_row_spans and default_spans and fused is None:
+            attn_spans = one_row_spans
         if attn_spans is None:
             attn_spans = max(1, min(self.cap // 64, (card.sms + Hk - 1) // Hk, (2 * card.sms) // (Hk * self.T)))
             if self.T == 1 and D == 128 and Hq // Hk >= 4:
@@ -208,6 +229,16 @@ class DecodeStep:
         self.glu_fold = (chosen or bool(fused)) and T > 1
         self.rows_attn_fused = (chosen or bool(fused)) and T > 1 and bool(
             card.attn_rows_fused(T, cfg.q_heads, cfg.kv_heads, cfg.head_dim, self.cap, self.S))
+        # ... or, over spans of more than one batch of keys, in the attention that walks them: long caches at one row
+        # (`step_on_spans`), and passes whose rows the kernel above does not take (28 rows x 32 / 8 heads over 2395 keys:
+        # 1469 -> 1434 us a pass of 15 layers against norm_rope_kv + attn_decode; over spans of 128 keys it loses, the
+        # 32-row pass over 1536 keys 4120 -> 4194)
+        if self.T == 1:
+            self.span_fused = default_spans and chosen and one_row_spans > 0
+        else:
+            self.span_fused = (default_spans and chosen and not self.rows_attn_fused and D == 128 and self.T <= 32
+                               and Hq // Hk in (1, 2, 4, 8) and -(-self.cap // self.S) > 128
+                               and self.T * Hq * self.S % 2 == 0)
         # the handoff to the host: token, cache length and the GPU's clock in pinned memory
         self.host_tok = torch.zeros(1, dtype=torch.int32).pin_memory()
         self.host_n0 = torch.zeros(1, dtype=torch.int32).pin_memory()
@@ -284,7 +315,10 @@ class DecodeStep:
             K, V = self.kv[i, 0], self.kv[i, 1]
             k.add_rmsnorm(self.h, y_prev, w[L + "ln1"], cfg.eps, self.x)
             w[L + "qkv"].matvec(self.x, self.qkv)
-            if self.rows_attn_fused:
+            if self.span_fused:
+                k.attn_decode_qkv_span(self.qkv, w.get(L + "wq"), w.get(L + "wk"), cfg.eps, self.cos, self.sin, self.n0, K, V,
+                                       self.att, Hq, Hk, D, self.scale, self.S, self.scratch, depth=self.depth, par=self.par)
+            elif self.rows_attn_fused:
                 k.attn_decode_qkv_rows(self.qkv, w.get(L + "wq"), w.get(L + "wk"), cfg.eps, self.cos, self.sin,
                                        self.n0, K, V, self.att, Hq, Hk, D, self.scale, self.S, self.scratch,
                                        depth=self.depth, par=self.par)
@@ -329,7 +363,10 @@ class DecodeStep:
                 k.gemv_embed_norm(w[L + "qkv"].w, w["embed"], self.ids, w[L + "ln1"], cfg.eps, hb, self.qkv)
             else:
                 k.gemv_norm(w[L + "qkv"].w, ha, y_prev, w[L + "ln1"], cfg.eps, hb, self.qkv)
-            if self.T == 1 and D == 128:
+            if self.span_fused:
+                k.attn_decode_qkv_span(self.qkv, w.get(L + "wq"), w.get(L + "wk"), cfg.eps, self.cos, self.sin, self.n0, K, V,
+                                       self.att, Hq, Hk, D, self.scale, self.S, self.scratch, depth=self.depth, par=self.par)
+            elif self.T == 1 and D == 128:
                 k.attn_decode_qkv(self.qkv, w.get(L + "wq"), w.get(L + "wk"), cfg.eps, self.cos, self.sin, self.n0, K,
                                   V, self.att, Hq, Hk, D, self.scale, self.S, self.scratch)
             elif self.rows_attn_fused:

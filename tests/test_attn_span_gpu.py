@@ -73,3 +73,58 @@ def test_attention_over_long_spans(card, n0, T, Hq, Hk, S, tree, win, mapped):
         # weights and outputs are rounded to bf16 (2^-9 each), as in the other attention kernels' tests
         worst = np.abs(got[t].reshape(Hq, D) - want).max() / np.abs(want).max()
         assert worst <= 2.0**-7, (t, worst)
+
+
+# one row and several; one, two and four tiles of pairs, several workgroups a kv head; the rows' own slots within one
+# batch, across two and across two spans, the first and the last slot of the cache; with and without norm weights
+@pytest.mark.parametrize("n0,T,Hq,Hk,S,tree", [
+    (1000, 1, 16, 2, 2, False), (255, 1, 32, 8, 1, False), (256, 1, 8, 8, 2, False), (0, 1, 4, 2, 1, False),
+    (1000, 2, 16, 2, 3, True), (383, 5, 8, 2, 2, False), (250, 17, 32, 8, 1, False), (0, 32, 16, 2, 1, True),
+    (500, 32, 8, 8, 2, False), (250, 21, 4, 1, 2, True), (2047, 8, 32, 8, 5, True), (246, 10, 8, 1, 1, False)])
+@pytest.mark.parametrize("with_norm", [True, False])
+def test_long_spans_from_the_fused_qkv_rows(card, n0, T, Hq, Hk, S, tree, with_norm):
+    """`attn_decode_qkv_span` against `norm_rope_kv` and `attn_decode` at the same span count: the same cache, nothing else
+    in it touched, and from two rows on the same output bits (one row: both within bf16's bar of f64 attention)"""
+    from btb_amd.decode import StackConfig, rope_tables
+
+    D = 128
+    cap = n0 + T
+    cap = 256 if n0 + T == 256 else cap + 150
+    g = gen(1300 + n0 + T)
+    K = torch.randn(Hk, cap, D, generator=g).to(torch.bfloat16)
+    V = torch.randn(Hk, cap, D, generator=g).to(torch.bfloat16)
+    K[:, n0:] = float("nan")
+    V[:, n0:] = float("nan")
+    qkv = torch.randn(T, (Hq + 2 * Hk) * D, generator=g).to(torch.bfloat16).cuda()
+    wn = (1 + 0.1 * torch.randn(D, generator=g)).to(torch.bfloat16).cuda() if with_norm else None
+    cos, sin = rope_tables(StackConfig(q_heads=Hq, kv_heads=Hk), cap + 64, torch.device("cuda"))
+    par = [-1] + [int(torch.randint(-1, t, (1,), generator=g)) for t in range(1, T)] if tree else None
+    part, depth = None, None
+    if tree:
+        d = []
+        for p in par:
+            d.append(0 if p < 0 else d[p] + 1)
+        part = torch.tensor(par, dtype=torch.int32, device="cuda")
+        depth = torch.tensor(d, dtype=torch.int32, device="cuda")
+    scale = 1.0 / np.sqrt(D)
+    n0t = torch.tensor([n0], dtype=torch.int32, device="cuda")
+    scratch = card.attn_scratch(T, Hq, Hk, D, S)
+    K1, V1, K2, V2 = K.cuda(), V.cuda(), K.cuda(), V.cuda()
+    q = torch.empty(T, Hq * D, dtype=torch.bfloat16, device="cuda")
+    want, got = torch.zeros_like(q), torch.zeros_like(q)
+    card.norm_rope_kv(qkv, wn, wn, 1e-6, cos, sin, n0t, K1, V1, q, Hq, Hk, D, depth=depth)
+    card.attn_decode(q, K1, V1, want, n0t, Hq, Hk, D, scale, S, scratch, par=part)
+    card.attn_decode_qkv_span(qkv, wn, wn, 1e-6, cos, sin, n0t, K2, V2, got, Hq, Hk, D, scale, S, scratch, depth=depth,
+                              par=part)
+    for a, b in ((K1, K2), (V1, V2)):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+    span = -(-(-(-cap // S)) // 128) * 128
+    if T > 1 and not (span == 128 and Hq // Hk in (2, 4)):  # there attn_decode is the one-batch kernel
+        assert torch.equal(want.view(torch.int16), got.view(torch.int16))
+    assert bool(torch.isfinite(got.float()).all())
+    for t in range(T):
+        keep = seen_by(t, n0, par, 0)
+        ref = od.attention(q[t].float().cpu().numpy().reshape(Hq, D), K1[:, keep].float().cpu().numpy(),
+                           V1[:, keep].float().cpu().numpy(), scale)
+        worst = np.abs(got[t].float().cpu().numpy().reshape(Hq, D) - ref).max() / np.abs(ref).max()
+        assert worst <= 2.0**-7, (t, worst)
