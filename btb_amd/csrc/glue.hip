@@ -828,7 +828,9 @@ static int32_t attn_decode_any(const void* q, const void* K, const void* V, void
         else launch_merge<2>(st, att, T, Hq, Hk, S, part_m, part_l, part_acc, nullptr);
         return hip_status(hipGetLastError(), "attn_decode launch");
     }
-    if (parts == nullptr && attn_span_fits(T, G) && al(part_acc, 16)) {
+    // Longer spans, and 1 or 8 query heads a kv head: the matrix cores too, a span walked in batches (attn_span.hip). With
+    // the caller's state arrays spans of one and two batches stay on the general kernel.
+    if (rw == nullptr && (parts == nullptr || span > 256) && attn_span_fits(T, G) && al(part_acc, 16)) {
         const int32_t rc = attn_decode_span(q, K, V, n0, par, T, Hq, Hk, (long long)hs, (long long)rs, scale_log2, part_m,
                                             part_l, part_acc, S, span, (int)win, tbl, st);
         if (rc != OK) return rc;
