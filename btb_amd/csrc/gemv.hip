@@ -524,6 +524,10 @@ int32_t gemv_mfma_dl_p12(const uint8_t* lo, const uint8_t* hi4, const uint8_t* t
 // gemv_mfma_from, when set, replaces every form's own figure)
 static bool wide_pass(size_t M, size_t R, size_t C, bool packed, size_t from = 5) {
     if (tuning("gemv_mfma_from") > 0) from = (size_t)tuning("gemv_mfma_from");
+    // bf16 and more than 16 rows of x: the column-interleaved kernel over rows of more than 10240 columns ([4096 x 12288]
+    // at 32 rows 44.0 us against 53.1) and, where the last tile is not whole, of more than 4096 ([5001 x 9728] 66.8
+    // against 73.7, [12345 x 7168] at 20 rows 79.0 against 84.2)
+    if (!packed && M > 16 && (C > 10240 || (R % 16 != 0 && C > 4096))) return false;
     return M >= from && (packed ? mfma_lds_fits_packed((int)R, (int)C) : mfma_lds_fits_bf16((int)R, (int)C)) &&
            tuning("gemv_no_mfma") <= 0 && tuning("mfma_lds") != 0;
 }
@@ -534,9 +538,14 @@ static bool wide_pass(size_t M, size_t R, size_t C, bool packed, size_t from = 5
 // cores; FP8 33.3 / 45.1 us at 3 / 4 rows against 30.7; under 4 M weights the vector kernel wins to four rows)
 static size_t mx4_matrix_from(size_t R, size_t C) {
     const size_t n = R * C;
+    // x of more than 10240 columns is streamed beside the weights, which the vector kernel's few rows beat for longer
+    // ([4096 x 12288] at 2 / 3 / 4 rows 13.8 / 18.1 / 30.9 us on the vector kernel, 17.9 / 18.3 / 18.7 here; [1024 x 12288]
+    // 6.1 / 8.4 / 11.2 against 17.5)
+    if (C > 10240) return n >= (1u << 25) ? 4 : 5;
     return n >= (1u << 25) ? 2 : n >= (1u << 23) ? 3 : n >= (1u << 22) ? 4 : 5;
 }
-static size_t fp8_matrix_from(size_t R, size_t C) { return R * C >= (1u << 25) ? 3 : 5; }
+// (FP8 likewise: [4096 x 12288] at 3 / 4 rows 15.9 / 24.8 us on the vector kernel, 28.8 / 29.0 here)
+static size_t fp8_matrix_from(size_t R, size_t C) { return R * C >= (1u << 25) && C <= 10240 ? 3 : 5; }
 
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 static bool aligned2(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 1u) == 0; }

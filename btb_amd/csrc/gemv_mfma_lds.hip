@@ -248,7 +248,7 @@ struct MfP12 {
         }
     }
     // the thirty-two escapes in t: their terms into LDS, then added to the lane's rows in list order
-    __device__ static __forceinline__ void tail_chunk(const uint4& tbl, const Tail& t, int tile, int first, int lane,
+    __device__ static __forceinline__ void tail_chunk(const uint4& tbl, const Tail& t, int tile_row, int first, int lane,
                                                       uint8_t* scratch, f32x4& s) {
         float* dl = reinterpret_cast<float*>(scratch);            // [32 escapes][16 x rows]
         int* rw = reinterpret_cast<int*>(scratch + 32 * 16 * 4);  // [32] the escape's row within the tile
@@ -265,7 +265,7 @@ struct MfP12 {
         float4* o = reinterpret_cast<float4*>(dl + (lane & 31) * 16 + (lane >> 5) * 8);
         o[0] = make_float4(d[0], d[1], d[2], d[3]);
         o[1] = make_float4(d[4], d[5], d[6], d[7]);
-        rw[lane & 31] = t.row - tile * 16;  // both halves write the same value
+        rw[lane & 31] = t.row - tile_row;  // both halves write the same value
         const int cnt = max(min(32, t.e1 - first), 0);
 #pragma unroll 2
         for (int j = 0; j < cnt; ++j) {
@@ -278,18 +278,18 @@ struct MfP12 {
         }
     }
     // fetched: the first thirty-two are already in t (tail_begin, tail_loads with these x rows)
-    __device__ static __forceinline__ void tail_apply(const Mat& mat, const uint4& tbl, Tail& t, int tile,
+    __device__ static __forceinline__ void tail_apply(const Mat& mat, const uint4& tbl, Tail& t, int tile_row,
                                                       const uint16_t* xrows, int C, int have, int lane, uint8_t* scratch,
                                                       bool fetched, f32x4& s) {
         if (!fetched) {  // other x rows than the ones asked for ahead
             tail_request(mat, t, t.e0, lane);
             tail_loads(mat, t, xrows, C, have, lane);
         }
-        tail_chunk(tbl, t, tile, t.e0, lane, scratch, s);
+        tail_chunk(tbl, t, tile_row, t.e0, lane, scratch, s);
         for (int first = t.e0 + 32; first < t.e1; first += 32) {  // a crowd: fetched here
             tail_request(mat, t, first, lane);
             tail_loads(mat, t, xrows, C, have, lane);
-            tail_chunk(tbl, t, tile, first, lane, scratch, s);
+            tail_chunk(tbl, t, tile_row, first, lane, scratch, s);
         }
     }
 };
@@ -312,7 +312,10 @@ struct MfP12 {
 // TR: the rows of a tile that are rows of the matrix (a divisor of R, a multiple of a load's rows): the tile is rows
 // TR tile .. + TR - 1, its other rows are not read and what the matrix cores make of them is not written. A template
 // argument: a load that a run-time test decides on is a load the compiler cannot count, and it then waits for all.
-template <class MF, int KS, int MT, int SPW, int SB, bool XS = false, bool XN = false, int TR = 16>
+// RAG: R is no multiple of sixteen (and at least that): the last tile starts sixteen rows before the end and writes only
+// the rows no other tile has, so every load stays whole and no row is masked. A template argument: the minimum in every
+// tile's address made the 8-row pass of the [2560 / 9728] stack 2.65 -> 2.84 ms where no tile needs it.
+template <class MF, int KS, int MT, int SPW, int SB, bool XS = false, bool XN = false, int TR = 16, bool RAG = false>
 __global__ void __launch_bounds__(KS * 64) gemv_mfma_lds(typename MF::Mat mat, const uint4* __restrict__ x,
                                                          uint16_t* __restrict__ y, int R, int C, int M, int half,
                                                          XArgs xa) {
@@ -408,7 +411,8 @@ __global__ void __launch_bounds__(KS * 64) gemv_mfma_lds(typename MF::Mat mat, c
     uint4 raw[NLD] = {};
     uint4 raw2[TWO ? NLD2 : 1] = {};
     uint32_t scl[SB] = {};  // the scales of the sub-block in flight, one per step, for this lane's row and column group
-    auto request = [&](int tile, int sb) {  // the loads of sub-block sb of the tile (R is a multiple of 16)
+    auto row_of = [&](int tile) { return RAG ? min(tile * tr, R - tr) : tile * tr; };  // the first row a tile reads
+    auto request = [&](int tile, int sb) {  // the loads of sub-block sb of the tile
         if constexpr (XS) {  // out of L2, ahead of the weights they will meet: a step past the wave's last takes the last
             // the same addresses every tile: a zero the compiler cannot see through keeps it from loading them all
             // once, ahead of the loop, into the registers this form is there to save
@@ -422,12 +426,12 @@ __global__ void __launch_bounds__(KS * 64) gemv_mfma_lds(typename MF::Mat mat, c
             }
         }
         const uint32_t valid = (uint32_t)(min(SB, n - sb * SB) * MF::STEPB);
-        const typename MF::RowInfo rn = MF::row_info(mat, tile * 16 + li, nsteps);
+        const typename MF::RowInfo rn = MF::row_info(mat, row_of(tile) + li, nsteps);
         MF::template scales<SB>(mat, rn, lg, s0 + sb * SB, nsteps, scl);
 #pragma unroll
         for (int q = 0; q < NLD; ++q) {
             // half > 0: the tile's rows 0..7 are gate rows 8 tile .., its rows 8..15 the up rows of the same outputs
-            const int row0 = half ? tile * 8 + q * RPI + (q * RPI >= 8 ? half * 16 - 8 : 0) : tile * tr + q * RPI;
+            const int row0 = half ? tile * 8 + q * RPI + (q * RPI >= 8 ? half * 16 - 8 : 0) : row_of(tile) + q * RPI;
             const uint8_t* base = mat.w + (size_t)row0 * rowbytes + (size_t)(s0 + sb * SB) * MF::STEPB;
             if (q * RPI < tr) {
                 if (lane_byte < valid) raw[q] = load_stream16(reinterpret_cast<const uint4*>(base + goff));
@@ -438,13 +442,13 @@ __global__ void __launch_bounds__(KS * 64) gemv_mfma_lds(typename MF::Mat mat, c
 #pragma unroll
             for (int q = 0; q < NLD2; ++q) {
                 const uint8_t* base =
-                    mat.w2 + (size_t)(tile * 16 + q * RPI2) * rowbytes2 + (size_t)(s0 + sb * SB) * STEPB2;
+                    mat.w2 + (size_t)(row_of(tile) + q * RPI2) * rowbytes2 + (size_t)(s0 + sb * SB) * STEPB2;
                 if (lane_byte2 < valid2) raw2[q] = load_stream16(reinterpret_cast<const uint4*>(base + goff2));
             }
         }
     };
 
-    const int ntiles = R / tr;
+    const int ntiles = RAG ? (R + tr - 1) / tr : R / tr;
     const int nsb = (n + SB - 1) / SB;
     // The tiles a workgroup visits: blockIdx.x, + gridDim.x, ... With half > 0 (W is a gate matrix over an up matrix,
     // half tiles of 16 rows each, and y their fold bf16(bf16(silu(g)) * u), [M, R / 2]) a tile is eight gate rows over
@@ -462,7 +466,7 @@ __global__ void __launch_bounds__(KS * 64) gemv_mfma_lds(typename MF::Mat mat, c
     [[maybe_unused]] int2 span_next = make_int2(0, 0);
     constexpr int TROWS = 16 / KS;  // the rows of a tile whose escapes this wave takes
     if constexpr (MF::TAIL) {
-        if (tile < ntiles) tnext = MF::tail_begin(mat, MF::tail_span(mat, tile * 16 + wv * TROWS, TROWS), lane);
+        if (tile < ntiles) tnext = MF::tail_begin(mat, MF::tail_span(mat, row_of(tile) + wv * TROWS, TROWS), lane);
     }
     if (tile < ntiles && nsb > 0) request(tile, 0);
     if constexpr (XN) {
@@ -563,7 +567,7 @@ __global__ void __launch_bounds__(KS * 64) gemv_mfma_lds(typename MF::Mat mat, c
                 if constexpr (MF::TAIL) {
                     if (sb == 0) {
                         MF::tail_loads(mat, tl, xrows, C, min(M, 16), lane);
-                        span_next = MF::tail_span(mat, min(next, ntiles - 1) * 16 + wv * TROWS, TROWS);
+                        span_next = MF::tail_span(mat, row_of(min(next, ntiles - 1)) + wv * TROWS, TROWS);
                     }
                 }
                 // the next sub-block - of this tile, or the first of the workgroup's next tile - on its way
@@ -597,13 +601,13 @@ __global__ void __launch_bounds__(KS * 64) gemv_mfma_lds(typename MF::Mat mat, c
             if (nsb == 0) {
                 MF::tail_loads(mat, tl, xrows, C, min(M, 16), lane);
                 if (more)
-                    tnext = MF::tail_begin(mat, MF::tail_span(mat, next * 16 + wv * TROWS, TROWS), lane);
+                    tnext = MF::tail_begin(mat, MF::tail_span(mat, row_of(next) + wv * TROWS, TROWS), lane);
             }
             if (MF::tail_any(tl)) {  // the same for the whole wave
 #pragma unroll
                 for (int t = 0; t < MT; ++t)
                     if (t == 0 || t * 16 < M)
-                        MF::tail_apply(mat, tbl, tl, tile, xrows + (size_t)t * 16 * C, C, min(M - t * 16, 16), lane,
+                        MF::tail_apply(mat, tbl, tl, row_of(tile), xrows + (size_t)t * 16 * C, C, min(M - t * 16, 16), lane,
                                        tailbuf, t == 0, acc[t]);
             }
         }
@@ -638,20 +642,21 @@ __global__ void __launch_bounds__(KS * 64) gemv_mfma_lds(typename MF::Mat mat, c
                     o[3] = fold(s.w, up.w);
                 }
             } else {
-                const int in_tile = lg * 4, row = tile * tr + in_tile;
+                const int in_tile = lg * 4, row = row_of(tile) + in_tile;
+                const int own = RAG ? tile * tr : 0;  // the tile's own rows begin here
                 if (m < M) {
                     uint16_t* o = y + (size_t)m * R + row;
-                    if (in_tile + 0 < tr && row + 0 < R) o[0] = f32_bf16(s.x);
-                    if (in_tile + 1 < tr && row + 1 < R) o[1] = f32_bf16(s.y);
-                    if (in_tile + 2 < tr && row + 2 < R) o[2] = f32_bf16(s.z);
-                    if (in_tile + 3 < tr && row + 3 < R) o[3] = f32_bf16(s.w);
+                    if (in_tile + 0 < tr && row + 0 >= own && row + 0 < R) o[0] = f32_bf16(s.x);
+                    if (in_tile + 1 < tr && row + 1 >= own && row + 1 < R) o[1] = f32_bf16(s.y);
+                    if (in_tile + 2 < tr && row + 2 >= own && row + 2 < R) o[2] = f32_bf16(s.z);
+                    if (in_tile + 3 < tr && row + 3 >= own && row + 3 < R) o[3] = f32_bf16(s.w);
                 }
             }
         }
     }
 }
 
-template <class MF, int KS, int MT, int SPW, int SB, bool XS, bool XN, int TR>
+template <class MF, int KS, int MT, int SPW, int SB, bool XS, bool XN, int TR, bool RAG = false>
 static int32_t launch_lds_tr(const typename MF::Mat& mat, const void* x, void* y, int R, int C, int M, hipStream_t st,
                              int half, const XArgs& xa, int cap) {
     constexpr int SLAB = 16 * (SB * MF::STEPB + 16) + (MF::STEPB2 > 0 ? 16 * (SB * MF::STEPB2 + 16) : 0) + MF::TAIL_BYTES;
@@ -660,11 +665,11 @@ static int32_t launch_lds_tr(const typename MF::Mat& mat, const void* x, void* y
         const size_t rows = 16 * ((size_t)C * 2 + 16) + 16 * 4 * sizeof(float);
         if (rows > lds) lds = rows;
     }
-    const int ntiles = R / TR;
+    const int ntiles = RAG ? (R + TR - 1) / TR : R / TR;
     // whole turns of the grid over the tiles: the smallest grid that walks them in ceil(ntiles / cap) turns
     const int turns = (ntiles + cap - 1) / cap;
     const int grid = (ntiles + turns - 1) / turns;
-    auto kern = gemv_mfma_lds<MF, KS, MT, SPW, SB, XS, XN, TR>;
+    auto kern = gemv_mfma_lds<MF, KS, MT, SPW, SB, XS, XN, TR, RAG>;
     if (lds > 64 * 1024) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -689,7 +694,7 @@ static int32_t launch_lds(const typename MF::Mat& mat, const void* x, void* y, i
     // [2560 x 4096] 7.8 -> 7.6.
     if constexpr (std::is_same<MF, MfBf16>::value && KS == 8 && !XN) {
         if (half == 0 && tuning("mfma_tile_rows") != 0) {
-            auto rows_of = [&](int t) { return (long)((R / t + cap - 1) / cap) * t; };
+            auto rows_of = [&](int t) { return (long)(((R + t - 1) / t + cap - 1) / cap) * t; };
             int tr = 16;
             // (a lower tile has fewer bytes in flight a workgroup, which costs where the tiles are many: eight rows a
             // tile took [9728 x 2560] from 12.7 to 14.2 us and the head [151936 x 2560] from 130 to 173 although both
@@ -701,17 +706,20 @@ static int32_t launch_lds(const typename MF::Mat& mat, const void* x, void* y, i
             if (tr == 10) return launch_lds_tr<MF, KS, MT, SPW, SB, XS, XN, 10>(mat, x, y, R, C, M, st, half, xa, cap);
         }
     }
+    if constexpr (!XN) {
+        if (R % 16 != 0) return launch_lds_tr<MF, KS, MT, SPW, SB, XS, XN, 16, true>(mat, x, y, R, C, M, st, half, xa, cap);
+    }
     return launch_lds_tr<MF, KS, MT, SPW, SB, XS, XN, 16>(mat, x, y, R, C, M, st, half, xa, cap);
 }
 
 // The split of the columns over a workgroup's waves comes from the row length alone: at most eight waves (a workgroup
 // of sixteen would leave each wave 128 registers, less than the x fragments and a sub-block in flight need), each
-// holding x for 10, 16 or 28 steps. Up to 16 steps a wave there is room for two tiles of x rows; at 28 for one, and a
-// pass of more than 16 rows runs as two. Rows up to 7168 wide fit that way; up to 10240 the x fragments are streamed
-// (XS); wider ones stay with the column-interleaved kernel (bf16) or the vector-ALU passes (packed forms).
+// holding x for 10, 16 or 28 steps. Up to 16 steps a wave there is room for two tiles of x rows; at 28 for one. Rows up
+// to 7168 wide fit that way; up to 16384 the x fragments are streamed (XS), as they are for two tiles of x rows over rows
+// of more than 4096; wider ones stay with the column-interleaved kernel (bf16) or the vector-ALU passes (packed forms).
 template <class MF>
 static bool lds_fits(int R, int C) {
-    return R % 16 == 0 && C % 32 == 0 && C / 32 <= 8 * 40;
+    return R >= 16 && C % 32 == 0 && C / 32 <= 8 * 64;
 }
 bool mfma_lds_fits_bf16(int R, int C) { return lds_fits<MfBf16>(R, C); }
 bool mfma_lds_fits_packed(int R, int C) { return lds_fits<MfF8>(R, C); }
@@ -745,20 +753,48 @@ static int32_t run_lds(const typename MF::Mat& mat, const void* x, void* y, int 
     }
     constexpr int SBW = MF::SB_WIDE;
     // (sixteen steps a sub-block for the streamed rows - twice the bytes in flight - spills: [2560 x 9728] 13.7 -> 22.5 us)
-    // up to 28 steps a wave the x fragments stay in registers; longer rows (to 40 steps: 10240 columns) stream them
-    const bool stream_x = nsteps > 8 * 28 || tuning("mfma_stream_x") > 0;
-    for (int m0 = 0; m0 < M; m0 += 16) {
-        const int mm = M - m0 < 16 ? M - m0 : 16;
-        int32_t rc = stream_x ? (nsteps > 8 * 28
-                                     ? launch_lds<MF, 8, 1, 40, 8, true>(mat, xp + (size_t)m0 * C, yp + (size_t)m0 * yrow, R, C, mm, st, half)
-                                     : launch_lds<MF, 8, 1, 28, 8, true>(mat, xp + (size_t)m0 * C, yp + (size_t)m0 * yrow, R, C, mm, st, half))
-                              : launch_lds<MF, 8, 1, 28, SBW>(mat, xp + (size_t)m0 * C, yp + (size_t)m0 * yrow, R, C, mm, st, half);
+    // Up to 28 steps a wave the x fragments stay in registers; longer rows (to 64 steps: 16384 columns) stream them.
+    // Measured at 16 rows of x, [4096 x 12288], against the vector kernel's passes of four rows (bf16: the
+    // column-interleaved kernel): FP8 105.9 -> 32.3 us, MXFP4 129.5 -> 24.2, pack12 143.1 -> 29.0, bf16 33.9 -> 27.0.
+    // More than 16 rows of x: streamed, both tiles of x rows fit beside one pass over the weights. 32 rows, two passes
+    // against one: bf16 [4096 x 6144] 33.1 -> 26.5 us, [2560 x 9728] 36.4 -> 30.8, [8192 x 7040] 57.6 -> 55.1; FP8 [4096 x
+    // 6144] 36.2 -> 27.5, [8192 x 7040] 57.3 -> 49.4; MXFP4 [4096 x 6144] 25.8 -> 19.0 but [8192 x 7040] 38.3 -> 40.7,
+    // so MXFP4 only where the CUs go round once; pack12 loses ([5120 x 6144] 50.0 -> 57.9).
+    const bool two = M > 16 && !MF::TAIL && (!std::is_same<MF, MfMx4>::value || R <= 16 * device_info().cus);
+    const int step = two ? 32 : 16;
+    for (int m0 = 0; m0 < M; m0 += step) {
+        const int mm = M - m0 < step ? M - m0 : step;
+        const uint16_t* xm = xp + (size_t)m0 * C;
+        uint16_t* ym = yp + (size_t)m0 * yrow;
+        int32_t rc;
+        if constexpr (!MF::TAIL) {
+            if (two) {
+                if (nsteps <= 8 * 28)
+                    rc = launch_lds<MF, 8, 2, 28, 8, true>(mat, xm, ym, R, C, mm, st, half);
+                else if (nsteps <= 8 * 40)
+                    rc = launch_lds<MF, 8, 2, 40, 8, true>(mat, xm, ym, R, C, mm, st, half);
+                else if constexpr (!std::is_same<MF, MfBf16>::value)
+                    rc = launch_lds<MF, 8, 2, 64, 8, true>(mat, xm, ym, R, C, mm, st, half);
+                else
+                    rc = ERR_UNSUPPORTED;  // such passes go to the column-interleaved kernel
+                if (rc != OK) return rc;
+                continue;
+            }
+        }
+        if (nsteps > 8 * 40)
+            rc = launch_lds<MF, 8, 1, 64, 8, true>(mat, xm, ym, R, C, mm, st, half);
+        else if (nsteps > 8 * 28)
+            rc = launch_lds<MF, 8, 1, 40, 8, true>(mat, xm, ym, R, C, mm, st, half);
+        else if (tuning("mfma_stream_x") > 0)
+            rc = launch_lds<MF, 8, 1, 28, 8, true>(mat, xm, ym, R, C, mm, st, half);
+        else
+            rc = launch_lds<MF, 8, 1, 28, SBW>(mat, xm, ym, R, C, mm, st, half);
         if (rc != OK) return rc;
     }
     return OK;
 }
 
-// M = 5..32 and a shape the fits() above take (whole 16-row tiles among them): the callers (gemv.hip) check before
+// M = 5..32 and a shape the fits() above take (a whole tile of 16 rows at least): the callers (gemv.hip) check before
 // they come here
 int32_t gemv_mfma_lds_bf16(const void* w, const void* x, void* y, int R, int C, int M, hipStream_t st) {
     return run_lds<MfBf16>(MfBf16::Mat{static_cast<const uint8_t*>(w)}, x, y, R, C, M, st);
@@ -771,7 +807,7 @@ int32_t gemv_mfma_lds_glu_bf16(const void* w, const void* x, void* y, int I, int
 // 1312 .. 2560 columns (the widths whose workgroups are 512 threads: two rows in the making at once), 16 rows of the
 // residual stream a pass.
 bool mfma_lds_norm_fits(int R, int C, int M) {
-    return lds_fits<MfBf16>(R, C) && C / 32 > 40 && C / 32 <= 80 && M >= 5 && tuning("mfma_lds_norm") != 0;
+    return R % 16 == 0 && lds_fits<MfBf16>(R, C) && C / 32 > 40 && C / 32 <= 80 && M >= 5 && tuning("mfma_lds_norm") != 0;
 }
 int32_t gemv_mfma_lds_norm_bf16(const void* w, const XArgs& xa, void* y, int R, int C, int M, int I, hipStream_t st) {
     const MfBf16::Mat mat{static_cast<const uint8_t*>(w)};

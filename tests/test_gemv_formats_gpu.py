@@ -624,3 +624,32 @@ def test_fp8_add_norm_and_activation_in_the_matvec(card, R, C, block, M, glu, wi
         card.gemv_embed_norm(w, h, ids, nw, 1e-6, h3, out3)
         assert torch.equal(out3.view(torch.int16), want.view(torch.int16))
         assert torch.equal(h3.view(torch.int16), h1.view(torch.int16))
+
+
+# one row past a tile, one before two, one tile and the smallest past it, every wave's split (2, 4, 8 waves), short rows
+# that leave waves without a step, streamed x; one and two tiles of x rows
+@pytest.mark.parametrize("R,C", [(17, 512), (31, 1216), (16, 2592), (1009, 2560), (4107, 736), (345, 7200), (515, 9600),
+                                 (25, 96), (650, 5120), (144, 12288), (257, 16384)])
+@pytest.mark.parametrize("form", ["bf16", "pack12", "mxfp4"])
+@pytest.mark.parametrize("M", [5, 16, 27])
+def test_row_counts_that_end_inside_a_tile(card, R, C, form, M):
+    """matrices whose rows are no whole number of sixteen-row tiles on the matrix cores (the last tile starts sixteen rows
+    before the end): against the oracle, every row of a wide pass, escapes in the last rows among them, nothing written
+    past the last"""
+    x = acts_bf16(M, C, seed=400 + R)
+    if form == "mxfp4":
+        b, s = mxfp4.quantize(torch.randn(R, C, generator=gen(R + C)) * 0.02)
+        w, op = mxfp4.MxWeight(b.reshape(-1).cuda(), s.reshape(-1).cuda(), R, C), card.gemv_mx4
+        ref = oracle.gemv_mxfp4(b.reshape(-1).numpy(), s.reshape(-1).numpy(), R, C, x.float().numpy(), threads=0)
+    else:
+        wb = bits16(weights_bf16(R, C, seed=401 + R)).copy().reshape(R, C)
+        wb[R - 1, ::7] = (wb[R - 1, ::7] & 0x00FF) | 0x4200  # large weights: escapes in the last row, and in its neighbours
+        wb[max(R - 17, 0), 3] = (wb[max(R - 17, 0), 3] & 0x00FF) | 0x3100
+        t = torch.from_numpy(wb.view(np.int16)).view(torch.bfloat16).cuda()
+        w, op = (P12Weight.pack(t, card), card.gemv_p12) if form == "pack12" else (t, card.gemv)
+        ref = oracle.gemv_bf16(wb, x.float().numpy(), threads=0)
+    room = torch.full((M * R + 64,), 7.0, dtype=torch.bfloat16, device="cuda")
+    y = room[: M * R].view(M, R)
+    op(w, x.cuda(), y)
+    check(y, ref)
+    assert bool((room[M * R:] == 7.0).all())
