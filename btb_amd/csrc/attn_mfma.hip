@@ -22,7 +22,14 @@
 //
 // What comes out is the (m, l, acc[128]) state per (row, head, span) that attn_decode_kernel leaves, for the same
 // merge kernel; the arithmetic is the same up to the order of the f32 sums (the matrix cores' instead of the
-// 16-stream fold's). Which keys a row sees - chain or tree, window - is row_view's, as there.
+// 16-stream fold's) and the maximum a weight is taken against (the span's instead of its stream's). Which keys a row
+// sees - chain or tree, window - is row_view's, as there.
+//
+// SPLIT, passes of more than sixteen rows: a weight goes to the matrix cores as two bf16 terms, as in attn_span.hip and for
+// its reason - a step's pass of so many rows over spans of 128 keys is what the vector kernels served in longer spans,
+// closer to f64 (32 rows x 32 / 8 heads, 1536 keys: 1.99e-3 off there, 2.15e-3 here with one term, 1.66e-3 with two;
+// norm_rope_kv, this and the fold 18.6 us a layer with one term, 19.1 with two, 37.3 on the vector kernel). The second terms have sums of their own, left out where they are not finite: of an
+// infinite value and a weight's two terms the first alone says what the output is.
 
 #include "btb_attn.hpp"
 #include "btb_common.hpp"
@@ -37,11 +44,13 @@ constexpr int AM_SPAN = 128;  // keys a workgroup
 constexpr int AM_VROW = 272;  // bytes a V row takes in LDS: 256 + 16, so the eight rows a fragment read touches differ in bank
 constexpr int AM_PROW = 80;   // bytes a pair's 32 weights of a step take: 64 + 16, sixteen pairs in sixteen bank groups
 
+constexpr int AM_PROW2 = 144;  // the same with the weights' second terms behind them
+
 constexpr int AM_QROW = 272;  // bytes a prepared q or k row takes in LDS: 256 + 16, as for V
 
-__host__ __device__ constexpr size_t am_lds_bytes(int G, int NQT, bool QKV, int ZG = 1) {
+__host__ __device__ constexpr size_t am_lds_bytes(int G, int NQT, bool QKV, int ZG = 1, bool SPLIT = false) {
     const size_t NQ = 16 * (size_t)NQT, TPW = NQ / (size_t)G;
-    const size_t weights = 4 * NQ * AM_PROW, heads = QKV ? (NQ + (size_t)ZG * TPW) * AM_QROW : 0;
+    const size_t weights = 4 * NQ * (SPLIT ? AM_PROW2 : AM_PROW), heads = QKV ? (NQ + (size_t)ZG * TPW) * AM_QROW : 0;
     return (size_t)AM_SPAN * AM_VROW + 2 * 4 * NQ * sizeof(float) + (weights > heads ? weights : heads);
 }
 
@@ -56,20 +65,20 @@ __host__ __device__ constexpr size_t am_lds_bytes(int G, int NQT, bool QKV, int 
 // norm_rope_kv_kernel's, then this kernel's. ZG = 2: the pass's pairs are two workgroups' (gridDim.z = 2, up to 64 pairs
 // a kv head): each prepares the q heads of its own rows and the k heads of all the rows, the first of the two writes
 // the cache.
-template <int G, int NQT, bool TBL, bool QKV, bool DEPTH, int ZG = 1>
+template <int G, int NQT, bool TBL, bool QKV, bool DEPTH, int ZG = 1, bool SPLIT = false>
 __global__ void __launch_bounds__(256) attn_decode_mfma_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ K, const uint16_t* __restrict__ V,
     const int32_t* __restrict__ n0p, const int32_t* __restrict__ par, int T, int Hq, int Hk, long long hs, long long rs,
     float scale_log2, float* __restrict__ part_m, float* __restrict__ part_l, float* __restrict__ part_acc, int cap,
     int win, const int32_t* __restrict__ tbl, AmQkv x) {
-    constexpr int D = AD, NQ = 16 * NQT, TPW = NQ / G;
+    constexpr int D = AD, NQ = 16 * NQT, TPW = NQ / G, PROW = SPLIT ? AM_PROW2 : AM_PROW;
     static_assert(NQ % G == 0, "whole rows a workgroup");
     static_assert(!(QKV && TBL), "the fused rows go with a cache without a row map");
     extern __shared__ __align__(16) uint8_t lds[];
     uint8_t* v_lds = lds;                                                 // [128 keys][AM_VROW]
     float* red_m = reinterpret_cast<float*>(lds + AM_SPAN * AM_VROW);     // [4 waves][NQ]
     float* red_l = red_m + 4 * NQ;                                        // [4 waves][NQ]
-    // [4 steps of 32 keys][NQ pairs][AM_PROW]; before the scores are done the prepared heads lie here:
+    // [4 steps of 32 keys][NQ pairs][PROW]; before the scores are done the prepared heads lie here:
     // q [NQ][AM_QROW], then the pass's own k rows [ZG TPW][AM_QROW]
     uint8_t* p_lds = reinterpret_cast<uint8_t*>(red_l + 4 * NQ);
     const int g = blockIdx.x, sp = blockIdx.y, S = gridDim.y;
@@ -277,7 +286,7 @@ __global__ void __launch_bounds__(256) attn_decode_mfma_kernel(
         float l = 0.f;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            uint32_t pw[2];
+            uint32_t pw[2], pw2[2];
 #pragma unroll
             for (int i2 = 0; i2 < 2; ++i2) {
                 const float s0 = st[h][qt][2 * i2], s1 = st[h][qt][2 * i2 + 1];
@@ -285,11 +294,19 @@ __global__ void __launch_bounds__(256) attn_decode_mfma_kernel(
                 const float p1 = s1 == ninf ? 0.f : __builtin_amdgcn_exp2f(s1 - m);
                 const bf16x2 pr = {(__bf16)p0, (__bf16)p1};
                 pw[i2] = __builtin_bit_cast(uint32_t, pr);
-                l += bf16lo_f32(pw[i2]);
-                l += bf16hi_f32(pw[i2]);
+                if constexpr (SPLIT) {
+                    pw2[i2] = f32x2_bf16(p0 - bf16lo_f32(pw[i2]), p1 - bf16hi_f32(pw[i2]));
+                    l += p0;
+                    l += p1;
+                } else {
+                    l += bf16lo_f32(pw[i2]);
+                    l += bf16hi_f32(pw[i2]);
+                }
             }
             // step wv (the wave's 32 keys), pair r, slots 16 h + 4 a .. + 3
-            *reinterpret_cast<uint2*>(p_lds + (wv * NQ + r) * AM_PROW + (16 * h + 4 * a) * 2) = make_uint2(pw[0], pw[1]);
+            uint8_t* to = p_lds + (wv * NQ + r) * PROW + (16 * h + 4 * a) * 2;
+            *reinterpret_cast<uint2*>(to) = make_uint2(pw[0], pw[1]);
+            if constexpr (SPLIT) *reinterpret_cast<uint2*>(to + 64) = make_uint2(pw2[0], pw2[1]);
         }
         l += xor_lanes16(l);
         l += xor_lanes32(l);
@@ -310,16 +327,24 @@ __global__ void __launch_bounds__(256) attn_decode_mfma_kernel(
     }
     // outputs: O^T tile [dt][qt], lane: pair c of tile qt, dims 32 wv + 16 dt + 4 a .. + 3
     f32x4 ot[2][NQT];
+    [[maybe_unused]] f32x4 ot2[2][NQT];  // SPLIT: of the weights' second terms
 #pragma unroll
     for (int dt = 0; dt < 2; ++dt)
 #pragma unroll
-        for (int qt = 0; qt < NQT; ++qt) ot[dt][qt] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int qt = 0; qt < NQT; ++qt) {
+            ot[dt][qt] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if constexpr (SPLIT) ot2[dt][qt] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
         uint4 pfrag[NQT];
+        [[maybe_unused]] uint4 pfrag2[NQT];
 #pragma unroll
-        for (int qt = 0; qt < NQT; ++qt)
-            pfrag[qt] = *reinterpret_cast<const uint4*>(p_lds + (ks * NQ + qt * 16 + c) * AM_PROW + a * 16);
+        for (int qt = 0; qt < NQT; ++qt) {
+            const uint8_t* from = p_lds + (ks * NQ + qt * 16 + c) * PROW + a * 16;
+            pfrag[qt] = *reinterpret_cast<const uint4*>(from);
+            if constexpr (SPLIT) pfrag2[qt] = *reinterpret_cast<const uint4*>(from + 64);
+        }
 #pragma unroll
         for (int dt = 0; dt < 2; ++dt) {
             // V^T fragment: dim 32 wv + 16 dt + c, keys 32 ks + 8 a .. + 7
@@ -336,7 +361,22 @@ __global__ void __launch_bounds__(256) attn_decode_mfma_kernel(
             for (int qt = 0; qt < NQT; ++qt)
                 ot[dt][qt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vfrag, __builtin_bit_cast(bf16x8, pfrag[qt]),
                                                                      ot[dt][qt], 0, 0, 0);
+            if constexpr (SPLIT) {
+#pragma unroll
+                for (int qt = 0; qt < NQT; ++qt)
+                    ot2[dt][qt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vfrag, __builtin_bit_cast(bf16x8, pfrag2[qt]),
+                                                                          ot2[dt][qt], 0, 0, 0);
+            }
         }
+    }
+    if constexpr (SPLIT) {
+#pragma unroll
+        for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+            for (int qt = 0; qt < NQT; ++qt)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    ot[dt][qt][i] += fabsf(ot2[dt][qt][i]) < __builtin_inff() ? ot2[dt][qt][i] : 0.f;
     }
 #pragma unroll
     for (int qt = 0; qt < NQT; ++qt) {
@@ -352,36 +392,40 @@ __global__ void __launch_bounds__(256) attn_decode_mfma_kernel(
     }
 }
 
-template <int G, int NQT>
-static void launch_am(const uint16_t* q, const uint16_t* K, const uint16_t* V, const int32_t* n0, const int32_t* par, int T,
-               int Hq, int Hk, long long hs, long long rs, float scale_log2, float* part_m, float* part_l,
-               float* part_acc, int S, int cap, int win, const int32_t* tbl, hipStream_t st) {
+template <int G, int NQT, bool SPLIT = false>
+static hipError_t launch_am(const uint16_t* q, const uint16_t* K, const uint16_t* V, const int32_t* n0, const int32_t* par,
+                            int T, int Hq, int Hk, long long hs, long long rs, float scale_log2, float* part_m,
+                            float* part_l, float* part_acc, int S, int cap, int win, const int32_t* tbl, hipStream_t st) {
     constexpr int NQ = 16 * NQT, TPW = NQ / G;
-    const size_t lds = am_lds_bytes(G, NQT, false);
+    constexpr size_t lds = am_lds_bytes(G, NQT, false, 1, SPLIT);
     const dim3 grid((unsigned)Hk, (unsigned)S, (unsigned)((T + TPW - 1) / TPW));
     const AmQkv none{};
-    if (tbl != nullptr)
-        hipLaunchKernelGGL((attn_decode_mfma_kernel<G, NQT, true, false, false>), grid, dim3(256), lds, st, q, K, V, n0,
-                           par, T, Hq, Hk, hs, rs, scale_log2, part_m, part_l, part_acc, cap, win, tbl, none);
-    else
-        hipLaunchKernelGGL((attn_decode_mfma_kernel<G, NQT, false, false, false>), grid, dim3(256), lds, st, q, K, V, n0,
-                           par, T, Hq, Hk, hs, rs, scale_log2, part_m, part_l, part_acc, cap, win, tbl, none);
+    auto kern = tbl != nullptr ? attn_decode_mfma_kernel<G, NQT, true, false, false, 1, SPLIT>
+                               : attn_decode_mfma_kernel<G, NQT, false, false, false, 1, SPLIT>;
+    if (lds > 64 * 1024) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return e;
+    }
+    hipLaunchKernelGGL(kern, grid, dim3(256), lds, st, q, K, V, n0, par, T, Hq, Hk, hs, rs, scale_log2, part_m, part_l,
+                       part_acc, cap, win, tbl, none);
+    return hipGetLastError();
 }
 
 // the variant that starts from the fused qkv rows: one workgroup per (kv head, span), the whole pass in it
-template <int G, int NQT, int ZG>
+template <int G, int NQT, int ZG, bool SPLIT = false>
 static void launch_am_qkv(const AmQkv& x, const int32_t* n0, const int32_t* par, int T, int Hq, int Hk, long long hs,
                           long long rs, float scale_log2, float* part_m, float* part_l, float* part_acc, int S, int cap,
                           hipStream_t st) {
-    const size_t lds = am_lds_bytes(G, NQT, true, ZG);
-    static_assert(am_lds_bytes(G, NQT, true, ZG) <= 64 * 1024, "within what a workgroup gets without asking for more");
+    const size_t lds = am_lds_bytes(G, NQT, true, ZG, SPLIT);
+    static_assert(am_lds_bytes(G, NQT, true, ZG, SPLIT) <= 64 * 1024, "within what a workgroup gets without asking for more");
     const dim3 grid((unsigned)Hk, (unsigned)S, (unsigned)ZG);
     const uint16_t* none = nullptr;
     if (x.depth != nullptr)
-        hipLaunchKernelGGL((attn_decode_mfma_kernel<G, NQT, false, true, true, ZG>), grid, dim3(256), lds, st, none, x.Kw,
+        hipLaunchKernelGGL((attn_decode_mfma_kernel<G, NQT, false, true, true, ZG, SPLIT>), grid, dim3(256), lds, st, none, x.Kw,
                            x.Vw, n0, par, T, Hq, Hk, hs, rs, scale_log2, part_m, part_l, part_acc, cap, 0, nullptr, x);
     else
-        hipLaunchKernelGGL((attn_decode_mfma_kernel<G, NQT, false, true, false, ZG>), grid, dim3(256), lds, st, none, x.Kw,
+        hipLaunchKernelGGL((attn_decode_mfma_kernel<G, NQT, false, true, false, ZG, SPLIT>), grid, dim3(256), lds, st, none, x.Kw,
                            x.Vw, n0, par, T, Hq, Hk, hs, rs, scale_log2, part_m, part_l, part_acc, cap, 0, nullptr, x);
 }
 
@@ -406,18 +450,20 @@ int32_t attn_decode_mfma(const void* q, const void* K, const void* V, const int3
     const size_t G = Hq / Hk;
     const size_t pairs = T * G;  // of one kv head
     const int nqt = pairs <= 16 ? 1 : pairs <= 32 ? 2 : 4;
+    const bool split = T > 16;  // more than 32 pairs then
+    hipError_t e;
     const int capi = (int)(cap < 0x7FFFFFFFu ? cap : 0x7FFFFFFFu);
-#define AM(GG, NN)                                                                                                    \
-    launch_am<GG, NN>(static_cast<const uint16_t*>(q), static_cast<const uint16_t*>(K), static_cast<const uint16_t*>(V), \
+#define AM(...)                                                                                                       \
+    e = launch_am<__VA_ARGS__>(static_cast<const uint16_t*>(q), static_cast<const uint16_t*>(K), static_cast<const uint16_t*>(V), \
                       n0, par, (int)T, (int)Hq, (int)Hk, hs, rs, scale_log2, part_m, part_l, part_acc, (int)S, capi, win, \
                       tbl, st)
     if (G == 4) {
-        if (nqt == 1) AM(4, 1); else if (nqt == 2) AM(4, 2); else AM(4, 4);
+        if (nqt == 1) AM(4, 1); else if (nqt == 2) AM(4, 2); else if (split) AM(4, 4, true); else AM(4, 4);
     } else {
-        if (nqt == 1) AM(2, 1); else if (nqt == 2) AM(2, 2); else AM(2, 4);
+        if (nqt == 1) AM(2, 1); else if (nqt == 2) AM(2, 2); else if (split) AM(2, 4, true); else AM(2, 4);
     }
 #undef AM
-    return hip_status(hipGetLastError(), "attn_decode_mfma launch");
+    return hip_status(e, "attn_decode_mfma launch");
 }
 
 // the same states from the fused qkv rows; the new K / V rows land in the cache on the way
@@ -440,13 +486,13 @@ int32_t attn_decode_mfma_qkv(const void* qkv, const void* wq, const void* wk, fl
     x.Vw = static_cast<uint16_t*>(V);
     x.eps = eps;
     x.centered = centered;
-#define AMQ(GG, NN, ZZ)                                                                                               \
-    launch_am_qkv<GG, NN, ZZ>(x, n0, par, (int)T, (int)Hq, (int)Hk, hs, rs, scale_log2, part_m, part_l, part_acc,     \
+#define AMQ(...)                                                                                                      \
+    launch_am_qkv<__VA_ARGS__>(x, n0, par, (int)T, (int)Hq, (int)Hk, hs, rs, scale_log2, part_m, part_l, part_acc,     \
                               (int)S, capi, st)
     if (G == 4) {
         if (nqt == 1) AMQ(4, 1, 1); else if (pairs <= 32) AMQ(4, 2, 1); else AMQ(4, 2, 2);
     } else {
-        if (nqt == 1) AMQ(2, 1, 1); else if (pairs <= 32) AMQ(2, 2, 1); else AMQ(2, 2, 2);
+        if (nqt == 1) AMQ(2, 1, 1); else if (pairs <= 32) AMQ(2, 2, 1); else if (T > 16) AMQ(2, 2, 2, true); else AMQ(2, 2, 2);
     }
 #undef AMQ
     return hip_status(hipGetLastError(), "attn_decode_mfma_qkv launch");

@@ -7,8 +7,18 @@
 // A workgroup: one kv head, one span, up to 64 of the pass's (row, head) pairs; wider passes are more workgroups (the
 // z axis), which read the same keys out of the last-level cache. Four waves; the products' layout is attn_mfma.hip's:
 // scores S^T = K Q^T with wave w on keys 32 w .. + 31 of the batch, outputs O^T = V^T P^T with wave w on dims 32 w ..
-// + 31, weights rounded to bf16 and their sum made of the rounded ones. Between batches a pair's maximum moves in every
-// lane that holds the pair, so the rescaling needs no exchange; the sums stay a lane's own until the span ends.
+// + 31. Between batches a pair's maximum moves in every lane that holds the pair, so the rescaling needs no exchange; the
+// sums stay a lane's own until the span ends.
+//
+// A weight goes to the matrix cores as two bf16 terms, its rounding and what the rounding left (2^-17 of it stays out),
+// one product each into the same sum. A weight rounded once is not enough here: the vector kernels take a weight against
+// the maximum of its own stream of 16 keys or fewer a batch, so the heaviest of them are 1 and exact, and against f64 their
+// outputs lie 1.8e-3 to 2.2e-3 off (relative 2-norm, normal q and k, 100 to 32000 keys) where weights taken against a whole
+// batch's maximum and rounded once lie 2.1e-3 to 2.2e-3 off; with two terms 1.66e-3, what rounding the outputs to bf16
+// alone makes. With the fold, one term / two: one row x 32 / 8 heads over 32000 keys 26.7 / 27.8 us, 8 rows over 6125
+// 15.1 / 15.9, 32 rows over 6125 34.2 / 39.6, over 23367 54.8 / 65.2 (the vector kernels 32.7, 32.8, 97, 349).
+// Two terms of unlike sign, or a zero, must not meet an infinite value: a workgroup that ends with an output that is not
+// finite walks its span once more with such values taken out of the product and added by their whole weight.
 //
 // The next batch's K is asked for as soon as the scores are made and its V as soon as this one's lies in LDS, into the
 // registers just freed: a batch's arithmetic (about 1 us for 64 pairs) hides the next one's trip. Two barriers a batch:
@@ -22,20 +32,34 @@
 #include "btb_head_tile.hpp"
 #include "btb_tuning.hpp"
 
+#include <type_traits>
+
 #include "../../include/btb_hip.h"
 
 namespace btb {
 
 constexpr int AS_KEYS = 128;  // keys a batch
 constexpr int AS_VROW = 272;  // bytes a V row takes in LDS: 256 + 16, so the eight rows a fragment read touches differ in bank
-constexpr int AS_PROW = 80;   // bytes a pair's 32 weights of a step take: 64 + 16, sixteen pairs in sixteen bank groups
-
+constexpr int AS_PROW = 144;  // bytes a pair's 32 weights of a step take: 64 a term and 16, so that pairs differ in bank
 constexpr int AS_HROW = 272;  // bytes a prepared q, k or v row takes in LDS: as a V row
+constexpr int AS_VOWN = 16;   // a pass of more rows reads its own v rows out of the fused rows when it needs them: with
+                              // them in LDS too (8.7 KB at 32 rows) a CU would hold one workgroup and not two
 
 // own: the pass's own rows kept in LDS (their k, then their v), none where q is given
 __host__ __device__ constexpr size_t as_lds_bytes(int NQT, int own) {
     const size_t NQ = 16 * (size_t)NQT;
-    return (size_t)AS_KEYS * AS_VROW + 4 * NQ * sizeof(float) + 4 * NQ * AS_PROW + 2 * (size_t)own * AS_HROW;
+    return (size_t)AS_KEYS * AS_VROW + 4 * NQ * sizeof(float) + 4 * sizeof(int) + 4 * NQ * AS_PROW +
+           (size_t)(own > AS_VOWN ? own : 2 * own) * AS_HROW;
+}
+
+// eight bf16 values with those that are not finite as zeros
+__device__ __forceinline__ uint32_t finite2(uint32_t w) {
+    if ((w & 0x7F80u) == 0x7F80u) w &= 0xFFFF0000u;
+    if ((w & 0x7F800000u) == 0x7F800000u) w &= 0x0000FFFFu;
+    return w;
+}
+__device__ __forceinline__ uint4 finite8(const uint4& v) {
+    return make_uint4(finite2(v.x), finite2(v.y), finite2(v.z), finite2(v.w));
 }
 
 // NQT tiles of 16 (row, head) pairs a workgroup: pair r is row t_base + r / G, head r % G, G = 1 << gs. TBL: the cache
@@ -44,8 +68,7 @@ __host__ __device__ constexpr size_t as_lds_bytes(int NQT, int own) {
 // QKV: the rows come as the fused qkv rows, before the q / k norm and rope. A workgroup prepares the q heads of its own
 // rows, a tile of 16 a wave and turn, while the first batch's K travels (its addresses then wait for nothing: they stay
 // within the cache's capacity); where its span holds some of the pass's own slots *n0 .. *n0 + T - 1 it prepares the
-// pass's k heads too, takes those keys and values from LDS, and the last of the z axis - whose rows see all of them -
-// writes them into the cache. T <= 32. The arithmetic is norm_rope_kv_kernel's, then this kernel's.
+// pass's k heads too, takes those keys and values from there, and the last of the z axis - whose rows see all of them - writes them into the cache. T <= 32. The arithmetic is norm_rope_kv_kernel's, then this kernel's.
 template <int NQT, bool TBL, bool QKV>
 __global__ void __launch_bounds__(256, 2) attn_span_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ K, const uint16_t* __restrict__ V,
@@ -57,7 +80,8 @@ __global__ void __launch_bounds__(256, 2) attn_span_kernel(
     extern __shared__ __align__(16) uint8_t lds[];
     uint8_t* v_lds = lds;                                             // [128 keys][AS_VROW]
     float* red = reinterpret_cast<float*>(lds + AS_KEYS * AS_VROW);   // [4 waves][NQ]: maxima, at the end the sums
-    uint8_t* p_lds = reinterpret_cast<uint8_t*>(red + 4 * NQ);        // [4 steps of 32 keys][NQ pairs][AS_PROW]
+    int* odd = reinterpret_cast<int*>(red + 4 * NQ);                  // [4 waves]: an output of the wave is not finite
+    uint8_t* p_lds = reinterpret_cast<uint8_t*>(odd + 4);             // [4 steps of 32 keys][NQ pairs][AS_PROW]
     uint8_t* q_lds = p_lds;                                           // QKV, before the first weights: [NQ][AS_HROW]
     uint8_t* kn_lds = p_lds + 4 * NQ * AS_PROW;                       // QKV: the pass's own k rows, then their v rows
     uint8_t* vn_lds = kn_lds + T * AS_HROW;
@@ -129,7 +153,7 @@ __global__ void __launch_bounds__(256, 2) attn_span_kernel(
 #pragma unroll
                     for (int ds = 0; ds < 4; ++ds) {
                         *reinterpret_cast<uint4*>(kn_lds + tr * AS_HROW + ds * 64 + a * 16) = out[ds];
-                        *reinterpret_cast<uint4*>(vn_lds + tr * AS_HROW + ds * 64 + a * 16) = h.vrow[ds];
+                        if (T <= AS_VOWN) *reinterpret_cast<uint4*>(vn_lds + tr * AS_HROW + ds * 64 + a * 16) = h.vrow[ds];
                     }
                     // (a slot at or past the cache's capacity is not written: the caller has let the cache overflow)
                     if (blockIdx.z == gridDim.z - 1 && slot >= k_begin && slot < min(k_begin + span, cap)) {
@@ -167,14 +191,14 @@ __global__ void __launch_bounds__(256, 2) attn_span_kernel(
 
     f32x4 ot[2][NQT];      // O^T tile [dt][qt], lane: pair c of tile qt, dims 32 wv + 16 dt + 4 a .. + 3
     float m[NQT], l[NQT];  // pair c's running maximum (the same in its lanes of every wave), the lane's share of its sum
-#pragma unroll
-    for (int qt = 0; qt < NQT; ++qt) {
-        m[qt] = ninf;
-        l[qt] = 0.f;
-        ot[0][qt] = ot[1][qt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
     const uint32_t rows = tree_rows(parent, T);  // while the first batch travels
-    for (int kb = k_begin; kb < k_lim; kb += AS_KEYS) {
+    // one batch of keys; CAREFUL: values that are not finite are taken out of the product and added by their whole weight
+    auto batch = [&](auto mode, int kb) {
+        constexpr bool CAREFUL = decltype(mode)::value;
+        if constexpr (CAREFUL) {
+            request_k(kb, last);
+            request_v(kb, last);
+        }
         const bool own = own_here && kb < n0 + T && n0 < kb + AS_KEYS;
         if constexpr (QKV) {
             if (own) {
@@ -203,7 +227,7 @@ __global__ void __launch_bounds__(256, 2) attn_span_kernel(
                                                                   __builtin_bit_cast(bf16x8, qreg[qt][ds]), acc, 0, 0, 0);
                 st[h][qt] = acc;
             }
-        const bool more = kb + AS_KEYS < k_lim;
+        const bool more = !CAREFUL && kb + AS_KEYS < k_lim;
         if (more) request_k(kb + AS_KEYS, last);
         // scaled, masked where a row may not see a key (a batch wholly in the cache, without a window, needs no mask)
         if (kb + AS_KEYS <= n0 && win == 0) {
@@ -253,17 +277,23 @@ __global__ void __launch_bounds__(256, 2) attn_span_kernel(
         }
         if constexpr (QKV) {
             if (own) {  // the rows of the pass among them, by the threads that have just written their places
+                const uint16_t* v_own = x.qkv + (size_t)(Hq + Hk + g) * D + (tid & 15) * 8;
 #pragma unroll
                 for (int i = 0; i < 8; ++i) {
                     const int key = kb + (tid >> 4) + 16 * i, tr = key - n0;
-                    if (tr >= 0 && tr < T && key < k_lim)
-                        *reinterpret_cast<uint4*>(v_lds + (key - kb) * AS_VROW + (tid & 15) * 16) =
-                            *reinterpret_cast<const uint4*>(vn_lds + tr * AS_HROW + (tid & 15) * 16);
+                    if (tr >= 0 && tr < T && key < k_lim) {
+                        uint4 v;
+                        if (T <= AS_VOWN)
+                            v = *reinterpret_cast<const uint4*>(vn_lds + tr * AS_HROW + (tid & 15) * 16);
+                        else
+                            v = *reinterpret_cast<const uint4*>(v_own + (size_t)tr * (Hq + 2 * Hk) * D);
+                        *reinterpret_cast<uint4*>(v_lds + (key - kb) * AS_VROW + (tid & 15) * 16) = v;
+                    }
                 }
             }
         }
         if (more) request_v(kb + AS_KEYS, last);
-        // the pairs' maxima move; weights, rounded to bf16, P^T into LDS
+        // the pairs' maxima move; weights in two terms, P^T into LDS
 #pragma unroll
         for (int qt = 0; qt < NQT; ++qt) {
             const int r = qt * 16 + c;
@@ -274,18 +304,21 @@ __global__ void __launch_bounds__(256, 2) attn_span_kernel(
             float sum = 0.f;
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-                uint32_t pw[2];
+                uint32_t pw[2], pw2[2];
 #pragma unroll
                 for (int i2 = 0; i2 < 2; ++i2) {
                     const float s0 = st[h][qt][2 * i2], s1 = st[h][qt][2 * i2 + 1];
                     const float p0 = s0 == ninf ? 0.f : __builtin_amdgcn_exp2f(s0 - mn);
                     const float p1 = s1 == ninf ? 0.f : __builtin_amdgcn_exp2f(s1 - mn);
                     pw[i2] = f32x2_bf16(p0, p1);
-                    sum += bf16lo_f32(pw[i2]);
-                    sum += bf16hi_f32(pw[i2]);
+                    pw2[i2] = f32x2_bf16(p0 - bf16lo_f32(pw[i2]), p1 - bf16hi_f32(pw[i2]));
+                    sum += p0;
+                    sum += p1;
                 }
                 // step wv (the wave's 32 keys), pair r, slots 16 h + 4 a .. + 3
-                *reinterpret_cast<uint2*>(p_lds + (wv * NQ + r) * AS_PROW + (16 * h + 4 * a) * 2) = make_uint2(pw[0], pw[1]);
+                const int at = (wv * NQ + r) * AS_PROW + (16 * h + 4 * a) * 2;
+                *reinterpret_cast<uint2*>(p_lds + at) = make_uint2(pw[0], pw[1]);
+                *reinterpret_cast<uint2*>(p_lds + at + 64) = make_uint2(pw2[0], pw2[1]);
             }
             l[qt] = fmaf(l[qt], corr, sum);
 #pragma unroll
@@ -294,12 +327,34 @@ __global__ void __launch_bounds__(256, 2) attn_span_kernel(
                 for (int i = 0; i < 4; ++i) ot[dt][qt][i] *= corr;
         }
         __syncthreads();
+        if constexpr (CAREFUL) {
+#pragma unroll 1
+            for (int key = 0; key < AS_KEYS; ++key)
+#pragma unroll
+                for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const uint32_t v =
+                            *reinterpret_cast<const uint16_t*>(v_lds + key * AS_VROW + (32 * wv + 16 * dt + 4 * a + i) * 2);
+                        if ((v & 0x7F80u) != 0x7F80u) continue;
+#pragma unroll
+                        for (int qt = 0; qt < NQT; ++qt) {
+                            const uint32_t p = *reinterpret_cast<const uint16_t*>(
+                                p_lds + ((key >> 5) * NQ + qt * 16 + c) * AS_PROW + (key & 31) * 2);
+                            ot[dt][qt][i] = fmaf(bits_f32(p << 16), bits_f32(v << 16), ot[dt][qt][i]);
+                        }
+                    }
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                uint4* v = reinterpret_cast<uint4*>(v_lds + ((tid >> 4) + 16 * i) * AS_VROW + (tid & 15) * 16);
+                *v = finite8(*v);
+            }
+            __syncthreads();
+        }
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
-            uint4 pfrag[NQT];
-#pragma unroll
-            for (int qt = 0; qt < NQT; ++qt)
-                pfrag[qt] = *reinterpret_cast<const uint4*>(p_lds + (ks * NQ + qt * 16 + c) * AS_PROW + a * 16);
+            bf16x8 vfrag[2];
 #pragma unroll
             for (int dt = 0; dt < 2; ++dt) {
                 // V^T fragment: dim 32 wv + 16 dt + c, keys 32 ks + 8 a .. + 7
@@ -311,16 +366,48 @@ __global__ void __launch_bounds__(256, 2) attn_span_kernel(
                     const uint32_t hi = *reinterpret_cast<const uint16_t*>(col + (2 * e2 + 1) * AS_VROW);
                     vw[e2] = lo | (hi << 16);
                 }
-                const bf16x8 vfrag = __builtin_bit_cast(bf16x8, make_uint4(vw[0], vw[1], vw[2], vw[3]));
+                vfrag[dt] = __builtin_bit_cast(bf16x8, make_uint4(vw[0], vw[1], vw[2], vw[3]));
+            }
+#pragma unroll
+            for (int term = 1; term >= 0; --term) {  // the weights' second terms, then their first
+                const uint8_t* pt = p_lds + (ks * NQ + c) * AS_PROW + term * 64 + a * 16;
+                bf16x8 pfrag[NQT];
 #pragma unroll
                 for (int qt = 0; qt < NQT; ++qt)
-                    ot[dt][qt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vfrag, __builtin_bit_cast(bf16x8, pfrag[qt]),
-                                                                         ot[dt][qt], 0, 0, 0);
+                    pfrag[qt] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(pt + qt * 16 * AS_PROW));
+#pragma unroll
+                for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+                    for (int qt = 0; qt < NQT; ++qt)
+                        ot[dt][qt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vfrag[dt], pfrag[qt], ot[dt][qt], 0, 0, 0);
             }
         }
+    };
+    auto walk = [&](auto mode) {
+#pragma unroll
+        for (int qt = 0; qt < NQT; ++qt) {
+            m[qt] = ninf;
+            l[qt] = 0.f;
+            ot[0][qt] = ot[1][qt] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+        for (int kb = k_begin; kb < k_lim; kb += AS_KEYS) batch(mode, kb);
+    };
+    walk(std::false_type{});
+    bool strange = false;
+#pragma unroll
+    for (int qt = 0; qt < NQT; ++qt)
+#pragma unroll
+        for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) strange = strange || !(fabsf(ot[dt][qt][i]) < __builtin_inff());
+    const bool strange_here = __ballot(strange) != 0;
+    if (lane == 0) odd[wv] = strange_here ? 1 : 0;
+    __syncthreads();  // the last batch's maxima have been read
+    if ((odd[0] | odd[1] | odd[2] | odd[3]) != 0) {  // the same in all four waves
+        walk(std::true_type{});
+        __syncthreads();
     }
     // the span's state out: the sums meet across the pair's lanes and the waves
-    __syncthreads();  // the last batch's maxima have been read
 #pragma unroll
     for (int qt = 0; qt < NQT; ++qt) {
         float s = l[qt];

@@ -128,3 +128,71 @@ def test_long_spans_from_the_fused_qkv_rows(card, n0, T, Hq, Hk, S, tree, with_n
                            V1[:, keep].float().cpu().numpy(), scale)
         worst = np.abs(got[t].float().cpu().numpy().reshape(Hq, D) - ref).max() / np.abs(ref).max()
         assert worst <= 2.0**-7, (t, worst)
+
+
+# one row and several, from the fused rows and from q; one, two and four tiles of pairs; passes of more than sixteen rows
+# over spans of one batch (the one-batch kernel's two terms); few keys, whose weights are heaviest, and many
+@pytest.mark.parametrize("n0,T,Hq,Hk,S", [(9000, 1, 32, 8, 16), (20000, 1, 8, 2, 32), (100, 2, 32, 4, 1), (1500, 3, 16, 2, 4),
+                                          (6000, 8, 32, 8, 16), (700, 5, 8, 8, 3), (1536, 32, 32, 8, 13),
+                                          (300, 17, 16, 8, 3), (260, 32, 8, 2, 3), (3000, 26, 32, 8, 6), (5000, 32, 16, 2, 8)])
+def test_weights_lose_nothing_the_output_would_show(card, n0, T, Hq, Hk, S):
+    """against f64 the outputs are off by their own rounding to bf16 and no more: 2^-8 / sqrt(3) of a unit whose values lie
+    log-uniform in it, 1.66e-3 in the relative 2-norm, and a twentieth over that; weights rounded once to bf16 against a
+    batch's maximum make it 2.1e-3"""
+    D = 128
+    cap = n0 + T + 30
+    g = torch.Generator(device="cuda").manual_seed(1400 + n0 + T)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda").to(torch.bfloat16)
+    K, V, q = rnd(Hk, cap, D), rnd(Hk, cap, D), rnd(T, Hq * D)
+    n0t = torch.tensor([n0], dtype=torch.int32, device="cuda")
+    scratch = card.attn_scratch(T, Hq, Hk, D, S)
+    att = torch.zeros(T, Hq * D, dtype=torch.bfloat16, device="cuda")
+    scale = 1.0 / np.sqrt(D)
+    if T == 1:  # no norm, and a rope that leaves q and k as they are
+        cos, sin = torch.ones(cap, D, device="cuda").to(torch.bfloat16), torch.zeros(cap, D, device="cuda").to(torch.bfloat16)
+        qkv = torch.cat([q[0], rnd(2 * Hk * D)])[None]
+        card.attn_decode_qkv_span(qkv, None, None, 1e-6, cos, sin, n0t, K, V, att, Hq, Hk, D, scale, S, scratch)
+    else:
+        card.attn_decode(q, K, V, att, n0t, Hq, Hk, D, scale, S, scratch)
+    ref = torch.empty(T, Hq, D, dtype=torch.float64, device="cuda")
+    hidden = torch.ones(T, n0 + T, dtype=torch.bool, device="cuda").triu(n0 + 1)
+    for h in range(Hq):
+        k, v = K[h // (Hq // Hk), : n0 + T].double(), V[h // (Hq // Hk), : n0 + T].double()
+        s = (q.view(T, Hq, D)[:, h].double() @ k.t()) * scale
+        ref[:, h] = torch.softmax(s.masked_fill(hidden, float("-inf")), 1) @ v
+    off = float((att.double() - ref.view(T, -1)).norm() / ref.norm())
+    assert off <= 1.05 * 1.66e-3, off
+
+
+@pytest.mark.parametrize("n0,T,Hq,Hk,S", [(1000, 2, 8, 8, 2), (700, 17, 32, 8, 1), (300, 5, 16, 2, 1), (520, 20, 8, 2, 5)])
+def test_values_that_are_not_finite(card, n0, T, Hq, Hk, S):
+    """an infinite or NaN value every row sees: an output is what the vector kernels make of it - the same infinity, NaN
+    where they are NaN -, and the other outputs are finite and what they would be"""
+    D = 128
+    cap = n0 + T + 30
+    g = gen(1500 + n0 + T)
+    K = torch.randn(Hk, cap, D, generator=g).to(torch.bfloat16).cuda()
+    V = torch.randn(Hk, cap, D, generator=g).to(torch.bfloat16)
+    for slot, dim, v in ((17, 3, "inf"), (n0 - 1, 5, "-inf"), (130, 7, "nan"), (20, 9, "inf"), (21, 9, "-inf")):
+        V[0, slot, dim] = float(v)
+    V = V.cuda()
+    q = torch.randn(T, Hq * D, generator=g).to(torch.bfloat16).cuda()
+    par = torch.arange(-1, T - 1, dtype=torch.int32, device="cuda")
+    n0t = torch.tensor([n0], dtype=torch.int32, device="cuda")
+    scratch = card.attn_scratch(T, Hq, Hk, D, S)
+
+    def run(knob):
+        att = torch.zeros(T, Hq * D, dtype=torch.bfloat16, device="cuda")
+        card.set_tuning("attn_mfma", knob)
+        try:
+            card.attn_decode(q, K, V, att, n0t, Hq, Hk, D, 1.0 / np.sqrt(D), S, scratch, par=par)
+        finally:
+            card.set_tuning("attn_mfma", -1)
+        return att.float()
+
+    want, got = run(0), run(-1)
+    assert torch.equal(torch.isnan(want), torch.isnan(got)) and int(torch.isnan(want).sum()) == T * (Hq // Hk) * 2
+    assert torch.equal(want[want.isinf()], got[want.isinf()]) and int(want.isinf().sum()) == T * (Hq // Hk) * 2
+    fin = torch.isfinite(want)
+    assert bool(torch.isfinite(got[fin]).all())
+    assert float((want[fin] - got[fin]).abs().max()) <= float(want[fin].abs().max()) * 2.0**-7
