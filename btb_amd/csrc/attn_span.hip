@@ -18,7 +18,8 @@
 // alone makes. With the fold, one term / two: one row x 32 / 8 heads over 32000 keys 26.7 / 27.8 us, 8 rows over 6125
 // 15.1 / 15.9, 32 rows over 6125 34.2 / 39.6, over 23367 54.8 / 65.2 (the vector kernels 32.7, 32.8, 97, 349).
 // Two terms of unlike sign, or a zero, must not meet an infinite value: a workgroup that ends with an output that is not
-// finite walks its span once more with such values taken out of the product and added by their whole weight.
+// finite walks its span once more with such values taken out of the product and added by their whole weight, to the rows
+// that see their keys and to no other - what a later row of the pass holds never reaches an earlier one.
 //
 // The next batch's K is asked for as soon as the scores are made and its V as soon as this one's lies in LDS, into the
 // registers just freed: a batch's arithmetic (about 1 us for 64 pairs) hides the next one's trip. Two barriers a batch:
@@ -60,6 +61,14 @@ __device__ __forceinline__ uint32_t finite2(uint32_t w) {
 }
 __device__ __forceinline__ uint4 finite8(const uint4& v) {
     return make_uint4(finite2(v.x), finite2(v.y), finite2(v.z), finite2(v.w));
+}
+
+// whether a row sees the key of this slot, below `lim`; branch-free
+__device__ __forceinline__ bool sees(const RowView& v, int key, int lim) {
+    const int tb = v.tree_base >= 0 ? v.tree_base : 0x7FFFFFFF;  // the first of the pass's own slots, if a tree
+    const uint32_t named = (v.tree_mask >> min(max(key - tb, 0), 31)) & 1u;
+    const bool inside = key >= tb ? named != 0u : key >= v.k_first;
+    return (key < min(v.n, lim)) & inside;
 }
 
 // NQT tiles of 16 (row, head) pairs a workgroup: pair r is row t_base + r / G, head r % G, G = 1 << gs. TBL: the cache
@@ -242,16 +251,12 @@ __global__ void __launch_bounds__(256, 2) attn_span_kernel(
             for (int qt = 0; qt < NQT; ++qt) {
                 const int t = t_base + ((qt * 16 + c) >> gs);
                 const RowView rv = row_view_of(rows, par, min(t, T - 1), T, n0, win);
-                const int k_end = t < T ? min(rv.n, k_lim) : 0;
-                const int tb = rv.tree_base >= 0 ? rv.tree_base : 0x7FFFFFFF;  // the first of the pass's own slots, if a tree
+                const int lim = t < T ? k_lim : 0;
 #pragma unroll
                 for (int h = 0; h < 2; ++h)
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
-                        const int key = kb + 32 * wv + 16 * h + 4 * a + i;
-                        const uint32_t named = (rv.tree_mask >> min(max(key - tb, 0), 31)) & 1u;
-                        const bool inside = key >= tb ? named != 0u : key >= rv.k_first;
-                        const bool live = (key < k_end) & inside;
+                        const bool live = sees(rv, kb + 32 * wv + 16 * h + 4 * a + i, lim);
                         st[h][qt][i] = live ? st[h][qt][i] * scale_log2 : ninf;
                     }
             }
@@ -328,6 +333,10 @@ __global__ void __launch_bounds__(256, 2) attn_span_kernel(
         }
         __syncthreads();
         if constexpr (CAREFUL) {
+            RowView see[NQT];
+#pragma unroll
+            for (int qt = 0; qt < NQT; ++qt)
+                see[qt] = row_view_of(rows, par, min(t_base + ((qt * 16 + c) >> gs), T - 1), T, n0, win);
 #pragma unroll 1
             for (int key = 0; key < AS_KEYS; ++key)
 #pragma unroll
@@ -339,6 +348,7 @@ __global__ void __launch_bounds__(256, 2) attn_span_kernel(
                         if ((v & 0x7F80u) != 0x7F80u) continue;
 #pragma unroll
                         for (int qt = 0; qt < NQT; ++qt) {
+                            if (!sees(see[qt], kb + key, k_lim)) continue;
                             const uint32_t p = *reinterpret_cast<const uint16_t*>(
                                 p_lds + ((key >> 5) * NQ + qt * 16 + c) * AS_PROW + (key & 31) * 2);
                             ot[dt][qt][i] = fmaf(bits_f32(p << 16), bits_f32(v << 16), ot[dt][qt][i]);

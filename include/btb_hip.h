@@ -370,9 +370,9 @@ int32_t btb_hip_attn_decode_win(const void* q, const void* K, const void* V, voi
  * the sizes the reference's card graph allocates (btb/engine/cuda.py:1563-1583), in this library's own order - so a
  * launch by the reference's kernel name allocates nothing and a captured graph keeps reading the arrays it was recorded
  * with. `span` keys a span (a multiple of 128; the reference's key group is 512), S spans: S * span need not be the
- * cache's capacity, only reach it - every load stays on a key the row sees. The bits are btb_hip_attn_decode_win's at
- * cap = S * span, on its general kernel for spans of up to 256 keys; the reference's arrival counter is not needed (a
- * second launch folds). */
+ * cache's capacity, only reach it - no load goes past the last slot of the pass, and in a chain a row's output does not
+ * depend on the rows after it. The bits are btb_hip_attn_decode_win's at cap = S * span, on its general kernel for spans of
+ * up to 256 keys; the reference's arrival counter is not needed (a second launch folds). */
 int32_t btb_hip_attn_decode_parts(const void* q, const void* K, const void* V, void* att, const int32_t* n0,
                                   const int32_t* par, size_t T, size_t Hq, size_t Hk, size_t D, int64_t hs, int64_t rs,
                                   float scale, size_t span, size_t S, int64_t win, const int32_t* tbl, float* part_m,

@@ -196,3 +196,33 @@ def test_values_that_are_not_finite(card, n0, T, Hq, Hk, S):
     fin = torch.isfinite(want)
     assert bool(torch.isfinite(got[fin]).all())
     assert float((want[fin] - got[fin]).abs().max()) <= float(want[fin].abs().max()) * 2.0**-7
+
+
+# a chain without a tree and a tree; the pass's own rows within a batch and across two; several workgroups a kv head
+@pytest.mark.parametrize("n0,T,Hq,Hk,S,tree", [(1000, 3, 8, 2, 2, False), (300, 9, 8, 8, 1, False), (250, 17, 32, 8, 1, False),
+                                               (300, 20, 16, 2, 1, False), (120, 12, 8, 8, 1, True)])
+@pytest.mark.parametrize("what", ["inf", "nan"])
+def test_a_later_row_never_reaches_an_earlier_one(card, n0, T, Hq, Hk, S, tree, what):
+    """the last row's k and v not finite - a padding row, or one that overflowed: the rows that do not see it keep their
+    bits"""
+    D = 128
+    cap = n0 + T + 30
+    g = gen(1600 + n0 + T)
+    K = torch.randn(Hk, cap, D, generator=g).to(torch.bfloat16).cuda()
+    V = torch.randn(Hk, cap, D, generator=g).to(torch.bfloat16).cuda()
+    q = torch.randn(T, Hq * D, generator=g).to(torch.bfloat16).cuda()
+    par = torch.tensor([-1] + [0] * (T - 1), dtype=torch.int32, device="cuda") if tree else None
+    n0t = torch.tensor([n0], dtype=torch.int32, device="cuda")
+    scratch = card.attn_scratch(T, Hq, Hk, D, S)
+
+    def run():
+        att = torch.zeros(T, Hq * D, dtype=torch.bfloat16, device="cuda")
+        card.attn_decode(q, K, V, att, n0t, Hq, Hk, D, 1.0 / np.sqrt(D), S, scratch, par=par)
+        return att
+
+    want = run()
+    V[:, n0 + T - 1] = float(what)
+    K[:, n0 + T - 1] = float(what)
+    got = run()
+    assert torch.equal(got[: T - 1], want[: T - 1])
+    assert not bool(torch.isfinite(got[T - 1].float()).any())
