@@ -161,7 +161,7 @@ __global__ void __launch_bounds__(256) attn_decode_mfma_kernel(
     // the keys any of the workgroup's rows may see end at n_max (a chain's last row, or the whole pass for a tree)
     const int n_max = par != nullptr ? n0 + T : n0 + t_end;
     const int k_lim = min(n_max, k_begin + AM_SPAN);
-    const uint32_t rows = tree_rows(parent, T);
+    const TreeRows rows = tree_rows(parent, T, win);
     if constexpr (QKV) {
         auto tables = [&](int id, HeadTile& h) {
             const int t = min(task_row(id), T - 1);
@@ -254,7 +254,7 @@ __global__ void __launch_bounds__(256) attn_decode_mfma_kernel(
     for (int qt = 0; qt < NQT; ++qt) {
         const int r = qt * 16 + c, t = t_base + r / G;
         const bool row_ok = t < T;
-        const RowView rv = row_view_of(rows, par, min(t, T - 1), T, n0, win);
+        const RowView rv = row_view_of(rows, par != nullptr, min(t, T - 1), T, n0, win);
         // branch-free: this runs once a workgroup, and a path that short is bound by how fast its code arrives
         const int k_end = row_ok ? min(rv.n, k_lim) : 0;
         const int tb = rv.tree_base >= 0 ? rv.tree_base : 0x7FFFFFFF;  // the first of the pass's own slots, if a tree

@@ -130,7 +130,22 @@ __global__ void __launch_bounds__(256, 2) attn_span_kernel(
     const int k_lim = min(n_max, k_begin + span);
     const int last = max(QKV ? min(k_lim - 1, cap - 1) : k_lim - 1, 0);
     const bool own_here = QKV && k_begin < n0 + T && n0 < k_begin + span;  // some of the pass's own slots lie in this span
-    const bool any = k_begin < k_lim;
+    // Under a window the walk starts with the first batch that any of the workgroup's rows sees
+    TreeRows rows;
+    int k_walk = k_begin;
+    if (!QKV && win > 0) {  // uniform
+        rows = tree_rows(parent, T, win);
+        int first = n0 + t_base + 1;
+        if (par != nullptr) {
+            const int r = lane & 31;
+            first = r >= t_base && r < min(T, t_base + TPW) ? n0 + rows.path : n0 + T;
+#pragma unroll
+            for (int d = 1; d < 32; d <<= 1) first = min(first, lane_value(first, lane ^ d));
+        }
+        first = min(max(first - win, 0), n0);  // (the pass's own slots are all seen, each by its row)
+        k_walk += max(first - k_begin, 0) / AS_KEYS * AS_KEYS;
+    }
+    const bool any = k_walk < k_lim;
 
     uint4 qreg[NQT][4];
     if constexpr (QKV) {
@@ -193,14 +208,14 @@ __global__ void __launch_bounds__(256, 2) attn_span_kernel(
             for (int ds = 0; ds < 4; ++ds) qreg[qt][ds] = *reinterpret_cast<const uint4*>(qr + ds * 32);
         }
         if (any) {
-            request_k(k_begin, last);
-            request_v(k_begin, last);
+            request_k(k_walk, last);
+            request_v(k_walk, last);
         }
     }
 
     f32x4 ot[2][NQT];      // O^T tile [dt][qt], lane: pair c of tile qt, dims 32 wv + 16 dt + 4 a .. + 3
     float m[NQT], l[NQT];  // pair c's running maximum (the same in its lanes of every wave), the lane's share of its sum
-    const uint32_t rows = tree_rows(parent, T);  // while the first batch travels
+    if (QKV || win <= 0) rows = tree_rows(parent, T, 0);  // while the first batch travels
     // one batch of keys; CAREFUL: values that are not finite are taken out of the product and added by their whole weight
     auto batch = [&](auto mode, int kb) {
         constexpr bool CAREFUL = decltype(mode)::value;
@@ -250,7 +265,7 @@ __global__ void __launch_bounds__(256, 2) attn_span_kernel(
 #pragma unroll
             for (int qt = 0; qt < NQT; ++qt) {
                 const int t = t_base + ((qt * 16 + c) >> gs);
-                const RowView rv = row_view_of(rows, par, min(t, T - 1), T, n0, win);
+                const RowView rv = row_view_of(rows, par != nullptr, min(t, T - 1), T, n0, win);
                 const int lim = t < T ? k_lim : 0;
 #pragma unroll
                 for (int h = 0; h < 2; ++h)
@@ -336,7 +351,7 @@ __global__ void __launch_bounds__(256, 2) attn_span_kernel(
             RowView see[NQT];
 #pragma unroll
             for (int qt = 0; qt < NQT; ++qt)
-                see[qt] = row_view_of(rows, par, min(t_base + ((qt * 16 + c) >> gs), T - 1), T, n0, win);
+                see[qt] = row_view_of(rows, par != nullptr, min(t_base + ((qt * 16 + c) >> gs), T - 1), T, n0, win);
 #pragma unroll 1
             for (int key = 0; key < AS_KEYS; ++key)
 #pragma unroll
@@ -400,7 +415,7 @@ __global__ void __launch_bounds__(256, 2) attn_span_kernel(
             l[qt] = 0.f;
             ot[0][qt] = ot[1][qt] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
-        for (int kb = k_begin; kb < k_lim; kb += AS_KEYS) batch(mode, kb);
+        for (int kb = k_walk; kb < k_lim; kb += AS_KEYS) batch(mode, kb);
     };
     walk(std::false_type{});
     bool strange = false;

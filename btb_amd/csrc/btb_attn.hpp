@@ -553,36 +553,67 @@ __device__ __forceinline__ RowView row_view(const int32_t* __restrict__ par, int
     return v;
 }
 
-// The same for many (row, head) pairs a wave without a window: every row's ancestors at once, lane l holding those of row
-// l % 32. Walking par hop by hop is a chain of dependent loads per pair - a chunk of a prompt is a chain of 32 rows, 64
-// hops a tile of pairs: 24 of the 36.8 us of its attention (32 rows x 32 / 8 heads over 1536 keys). Here each lane loads
-// its row's parent once and the sets double in five exchanges: after k of them a lane knows its first 2^k ancestors.
-// A parent outside 0 .. T - 1 is none; T <= 32. All 64 lanes call.
+// The same for many (row, head) pairs a wave: every row's ancestors at once, lane l holding those of row l % 32. Walking
+// par hop by hop is a chain of dependent loads per pair - a chunk of a prompt is a chain of 32 rows, 64 hops a tile of
+// pairs: 24 of the 36.8 us of its attention (32 rows x 32 / 8 heads over 1536 keys), and once a batch of keys where a span
+// is walked. Here each lane loads its row's parent once and the sets double in five exchanges: after k of them a lane
+// knows its first 2^k ancestors. Under a window a row sees itself and its first win - 1 ancestors: the sets of the window's
+// bits, one behind the other (a tree of 32 rows over 8000 keys, spans of 1024, a window of 1024: 282 -> 63 us, of which the
+// batches before the window, not walked any more, are the most). A parent outside 0 .. T - 1 is none; T <= 32 where par is
+// given. All 64 lanes call.
+struct TreeRows {
+    uint32_t mask;  // the pass's rows that row l % 32 sees, itself among them
+    int path;       // how many rows its path from the root holds (32 at most): it stands at *n0 + path - 1
+};
 __device__ __forceinline__ int tree_parent(const int32_t* __restrict__ par, int T) {  // ask early, use in tree_rows
     const int r = (int)(threadIdx.x & 31);
     return par != nullptr ? par[min(r, T - 1)] : -1;
 }
-__device__ __forceinline__ uint32_t tree_rows(int parent, int T) {
+__device__ __forceinline__ int lane_value(int v, int lane) { return __builtin_amdgcn_ds_bpermute(max(lane, 0) << 2, v); }
+__device__ __forceinline__ TreeRows tree_rows(int parent, int T, int win) {
     const int r = (int)(threadIdx.x & 31);
     int up = r < T && parent >= 0 && parent < T ? parent : -1;  // the ancestor 2^k hops up
-    uint32_t mask = 1u << r;
+    TreeRows own{1u << r, 1};  // the first 2^k rows of the path, counted from the row up
+    if (win > 0) {  // uniform
+        uint32_t seen = 0u;
+        int at = r;  // the next row of the path that the window has not taken yet
+#pragma unroll
+        for (int k = 0; k < 5; ++k) {
+            const uint32_t theirs = (uint32_t)lane_value((int)own.mask, at);
+            const int next = lane_value(up, at);
+            if ((win >> k) & 1) {
+                seen |= at >= 0 ? theirs : 0u;
+                at = at >= 0 ? next : -1;
+            }
+            const uint32_t mask2 = (uint32_t)lane_value((int)own.mask, up);
+            const int path2 = lane_value(own.path, up), up2 = lane_value(up, up);
+            own.mask |= up >= 0 ? mask2 : 0u;
+            own.path += up >= 0 ? path2 : 0;
+            up = up >= 0 ? up2 : -1;
+        }
+        if (win < 32) own.mask = seen;
+        return own;
+    }
 #pragma unroll
     for (int k = 0; k < 5; ++k) {
-        const uint32_t theirs = (uint32_t)__builtin_amdgcn_ds_bpermute(max(up, 0) << 2, (int)mask);
-        const int next = __builtin_amdgcn_ds_bpermute(max(up, 0) << 2, up);
-        mask |= up >= 0 ? theirs : 0u;
-        up = up >= 0 ? next : -1;
+        const uint32_t mask2 = (uint32_t)lane_value((int)own.mask, up);
+        const int up2 = lane_value(up, up);
+        own.mask |= up >= 0 ? mask2 : 0u;
+        up = up >= 0 ? up2 : -1;
     }
-    return mask;
+    return own;
 }
 // row t's view given tree_rows' sets (`rows`: this lane's); all 64 lanes call
-__device__ __forceinline__ RowView row_view_of(uint32_t rows, const int32_t* __restrict__ par, int t, int T, int n0, int win) {
-    if (win > 0) return row_view(par, t, T, n0, win);  // uniform
+__device__ __forceinline__ RowView row_view_of(const TreeRows& rows, bool tree, int t, int T, int n0, int win) {
     RowView v;
-    v.tree_base = par != nullptr ? n0 : -1;
-    v.n = par != nullptr ? n0 + T : n0 + t + 1;
-    v.tree_mask = (uint32_t)__builtin_amdgcn_ds_bpermute((t & 31) << 2, (int)rows);
+    v.tree_base = tree ? n0 : -1;
+    v.n = tree ? n0 + T : n0 + t + 1;
+    v.tree_mask = (uint32_t)lane_value((int)rows.mask, t & 31);
     v.k_first = 0;
+    if (win > 0) {  // uniform
+        const int path = lane_value(rows.path, t & 31);
+        v.k_first = max(n0 + (tree ? path : t + 1) - win, 0);
+    }
     return v;
 }
 

@@ -226,3 +226,41 @@ def test_a_later_row_never_reaches_an_earlier_one(card, n0, T, Hq, Hk, S, tree, 
     got = run()
     assert torch.equal(got[: T - 1], want[: T - 1])
     assert not bool(torch.isfinite(got[T - 1].float()).any())
+
+
+# windows shorter than the path, of a power of two and around it, as long as the pass; whole spans and the first batches of
+# one before every row's window; deep and bushy trees and a chain; both matrix-core kernels (spans of 128 keys: one batch)
+@pytest.mark.parametrize("n0,T,Hq,Hk,S,shape,win", [
+    (900, 32, 8, 8, 2, "deep", 1), (900, 32, 8, 8, 2, "deep", 7), (900, 32, 16, 2, 1, "deep", 31), (900, 32, 8, 2, 3, "deep", 32),
+    (900, 32, 8, 2, 3, "deep", 33), (700, 20, 32, 8, 2, "bushy", 4), (700, 9, 8, 8, 6, "bushy", 130), (700, 9, 8, 2, 6, "deep", 16),
+    (900, 40, 8, 8, 2, None, 5), (900, 17, 32, 8, 8, None, 200), (20, 6, 8, 1, 1, "deep", 3)])
+def test_windows_over_trees(card, n0, T, Hq, Hk, S, shape, win):
+    D = 128
+    cap = n0 + T + 60
+    span = -(-(-(-cap // S)) // 128) * 128
+    g = gen(1700 + n0 + T + win)
+    K = torch.randn(Hk, cap, D, generator=g).to(torch.bfloat16)
+    V = torch.randn(Hk, cap, D, generator=g).to(torch.bfloat16)
+    q = (2 * torch.randn(T, Hq * D, generator=g)).to(torch.bfloat16)
+    par = None
+    if shape == "deep":  # a long path with a leaf beside every fifth row
+        par = [-1] + [t - 2 if t % 5 == 4 else t - 1 for t in range(1, T)]
+        par = [p if p < 0 or p % 5 != 4 else p - 1 for p in par]
+    elif shape == "bushy":
+        par = [-1] + [int(torch.randint(-1, t, (1,), generator=g)) for t in range(1, T)]
+    seen = [seen_by(t, n0, par, win) for t in range(T)]
+    first = min(min(s) for s in seen)
+    if span > 128:  # slots that the window has left behind, and what lies past the pass, hold anything
+        K[:, :first], V[:, :first] = float("nan"), float("nan")
+    K[:, n0 + T:], V[:, n0 + T:] = float("nan"), float("nan")
+    part = None if par is None else torch.tensor(par, dtype=torch.int32, device="cuda")
+    scale = 1.0 / np.sqrt(D)
+    att = torch.zeros(T, Hq * D, dtype=torch.bfloat16, device="cuda")
+    card.attn_decode(q.cuda(), K.cuda(), V.cuda(), att, torch.tensor([n0], dtype=torch.int32, device="cuda"), Hq, Hk, D,
+                     scale, S, card.attn_scratch(T, Hq, Hk, D, S), par=part, win=win)
+    got = att.float().cpu().numpy()
+    for t in range(T):
+        want = od.attention(q[t].float().numpy().reshape(Hq, D), K[:, seen[t]].float().numpy(),
+                            V[:, seen[t]].float().numpy(), scale)
+        worst = np.abs(got[t].reshape(Hq, D) - want).max() / np.abs(want).max()
+        assert worst <= 2.0**-7, (t, worst)  # weights and outputs in bf16, as above
