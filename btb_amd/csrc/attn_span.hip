@@ -4,7 +4,7 @@
 // long cache is cut into as many spans as fill the chip and not into one per 128 keys, whose partial states (520 bytes
 // a (row, head, span), written and read back) come to outweigh the keys.
 //
-// A workgroup: one kv head, one span, up to 64 of the pass's (row, head) pairs; wider passes are more workgroups (the
+// A workgroup: one kv head, one span, up to 32 of the pass's (row, head) pairs; wider passes are more workgroups (the
 // z axis), which read the same keys out of the last-level cache. Four waves; the products' layout is attn_mfma.hip's:
 // scores S^T = K Q^T with wave w on keys 32 w .. + 31 of the batch, outputs O^T = V^T P^T with wave w on dims 32 w ..
 // + 31. Between batches a pair's maximum moves in every lane that holds the pair, so the rescaling needs no exchange; the
@@ -15,18 +15,18 @@
 // the maximum of its own stream of 16 keys or fewer a batch, so the heaviest of them are 1 and exact, and against f64 their
 // outputs lie 1.8e-3 to 2.2e-3 off (relative 2-norm, normal q and k, 100 to 32000 keys) where weights taken against a whole
 // batch's maximum and rounded once lie 2.1e-3 to 2.2e-3 off; with two terms 1.66e-3, what rounding the outputs to bf16
-// alone makes. With the fold, one term / two: one row x 32 / 8 heads over 32000 keys 26.7 / 27.8 us, 8 rows over 6125
-// 15.1 / 15.9, 32 rows over 6125 34.2 / 39.6, over 23367 54.8 / 65.2 (the vector kernels 32.7, 32.8, 97, 349).
+// alone makes. The second product costs 3 to 8 %: 8 rows x 32 / 8 heads over 6125 keys, with the fold, 15.2 -> 16.4 us
+// (the vector kernel 32.8).
 // Two terms of unlike sign, or a zero, must not meet an infinite value: a workgroup that ends with an output that is not
 // finite walks its span once more with such values taken out of the product and added by their whole weight, to the rows
 // that see their keys and to no other - what a later row of the pass holds never reaches an earlier one.
 //
 // The next batch's K is asked for as soon as the scores are made and its V as soon as this one's lies in LDS, into the
-// registers just freed: a batch's arithmetic (about 1 us for 64 pairs) hides the next one's trip. Two barriers a batch:
+// registers just freed: a batch's arithmetic (2.0 us for 16 pairs, 2.5 for 32) hides the next one's trip. Two barriers a batch:
 // the maxima, which are also the sign that the last batch's V and weights have been read, and the weights.
 //
-// Bound: HBM for the keys (one read of the span), then the vector ALUs' softmax: 10 instructions a score against
-// a quarter of an MFMA.
+// Bound: a batch's chain of phases - scores, maxima, weights, outputs, a barrier between - at one or two workgroups a CU;
+// one row x 32 / 8 heads over 32000 keys reads its 131 MB in 27.8 us with the fold, 4.7 TB/s.
 
 #include "btb_attn.hpp"
 #include "btb_common.hpp"
@@ -43,14 +43,12 @@ constexpr int AS_KEYS = 128;  // keys a batch
 constexpr int AS_VROW = 272;  // bytes a V row takes in LDS: 256 + 16, so the eight rows a fragment read touches differ in bank
 constexpr int AS_PROW = 144;  // bytes a pair's 32 weights of a step take: 64 a term and 16, so that pairs differ in bank
 constexpr int AS_HROW = 272;  // bytes a prepared q, k or v row takes in LDS: as a V row
-constexpr int AS_VOWN = 16;   // a pass of more rows reads its own v rows out of the fused rows when it needs them: with
-                              // them in LDS too (8.7 KB at 32 rows) a CU would hold one workgroup and not two
 
 // own: the pass's own rows kept in LDS (their k, then their v), none where q is given
 __host__ __device__ constexpr size_t as_lds_bytes(int NQT, int own) {
     const size_t NQ = 16 * (size_t)NQT;
     return (size_t)AS_KEYS * AS_VROW + 4 * NQ * sizeof(float) + 4 * sizeof(int) + 4 * NQ * AS_PROW +
-           (size_t)(own > AS_VOWN ? own : 2 * own) * AS_HROW;
+           2 * (size_t)own * AS_HROW;
 }
 
 // eight bf16 values with those that are not finite as zeros
@@ -177,7 +175,7 @@ __global__ void __launch_bounds__(256, 2) attn_span_kernel(
 #pragma unroll
                     for (int ds = 0; ds < 4; ++ds) {
                         *reinterpret_cast<uint4*>(kn_lds + tr * AS_HROW + ds * 64 + a * 16) = out[ds];
-                        if (T <= AS_VOWN) *reinterpret_cast<uint4*>(vn_lds + tr * AS_HROW + ds * 64 + a * 16) = h.vrow[ds];
+                        *reinterpret_cast<uint4*>(vn_lds + tr * AS_HROW + ds * 64 + a * 16) = h.vrow[ds];
                     }
                     // (a slot at or past the cache's capacity is not written: the caller has let the cache overflow)
                     if (blockIdx.z == gridDim.z - 1 && slot >= k_begin && slot < min(k_begin + span, cap)) {
@@ -297,18 +295,12 @@ __global__ void __launch_bounds__(256, 2) attn_span_kernel(
         }
         if constexpr (QKV) {
             if (own) {  // the rows of the pass among them, by the threads that have just written their places
-                const uint16_t* v_own = x.qkv + (size_t)(Hq + Hk + g) * D + (tid & 15) * 8;
 #pragma unroll
                 for (int i = 0; i < 8; ++i) {
                     const int key = kb + (tid >> 4) + 16 * i, tr = key - n0;
-                    if (tr >= 0 && tr < T && key < k_lim) {
-                        uint4 v;
-                        if (T <= AS_VOWN)
-                            v = *reinterpret_cast<const uint4*>(vn_lds + tr * AS_HROW + (tid & 15) * 16);
-                        else
-                            v = *reinterpret_cast<const uint4*>(v_own + (size_t)tr * (Hq + 2 * Hk) * D);
-                        *reinterpret_cast<uint4*>(v_lds + (key - kb) * AS_VROW + (tid & 15) * 16) = v;
-                    }
+                    if (tr >= 0 && tr < T && key < k_lim)
+                        *reinterpret_cast<uint4*>(v_lds + (key - kb) * AS_VROW + (tid & 15) * 16) =
+                            *reinterpret_cast<const uint4*>(vn_lds + tr * AS_HROW + (tid & 15) * 16);
                 }
             }
         }
@@ -481,6 +473,15 @@ static int32_t launch_span(const void* q, const void* K, const void* V, const in
 
 static int group_shift(size_t G) { return G == 1 ? 0 : G == 2 ? 1 : G == 4 ? 2 : G == 8 ? 3 : -1; }
 
+// Tiles of 16 pairs a workgroup takes: two, one where the pass has no more or where workgroups of one do not outnumber the
+// CUs - a batch is 2.0 us for one tile, 2.5 for two. (8 rows x 32 / 8 heads over 14000 keys, one tile / two: 16 spans, 256
+// workgroups of one, 22.6 / 26.4 us; 21 spans, 336 workgroups of one, 27.0 / 22.5. Four tiles want 360 registers, a
+// workgroup a CU, and lose everywhere: 32 rows over 14000 keys, 16 spans, 64.2 / 40.2 / 43.7.) The bits are the same.
+static int tiles_of(size_t T, size_t Hk, int gs, size_t S) {
+    const size_t rows = 16u >> gs;
+    return T <= rows || Hk * S * ((T + rows - 1) / rows) <= (size_t)device_info().cus ? 1 : 2;
+}
+
 // whether a pass takes this kernel: several rows, 1, 2, 4 or 8 query heads a kv head
 bool attn_span_fits(size_t T, size_t G) { return T >= 2 && group_shift(G) >= 0 && tuning("attn_mfma") != 0; }
 
@@ -488,19 +489,16 @@ bool attn_span_fits(size_t T, size_t G) { return T >= 2 && group_shift(G) >= 0 &
 int32_t attn_decode_span(const void* q, const void* K, const void* V, const int32_t* n0, const int32_t* par, size_t T,
                          size_t Hq, size_t Hk, long long hs, long long rs, float scale_log2, float* part_m, float* part_l,
                          float* part_acc, size_t S, int span, int win, const int32_t* tbl, hipStream_t st) {
-    const size_t pairs = T * (Hq / Hk);  // of one kv head
-    const int gs = group_shift(Hq / Hk);
+    const int gs = group_shift(Hq / Hk), tiles = tiles_of(T, Hk, gs, S);
 #define AS(NN, TBL)                                                                                                      \
     return launch_span<NN, TBL, false>(q, K, V, n0, par, T, Hq, Hk, gs, hs, rs, scale_log2, part_m, part_l, part_acc, S, \
                                        span, win, tbl, 0, AmQkv{}, st)
     if (tbl != nullptr) {
-        if (pairs <= 16) AS(1, true);
-        if (pairs <= 32) AS(2, true);
-        AS(4, true);
+        if (tiles == 1) AS(1, true);
+        AS(2, true);
     }
-    if (pairs <= 16) AS(1, false);
-    if (pairs <= 32) AS(2, false);
-    AS(4, false);
+    if (tiles == 1) AS(1, false);
+    AS(2, false);
 #undef AS
 }
 
@@ -508,14 +506,12 @@ int32_t attn_decode_span(const void* q, const void* K, const void* V, const int3
 int32_t attn_decode_span_qkv(const AmQkv& x, const int32_t* n0, const int32_t* par, size_t T, size_t Hq, size_t Hk,
                              long long hs, long long rs, float scale_log2, float* part_m, float* part_l, float* part_acc,
                              size_t S, int span, size_t cap, hipStream_t st) {
-    const size_t pairs = T * (Hq / Hk);
-    const int gs = group_shift(Hq / Hk), capi = (int)(cap < 0x7FFFFFFFu ? cap : 0x7FFFFFFFu);
+    const int gs = group_shift(Hq / Hk), tiles = tiles_of(T, Hk, gs, S), capi = (int)(cap < 0x7FFFFFFFu ? cap : 0x7FFFFFFFu);
 #define AS(NN)                                                                                                          \
     return launch_span<NN, false, true>(nullptr, x.Kw, x.Vw, n0, par, T, Hq, Hk, gs, hs, rs, scale_log2, part_m, part_l, \
                                         part_acc, S, span, 0, nullptr, capi, x, st)
-    if (pairs <= 16) AS(1);
-    if (pairs <= 32) AS(2);
-    AS(4);
+    if (tiles == 1) AS(1);
+    AS(2);
 #undef AS
 }
 

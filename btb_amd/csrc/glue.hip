@@ -758,6 +758,18 @@ size_t btb_hip_attn_scratch_floats(size_t T, size_t Hq, size_t Hk, size_t D, siz
     return T * Hq * S * (2 + D);
 }
 
+// Whether a pass's spans are walked on the matrix cores: from four query heads a kv head on always; with one or two, whose
+// vector arithmetic is less, once the vector kernels' workgroups, one a (kv head, span, row), outnumber the CUs or nearly.
+// Measured on MI355X with the fold, us, vector kernel / this: 16 / 8 heads, spans of 256, 96 workgroups 10.2 / 10.7, 256
+// 9.2 / 10.3, 384 10.2 / 10.2; spans of 1024, 48 workgroups 20.0 / 21.0, 192 21.3 / 21.1, 256 26.4 / 21.8; 8 / 8 heads, spans
+// of 2048, 16 workgroups 29.3 / 34.4, 256 51.6 / 35.5 (of 8 spans; of 2, whose rows share their keys, 32.4 / 34.8).
+static bool span_walk_fits(size_t T, size_t G, size_t Hk, size_t S, int span) {
+    if (!attn_span_fits(T, G)) return false;
+    const size_t cus = (size_t)device_info().cus, wgs = Hk * S * T;
+    if (G > 2) return true;
+    return span <= 256 ? wgs > cus : G == 1 ? wgs >= cus : 4 * wgs >= 3 * cus;
+}
+
 // `work` is the caller's workspace, or nullptr for the library's own static array on the current device
 // `parts`: the caller's own three state arrays (part_m, part_l [T Hq S], part_acc [T Hq S D]) in place of one workspace;
 // the call then takes spans of `cap / S` keys exactly and only the kernel whose loads stay on live keys, so `cap` need
@@ -818,8 +830,8 @@ static int32_t attn_decode_any(const void* q, const void* K, const void* V, void
     launch_merge<GG>(st, att, T, Hq, Hk, S, part_m, part_l, part_acc, rw)
     // Several rows and spans of 128 keys: the matrix cores, every row of the pass that shares a kv head in one workgroup
     // (attn_mfma.hip). A pass of 8 rows over 4096 keys: 22.7 us a layer on the vector kernel below (spans of one or two
-    // batches of keys, asked for at once and kept in registers, a workgroup a row), which stays for spans of 256 keys
-    // and behind the knob attn_mfma = 0.
+    // batches of keys, asked for at once and kept in registers, a workgroup a row), which stays for spans of 256 keys and
+    // two query heads a kv head where span_walk_fits leaves them, and behind the knob attn_mfma = 0.
     if (parts == nullptr && attn_mfma_fits(T, G, span)) {
         const int32_t rc = attn_decode_mfma(q, K, V, n0, par, T, Hq, Hk, (long long)hs, (long long)rs, scale_log2, part_m,
                                             part_l, part_acc, S, cap, (int)win, tbl, st);
@@ -830,7 +842,7 @@ static int32_t attn_decode_any(const void* q, const void* K, const void* V, void
     }
     // Longer spans, and 1 or 8 query heads a kv head: the matrix cores too, a span walked in batches (attn_span.hip). With
     // the caller's state arrays spans of one and two batches stay on the general kernel.
-    if (rw == nullptr && (parts == nullptr || span > 256) && attn_span_fits(T, G) && al(part_acc, 16)) {
+    if (rw == nullptr && (parts == nullptr || span > 256) && span_walk_fits(T, G, Hk, S, span) && al(part_acc, 16)) {
         const int32_t rc = attn_decode_span(q, K, V, n0, par, T, Hq, Hk, (long long)hs, (long long)rs, scale_log2, part_m,
                                             part_l, part_acc, S, span, (int)win, tbl, st);
         if (rc != OK) return rc;

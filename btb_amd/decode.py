@@ -84,13 +84,13 @@ def rope_tables(cfg: StackConfig, positions: int, device: Any) -> tuple[torch.Te
 
 def pass_spans(cus: int, T: int, Hq: int, Hk: int, cap: int) -> int:
     """how many spans the attention of a pass of T rows cuts a cache of `cap` slots into. Its workgroup walks a span in
-    batches of 128 keys for up to 64 (row, head) pairs of a kv head, so: a workgroup a CU, spans whole batches. Where a
-    kv head's pairs take several workgroups, which read the same keys, and spans stay at 512 keys or more, two a CU.
-    Measured on MI355X with the fold, us a layer: 8 rows x 32 / 8 heads, 4096 keys: 18 spans 11.9, 9 15.8, 36 15.1; 2
-    rows, 32000 keys: 31 spans 30.8, 16 46.5, 56 32.7; 13 rows x 32 / 4, 6125 keys: 27 spans 19.9, 53 22.6; two a CU: 26
-    rows x 32 / 8, 23367 keys: 29 spans 54.5, 16 61.4, 51 64.8; 32 rows x 64 / 8, 8000 keys: 14 spans 42.6, 8 47.7."""
+    batches of 128 keys for up to 32 (row, head) pairs of a kv head, so: a workgroup a CU, spans whole batches. Where a kv
+    head's pairs take several workgroups, which read the same keys, and spans stay at 512 keys or more, two a CU.
+    Measured on MI355X with the q / k norm and the fold, us a layer, at a workgroup a CU / at two: 8 rows x 32 / 8 heads,
+    6125 keys 16.4 / 17.8, 32000 32.1 / 32.0; 17 rows x 32 / 8, 3000 keys 18.3 / 19.4, 6125 25.8 / 24.1, 23367 58.6 / 47.8;
+    32 rows x 32 / 8, 6125 31.0 / 28.9, 23367 70.5 / 57.8; 16 rows x 32 / 4, 6125 20.7 / 21.7, 32000 52.0 / 45.8."""
     G = Hq // Hk
-    z = -(-T * G // 64)
+    z = -(-T * G // 32)
     most = 1024 // G  # the fold's limit
 
     def keys(per_cu: int) -> int:

@@ -133,7 +133,7 @@ def test_long_spans_from_the_fused_qkv_rows(card, n0, T, Hq, Hk, S, tree, with_n
 # one row and several, from the fused rows and from q; one, two and four tiles of pairs; passes of more than sixteen rows
 # over spans of one batch (the one-batch kernel's two terms); few keys, whose weights are heaviest, and many
 @pytest.mark.parametrize("n0,T,Hq,Hk,S", [(9000, 1, 32, 8, 16), (20000, 1, 8, 2, 32), (100, 2, 32, 4, 1), (1500, 3, 16, 2, 4),
-                                          (6000, 8, 32, 8, 16), (700, 5, 8, 8, 3), (1536, 32, 32, 8, 13),
+                                          (6000, 8, 32, 8, 16), (700, 12, 8, 8, 3), (1536, 32, 32, 8, 13),
                                           (300, 17, 16, 8, 3), (260, 32, 8, 2, 3), (3000, 26, 32, 8, 6), (5000, 32, 16, 2, 8)])
 def test_weights_lose_nothing_the_output_would_show(card, n0, T, Hq, Hk, S):
     """against f64 the outputs are off by their own rounding to bf16 and no more: 2^-8 / sqrt(3) of a unit whose values lie
@@ -164,7 +164,7 @@ def test_weights_lose_nothing_the_output_would_show(card, n0, T, Hq, Hk, S):
     assert off <= 1.05 * 1.66e-3, off
 
 
-@pytest.mark.parametrize("n0,T,Hq,Hk,S", [(1000, 2, 8, 8, 2), (700, 17, 32, 8, 1), (300, 5, 16, 2, 1), (520, 20, 8, 2, 5)])
+@pytest.mark.parametrize("n0,T,Hq,Hk,S", [(1000, 20, 8, 8, 2), (700, 17, 32, 8, 1), (300, 5, 16, 2, 1), (520, 20, 8, 2, 5)])
 def test_values_that_are_not_finite(card, n0, T, Hq, Hk, S):
     """an infinite or NaN value every row sees: an output is what the vector kernels make of it - the same infinity, NaN
     where they are NaN -, and the other outputs are finite and what they would be"""
@@ -200,7 +200,7 @@ def test_values_that_are_not_finite(card, n0, T, Hq, Hk, S):
 
 # a chain without a tree and a tree; the pass's own rows within a batch and across two; several workgroups a kv head
 @pytest.mark.parametrize("n0,T,Hq,Hk,S,tree", [(1000, 3, 8, 2, 2, False), (300, 9, 8, 8, 1, False), (250, 17, 32, 8, 1, False),
-                                               (300, 20, 16, 2, 1, False), (120, 12, 8, 8, 1, True)])
+                                               (300, 20, 16, 2, 1, False), (300, 33, 8, 8, 1, False), (120, 12, 16, 2, 1, True)])
 @pytest.mark.parametrize("what", ["inf", "nan"])
 def test_a_later_row_never_reaches_an_earlier_one(card, n0, T, Hq, Hk, S, tree, what):
     """the last row's k and v not finite - a padding row, or one that overflowed: the rows that do not see it keep their
@@ -264,3 +264,33 @@ def test_windows_over_trees(card, n0, T, Hq, Hk, S, shape, win):
                             V[:, seen[t]].float().numpy(), scale)
         worst = np.abs(got[t].reshape(Hq, D) - want).max() / np.abs(want).max()
         assert worst <= 2.0**-7, (t, worst)  # weights and outputs in bf16, as above
+
+
+@pytest.mark.parametrize("n0,T,Hq,Hk,S,tree", [(2100, 16, 32, 8, 16, False), (3000, 21, 16, 2, 23, True), (2100, 17, 16, 8, 12, True)])
+def test_a_workgroups_tiles_change_no_bit(card, n0, T, Hq, Hk, S, tree):
+    """a kv head's rows in workgroups of two tiles of pairs (all the kv heads: more workgroups of one than CUs) and of one (the
+    kv head by itself)"""
+    D, G = 128, Hq // Hk
+    cap = n0 + T + 30
+    g = gen(1900 + n0 + T)
+    K = torch.randn(Hk, cap, D, generator=g).to(torch.bfloat16).cuda()
+    V = torch.randn(Hk, cap, D, generator=g).to(torch.bfloat16).cuda()
+    q = torch.randn(T, Hk, G * D, generator=g).to(torch.bfloat16).cuda()
+    par = [-1] + [int(torch.randint(-1, t, (1,), generator=g)) for t in range(1, T)] if tree else None
+    part = None if par is None else torch.tensor(par, dtype=torch.int32, device="cuda")
+    n0t = torch.tensor([n0], dtype=torch.int32, device="cuda")
+
+    def run(q, K, V, heads, kv_heads):
+        att = torch.zeros(T, heads * D, dtype=torch.bfloat16, device="cuda")
+        card.attn_decode(q.reshape(T, -1), K, V, att, n0t, heads, kv_heads, D, 1.0 / np.sqrt(D), S,
+                         card.attn_scratch(T, heads, kv_heads, D, S), par=part)
+        return att
+
+    both = run(q, K, V, Hq, Hk).view(T, Hk, G * D)
+    for h in range(0, Hk, max(1, Hk - 1) if G > 2 else Hk):
+        if G > 2:  # with two heads a kv head so few workgroups stay with the vector kernels
+            assert torch.equal(run(q[:, h].contiguous(), K[h : h + 1], V[h : h + 1], G, 1), both[:, h])
+    if G <= 2:
+        half = Hk // 2
+        part_of = run(q[:, :half].contiguous(), K[:half], V[:half], Hq // 2, half).view(T, half, G * D)
+        assert torch.equal(part_of, both[:, :half])
