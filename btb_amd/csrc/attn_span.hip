@@ -26,7 +26,11 @@
 // the maxima, which are also the sign that the last batch's V and weights have been read, and the weights.
 //
 // Bound: a batch's chain of phases - scores, maxima, weights, outputs, a barrier between - at one or two workgroups a CU;
-// one row x 32 / 8 heads over 32000 keys reads its 131 MB in 27.8 us with the fold, 4.7 TB/s.
+// one row x 32 / 8 heads over 32000 keys reads its 131 MB in 26.5 us with the fold, 4.9 TB/s.
+//
+// ONE, the one-row step: the spans are cut from the keys the cache holds and not from its capacity, so that a large cache
+// with few keys in it is spread over the workgroups as a full one is (35200 slots, 704 keys: 19.5 -> 10.0 us; full ones
+// as before). Its keys are asked for when *n0 is there; the row's own words travel meanwhile.
 
 #include "btb_attn.hpp"
 #include "btb_common.hpp"
@@ -73,10 +77,10 @@ __device__ __forceinline__ bool sees(const RowView& v, int key, int lim) {
 // has a row map. Every load stays on a slot one of the workgroup's rows may see, so the cache's capacity need not be
 // known and what lies past the rows is never read.
 // QKV: the rows come as the fused qkv rows, before the q / k norm and rope. A workgroup prepares the q heads of its own
-// rows, a tile of 16 a wave and turn, while the first batch's K travels (its addresses then wait for nothing: they stay
+// rows, a tile of 16 a wave, while the first batch's K travels (but for ONE its addresses wait for nothing: they stay
 // within the cache's capacity); where its span holds some of the pass's own slots *n0 .. *n0 + T - 1 it prepares the
 // pass's k heads too, takes those keys and values from there, and the last of the z axis - whose rows see all of them - writes them into the cache. T <= 32. The arithmetic is norm_rope_kv_kernel's, then this kernel's.
-template <int NQT, bool TBL, bool QKV>
+template <int NQT, bool TBL, bool QKV, bool ONE = false>
 __global__ void __launch_bounds__(256, 2) attn_span_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ K, const uint16_t* __restrict__ V,
     const int32_t* __restrict__ n0p, const int32_t* __restrict__ par, int T, int Hq, int Hk, int gs, long long hs,
@@ -84,6 +88,7 @@ __global__ void __launch_bounds__(256, 2) attn_span_kernel(
     int span, int win, const int32_t* __restrict__ tbl, int cap, AmQkv x) {
     constexpr int D = AD, NQ = 16 * NQT;
     static_assert(!(QKV && TBL), "the fused rows go with a cache without a row map");
+    static_assert(!ONE || (QKV && NQT == 1), "one row comes as its fused row");
     extern __shared__ __align__(16) uint8_t lds[];
     uint8_t* v_lds = lds;                                             // [128 keys][AS_VROW]
     float* red = reinterpret_cast<float*>(lds + AS_KEYS * AS_VROW);   // [4 waves][NQ]: maxima, at the end the sums
@@ -99,7 +104,7 @@ __global__ void __launch_bounds__(256, 2) attn_span_kernel(
     const int c = lane & 15, a = lane >> 4;
     const float ninf = bits_f32(0xff800000u);
     const int parent = tree_parent(par, T);
-    const int k_begin = sp * span;
+    int k_begin = sp * span;
     const uint16_t* Kg = K + (size_t)g * hs + a * 8;
     const uint16_t* Vg = V + (size_t)g * hs + (tid & 15) * 8;
     uint4 kreg[2][4], vreg[8];
@@ -121,8 +126,25 @@ __global__ void __launch_bounds__(256, 2) attn_span_kernel(
         }
     };
     const int in_cap = min(k_begin + span, cap) - 1;
-    if constexpr (QKV) request_k(k_begin, in_cap);
+    // QKV: the heads to prepare come as tiles of 16 - the workgroup's q heads, then the pass's k heads -, a tile a wave. What
+    // does not wait for *n0 is asked for first, a k tile's words whether or not this span turns out to hold the pass's rows.
+    constexpr int MAX_TASKS = NQT + 2;
+    static_assert(MAX_TASKS <= 4, "a tile a wave");
+    const bool k_tile = wv >= NQT;
+    const int task_row = k_tile ? (wv - NQT) * 16 + c : t_base + ((wv * 16 + c) >> gs);  // unclamped
+    const uint16_t* qkv_row = x.qkv + (size_t)min(task_row, T - 1) * (Hq + 2 * Hk) * D;
+    const uint16_t* wn = k_tile ? x.wk : x.wq;
+    HeadTile task;
+    if constexpr (QKV) {
+        const uint16_t* src = qkv_row + (size_t)(k_tile ? Hq + g : g * G + ((wv * 16 + c) & (G - 1))) * D;
+        if (wv < NQT || (wv - NQT) * 16 < T) tile_request(task, src, wn, a);
+        if constexpr (!ONE) request_k(k_begin, in_cap);
+    }
     const int n0 = *n0p;
+    if constexpr (ONE) {  // the spans of the keys there are
+        span = ((n0 + S) / S + AS_KEYS - 1) / AS_KEYS * AS_KEYS;
+        k_begin = sp * span;
+    }
     // the keys any of the workgroup's rows may see end at n_max (a chain's last row, or the whole pass for a tree)
     const int n_max = par != nullptr ? n0 + T : n0 + min(T, t_base + TPW);
     const int k_lim = min(n_max, k_begin + span);
@@ -148,34 +170,33 @@ __global__ void __launch_bounds__(256, 2) attn_span_kernel(
     uint4 qreg[NQT][4];
     if constexpr (QKV) {
         if (any) {
-            const size_t width = (size_t)(Hq + 2 * Hk) * D;
-            const int ntask = NQT + (own_here ? (T + 15) / 16 : 0);
-            for (int id = wv; id < ntask; id += 4) {  // uniform in the wave
-                const bool is_k = id >= NQT;
-                const int tr = is_k ? (id - NQT) * 16 + c : t_base + ((id * 16 + c) >> gs), t = min(tr, T - 1);
-                const uint16_t* row = x.qkv + (size_t)t * width;
-                const uint16_t* src = row + (size_t)(is_k ? Hq + g : g * G + ((id * 16 + c) & (G - 1))) * D;
-                const uint16_t* wn = is_k ? x.wk : x.wq;
-                HeadTile h;
-                tile_request(h, src, wn, a);
-                cs_sn_request(h, x.cos_t, x.sin_t, n0 + (x.depth != nullptr ? x.depth[t] : t), a);
-                const uint16_t* vsrc = is_k ? row + (size_t)(Hq + Hk + g) * D : src;
+            if constexpr (ONE) request_k(k_begin, last);
+            const bool mine = wv < NQT || (own_here && (wv - NQT) * 16 < T);  // uniform in the wave
+            if (mine) {
+                const int t = min(task_row, T - 1);
+                cs_sn_request(task, x.cos_t, x.sin_t, n0 + (x.depth != nullptr ? x.depth[t] : t), a);
+                if (k_tile) {
+                    const uint16_t* vsrc = qkv_row + (size_t)(Hq + Hk + g) * D + a * 8;
 #pragma unroll
-                for (int ds = 0; ds < 4; ++ds) h.vrow[ds] = *reinterpret_cast<const uint4*>(vsrc + ds * 32 + a * 8);
+                    for (int ds = 0; ds < 4; ++ds) task.vrow[ds] = *reinterpret_cast<const uint4*>(vsrc + ds * 32);
+                }
+            }
+            request_v(k_begin, last);
+            if (mine) {
                 float v[4][8];
-                tile_norm(h, wn != nullptr, x.eps, x.centered, v);
+                tile_norm(task, wn != nullptr, x.eps, x.centered, v);
                 uint4 out[4];
-                tile_rope(v, h, out);
-                if (!is_k) {
+                tile_rope(v, task, out);
+                if (!k_tile) {
 #pragma unroll
                     for (int ds = 0; ds < 4; ++ds)
-                        *reinterpret_cast<uint4*>(q_lds + (id * 16 + c) * AS_HROW + ds * 64 + a * 16) = out[ds];
-                } else if (tr < T) {
-                    const int slot = n0 + tr;
+                        *reinterpret_cast<uint4*>(q_lds + (wv * 16 + c) * AS_HROW + ds * 64 + a * 16) = out[ds];
+                } else if (task_row < T) {
+                    const int slot = n0 + task_row;
 #pragma unroll
                     for (int ds = 0; ds < 4; ++ds) {
-                        *reinterpret_cast<uint4*>(kn_lds + tr * AS_HROW + ds * 64 + a * 16) = out[ds];
-                        *reinterpret_cast<uint4*>(vn_lds + tr * AS_HROW + ds * 64 + a * 16) = h.vrow[ds];
+                        *reinterpret_cast<uint4*>(kn_lds + task_row * AS_HROW + ds * 64 + a * 16) = out[ds];
+                        *reinterpret_cast<uint4*>(vn_lds + task_row * AS_HROW + ds * 64 + a * 16) = task.vrow[ds];
                     }
                     // (a slot at or past the cache's capacity is not written: the caller has let the cache overflow)
                     if (blockIdx.z == gridDim.z - 1 && slot >= k_begin && slot < min(k_begin + span, cap)) {
@@ -184,12 +205,11 @@ __global__ void __launch_bounds__(256, 2) attn_span_kernel(
 #pragma unroll
                         for (int ds = 0; ds < 4; ++ds) {
                             *reinterpret_cast<uint4*>(kc + ds * 32) = out[ds];
-                            *reinterpret_cast<uint4*>(vc + ds * 32) = h.vrow[ds];
+                            *reinterpret_cast<uint4*>(vc + ds * 32) = task.vrow[ds];
                         }
                     }
                 }
             }
-            request_v(k_begin, last);
             __syncthreads();
 #pragma unroll
             for (int qt = 0; qt < NQT; ++qt)
@@ -451,14 +471,14 @@ __global__ void __launch_bounds__(256, 2) attn_span_kernel(
     }
 }
 
-template <int NQT, bool TBL, bool QKV>
+template <int NQT, bool TBL, bool QKV, bool ONE = false>
 static int32_t launch_span(const void* q, const void* K, const void* V, const int32_t* n0, const int32_t* par, size_t T,
                            size_t Hq, size_t Hk, int gs, long long hs, long long rs, float scale_log2, float* part_m,
                            float* part_l, float* part_acc, size_t S, int span, int win, const int32_t* tbl, int cap,
                            const AmQkv& x, hipStream_t st) {
     const size_t TPW = (16 * NQT) >> gs;
     const dim3 grid((unsigned)Hk, (unsigned)S, (unsigned)((T + TPW - 1) / TPW));
-    auto kern = attn_span_kernel<NQT, TBL, QKV>;
+    auto kern = attn_span_kernel<NQT, TBL, QKV, ONE>;
     const size_t lds = as_lds_bytes(NQT, QKV ? (int)T : 0);
     if (lds > 64 * 1024) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
@@ -507,11 +527,12 @@ int32_t attn_decode_span_qkv(const AmQkv& x, const int32_t* n0, const int32_t* p
                              long long hs, long long rs, float scale_log2, float* part_m, float* part_l, float* part_acc,
                              size_t S, int span, size_t cap, hipStream_t st) {
     const int gs = group_shift(Hq / Hk), tiles = tiles_of(T, Hk, gs, S), capi = (int)(cap < 0x7FFFFFFFu ? cap : 0x7FFFFFFFu);
-#define AS(NN)                                                                                                          \
-    return launch_span<NN, false, true>(nullptr, x.Kw, x.Vw, n0, par, T, Hq, Hk, gs, hs, rs, scale_log2, part_m, part_l, \
+#define AS(...)                                                                                                         \
+    return launch_span<__VA_ARGS__>(nullptr, x.Kw, x.Vw, n0, par, T, Hq, Hk, gs, hs, rs, scale_log2, part_m, part_l, \
                                         part_acc, S, span, 0, nullptr, capi, x, st)
-    if (tiles == 1) AS(1);
-    AS(2);
+    if (T == 1) AS(1, false, true, true);
+    if (tiles == 1) AS(1, false, true);
+    AS(2, false, true);
 #undef AS
 }
 

@@ -100,20 +100,41 @@ def pass_spans(cus: int, T: int, Hq: int, Hk: int, cap: int) -> int:
     return -(-cap // span)
 
 
+def step_spans(cus: int, Hq: int, Hk: int, cap: int) -> int:
+    """how many spans a one-row step's attention cuts a cache of `cap` slots into for the kernel that keeps a batch of a
+    span's keys in registers: a workgroup a CU or two, a span at least 64 keys"""
+    if Hq // Hk >= 4:
+        # it splits a kv head's query heads over workgroups of two heads, and a workgroup folds its span 128 keys at a time:
+        # about a CU's worth of (kv head, head pair, span) triples, each span a whole number of those batches (the
+        # library rounds a span up to one)
+        per = max(128, cap // max(1, cus // (Hk * (Hq // Hk // 2))) // 128 * 128)
+        return max(1, -(-cap // per))
+    return max(1, min(cap // 64, (cus + Hk - 1) // Hk, (2 * cus) // Hk))
+
+
 def step_on_spans(cus: int, Hq: int, Hk: int, cap: int) -> int:
     """the span count with which a one-row step's attention over a cache of `cap` slots walks its spans on the matrix
-    cores, 0 where it stays with the kernel that holds a span's keys in registers. One workgroup a CU takes all query
-    heads of a kv head, 64 spans at most (more take the fold's slow form). Its launch has a longer start, so it pays from
-    8192 slots on - with one or two heads a kv head, whose vector arithmetic is less, from 16384, or where the other
-    kernel's spans would be more than 64. Measured on MI355X, us a step, register kernel / this: 20 layers [2048 / 6144],
-    32 / 8 heads, 6000 keys 871 / 865, 12000 990 / 958, 24000 1209 / 1100; 32 / 4: 4000 keys 792 / 800, 8000 892 / 846, 16000
-    1030 / 916; 8 / 2: 4000 685 / 738, 8000 852 / 763; 16 / 8: 8000 851 / 855, 16000 964 / 957; 36 layers [2560 / 9728], 32 / 8,
-    32000 keys 3022 / 2715."""
+    cores, 0 where it stays with the kernel that keeps a batch of keys in registers. One workgroup a CU takes all query
+    heads of a kv head, 64 spans at most; the spans are cut from the keys there are, so a large cache with few keys is
+    spread over them too. It starts about 3 us later, and a batch of its spans costs 2.1 us where one of the other's
+    costs 1.6 to 3.6: it pays from four query heads a kv head on, where its spans are two thirds of the other's or
+    shorter and those hold three batches - and wherever the other's would be more than 64, whose fold is slow. Measured
+    on MI355X with the fold, us a layer, the other / this, the cache 2 % / 30 % / 91 % full:
+    32 / 8 heads, 6144 slots 7.2 / 10.3, 10.4 / 10.1, 10.3 / 12.4; 8192 8.9 / 9.9, 11.7 / 10.1, 12.4 / 12.1; 8800 9.0 / 9.9,
+    11.0 / 10.3, 12.6 / 14.6; 12288 8.9 / 10.3, 13.1 / 10.5, 17.2 / 15.1; 35200 14.1 / 10.0, 28.7 / 14.9, 32.2 / 26.5.
+    32 / 4, 8192 9.0 / 10.7, 11.8 / 10.6, 12.2 / 10.8; 35200 14.1 / 10.7, 29.2 / 12.7, 32.7 / 19.1.
+    16 / 4, 8192 9.3 / 10.5, 9.4 / 10.5, 9.5 / 10.6; 12288 9.3 / 10.9, 10.0 / 10.9, 15.0 / 12.8.
+    16 / 8, 16384 10.5 / 9.9, 11.1 / 11.3, 17.2 / 17.3. 8 / 2, 16384 (64 spans) 9.3 / 10.6, 9.6 / 10.5, 10.1 / 11.9; 15808
+    (124 spans) 22.0 / 10.7, 22.0 / 10.5, 23.4 / 11.8."""
     G = Hq // Hk
-    if G not in (1, 2, 4, 8) or cap < 8192 or (G <= 2 and cap < 16384 and Hk > cus // 64):
+    if G not in (1, 2, 4, 8) or cap < 8192:
         return 0
-    spans = max(1, min(64, cus // Hk))
-    spans = -(-cap // (-(-cap // (spans * 128)) * 128))
+    others = step_spans(cus, Hq, Hk, cap)
+    theirs = -(-cap // (others * 128))  # batches of 128 keys a span
+    ours = -(-cap // (max(1, min(64, cus // Hk)) * 128))
+    if others <= 64 and (G < 4 or theirs < 3 or 3 * ours > 2 * theirs):
+        return 0
+    spans = -(-cap // (ours * 128))
     return spans if Hq * spans % 2 == 0 else 0  # the states' alignment
 
 
@@ -188,12 +209,8 @@ class DecodeStep:
             attn_spans = one_row_spans
         if attn_spans is None:
             attn_spans = max(1, min(self.cap // 64, (card.sms + Hk - 1) // Hk, (2 * card.sms) // (Hk * self.T)))
-            if self.T == 1 and D == 128 and Hq // Hk >= 4:
-                # the step's own attention kernel splits a kv head's query heads over workgroups of two heads, and a
-                # workgroup folds its span 128 keys at a time: about a CU's worth of (kv head, head pair, span)
-                # triples, each span a whole number of those batches (the library rounds a span up to one)
-                per = max(128, self.cap // max(1, card.sms // (Hk * (Hq // Hk // 2))) // 128 * 128)
-                attn_spans = max(1, -(-self.cap // per))
+            if self.T == 1 and D == 128:
+                attn_spans = step_spans(card.sms, Hq, Hk, self.cap)
             elif 2 <= self.T <= 16 and D == 128 and Hq // Hk in (2, 4) and self.cap <= 128 * (1024 // (Hq // Hk)):
                 # a pass of a few rows: spans of 128 keys, one batch of the attention's sixteen streams, which a
                 # workgroup asks for at once and keeps in registers (measured at 4096 keys, ms a pass with this

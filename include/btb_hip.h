@@ -434,7 +434,8 @@ int32_t btb_hip_attn_decode_qkv_rows(const void* qkv, const void* wq, const void
 /* The same over spans of any number of 128-key batches, for a pass of 1 .. 32 rows and 1, 2, 4 or 8 query heads a kv
  * head: each workgroup walks its span with an online softmax on the matrix cores. For T >= 2 the bits are
  * btb_hip_norm_rope_kv's followed by btb_hip_attn_decode's at the same span count (where that walks spans on the matrix
- * cores too); at T = 1 the sums are the matrix cores' where btb_hip_attn_decode_qkv's are the vector units'. qkv, the norm
+ * cores too); at T = 1 the S spans are cut from the *n0 + 1 keys there are, not from cap, and the sums are the matrix cores'
+ * where btb_hip_attn_decode_qkv's are the vector units'. qkv, the norm
  * weights, the tables and workspace 16-byte aligned; `cap` is the cache's capacity. */
 int32_t btb_hip_attn_decode_qkv_span(const void* qkv, const void* wq, const void* wk, float eps, int32_t centered,
                                      const void* cos_t, const void* sin_t, const int32_t* n0, const int32_t* depth,

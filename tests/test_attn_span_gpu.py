@@ -294,3 +294,31 @@ def test_a_workgroups_tiles_change_no_bit(card, n0, T, Hq, Hk, S, tree):
         half = Hk // 2
         part_of = run(q[:, :half].contiguous(), K[:half], V[:half], Hq // 2, half).view(T, half, G * D)
         assert torch.equal(part_of, both[:, :half])
+
+
+# a cache of 9000 slots with few keys, one batch and the first of the next, as many as the spans take in one batch each and
+# one more, the last slot; 32 spans (a workgroup a CU), 7 and 1
+@pytest.mark.parametrize("n0", [0, 1, 127, 128, 4094, 4095, 4096, 8999])
+@pytest.mark.parametrize("Hq,Hk,S", [(32, 8, 32), (16, 2, 7), (4, 2, 1)])
+def test_one_row_over_the_keys_there_are(card, n0, Hq, Hk, S):
+    """`attn_decode_qkv_span` at one row cuts its spans from the keys the cache holds: against f64 attention, the row in its
+    slot and nothing else in the cache touched, whatever the empty slots hold"""
+    D, cap = 128, 9000
+    g = torch.Generator(device="cuda").manual_seed(1800 + n0)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda").to(torch.bfloat16)
+    K, V, qkv = rnd(Hk, cap, D), rnd(Hk, cap, D), rnd(1, (Hq + 2 * Hk) * D)
+    K[:, n0:], V[:, n0:] = float("nan"), float("nan")
+    K0, V0 = K.clone(), V.clone()
+    cos, sin = torch.ones(cap, D, device="cuda").to(torch.bfloat16), torch.zeros(cap, D, device="cuda").to(torch.bfloat16)
+    att = torch.zeros(1, Hq * D, dtype=torch.bfloat16, device="cuda")
+    card.attn_decode_qkv_span(qkv, None, None, 1e-6, cos, sin, torch.tensor([n0], dtype=torch.int32, device="cuda"), K, V,
+                              att, Hq, Hk, D, 1.0 / np.sqrt(D), S, card.attn_scratch(1, Hq, Hk, D, S))
+    rows = qkv[0].view(Hq + 2 * Hk, D)
+    K0[:, n0], V0[:, n0] = rows[Hq : Hq + Hk], rows[Hq + Hk :]
+    for a, b in ((K, K0), (V, V0)):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+    for h in range(Hq):
+        k, v = K[h // (Hq // Hk), : n0 + 1].double(), V[h // (Hq // Hk), : n0 + 1].double()
+        want = torch.softmax((k @ rows[h].double()) / np.sqrt(D), 0) @ v
+        off = float((att.view(Hq, D)[h].double() - want).norm() / want.norm())
+        assert off <= 2.0**-8, (h, off)  # the outputs' rounding to bf16

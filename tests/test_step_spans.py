@@ -4,7 +4,7 @@ from __future__ import annotations
 
 import pytest
 
-from btb_amd.decode import pass_spans, step_on_spans
+from btb_amd.decode import pass_spans, step_on_spans, step_spans
 
 
 @pytest.mark.parametrize("T", [2, 3, 16, 17, 32])
@@ -26,3 +26,16 @@ def test_a_steps_spans_cover_the_cache(Hq, Hk, cap):
     if S:
         span = -(-(-(-cap // S)) // 128) * 128
         assert S <= 64 and S * Hq % 2 == 0 and S * span >= cap and (S - 1) * span < cap
+
+
+@pytest.mark.parametrize("Hq,Hk", [(8, 8), (16, 8), (32, 8), (64, 8), (16, 4), (32, 4), (8, 2), (16, 2), (4, 2), (8, 4)])
+@pytest.mark.parametrize("cap", [8192, 8800, 12288, 16384, 20000, 35200, 131072])
+def test_a_step_walks_its_spans_where_they_are_short_for_it(Hq, Hk, cap):
+    """the walk's batch of keys costs up to one and a half of the register kernel's, whose own batches have to be many - or
+    its spans, which are slow to fold beyond 64"""
+    S, others = step_on_spans(256, Hq, Hk, cap), step_spans(256, Hq, Hk, cap)
+    ours, theirs = -(-cap // (min(64, 256 // Hk) * 128)), -(-cap // (others * 128))
+    pays = Hq // Hk >= 4 and theirs >= 3 and 3 * ours <= 2 * theirs
+    assert bool(S) == (others > 64 or pays)
+    if S:
+        assert -(-(-(-cap // S)) // 128) == ours
