@@ -1038,6 +1038,15 @@ int32_t btb_hip_attn_decode_qkv_rows(const void* qkv, const void* wq, const void
     return hip_status(hipGetLastError(), "attn_decode_qkv_rows launch");
 }
 
+int32_t btb_hip_attn_span_fused(size_t T, size_t Hq, size_t Hk, size_t D, size_t cap, size_t S) {
+    if (T == 0 || T > 32 || Hq == 0 || Hk == 0 || S == 0 || S > 1024 || cap == 0 || cap > 0x7FFFFFFFull - 256 ||
+        Hq % Hk != 0 || D != (size_t)ATT_D)
+        return 0;
+    const size_t G = Hq / Hk;
+    // (T * Hq * S * 2) % 4: the states' outputs stand 16-byte aligned in an aligned workspace
+    return attn_span_fits(T < 2 ? 2 : T, G) && S * G <= (size_t)ATT_MAX_STATES && (T * Hq * S * 2) % 4 == 0 ? 1 : 0;
+}
+
 int32_t btb_hip_attn_decode_qkv_span(const void* qkv, const void* wq, const void* wk, float eps, int32_t centered,
                                      const void* cos_t, const void* sin_t, const int32_t* n0, const int32_t* depth,
                                      const int32_t* par, void* K, void* V, void* att, size_t T, size_t Hq, size_t Hk,

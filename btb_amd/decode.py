@@ -204,7 +204,13 @@ class DecodeStep:
         # rows launches T times the workgroups, so it takes longer spans - two workgroups a CU in all (measured on
         # the [2560 / 9728] stack at 4096 keys: 8 rows 4.32 ms a pass with 32 spans, 3.83 with 8; 16 rows 5.6 / 4.7)
         default_spans = attn_spans is None
-        one_row_spans = step_on_spans(card.sms, Hq, Hk, self.cap) if self.T == 1 and D == 128 else 0
+        # the attention kernels that start from the fused qkv rows read 16 bytes of a norm's weight at a time (at one row the
+        # register kernel does not: it takes views at any place)
+        qk_norms = [weights.get(f"layers.{i}.{n}") for i in range(cfg.layers) for n in ("wq", "wk")]
+        aligned = all(t is None or t.data_ptr() % 16 == 0 for t in qk_norms)
+        one_row_spans = step_on_spans(card.sms, Hq, Hk, self.cap) if self.T == 1 and aligned else 0
+        if one_row_spans and not card.attn_span_fused(1, Hq, Hk, D, self.cap, one_row_spans):
+            one_row_spans = 0
         if one_row_spans and default_spans and fused is None:
             attn_spans = one_row_spans
         if attn_spans is None:
@@ -244,7 +250,7 @@ class DecodeStep:
         # shape - in the fused sequence, and in the other one too unless the caller asked for a launch per operator
         # ... and the activation in the gate / up matvec's epilogue (bf16 matrices)
         self.glu_fold = (chosen or bool(fused)) and T > 1
-        self.rows_attn_fused = (chosen or bool(fused)) and T > 1 and bool(
+        self.rows_attn_fused = (chosen or bool(fused)) and T > 1 and aligned and bool(
             card.attn_rows_fused(T, cfg.q_heads, cfg.kv_heads, cfg.head_dim, self.cap, self.S))
         # ... or, over spans of more than one batch of keys, in the attention that walks them: long caches at one row
         # (`step_on_spans`), and passes whose rows the kernel above does not take (28 rows x 32 / 8 heads over 2395 keys:
@@ -253,9 +259,9 @@ class DecodeStep:
         if self.T == 1:
             self.span_fused = default_spans and chosen and one_row_spans > 0
         else:
-            self.span_fused = (default_spans and chosen and not self.rows_attn_fused and D == 128 and self.T <= 32
-                               and Hq // Hk in (1, 2, 4, 8) and -(-self.cap // self.S) > 128
-                               and self.T * Hq * self.S % 2 == 0)
+            self.span_fused = (default_spans and chosen and not self.rows_attn_fused and aligned
+                               and -(-self.cap // self.S) > 128
+                               and card.attn_span_fused(self.T, Hq, Hk, D, self.cap, self.S))
         # the handoff to the host: token, cache length and the GPU's clock in pinned memory
         self.host_tok = torch.zeros(1, dtype=torch.int32).pin_memory()
         self.host_n0 = torch.zeros(1, dtype=torch.int32).pin_memory()

@@ -102,6 +102,7 @@ SIGNATURES: dict[str, tuple[Any, list[Any]]] = {
     "btb_hip_attn_decode_qkv_rows": (_i32, [_vp, _vp, _vp, ctypes.c_float, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
                                             _sz, _sz, _sz, _sz, ctypes.c_int64, ctypes.c_int64, ctypes.c_float, _sz,
                                             _sz, _vp, _vp]),
+    "btb_hip_attn_span_fused": (_i32, [_sz, _sz, _sz, _sz, _sz, _sz]),
     "btb_hip_attn_decode_qkv_span": (_i32, [_vp, _vp, _vp, ctypes.c_float, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
                                             _sz, _sz, _sz, _sz, ctypes.c_int64, ctypes.c_int64, ctypes.c_float, _sz,
                                             _sz, _vp, _vp]),
@@ -945,6 +946,10 @@ class HipCard(CardLaunch):
         launch less (q stays on the chip; the new K / V rows are written by the workgroups whose spans hold them)"""
         self._attn_qkv("attn_decode_qkv_rows", qkv, wq, wk, eps, cos_t, sin_t, n0, K, V, att, Hq, Hk, D, scale, S, scratch,
                        depth, par, centered)
+
+    def attn_span_fused(self, T: int, Hq: int, Hk: int, D: int, cap: int, S: int) -> bool:
+        """whether `attn_decode_qkv_span` takes a pass of this shape and the matrix-core attention is not switched off"""
+        return bool(self.lib.btb_hip_attn_span_fused(T, Hq, Hk, D, cap, S))
 
     def attn_decode_qkv_span(self, qkv: torch.Tensor, wq: torch.Tensor | None, wk: torch.Tensor | None, eps: float,
                              cos_t: torch.Tensor, sin_t: torch.Tensor, n0: torch.Tensor, K: torch.Tensor,

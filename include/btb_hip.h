@@ -436,7 +436,9 @@ int32_t btb_hip_attn_decode_qkv_rows(const void* qkv, const void* wq, const void
  * btb_hip_norm_rope_kv's followed by btb_hip_attn_decode's at the same span count (where that walks spans on the matrix
  * cores too); at T = 1 the S spans are cut from the *n0 + 1 keys there are, not from cap, and the sums are the matrix cores'
  * where btb_hip_attn_decode_qkv's are the vector units'. qkv, the norm
- * weights, the tables and workspace 16-byte aligned; `cap` is the cache's capacity. */
+ * weights, the tables and workspace 16-byte aligned; `cap` is the cache's capacity. btb_hip_attn_span_fused returns 1 for a
+ * shape this call takes, 0 otherwise and where the knob attn_mfma has switched the matrix-core attention off. */
+int32_t btb_hip_attn_span_fused(size_t T, size_t Hq, size_t Hk, size_t D, size_t cap, size_t S);
 int32_t btb_hip_attn_decode_qkv_span(const void* qkv, const void* wq, const void* wk, float eps, int32_t centered,
                                      const void* cos_t, const void* sin_t, const int32_t* n0, const int32_t* depth,
                                      const int32_t* par, void* K, void* V, void* att, size_t T, size_t Hq, size_t Hk,

@@ -1,0 +1,98 @@
+"""Decode steps over caches whose attention walks spans on the matrix cores (`attn_decode_qkv_span`): one row from 8192 slots
+on, passes of more rows over spans of several batches; the same steps with a launch per operator, on the vector kernels'
+spans, are the reference."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from btb_amd.decode import DecodeStep, Linear, StackConfig
+
+from .helpers import gen
+
+pytestmark = pytest.mark.gpu
+
+# eight query heads a kv head and few kv heads: one row walks spans from 8192 slots on, 2 .. 32 rows over any spans
+CFG = StackConfig(layers=2, hidden=256, q_heads=16, kv_heads=2, head_dim=128, intermediate=512, vocab=1000)
+TOKENS = [17, 5, 901, 33, 4, 250, 7, 12]
+
+
+def weights(card, off: int = 0):
+    """random weights; the norms' as views `off` values into a larger tensor"""
+    g = gen(1700)
+
+    def mat(rows, cols):
+        return Linear(card, (torch.randn(rows, cols, generator=g) * 0.05).to(torch.bfloat16).cuda())
+
+    def vec(n):
+        t = torch.zeros(n + 8, dtype=torch.bfloat16)
+        t[off : off + n] = (1.0 + 0.1 * torch.randn(n, generator=g)).to(torch.bfloat16)
+        return t.cuda()[off : off + n]
+
+    H, I = CFG.hidden, CFG.intermediate
+    w = {}
+    for i in range(CFG.layers):
+        p = f"layers.{i}."
+        w[p + "qkv"], w[p + "o"] = mat(CFG.qkv_rows, H), mat(H, CFG.q_heads * CFG.head_dim)
+        w[p + "gu"], w[p + "down"] = mat(2 * I, H), mat(H, I)
+        for name, n in (("ln1", H), ("ln2", H), ("wq", CFG.head_dim), ("wk", CFG.head_dim)):
+            w[p + name] = vec(n)
+    w["embed"] = torch.randn(CFG.vocab, H, generator=g).to(torch.bfloat16).cuda()
+    w["norm"], w["head"] = vec(H), mat(CFG.vocab, H)
+    return w
+
+
+def make(card, w, cap, T, n0, kv, tree=None, **kw):
+    step = DecodeStep(card, CFG, w, cap, T=T, **kw)
+    fill(step, n0, kv)
+    if tree is not None:
+        step.set_tree(tree)
+    return step
+
+
+def fill(step, n0, kv):
+    step.kv.zero_()
+    step.kv[:, :, :, :n0].copy_(kv[:, :, :, :n0])
+    step.reset(n0, TOKENS[0])
+    if step.T > 1:
+        step.ids.copy_(torch.tensor([TOKENS[t % 8] + t for t in range(step.T)], dtype=torch.int32))
+
+
+def cache(cap):
+    return torch.randn(CFG.layers, 2, CFG.kv_heads, cap, CFG.head_dim, generator=torch.Generator(device="cuda").manual_seed(5),
+                       device="cuda").to(torch.bfloat16)
+
+
+def close(a, b):
+    """logits to the step's bar (tests/test_decode_gpu.py)"""
+    return float((a.float() - b.float()).abs().max()) <= 3e-2 * float(b.float().abs().max())
+
+
+def test_norm_weights_at_any_place(card):
+    """norm weights that are views into a larger tensor, not 16-byte aligned: such a step keeps the kernels that take
+    them, on a long cache too"""
+    cap, n0 = 16384, 9000
+    kv = cache(cap)
+    odd, even = make(card, weights(card, 1), cap, 1, n0, kv), make(card, weights(card), cap, 1, n0, kv)
+    assert even.span_fused and not odd.span_fused
+    for s in (odd, even):
+        s.body()
+    torch.cuda.synchronize()
+    assert close(odd.logits, even.logits)
+    odd, even = make(card, weights(card, 1), cap, 20, n0, kv), make(card, weights(card), cap, 20, n0, kv)
+    assert even.span_fused and not odd.span_fused
+    for s in (odd, even):
+        s.body()
+    torch.cuda.synchronize()
+    assert close(odd.logits, even.logits)
+
+
+def test_the_knob_switches_the_walk_off(card):
+    w = weights(card)
+    card.set_tuning("attn_mfma", 0)
+    try:
+        assert not DecodeStep(card, CFG, w, 16384).span_fused and not DecodeStep(card, CFG, w, 16384, T=20).span_fused
+    finally:
+        card.set_tuning("attn_mfma", -1)
+    assert DecodeStep(card, CFG, w, 16384).span_fused and DecodeStep(card, CFG, w, 16384, T=20).span_fused
