@@ -160,17 +160,18 @@ __global__ void __launch_bounds__(256) p12_row_esc_kernel(const uint8_t* __restr
                                                           const int32_t* __restrict__ row_ptr, int rows, int cols,
                                                           uint32_t* __restrict__ out) {
     const int slots = FmtP12::row_esc_slots(cols);
-    const size_t at = (size_t)blockIdx.x * 256 + threadIdx.x;
-    const size_t r = at / slots;  // slots: a power of two
-    const int k = (int)(at - r * slots);
-    if (r >= (size_t)rows) return;
-    const int e0 = row_ptr[r], e1 = row_ptr[r + 1];
-    uint32_t w = FmtP12::ROW_ESC_NONE << 16;
-    if (e0 + k < e1) {
-        const size_t i = (size_t)esc_idx[e0 + k];
-        w = (uint32_t)lo[i] | ((uint32_t)esc_val[e0 + k] << 8) | ((uint32_t)(i - r * cols) << 16);
+    const size_t words = (size_t)rows * slots;
+    for (size_t at = (size_t)blockIdx.x * 256 + threadIdx.x; at < words; at += (size_t)gridDim.x * 256) {
+        const size_t r = at / slots;  // slots: a power of two
+        const int k = (int)(at - r * slots);
+        const int e0 = row_ptr[r], e1 = row_ptr[r + 1];
+        uint32_t w = FmtP12::ROW_ESC_NONE << 16;
+        if (e0 + k < e1) {
+            const size_t i = (size_t)esc_idx[e0 + k];
+            w = (uint32_t)lo[i] | ((uint32_t)esc_val[e0 + k] << 8) | ((uint32_t)(i - r * cols) << 16);
+        }
+        out[at] = w | (e1 - e0 > slots ? 0x80000000u : 0u);
     }
-    out[at] = w | (e1 - e0 > slots ? 0x80000000u : 0u);
 }
 
 int32_t btb_hip_p12_row_esc(const void* lo, const void* esc_idx, const void* esc_val, size_t n_esc, const void* row_ptr,
@@ -180,7 +181,9 @@ int32_t btb_hip_p12_row_esc(const void* lo, const void* esc_idx, const void* esc
     if (rows == 0 || cols == 0 || cols > FmtP12::ROW_ESC_NONE || rows * cols > 0x7FFFFFFFull) return ERR_DOMAIN;
     if (!al(esc_idx, 4) || !al(row_ptr, 4) || !al(row_esc, 4)) return ERR_DOMAIN;
     const size_t words = rows * (size_t)FmtP12::row_esc_slots((int)cols);
-    hipLaunchKernelGGL(p12_row_esc_kernel, dim3((unsigned)((words + 255) / 256)), dim3(256), 0,
+    // a launch holds fewer than 2^32 threads, and a matrix of one column has up to 2^34 words
+    const size_t want = (words + 255) / 256, most = (size_t)1 << 23;
+    hipLaunchKernelGGL(p12_row_esc_kernel, dim3((unsigned)(want < most ? want : most)), dim3(256), 0,
                        static_cast<hipStream_t>(stream), static_cast<const uint8_t*>(lo),
                        static_cast<const int32_t*>(esc_idx), static_cast<const uint8_t*>(esc_val),
                        static_cast<const int32_t*>(row_ptr), (int)rows, (int)cols, static_cast<uint32_t*>(row_esc));

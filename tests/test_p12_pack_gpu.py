@@ -48,3 +48,18 @@ def test_a_view_that_is_not_16_byte_aligned(card):
     lo, hi4, _, idx, _ = codecs.pack12_pack(bits16(w[3:]))
     assert np.array_equal(pw.lo.cpu().numpy(), lo) and np.array_equal(pw.hi4.cpu().numpy(), hi4)
     assert np.array_equal(pw.esc_idx.cpu().numpy(), idx)
+
+
+def test_the_rows_words_of_the_tallest_matrices(card):
+    """more rows than a launch has threads for their words: one column, 2^29 + 3 rows, an escape in the first and the last"""
+    rows = 2**29 + 3
+    lo = torch.full((rows,), 7, dtype=torch.uint8, device="cuda")
+    idx = torch.tensor([0, rows - 1], dtype=torch.int32, device="cuda")
+    val = torch.tensor([0x41, 0x42], dtype=torch.uint8, device="cuda")
+    row_ptr = torch.ones(rows + 1, dtype=torch.int32, device="cuda")
+    row_ptr[0], row_ptr[-1] = 0, 2
+    words = card.p12_row_esc(lo, idx, val, row_ptr, rows, 1)
+    none = 0x7FFF << 16
+    assert words[0].tolist() == [7 | 0x41 << 8] + [none] * 7 and words[-1].tolist() == [7 | 0x42 << 8] + [none] * 7
+    for part in words[1:-1].split(2**27):
+        assert int(part.min()) == none and int(part.max()) == none
