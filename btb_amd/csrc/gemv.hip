@@ -520,15 +520,43 @@ int32_t gemv_mfma_dl_p12(const uint8_t* lo, const uint8_t* hi4, const uint8_t* t
                          const uint8_t* esc_val, const int32_t* row_ptr, const void* x, void* y, int R, int C, int M,
                          hipStream_t st);
 
+enum class Form { BF16, P12, FP8, MX4 };
+
+// The shapes the LDS-staged kernel takes by a last tile that starts inside the one before it (R % 16 != 0) or by streaming x
+// (C > 10240): not everywhere it can. The other side is the column-interleaved kernel (bf16 from eight rows of x on) or the
+// vector kernel's passes of four rows, cheap for small matrices. Measured on MI355X over 18 000 shapes of 16 to 40008 rows
+// by 96 to 16384 columns and 3 to 32 rows of x; what the staged kernel takes of the other side's time:
+//   bf16, 8 rows of x: [520 x 512] 1.10, [20008 x 1216] 1.0, [140 x 2560] 1.07, [264 x 2560] 0.85; 17 rows: [8200 x 1216]
+//   1.30; 5 rows: [520 x 512] 0.78, [264 x 7168] 1.12, [1000 x 7168] 0.98
+//   pack12, 5 rows: [1000 x 4096] 1.32, [2100 x 4096] 0.85, [4104 x 2560] 1.16; 17 rows: [520 x 5120] 1.21
+//   FP8, 5 rows: [1000 x 7168] 1.31, [4104 x 4608] 1.44, [1488 x 12288] 1.36; 3 rows: [4104 x 10240] 1.64
+//   MXFP4, 5 rows: [264 x 6144] 1.32, [992 x 12288] 1.44; 3 rows: [4104 x 2560] 1.70
+// where this rule now leaves them to it; what it takes, 0.2 to 1.0 (a few odd shapes 1.2).
+static bool staged_pays(Form f, size_t M, size_t R, size_t C) {
+    const bool whole = R % 16 == 0;
+    if (whole && C <= 10240) return true;
+    if (f == Form::BF16) return M >= 8 ? C > 1280 && R * C >= (1u << 19) : C <= 1280 || R * C >= (1u << 22);
+    if (whole) return R >= 2048;  // at any width: a row's bits are the same in every pass of five rows of x and more
+    if (M < 5) return false;
+    if (M <= 8) {
+        if (C <= 1280) return R <= 8192;
+        if (f == Form::P12) return C > 2560 && R >= 2048;
+        return C <= 4096 || (R >= 2048 && f == Form::MX4);
+    }
+    return f != Form::P12 || M <= 16 || M > 20 || R >= 1024;
+}
+
 // whether a pass of M rows goes to the matrix cores through the LDS-staged kernel: from `from` rows on (the knob
-// gemv_mfma_from, when set, replaces every form's own figure)
-static bool wide_pass(size_t M, size_t R, size_t C, bool packed, size_t from = 5) {
-    if (tuning("gemv_mfma_from") > 0) from = (size_t)tuning("gemv_mfma_from");
+// gemv_mfma_from, when set, replaces every form's own figures)
+static bool wide_pass(Form f, size_t M, size_t R, size_t C, size_t from = 5) {
+    const bool set = tuning("gemv_mfma_from") > 0;
+    if (set) from = (size_t)tuning("gemv_mfma_from");
     // bf16 and more than 16 rows of x: the column-interleaved kernel over rows of more than 10240 columns ([4096 x 12288]
     // at 32 rows 44.0 us against 53.1) and, where the last tile is not whole, of more than 4096 ([5001 x 9728] 66.8
     // against 73.7, [12345 x 7168] at 20 rows 79.0 against 84.2)
-    if (!packed && M > 16 && (C > 10240 || (R % 16 != 0 && C > 4096))) return false;
-    return M >= from && (packed ? mfma_lds_fits_packed((int)R, (int)C) : mfma_lds_fits_bf16((int)R, (int)C)) &&
+    if (f == Form::BF16 && M > 16 && (C > 10240 || (R % 16 != 0 && C > 4096))) return false;
+    return M >= from && (set || staged_pays(f, M, R, C)) &&
+           (f == Form::BF16 ? mfma_lds_fits_bf16((int)R, (int)C) : mfma_lds_fits_packed((int)R, (int)C)) &&
            tuning("gemv_no_mfma") <= 0 && tuning("mfma_lds") != 0;
 }
 
@@ -631,12 +659,12 @@ int32_t btb_hip_gemv_bf16(const void* w, const void* x, void* y, size_t R, size_
     if (!aligned16(w) || !aligned16(x) || !aligned2(y)) return ERR_DOMAIN;
     // the verify widths go to the matrix cores, 32 rows of x a pass (from five rows on where the LDS-staged kernel takes
     // the shape: one pass there against two of the vector ALUs'); narrower passes stay on the vector ALUs
-    if ((M >= 8 || wide_pass(M, R, C, false)) && C % 32 == 0 && tuning("gemv_no_mfma") <= 0) {
+    if ((M >= 8 || wide_pass(Form::BF16, M, R, C)) && C % 32 == 0 && tuning("gemv_no_mfma") <= 0) {
         const uint16_t* xp = static_cast<const uint16_t*>(x);
         uint16_t* yp = static_cast<uint16_t*>(y);
         for (size_t m0 = 0; m0 < M; m0 += 32) {
             const int mm = (int)(M - m0 < 32 ? M - m0 : 32);
-            rc = wide_pass(M, R, C, false) ? gemv_mfma_lds_bf16(w, xp + m0 * C, yp + m0 * R, (int)R, (int)C, mm,
+            rc = wide_pass(Form::BF16, M, R, C) ? gemv_mfma_lds_bf16(w, xp + m0 * C, yp + m0 * R, (int)R, (int)C, mm,
                                                       static_cast<hipStream_t>(stream))
                                  : gemv_mfma_bf16(w, xp + m0 * C, yp + m0 * R, (int)R, (int)C, mm,
                                                   static_cast<hipStream_t>(stream));
@@ -662,7 +690,7 @@ int32_t btb_hip_gemv_glu_silu_bf16(const void* w, const void* x, void* m, size_t
     int32_t rc = check_dims(2 * I, C, M, FmtBf16::UW);
     if (rc != OK) return rc;
     if (!aligned16(w) || !aligned16(x) || !aligned2(m)) return ERR_DOMAIN;
-    if (I % 16 == 0 && wide_pass(M, 2 * I, C, false)) {  // the verify widths: the matrix cores, 32 rows of x a pass
+    if (I % 16 == 0 && wide_pass(Form::BF16, M, 2 * I, C)) {  // the verify widths: the matrix cores, 32 rows of x a pass
         const uint16_t* xp = static_cast<const uint16_t*>(x);
         uint16_t* mp = static_cast<uint16_t*>(m);
         for (size_t m0 = 0; m0 < M; m0 += 32) {
@@ -725,7 +753,7 @@ int32_t btb_hip_gemv_p12(const void* lo, const void* hi4, const void* table, con
     if (!aligned16(x) || !aligned2(y)) return ERR_DOMAIN;
     // the verify widths: the matrix cores. Weights straight into LDS, 16 rows of x a pass, where that kernel has a
     // shape for the row length
-    if (wide_pass(M, R, C, true) && aligned16(hi4) && aligned16(lo) && (reinterpret_cast<uintptr_t>(table) & 3u) == 0 &&
+    if (wide_pass(Form::P12, M, R, C) && aligned16(hi4) && aligned16(lo) && (reinterpret_cast<uintptr_t>(table) & 3u) == 0 &&
         mfma_dl_fits_p12((int)R, (int)C, 16)) {
         const uint16_t* xp = static_cast<const uint16_t*>(x);
         uint16_t* yp = static_cast<uint16_t*>(y);
@@ -737,7 +765,7 @@ int32_t btb_hip_gemv_p12(const void* lo, const void* hi4, const void* table, con
         }
         return OK;
     }
-    if (wide_pass(M, R, C, true) && aligned16(hi4)) {  // through registers and LDS, 32 rows of x a pass
+    if (wide_pass(Form::P12, M, R, C) && aligned16(hi4)) {  // through registers and LDS, 32 rows of x a pass
         const uint16_t* xp = static_cast<const uint16_t*>(x);
         uint16_t* yp = static_cast<uint16_t*>(y);
         for (size_t m0 = 0; m0 < M; m0 += 32) {
@@ -813,7 +841,7 @@ int32_t btb_hip_gemv_fp8(const void* w, const void* scales, size_t sr, size_t sc
     if (rc != OK) return rc;
     if (!aligned16(x) || !aligned2(y)) return ERR_DOMAIN;
     const size_t from = fp8_matrix_from(R, C);
-    if (wide_pass(M, R, C, true, from) && mfma_dl_fits_fp8((int)R, (int)C, 16, (int)(R / sr), (int)(C / sc))) {
+    if (wide_pass(Form::FP8, M, R, C, from) && mfma_dl_fits_fp8((int)R, (int)C, 16, (int)(R / sr), (int)(C / sc))) {
         const uint16_t* xp = static_cast<const uint16_t*>(x);  // the long rows: weights straight into LDS, 16 rows a pass
         uint16_t* yp = static_cast<uint16_t*>(y);
         for (size_t m0 = 0; m0 < M; m0 += 16) {
@@ -824,7 +852,7 @@ int32_t btb_hip_gemv_fp8(const void* w, const void* scales, size_t sr, size_t sc
         }
         return OK;
     }
-    if (wide_pass(M, R, C, true, from)) {  // the verify widths: the matrix cores, 32 rows of x a pass
+    if (wide_pass(Form::FP8, M, R, C, from)) {  // the verify widths: the matrix cores, 32 rows of x a pass
         const uint16_t* xp = static_cast<const uint16_t*>(x);
         uint16_t* yp = static_cast<uint16_t*>(y);
         for (size_t m0 = 0; m0 < M; m0 += 32) {
@@ -876,7 +904,7 @@ int32_t btb_hip_gemv_mxfp4(const void* blocks, const void* scales, const void* x
     if (rc != OK) return rc;
     if (!aligned16(blocks) || !aligned16(x) || !aligned2(y)) return ERR_DOMAIN;
     const size_t from = mx4_matrix_from(R, C);
-    if (wide_pass(M, R, C, true, from) && mfma_dl_fits((int)R, (int)C, 16) &&
+    if (wide_pass(Form::MX4, M, R, C, from) && mfma_dl_fits((int)R, (int)C, 16) &&
         (reinterpret_cast<uintptr_t>(scales) & 3u) == 0) {
         const uint16_t* xp = static_cast<const uint16_t*>(x);  // the long rows: weights straight into LDS, 16 rows a pass
         uint16_t* yp = static_cast<uint16_t*>(y);
@@ -888,7 +916,7 @@ int32_t btb_hip_gemv_mxfp4(const void* blocks, const void* scales, const void* x
         }
         return OK;
     }
-    if (wide_pass(M, R, C, true, from)) {
+    if (wide_pass(Form::MX4, M, R, C, from)) {
         const uint16_t* xp = static_cast<const uint16_t*>(x);
         uint16_t* yp = static_cast<uint16_t*>(y);
         for (size_t m0 = 0; m0 < M; m0 += 32) {
