@@ -138,6 +138,16 @@ def step_on_spans(cus: int, Hq: int, Hk: int, cap: int) -> int:
     return spans if Hq * spans % 2 == 0 else 0  # the states' alignment
 
 
+def fp8_step_fused(T: int, hidden: int) -> bool:
+    """whether a pass of T rows over FP8 matrices takes the fused launches: one and two rows (from three on its large
+    matrices are faster on the matrix cores than on the streaming kernel the fused launches are: 30.7 against 33.3 us at
+    [18432 x 7168]) whose x rows and norm weight fit the 160 KB of LDS - two of them not over 3073 to 4096 columns, which
+    the add + norm's own launch holds in registers and the folded one makes row by row. Measured on MI355X, six layers, two
+    rows, a launch per operator / fused: 3072 / 9216 318.0 / 303.8 us, 3200 / 9600 338.2 / 355.0, 4096 / 12288 395.4 /
+    403.4, 4224 / 12672 535.6 / 472.7."""
+    return T <= 2 and 2 * hidden * (T + 1) <= 160 * 1024 and not (T == 2 and 3072 < hidden <= 4096)
+
+
 class Linear:
     """one linear's weight on the GPU in its stored form, multiplied as stored: a bf16 tensor or a `P12Weight`"""
 
@@ -240,12 +250,11 @@ class DecodeStep:
         if fold_silu is None:
             fold_silu = fused
         self.fold_silu = bool(fold_silu)
-        # The fused launches exist for bf16, 12-bit and FP8 matrices, FP8 for one and two rows (from three on its large
-        # matrices are faster on the matrix cores than on the streaming kernel the fused launches are: 30.7 against 33.3
-        # us at [18432 x 7168]); any other stored form takes one launch per operator.
+        # The fused launches exist for bf16, 12-bit and FP8 matrices; any other stored form takes one launch per operator.
         lins = [weights[f"layers.{i}.{k}"] for i in range(cfg.layers) for k in ("qkv", "o", "gu", "down")] + [weights["head"]]
         self.fused = bool(fused) and all(getattr(m, "fusable", False) or
-                                         (self.T <= 2 and isinstance(getattr(m, "w", None), F8Weight)) for m in lins)
+                                         (isinstance(getattr(m, "w", None), F8Weight) and fp8_step_fused(self.T, H))
+                                         for m in lins)
         # a pass's q / k norm, rope and cache write ride in its attention kernel where that kernel takes the pass's
         # shape - in the fused sequence, and in the other one too unless the caller asked for a launch per operator
         # ... and the activation in the gate / up matvec's epilogue (bf16 matrices)

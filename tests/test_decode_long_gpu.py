@@ -96,3 +96,32 @@ def test_the_knob_switches_the_walk_off(card):
     finally:
         card.set_tuning("attn_mfma", -1)
     assert DecodeStep(card, CFG, w, 16384).span_fused and DecodeStep(card, CFG, w, 16384, T=20).span_fused
+
+
+def test_fp8_rows_the_folded_norm_has_no_room_for(card):
+    """a residual stream whose two rows fit LDS but not with the norm's weight beside them: one launch per operator"""
+    from btb_amd import fp8
+
+    H, D = 32768, 128
+    cfg = StackConfig(layers=1, hidden=H, q_heads=2, kv_heads=1, head_dim=D, intermediate=256, vocab=64)
+    g = gen(1750)
+
+    def f8(rows, cols):
+        q, s = fp8.quantize(torch.randn(rows, cols, generator=g) * 0.01, (128, 128))
+        return Linear(card, fp8.F8Weight(q.view(torch.uint8).cuda(), s.cuda(), rows, cols))
+
+    ones = lambda n: torch.ones(n, dtype=torch.bfloat16, device="cuda")
+    p = "layers.0."
+    w = {p + "qkv": f8(4 * D, H), p + "o": f8(H, 2 * D), p + "gu": f8(512, H), p + "down": f8(H, 256), p + "ln1": ones(H),
+         p + "ln2": ones(H), p + "wq": ones(D), p + "wk": ones(D), "norm": ones(H),
+         "embed": torch.randn(64, H, generator=g).to(torch.bfloat16).cuda()}
+    w["head"] = Linear(card, w["embed"])
+    logits = []
+    for fused in (None, False):
+        step = DecodeStep(card, cfg, w, 64, T=2, fused=fused)
+        assert not step.fused
+        step.reset(3, 5)
+        step.body()
+        torch.cuda.synchronize()
+        logits.append(step.logits.clone())
+    assert bool(torch.isfinite(logits[0].float()).all()) and close(logits[0], logits[1])

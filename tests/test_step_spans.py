@@ -1,10 +1,10 @@
-"""The rules that cut a cache into the spans an attention launch walks."""
+"""The rules by which a step chooses its launches: the spans an attention launch walks, the fused sequence over FP8."""
 
 from __future__ import annotations
 
 import pytest
 
-from btb_amd.decode import pass_spans, step_on_spans, step_spans
+from btb_amd.decode import fp8_step_fused, pass_spans, step_on_spans, step_spans
 
 
 @pytest.mark.parametrize("T", [2, 3, 16, 17, 32])
@@ -39,3 +39,10 @@ def test_a_step_walks_its_spans_where_they_are_short_for_it(Hq, Hk, cap):
     assert bool(S) == (others > 64 or pays)
     if S:
         assert -(-(-(-cap // S)) // 128) == ours
+
+
+@pytest.mark.parametrize("T,hidden,fused", [(1, 4096, True), (2, 3072, True), (2, 3073, False), (2, 4096, False), (2, 4224, True),
+                                            (3, 1024, False), (1, 40960, True), (1, 40961, False), (2, 27306, True),
+                                            (2, 27392, False)])
+def test_fp8_steps_that_fit_and_pay(T, hidden, fused):
+    assert fp8_step_fused(T, hidden) == fused
