@@ -398,10 +398,15 @@ static int32_t launch_stream(const typename F::Params& p, const XArgs& xa, void*
                 // One row of x over FP8: a lane's 5 to 8 units of a row asked for at once, one row a wave - one trip to
                 // memory for the row instead of three or four spans of two units ([18432 x 7168], 7 units a lane:
                 // 26.3 -> 24.4 us; two rows by four units 25.1, by three 25.4, one row by four 27.2). 9 to 16 units: two
-                // trips (down [4096 x 12288] of a 32-layer step, 12 units a lane: the step 2051 -> 1999 us). Four units
-                // and the gate / up fold stay with two rows by two (one row by four, 2 x 4: the step 2051 -> 2091, 2099).
-                if (per_lane >= 9 && per_lane <= 12) return launch_variant<F, M, LPR, 1, 6, XMODE, E_PLAIN>(p, xa, y, R, C, st);
-                if (per_lane >= 13 && per_lane <= 16) return launch_variant<F, M, LPR, 1, 8, XMODE, E_PLAIN>(p, xa, y, R, C, st);
+                // trips (down [4096 x 12288] of a 32-layer step, 12 units a lane: the step 2051 -> 1999 us) - where the
+                // second trip is a whole one, or the rows are few enough that a trip's latency is what they cost:
+                // [1024 x 10240] 6.3 -> 4.4 us, [4096 x 10240] 9.4 -> 8.9, [8192 x 10240] 14.8 / 15.4; [3072 x 13312] 11.9 ->
+                // 10.0, [4096 x 13312] 12.5 / 13.9, [8192 x 14336] 20.6 / 24.8; [8192 x 12288] 18.3 -> 17.4. Four units and
+                // the gate / up fold stay with two rows by two (one row by four, 2 x 4: the step 2051 -> 2091, 2099).
+                if (per_lane >= 9 && per_lane <= 12 && (per_lane == 12 || R <= 4096))
+                    return launch_variant<F, M, LPR, 1, 6, XMODE, E_PLAIN>(p, xa, y, R, C, st);
+                if (per_lane >= 13 && per_lane <= 16 && R <= 3072)
+                    return launch_variant<F, M, LPR, 1, 8, XMODE, E_PLAIN>(p, xa, y, R, C, st);
                 switch (per_lane) {
                     case 5: return launch_variant<F, M, LPR, 1, 5, XMODE, E_PLAIN>(p, xa, y, R, C, st);
                     case 6: return launch_variant<F, M, LPR, 1, 6, XMODE, E_PLAIN>(p, xa, y, R, C, st);

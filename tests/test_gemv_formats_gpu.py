@@ -653,3 +653,31 @@ def test_row_counts_that_end_inside_a_tile(card, R, C, form, M):
     op(w, x.cuda(), y)
     check(y, ref)
     assert bool((room[M * R:] == 7.0).all())
+
+
+# one row of x over 5 to 16 units a lane: a row in one trip (5 .. 8), in two of six or eight - the second whole, short, of a
+# remainder that is no whole lane (9360, 16000) -, and the taller matrices that stay with two rows by two; odd row counts,
+# blocks of 16 columns
+@pytest.mark.parametrize("R,C,block", [(384, 5120, (128, 128)), (130, 7168, (2, 128)), (256, 8192, (64, 256)), (131, 9360, (1, 16)),
+                                       (258, 9728, (2, 128)), (4097, 9728, (1, 128)), (513, 12288, (1, 128)),
+                                       (4224, 12288, (128, 128)), (66, 13312, (2, 16)), (3200, 13312, (128, 128)),
+                                       (129, 16000, (1, 16)), (64, 16384, (64, 128))])
+def test_fp8_one_row_over_long_rows(card, R, C, block):
+    """`gemv_fp8` against the oracle, and `gemv_norm` / `gemv_embed_norm` with the bits of the launches they replace"""
+    g = gen(90 + R + C)
+    q, s = fp8.quantize(torch.randn(R, C, generator=g) * 0.02, block)
+    w = fp8.F8Weight(q.view(torch.uint8).cuda(), s.cuda(), R, C)
+    x = acts_bf16(1, C, seed=91 + R)
+    check(card.gemv_fp8(w, x.cuda()), oracle.gemv_fp8(q.view(torch.uint8).numpy(), s.numpy(), x.float().numpy(), threads=0))
+    h, y = (torch.randn(1, C, generator=g).to(torch.bfloat16).cuda() for _ in range(2))
+    nw = (1.0 + 0.1 * torch.randn(C, generator=g)).to(torch.bfloat16).cuda()
+    h1, x1 = h.clone(), torch.empty_like(h)
+    card.add_rmsnorm(h1, y, nw, 1e-6, x1)
+    want = card.gemv_fp8(w, x1)
+    h2, out = torch.empty_like(h), torch.empty_like(want)
+    card.gemv_norm(w, h, y, nw, 1e-6, h2, out)
+    assert torch.equal(out.view(torch.int16), want.view(torch.int16)) and torch.equal(h2, h1)
+    h1 = h.clone()
+    card.add_rmsnorm(h1, None, nw, 1e-6, x1)
+    card.gemv_embed_norm(w, h, torch.zeros(1, dtype=torch.int32, device="cuda"), nw, 1e-6, h2, out)
+    assert torch.equal(out.view(torch.int16), card.gemv_fp8(w, x1).view(torch.int16)) and torch.equal(h2, h1)
