@@ -69,6 +69,79 @@ def close(a, b):
     return float((a.float() - b.float()).abs().max()) <= 3e-2 * float(b.float().abs().max())
 
 
+def follow(step, n0, kv, steps, graph):
+    """logits and cache of `steps` steps, eager or replayed, with unrelated work and a synchronise between them"""
+    fill(step, n0, kv)
+    out = []
+    for _ in range(steps):
+        step.replay() if graph else step.body()
+        torch.cuda.synchronize()
+        out.append(step.logits.clone())
+        assert bool(torch.isfinite(torch.randn(1 << 14, device="cuda").sum()))
+        torch.cuda.synchronize()
+    return torch.stack(out), step.kv.clone()
+
+
+# the cache all but empty, one key short of a batch a span and at it (64 spans of 128), and near its end: the spans follow
+# the keys from step to step
+@pytest.mark.parametrize("n0", [0, 8189, 16380])
+def test_one_row_on_a_long_cache(card, n0):
+    """eager steps, replayed steps - the same bits - and the sequence with a launch per operator, to the step's bar; every
+    one writes its row into the cache"""
+    cap = 16384
+    w, kv = weights(card), cache(cap)
+    step, plain = DecodeStep(card, CFG, w, cap), DecodeStep(card, CFG, w, cap, fused=False)
+    assert step.span_fused and step.fused and not plain.span_fused and not plain.fused
+    eager, kv_e = follow(step, n0, kv, 4, False)
+    fill(step, n0, kv)
+    step.capture(warmup=1)
+    for _ in range(2):
+        again, kv_g = follow(step, n0, kv, 4, True)
+        assert torch.equal(again, eager) and torch.equal(kv_g, kv_e)
+    # the other sequence on the same tokens: its own picks may differ where two logits are close
+    fill(step, n0, kv)
+    fill(plain, n0, kv)
+    for t in range(4):
+        for s in (step, plain):
+            s.ids.fill_(TOKENS[t])
+            s.body()
+        torch.cuda.synchronize()
+        assert close(step.logits, plain.logits), t
+    new = slice(n0, n0 + 4)
+    a, b = step.kv[:, :, :, new].float(), plain.kv[:, :, :, new].float()
+    assert float((a - b).abs().max()) <= 3e-2 * float(b.abs().max())
+    assert torch.equal(step.kv[:, :, :, :n0], kv[:, :, :, :n0]) and not bool(step.kv[:, :, :, n0 + 4 :].any())
+
+
+@pytest.mark.parametrize("T,cap", [(2, 17000), (3, 17000), (20, 9000), (32, 9000)])
+@pytest.mark.parametrize("tree", [False, True])
+def test_passes_over_long_spans(card, T, cap, tree):
+    """a pass whose attention walks spans of several batches from the fused rows, the pass's rows in the middle of the cache,
+    across two spans and at its end"""
+    w, kv = weights(card), cache(cap)
+    par = [-1] + [t - 2 if t % 3 == 2 else t - 1 for t in range(1, T)] if tree else None
+    step, plain = DecodeStep(card, CFG, w, cap, T=T), DecodeStep(card, CFG, w, cap, T=T, fused=False)
+    span = -(-(-(-cap // step.S)) // 128) * 128
+    assert step.span_fused and not plain.span_fused and span > 128
+    for s in (step, plain):
+        s.set_tree(par)
+    fill(step, 5, kv)
+    step.capture(warmup=1)
+    for n0 in (5, 3 * span - 1, cap - T):
+        fill(step, n0, kv)
+        step.body()
+        torch.cuda.synchronize()
+        eager, kv_e = step.logits.clone(), step.kv.clone()
+        fill(step, n0, kv)
+        step.replay()
+        fill(plain, n0, kv)
+        plain.body()
+        torch.cuda.synchronize()
+        assert torch.equal(step.logits, eager) and torch.equal(step.kv, kv_e)
+        assert close(step.logits, plain.logits), n0
+        assert torch.equal(step.kv[:, :, :, :n0], kv[:, :, :, :n0]) and not bool(step.kv[:, :, :, n0 + T :].any())
+
+
 def test_norm_weights_at_any_place(card):
     """norm weights that are views into a larger tensor, not 16-byte aligned: such a step keeps the kernels that take
     them, on a long cache too"""

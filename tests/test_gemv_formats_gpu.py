@@ -681,3 +681,19 @@ def test_fp8_one_row_over_long_rows(card, R, C, block):
     card.add_rmsnorm(h1, None, nw, 1e-6, x1)
     card.gemv_embed_norm(w, h, torch.zeros(1, dtype=torch.int32, device="cuda"), nw, 1e-6, h2, out)
     assert torch.equal(out.view(torch.int16), card.gemv_fp8(w, x1).view(torch.int16)) and torch.equal(h2, h1)
+
+
+# FP8 rows past 10240 columns, x streamed beside the weights: one tile of x rows and two; matrices the vector kernel keeps
+# (fewer than 2048 rows) beside those the staged kernel takes, a last tile that starts inside the one before it
+@pytest.mark.parametrize("R,C,block", [(2048, 12288, (128, 128)), (2064, 16384, (16, 128)), (144, 12288, (16, 32)),
+                                       (2056, 11264, (8, 128)), (1000, 16384, (8, 64))])
+@pytest.mark.parametrize("M", [5, 16, 27])
+def test_fp8_rows_past_10240_columns(card, R, C, block, M):
+    q, s = fp8.quantize(torch.randn(R, C, generator=gen(95 + R + C)) * 0.02, block)
+    w = fp8.F8Weight(q.view(torch.uint8).cuda(), s.cuda(), R, C)
+    x = acts_bf16(M, C, seed=96 + R)
+    room = torch.full((M * R + 64,), 7.0, dtype=torch.bfloat16, device="cuda")
+    y = room[: M * R].view(M, R)
+    card.gemv_fp8(w, x.cuda(), y)
+    check(y, oracle.gemv_fp8(q.view(torch.uint8).numpy(), s.numpy(), x.float().numpy(), threads=0))
+    assert bool((room[M * R:] == 7.0).all())
