@@ -12,7 +12,7 @@
 //
 // A weight goes to the matrix cores as two bf16 terms, its rounding and what the rounding left (2^-17 of it stays out),
 // one product each into the same sum. A weight rounded once is not enough here: the vector kernels take a weight against
-// the maximum of its own stream of 16 keys or fewer a batch, so the heaviest of them are 1 and exact, and against f64 their
+// the maximum of its own stream, eight keys a batch, so the heaviest of them are 1 and exact, and against f64 their
 // outputs lie 1.8e-3 to 2.2e-3 off (relative 2-norm, normal q and k, 100 to 32000 keys) where weights taken against a whole
 // batch's maximum and rounded once lie 2.1e-3 to 2.2e-3 off; with two terms 1.66e-3, what rounding the outputs to bf16
 // alone makes. The second product costs 3 to 8 %: 8 rows x 32 / 8 heads over 6125 keys, with the fold, 15.2 -> 16.4 us

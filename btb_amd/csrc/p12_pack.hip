@@ -1,19 +1,18 @@
 // A bf16 tensor into its 12-bit form on the GPU (the reference packs in torch: btb/pack12.py:48-67): the bytes that
-// `pack12.pack_bf16` writes, in four launches where that is thirty-odd passes over the tensor.
+// `pack12.pack_bf16` writes, in five launches where that is thirty-odd passes over the tensor.
 //
-//   1. p12_hist_kernel    how often each high byte occurs (reads 2 B a weight)
+//   1. p12_clear_kernel, p12_hist_kernel   how often each high byte occurs (reads 2 B a weight)
 //   2. p12_table_kernel   the table: the 15 most frequent high bytes, equal counts by ascending byte value; with it the
 //                         pair table, the byte -> code map and the number of escapes (n less what the table covers)
 //   3. p12_encode_kernel  low bytes and codes (2 B read, 1.5 B written a weight), escapes counted a chunk of 2048
 //   4. p12_emit_kernel    the escape list in ascending order out of the codes (0.5 B a weight read back), and every
 //                         row's first entry in it
 //
-// The list's length has to be known on the host before the list can be allocated. It is known after the second launch,
-// so the host waits for that one (an event) while the third is already queued behind it.
+// The list's length has to be known on the host before the list can be allocated. It is known after the table's launch, so
+// the host waits for that one (an event) while the encoder is already queued behind it.
 //
 // Bound: HBM, 2 + 2 + 1.5 + 0.5 B a weight; the second read of a tensor that fits the 256 MB last-level cache comes out
-// of that. [19456 x 2560] packed,
-// with its rows' words, and widened back: 1456 us with the packing in torch, 118 in these launches: 27 us for the
+// of that. [19456 x 2560] packed, with its rows' words, and widened back: 1456 us with the packing in torch, 118 in these launches: 27 us for the
 // histogram, 4 for the table, 28 to encode (6.2 TB/s), 15 for the list.
 
 #include "btb_common.hpp"
@@ -192,8 +191,8 @@ __global__ void __launch_bounds__(256) p12_encode_kernel(const uint4* __restrict
 
 // The escape list out of the codes. A workgroup takes the chunks one of the encoding workgroups took; where its part
 // of the list begins is the sum of those workgroups' counts before it (summing the chunks' own counts, sixteen times
-// as many: 20 us for [19456 x 2560]); 15 us: a chain of three trips to memory - codes, the escapes' weights, the stores. Row r's first entry (row_ptr) is written by the chunk
-// that holds the row's first weight.
+// as many: 20 us for [19456 x 2560]); 15 us: a chain of three trips to memory - codes, the escapes' weights, the stores.
+// Row r's first entry (row_ptr) is written by the chunk that holds the row's first weight.
 __global__ void __launch_bounds__(256) p12_emit_kernel(const uint16_t* __restrict__ t, const uint8_t* __restrict__ hi4,
                                                        size_t n, const uint32_t* __restrict__ block_counts,
                                                        const uint32_t* __restrict__ counts, size_t n_esc,
@@ -335,7 +334,8 @@ int32_t btb_hip_p12_emit(const void* t, const void* hi4, size_t n, const void* w
     const size_t blocks = p12_blocks(n);
     hipLaunchKernelGGL(p12_emit_kernel, dim3((unsigned)blocks), dim3(256), 0, static_cast<hipStream_t>(stream),
                        static_cast<const uint16_t*>(t), static_cast<const uint8_t*>(hi4), n,
-                       static_cast<const uint32_t*>(work) + P12_BLOCKS, static_cast<const uint32_t*>(work) + P12_BLOCKS + blocks, n_esc, static_cast<int32_t*>(esc_idx),
+                       static_cast<const uint32_t*>(work) + P12_BLOCKS,
+                       static_cast<const uint32_t*>(work) + P12_BLOCKS + blocks, n_esc, static_cast<int32_t*>(esc_idx),
                        static_cast<uint8_t*>(esc_val), row_ptr != nullptr ? cols : 1, row_ptr != nullptr ? rows : 0,
                        static_cast<int32_t*>(row_ptr));
     return hip_status(hipGetLastError(), "p12_emit launch");

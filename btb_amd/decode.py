@@ -382,8 +382,9 @@ class DecodeStep:
     def _body_fused(self) -> None:
         """the same arithmetic in fewer launches: each residual add + norm rides in the x load of the matvec that
         follows it (the residual ping-pongs between two buffers), gate / up / activation are one kernel, the q / k norm
-        and rope ride in the attention kernel. Bit for bit
-        the plain sequence's result."""
+        and rope ride in the attention kernel. Bit for bit the plain sequence's result where both take the same span count
+        and the same attention arithmetic; a one-row step that walks its spans on the matrix cores (`step_on_spans`) adds in
+        another order than the plain sequence's register kernel."""
         k, cfg, w = self.card, self.cfg, self.w
         Hq, Hk, D = cfg.q_heads, cfg.kv_heads, cfg.head_dim
         ha, hb = self.h, self.h2

@@ -146,8 +146,8 @@ def split(body: torch.Tensor, meta: torch.Tensor):
 
 def check_escapes(esc_idx: torch.Tensor, esc_val: torch.Tensor, n: int) -> None:
     """ValueError unless the list is what the kernels index with: as many values as indices, every index in [0, n),
-    strictly ascending (the reference refuses the same lists with ERR_DOMAIN: native/src/gemv.rs:4171-4189). Runs where
-    the list lies (a few torch reductions; on the GPU for an uploaded matrix), once, at upload."""
+    strictly ascending (the reference refuses the same lists with ERR_DOMAIN: native/src/gemv.rs:4171-4189). A few torch
+    reductions where the list lies; an uploaded matrix's list is checked by the card (`HipCard.p12_check`)."""
     if esc_idx.numel() != esc_val.numel():
         raise ValueError(f"[pack12] {esc_idx.numel()} escape indices but {esc_val.numel()} escape values")
     if esc_idx.numel() == 0:
