@@ -28,8 +28,9 @@
 // SPLIT, passes of more than sixteen rows: a weight goes to the matrix cores as two bf16 terms, as in attn_span.hip and for
 // its reason - a step's pass of so many rows over spans of 128 keys is what the vector kernels served in longer spans,
 // closer to f64 (32 rows x 32 / 8 heads, 1536 keys: 1.99e-3 off there, 2.15e-3 here with one term, 1.66e-3 with two;
-// norm_rope_kv, this and the fold 18.6 us a layer with one term, 19.1 with two, 37.3 on the vector kernel). The second terms have sums of their own, left out where they are not finite: of an
-// infinite value and a weight's two terms the first alone says what the output is.
+// norm_rope_kv, this and the fold 18.6 us a layer with one term, 19.1 with two, 37.3 on the vector kernel). The second
+// terms have sums of their own, left out where they are not finite: of an infinite value and a weight's two terms the
+// first alone says what the output is.
 
 #include "btb_attn.hpp"
 #include "btb_common.hpp"

@@ -79,7 +79,8 @@ __device__ __forceinline__ bool sees(const RowView& v, int key, int lim) {
 // QKV: the rows come as the fused qkv rows, before the q / k norm and rope. A workgroup prepares the q heads of its own
 // rows, a tile of 16 a wave, while the first batch's K travels (but for ONE its addresses wait for nothing: they stay
 // within the cache's capacity); where its span holds some of the pass's own slots *n0 .. *n0 + T - 1 it prepares the
-// pass's k heads too, takes those keys and values from there, and the last of the z axis - whose rows see all of them - writes them into the cache. T <= 32. The arithmetic is norm_rope_kv_kernel's, then this kernel's.
+// pass's k heads too, takes those keys and their values from LDS, and the last of the z axis - whose rows see all of them -
+// writes them into the cache. T <= 32. The arithmetic is norm_rope_kv_kernel's, then this kernel's.
 template <int NQT, bool TBL, bool QKV, bool ONE = false>
 __global__ void __launch_bounds__(256, 2) attn_span_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ K, const uint16_t* __restrict__ V,
