@@ -85,13 +85,17 @@ def rope_tables(cfg: StackConfig, positions: int, device: Any) -> tuple[torch.Te
 def pass_spans(cus: int, T: int, Hq: int, Hk: int, cap: int) -> int:
     """how many spans the attention of a pass of T rows cuts a cache of `cap` slots into. Its workgroup walks a span in
     batches of 128 keys for up to 32 (row, head) pairs of a kv head, so: a workgroup a CU, spans whole batches. Where a kv
-    head's pairs take several workgroups, which read the same keys, and spans stay at 512 keys or more, two a CU.
-    Measured on MI355X with the q / k norm and the fold, us a layer, at a workgroup a CU / at two: 8 rows x 32 / 8 heads,
-    6125 keys 16.4 / 17.8, 32000 32.1 / 32.0; 17 rows x 32 / 8, 3000 keys 18.3 / 19.4, 6125 25.8 / 24.1, 23367 58.6 / 47.8;
-    32 rows x 32 / 8, 6125 31.0 / 28.9, 23367 70.5 / 57.8; 16 rows x 32 / 4, 6125 20.7 / 21.7, 32000 52.0 / 45.8."""
+    head's pairs take several workgroups, which read the same keys, and spans stay at 512 keys or more, two a CU. Beyond 64
+    spans the fold is slow, whatever the cache holds, so 64 at most: us a layer with the q / k norm and the fold, more / 64 at
+    most, the cache nearly empty and 90 % full: 4 rows x 16 / 2 heads, 12288 slots 27.8 / 11.6, 28.3 / 12.7; 33024 slots
+    27.8 / 11.5, 31.8 / 18.4; 8 rows x 8 / 1, 70016 32.6 / 11.5, 41.6 / 27.3; 32 rows x 2 / 1, 16384 24.2 / 11.9, 24.4 / 13.9.
+    Measured on MI355X in the same way, at a workgroup a CU / at two: 8 rows x 32 / 8 heads, 6125 keys 16.4 / 17.8, 32000
+    32.1 / 32.0; 17 rows x 32 / 8, 3000 keys 18.3 / 19.4, 6125 25.8 / 24.1, 23367 58.6 / 47.8; 32 rows x 32 / 8, 6125 31.0 /
+    28.9, 23367 70.5 / 57.8; 16 rows x 32 / 4, 6125 20.7 / 21.7, 32000 52.0 / 45.8."""
     G = Hq // Hk
     z = -(-T * G // 32)
-    most = 1024 // G  # the fold's limit
+    # (the walk leaves an odd number of (row, head, span) states, whose outputs are not aligned, to the vector kernels)
+    most = 1024 // G if T * Hq % 2 else min(64, 1024 // G)
 
     def keys(per_cu: int) -> int:
         return max(1, -(-cap // max(1, min(most, per_cu * cus // (Hk * z)) * 128))) * 128

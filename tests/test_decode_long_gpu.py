@@ -113,7 +113,7 @@ def test_one_row_on_a_long_cache(card, n0):
     assert torch.equal(step.kv[:, :, :, :n0], kv[:, :, :, :n0]) and not bool(step.kv[:, :, :, n0 + 4 :].any())
 
 
-@pytest.mark.parametrize("T,cap", [(2, 17000), (3, 17000), (20, 9000), (32, 9000)])
+@pytest.mark.parametrize("T,cap", [(2, 9000), (2, 17000), (3, 17000), (20, 9000), (32, 9000)])
 @pytest.mark.parametrize("tree", [False, True])
 def test_passes_over_long_spans(card, T, cap, tree):
     """a pass whose attention walks spans of several batches from the fused rows, the pass's rows in the middle of the cache,

@@ -17,6 +17,14 @@ def test_a_passs_spans_cover_the_cache_in_whole_batches(T, Hq, Hk, cap):
     assert S * span >= cap and (S - 1) * span < cap
 
 
+@pytest.mark.parametrize("T", [2, 4, 17, 32])
+@pytest.mark.parametrize("Hq,Hk", [(1, 1), (8, 1), (4, 2), (16, 2), (9, 3), (32, 4)])
+@pytest.mark.parametrize("cap", [8192, 8193, 16384, 33024, 70016, 2000000])
+def test_a_passs_spans_stay_with_the_fast_fold(T, Hq, Hk, cap):
+    """(an odd number of states is left to the kernels that cut as many spans as the fold takes)"""
+    assert pass_spans(256, T, Hq, Hk, cap) <= 64 or T * Hq % 2 == 1
+
+
 @pytest.mark.parametrize("Hq,Hk", [(1, 1), (8, 1), (4, 2), (16, 2), (32, 4), (32, 8), (8, 8), (512, 256), (12, 4)])
 @pytest.mark.parametrize("cap", [64, 8191, 8192, 16383, 16384, 35200, 1000000])
 def test_a_steps_spans_cover_the_cache(Hq, Hk, cap):
