@@ -135,31 +135,41 @@ __global__ void __launch_bounds__(256) lane16_kernel(W w, const XT* __restrict__
 // and hand them round through a slab of LDS the group owns, where lane j then finds its columns j, j + 16, ... - one
 // request a lane for eight of its columns instead of eight. x is staged once a workgroup, as f32. The sums are the same
 // chain of fused multiply-adds in the same column order. Writes and reads of a slab are one wave's, which LDS serves in
-// program order: no barrier between them.
-template <int B, int NB, class XT>
-__global__ void __launch_bounds__(256) lane16_bf16_wide_kernel(const uint16_t* __restrict__ w, const XT* __restrict__ x,
-                                                               float* __restrict__ y, size_t rows, size_t cols, size_t b0,
-                                                               size_t btotal) {
+// program order: no barrier between them. TAIL: the row ends inside its last step (a multiple of 8 columns, so that rows
+// and pieces stay 16-byte aligned): the pieces past its end are the row's last piece again and their products are
+// dropped (x's place there holds whatever LDS held). Bound by the chain of a lane's fused multiply-adds and the two LDS
+// reads each takes, so few waves a CU are best: a router's workgroup is eight rows (128 threads). Measured with the
+// routing behind it, us: [32 x 2880] one row 22.3 (lane16_kernel) -> 9.6, 32 rows 43.9 (passes of four) -> 10.1;
+// [128 x 2048] 7.1 -> 6.4 (sixteen rows a workgroup -> eight), [128 x 4096] 9.5 -> 8.6.
+template <int B, int NB, class XT, bool TAIL, int NT>
+__global__ void __launch_bounds__(NT) lane16_bf16_wide_kernel(const uint16_t* __restrict__ w, const XT* __restrict__ x,
+                                                              float* __restrict__ y, size_t rows, size_t cols, size_t b0,
+                                                              size_t btotal) {
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr int BP = B == 3 ? 4 : B;  // a column's B values of x side by side, one LDS read
-    float* xs = reinterpret_cast<float*>(smem);           // [cols][BP]
-    unsigned char* slabs = smem + (size_t)BP * cols * 4;  // [16 groups][NB][256]
+    const int nchunks = (int)((cols + 127) / 128);
+    float* xs = reinterpret_cast<float*>(smem);                           // [nchunks * 128][BP]
+    unsigned char* slabs = smem + (size_t)BP * (size_t)nchunks * 128 * 4;  // [NT / 16 groups][NB][256]
     b0 += (size_t)blockIdx.y * B;
     const int tid = threadIdx.x, j = tid & 15, grp = tid >> 4;
-    const size_t r = (size_t)blockIdx.x * 16 + grp;
+    const size_t r = (size_t)blockIdx.x * (NT / 16) + grp;
     const bool live = r < rows;
     const uint4* wrow = reinterpret_cast<const uint4*>(w + (live ? r : rows - 1) * cols);
-    const int nchunks = (int)(cols / 128);
+    const int last = (int)(cols / 8) - 1;  // the row's last piece
     // a compiler vector, not HIP's uint4: an array of the struct type that lives across the loop below is kept in scratch
     // memory - written there as soon as it is loaded, which waits for the loads at once - and a vector's is not
     u32x4 raw[NB];
     auto request = [&](int n0) {
 #pragma unroll
-        for (int n = 0; n < NB; ++n)
-            raw[n] = *reinterpret_cast<const u32x4*>(wrow + (size_t)min(n0 + n, nchunks - 1) * 16 + j);
+        for (int n = 0; n < NB; ++n) {
+            if (TAIL)
+                raw[n] = *reinterpret_cast<const u32x4*>(wrow + min((n0 + n) * 16 + j, last));
+            else
+                raw[n] = *reinterpret_cast<const u32x4*>(wrow + (size_t)min(n0 + n, nchunks - 1) * 16 + j);
+        }
     };
     request(0);
-    // x in 16-byte pieces (rows are 16-byte aligned: cols is a multiple of 128), every piece of every row requested
+    // x in 16-byte pieces (rows are 16-byte aligned: cols is a multiple of 8), every piece of every row requested
     // before the first is spread out
     constexpr int PER = 16 / (int)sizeof(XT);  // values a piece
     const size_t pieces = cols / PER;
@@ -167,7 +177,7 @@ __global__ void __launch_bounds__(256) lane16_bf16_wide_kernel(const uint16_t* _
     for (int b = 0; b < B; ++b) {
         const bool have = b0 + b < btotal;
         const uint4* src = reinterpret_cast<const uint4*>(x + (have ? b0 + b : b0) * cols);
-        for (size_t i = tid; i < pieces; i += 256) {
+        for (size_t i = tid; i < pieces; i += NT) {
             const uint4 v = src[i];
             const uint32_t d[4] = {v.x, v.y, v.z, v.w};
             float* dst = xs + i * PER * BP + b;
@@ -199,7 +209,10 @@ __global__ void __launch_bounds__(256) lane16_bf16_wide_kernel(const uint16_t* _
                     const float wv = bf16_f32(*reinterpret_cast<const uint16_t*>(mine + n * 256 + 2 * (j + 16 * u)));
                     const size_t c = (size_t)(n0 + n) * 128 + j + 16 * u;
 #pragma unroll
-                    for (int i = 0; i < B; ++i) acc[i] = fmaf(wv, xs[c * BP + i], acc[i]);
+                    for (int i = 0; i < B; ++i) {
+                        const float sum = fmaf(wv, xs[c * BP + i], acc[i]);
+                        acc[i] = !TAIL || c < cols ? sum : acc[i];
+                    }
                 }
             }
         }
@@ -211,12 +224,12 @@ __global__ void __launch_bounds__(256) lane16_bf16_wide_kernel(const uint16_t* _
     }
 }
 
-template <int B, int NB, class XT>
-static bool launch_wide(const uint16_t* w, const XT* x, float* y, size_t rows, size_t cols, size_t b0, size_t b,
+template <int B, int NB, bool TAIL, int NT, class XT>
+static bool launch_wide_as(const uint16_t* w, const XT* x, float* y, size_t rows, size_t cols, size_t b0, size_t b,
                         unsigned passes, hipStream_t st) {
-    const size_t lds = (size_t)(B == 3 ? 4 : B) * cols * 4 + 16 * NB * 256;  // x, the slabs
+    const size_t lds = (size_t)(B == 3 ? 4 : B) * ((cols + 127) / 128 * 128) * 4 + NT / 16 * NB * 256;  // x, the slabs
     if (lds > (size_t)device_info().lds_bytes) return false;
-    auto kern = lane16_bf16_wide_kernel<B, NB, XT>;
+    auto kern = lane16_bf16_wide_kernel<B, NB, XT, TAIL, NT>;
     static bool raised = false;  // per instance; the attribute is the function's, set before its first large launch
     if (lds > 64 * 1024 && !raised) {
         if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -224,8 +237,26 @@ static bool launch_wide(const uint16_t* w, const XT* x, float* y, size_t rows, s
             return false;
         raised = true;
     }
-    hipLaunchKernelGGL(kern, dim3((unsigned)((rows + 15) / 16), passes), dim3(256), lds, st, w, x, y, rows, cols, b0, b);
+    constexpr int PER_WG = NT / 16;
+    hipLaunchKernelGGL(kern, dim3((unsigned)((rows + PER_WG - 1) / PER_WG), passes), dim3(NT), lds, st, w, x, y, rows, cols,
+                       b0, b);
     return true;
+}
+
+// a matrix small enough that what bounds a pass is a row's chain, not its bytes
+static bool router_sized(size_t rows, size_t cols) { return rows * cols <= (1u << 20); }
+
+template <int B, int NB, class XT>
+static bool launch_wide(const uint16_t* w, const XT* x, float* y, size_t rows, size_t cols, size_t b0, size_t b,
+                        unsigned passes, hipStream_t st) {
+    if constexpr (B == 1) {
+        if (router_sized(rows, cols)) {
+            if (cols % 128 == 0) return launch_wide_as<B, NB, false, 128>(w, x, y, rows, cols, b0, b, passes, st);
+            return launch_wide_as<B, NB, true, 128>(w, x, y, rows, cols, b0, b, passes, st);
+        }
+    }
+    if (cols % 128 == 0) return launch_wide_as<B, NB, false, 256>(w, x, y, rows, cols, b0, b, passes, st);
+    return launch_wide_as<B, NB, true, 256>(w, x, y, rows, cols, b0, b, passes, st);
 }
 
 template <class W, class XT>
@@ -233,14 +264,15 @@ static int32_t launch_lane16(const W& w, const XT* x, float* y, size_t rows, siz
     const unsigned grid = (unsigned)((rows + 15) / 16);
     size_t b0 = 0;
     if constexpr (std::is_same<W, W16Bf16>::value) {
-        if (cols % 128 == 0 && ((reinterpret_cast<uintptr_t>(w.w) | reinterpret_cast<uintptr_t>(x)) & 15) == 0) {
+        if (cols % 8 == 0 && ((reinterpret_cast<uintptr_t>(w.w) | reinterpret_cast<uintptr_t>(x)) & 15) == 0) {
             // every pass of four rows of x in one launch (the pass is the grid's second dimension), then the rest
             bool done = true;
-            // A few rows of x against a small matrix (a router at the verify widths): a pass a row, all in one launch.
-            // The matrix is re-read once a row out of L2, but every row's sums start at once, where passes of four
-            // rows take four times the arithmetic each behind a fourfold staging (8 rows against the 128 x 2048
-            // router: 13.2 -> 8.9 us). A (row, vector) sum is the same chain of operations in every form.
-            if (b > 1 && b <= 16 && rows * cols <= (1u << 20)) {
+            // Rows of x against a small matrix (a router at the verify widths): a pass a row, all in one launch. The
+            // matrix is re-read once a row out of L2, but every row's sums start at once, where passes of four rows
+            // take four times the arithmetic each behind a fourfold staging (32 / 64 rows, with the routing: [32 x 2880]
+            // 25.2 / 25.4 -> 10.1 / 10.3 us, [128 x 2048] 12.3 / 12.4 -> 7.9 / 9.7, [128 x 4096] 19.6 / 19.7 -> 10.8 /
+            // 17.3). A (row, vector) sum is the same chain of operations in every form.
+            if (b > 1 && b <= 64 && router_sized(rows, cols)) {
                 done = launch_wide<1, 16>(w.w, x, y, rows, cols, 0, b, (unsigned)b, st);
                 if (done) b0 = b;
             }

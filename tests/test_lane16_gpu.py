@@ -34,6 +34,23 @@ def test_bf16_rows_bits(card, rows, cols, b):
     assert np.array_equal(f32_bits(got), f32_bits(want))
 
 
+@pytest.mark.parametrize("rows,cols", [(32, 2880), (5, 8), (9, 120), (17, 136), (8, 2040), (67, 2056), (16, 4088), (400, 2632)])
+@pytest.mark.parametrize("b", [1, 2, 6, 33, 64, 65])
+def test_bf16_rows_that_end_inside_a_step(card, rows, cols, b):
+    """Rows of a multiple of 8 columns but not of 128: the kernel that takes 128 columns a step, its last step part of one;
+    at the widths of one launch a row of x, of four rows a pass, and of a matrix past the router's size. Infinities in the
+    rows' last columns reach their own row's sums and no other."""
+    w = weights_bf16(rows, cols, seed=402, std=1.0)
+    x = xs(b, cols, 403)
+    w[0, cols - 1] = float("inf")
+    got = card.gemv_lane16(w.cuda(), x.cuda()).cpu().numpy()
+    want = oracle.gemv_bf16(bits16(w), x.numpy(), threads=0)
+    assert np.array_equal(f32_bits(got), f32_bits(want))
+    xb = x.to(torch.bfloat16)
+    picks = card.moe_router(w.cuda(), xb.cuda(), 1)[0].cpu().numpy()  # the same rows of x as bf16
+    assert np.array_equal(f32_bits(picks), f32_bits(oracle.gemv_bf16(bits16(w), xb.float().numpy(), threads=0)))
+
+
 @pytest.mark.parametrize("rows,cols", [(64, 512), (9, 1040), (3, 16)])
 def test_p12_rows_bits(card, rows, cols):
     w = weights_bf16(rows, cols, seed=410)
