@@ -65,7 +65,7 @@ class Experts:
         x = hidden_states.reshape(-1, self.hidden_dim)
         if x.dtype != torch.bfloat16:
             raise ValueError("[moe] the card's experts take bf16 rows")
-        T, k = (int(s) for s in top_k_index.shape)
+        T, k = top_k_index.shape
         if self._gu is None or self._gu.shape[0] < T or self._gu.shape[1] != k:
             self._gu = torch.empty(T, k, 2 * self.intermediate_dim, dtype=torch.bfloat16, device=x.device)
         return self.card.moe_experts(self.gate_up, self.down, x.contiguous(), top_k_index.to(torch.int32).contiguous(),
@@ -91,7 +91,7 @@ class MxExpertsLayer:
         x = hidden_states.reshape(-1, self.hidden_dim)
         if x.dtype != torch.bfloat16:
             raise ValueError("[moe] the card's experts take bf16 rows")
-        T, k = (int(s) for s in top_k_index.shape)
+        T, k = top_k_index.shape
         if self._h is None or self._h.shape[0] < T or self._h.shape[1] != k:
             self._h = torch.empty(T, k, self.intermediate_dim, dtype=torch.bfloat16, device=x.device)
         return self.card.moe_experts_mx4(self.stacks, x.contiguous(), top_k_index.to(torch.int32).contiguous(),
