@@ -2,6 +2,8 @@
 // (moe.hip): staging x in LDS, the span loads, and the pair-wise products of one unit against the rows of x.
 #pragma once
 
+#include <type_traits>
+
 #include "btb_common.hpp"
 #include "btb_formats.hpp"
 
@@ -12,9 +14,10 @@ namespace btb {
 // [M, 2C] gate/up block, or made by the residual add + RMSNorm from the residual stream
 // ------------------------------------------------------------------------------------------------------------
 
-enum XMode { X_PLAIN = 0, X_SILU = 1, X_ADDNORM = 2 };
+enum XMode { X_PLAIN = 0, X_SILU = 1, X_ADDNORM = 2, X_ADDNORM_4 = 3 };
 
-// where x comes from. X_PLAIN: x [M, C]. X_SILU: x is gu [M, 2C]. X_ADDNORM: x is the residual h [M, C]; y the block
+// where x comes from. X_PLAIN: x [M, C]. X_SILU: x is gu [M, 2C]. X_ADDNORM (one row of 3073 to 4096 values: X_ADDNORM_4, a
+// kernel of its own, whose registers the other lengths' kernels do not carry): x is the residual h [M, C]; y the block
 // output added to it (or null), norm_w the norm's weight, h_out where the new residual is written (not h itself:
 // other workgroups are still reading it). With `ids` (X_ADDNORM only) x is an embedding table [vocab, C] and row m of
 // the residual is table[ids[m]] (an id outside the table is clamped into it): the step's first layer, whose residual
@@ -52,7 +55,7 @@ __device__ __forceinline__ float block_sum256(float v, float* red) {
 // LDS the staging needs for M rows of C values: the rows themselves, and for X_ADDNORM three raw rows (h, y and the
 // norm's weight) behind them
 __host__ __device__ constexpr size_t stage_lds_bytes(int xmode, int M, int C) {
-    return (size_t)(M + (xmode == X_ADDNORM ? 1 : 0)) * (size_t)C * 2;
+    return (size_t)(M + (xmode == X_ADDNORM || xmode == X_ADDNORM_4 ? 1 : 0)) * (size_t)C * 2;
 }
 
 // Leaves the rows in xs (a barrier included). 256 threads. `after_issue` is called once, right after the first loads
@@ -111,60 +114,72 @@ __device__ __forceinline__ void stage_x(uint32_t* xs, const XArgs& a, int M, int
         uint2* wkeep = rows4 + (size_t)M * n4;
         constexpr int PER = 3;  // words a thread holds at once: rows up to 3072 wide take one pass
         const bool writer = blockIdx.x == 0 && blockIdx.y == 0 && a.h_out != nullptr;
-        if (KEEP && MR == 1 && n4 <= PER * 256) {
+        if constexpr (MR == 1 && (KEEP || XMODE == X_ADDNORM_4)) {
             // One row, one pass (the decode step's own launches): the thread's words stay in registers between the
             // sum of squares and the scaling - nothing of them goes to LDS and comes back - and the one sum needs
             // one barrier, not two (its four partial sums are not written again). The arithmetic, its order and the
             // stores are the loop's below. Taken by the forms that widen in registers (the packed step 2.063 ->
             // 2.054 ms); the bf16 kernels lose by it (qkv 7.40 -> 7.50 us, the step 2.026 -> 2.035 ms) and keep the
-            // loop.
-            uint2 hv[PER], yv[PER], wv[PER];
-            size_t hrow = 0;
-            if (a.ids != nullptr) hrow = (size_t)min(max(a.ids[0], 0), a.vocab - 1);
-            const uint2* hs = reinterpret_cast<const uint2*>(a.x + hrow * C);
-            const uint2* ys = a.y == nullptr ? hs : reinterpret_cast<const uint2*>(a.y);
-            const uint2* ws = reinterpret_cast<const uint2*>(a.norm_w);
+            // loop. Rows of 3073 to 4096 columns, of every form: four words a thread. The loop takes them in two rounds,
+            // and the second round's loads wait behind the first weights: FP8 [6144 x 4096] 8.85 -> 7.3 us, [5120 x 3584]
+            // 8.0 -> 6.4, [24576 x 4096] with the gate / up fold 21.2 -> 20.0; bf16 [6144 x 4096] 11.2 -> 9.6, [5120 x
+            // 3584] 11.2 -> 9.8.
+            auto kept = [&](auto words) {
+                constexpr int WORDS = decltype(words)::value;  // a thread's
+                uint2 hv[WORDS], yv[WORDS], wv[WORDS];
+                size_t hrow = 0;
+                if (a.ids != nullptr) hrow = (size_t)min(max(a.ids[0], 0), a.vocab - 1);
+                const uint2* hs = reinterpret_cast<const uint2*>(a.x + hrow * C);
+                const uint2* ys = a.y == nullptr ? hs : reinterpret_cast<const uint2*>(a.y);
+                const uint2* ws = reinterpret_cast<const uint2*>(a.norm_w);
 #pragma unroll
-            for (int q = 0; q < PER; ++q) {
-                const int i = min(q * 256 + tid, n4 - 1);
-                hv[q] = hs[i];
-                yv[q] = ys[i];
-                wv[q] = ws[i];
-            }
-            after_issue();
-            const bool has_y = a.y != nullptr;
-            float f[PER][4];
-            float ss = 0.f;
-#pragma unroll
-            for (int q = 0; q < PER; ++q) {
-                const bool live = q * 256 + tid < n4;
-                const float h4[4] = {bf16lo_f32(hv[q].x), bf16hi_f32(hv[q].x), bf16lo_f32(hv[q].y), bf16hi_f32(hv[q].y)};
-                const float g[4] = {bf16lo_f32(yv[q].x), bf16hi_f32(yv[q].x), bf16lo_f32(yv[q].y), bf16hi_f32(yv[q].y)};
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float sum = bfround(h4[e] + g[e]);
-                    f[q][e] = has_y ? sum : h4[e];
-                    const float sq = fmaf(f[q][e], f[q][e], ss);
-                    ss = live ? sq : ss;
+                for (int q = 0; q < WORDS; ++q) {
+                    const int i = min(q * 256 + tid, n4 - 1);
+                    hv[q] = hs[i];
+                    yv[q] = ys[i];
+                    wv[q] = ws[i];
                 }
-                if (writer)
-                    reinterpret_cast<uint2*>(a.h_out)[min(q * 256 + tid, n4 - 1)] =
-                        make_uint2(f32x2_bf16(f[q][0], f[q][1]), f32x2_bf16(f[q][2], f[q][3]));
-            }
-            ss = group_sum_last<64>(ss);
-            if ((tid & 63) == 63) red[tid >> 6] = ss;
-            __syncthreads();
-            const float rstd = rsqrtf((((red[0] + red[1]) + red[2]) + red[3]) / (float)C + a.eps);
+                after_issue();
+                const bool has_y = a.y != nullptr;
+                float f[WORDS][4];
+                float ss = 0.f;
 #pragma unroll
-            for (int q = 0; q < PER; ++q) {
-                const float g[4] = {bf16lo_f32(wv[q].x), bf16hi_f32(wv[q].x), bf16lo_f32(wv[q].y), bf16hi_f32(wv[q].y)};
-                float o[4];
+                for (int q = 0; q < WORDS; ++q) {
+                    const bool live = q * 256 + tid < n4;
+                    const float h4[4] = {bf16lo_f32(hv[q].x), bf16hi_f32(hv[q].x), bf16lo_f32(hv[q].y), bf16hi_f32(hv[q].y)};
+                    const float g[4] = {bf16lo_f32(yv[q].x), bf16hi_f32(yv[q].x), bf16lo_f32(yv[q].y), bf16hi_f32(yv[q].y)};
 #pragma unroll
-                for (int e = 0; e < 4; ++e) o[e] = f[q][e] * rstd * (a.centered ? 1.f + g[e] : g[e]);
-                rows4[min(q * 256 + tid, n4 - 1)] = make_uint2(f32x2_bf16(o[0], o[1]), f32x2_bf16(o[2], o[3]));
+                    for (int e = 0; e < 4; ++e) {
+                        const float sum = bfround(h4[e] + g[e]);
+                        f[q][e] = has_y ? sum : h4[e];
+                        const float sq = fmaf(f[q][e], f[q][e], ss);
+                        ss = live ? sq : ss;
+                    }
+                    if (writer)
+                        reinterpret_cast<uint2*>(a.h_out)[min(q * 256 + tid, n4 - 1)] =
+                            make_uint2(f32x2_bf16(f[q][0], f[q][1]), f32x2_bf16(f[q][2], f[q][3]));
+                }
+                ss = group_sum_last<64>(ss);
+                if ((tid & 63) == 63) red[tid >> 6] = ss;
+                __syncthreads();
+                const float rstd = rsqrtf((((red[0] + red[1]) + red[2]) + red[3]) / (float)C + a.eps);
+#pragma unroll
+                for (int q = 0; q < WORDS; ++q) {
+                    const float g[4] = {bf16lo_f32(wv[q].x), bf16hi_f32(wv[q].x), bf16lo_f32(wv[q].y), bf16hi_f32(wv[q].y)};
+                    float o[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) o[e] = f[q][e] * rstd * (a.centered ? 1.f + g[e] : g[e]);
+                    rows4[min(q * 256 + tid, n4 - 1)] = make_uint2(f32x2_bf16(o[0], o[1]), f32x2_bf16(o[2], o[3]));
+                }
+                __syncthreads();
+            };
+            if constexpr (XMODE == X_ADDNORM_4) {
+                kept(std::integral_constant<int, 4>{});
+                return;
+            } else if (n4 <= PER * 256) {
+                kept(std::integral_constant<int, PER>{});
+                return;
             }
-            __syncthreads();
-            return;
         }
         if (MR > 1 && n4 <= PER * 256) {
             // Several rows, each one pass: every row's words are requested before anything waits - and before the

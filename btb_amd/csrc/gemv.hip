@@ -311,9 +311,16 @@ static int32_t launch_variant(const typename F::Params& p, const XArgs& xa, void
     // made once a CU, not three times side by side: qkv 7.36 -> 6.97 us, the step 1.967 -> 1.961 ms (the head level;
     // from two rows of x on and for the packed form it loses: 2.16 -> 2.21 ms at two rows, packed qkv 6.63 -> 7.42 us).
     constexpr bool BF16_NORM_ROW =
-        std::is_same<F, FmtBf16>::value && M == 1 && XMODE == X_ADDNORM && EPI == E_PLAIN;
+        std::is_same<F, FmtBf16>::value && M == 1 && (XMODE == X_ADDNORM || XMODE == X_ADDNORM_4) && EPI == E_PLAIN;
+    // FP8's gate / up rows at one row of x: five. At four the even cut below could leave two workgroups a CU, whose waves
+    // are too few to hide the widening: [19456 x 2560] 15.4 -> 12.5 us, [28672 x 3584] 21.8 -> 20.7, [25600 x 3328] 20.9 ->
+    // 19.6, [24576 x 4096] 20.0 -> 19.6; at six [24576 x 4096] takes 20.7, [24576 x 3200] 19.4 (17.3 at five).
+    constexpr bool FP8_GLU_ROW = std::is_same<F, FmtF8>::value && M == 1 && EPI != E_PLAIN;
     if (per_cu <= 0)
-        per_cu = BF16_NORM_ROW ? 2 : (EPI != E_PLAIN && M <= 2) ? 4 : std::is_same<F, FmtP12G>::value ? 5 : 6;
+        per_cu = BF16_NORM_ROW ? 2
+                 : FP8_GLU_ROW ? 5
+                 : (EPI != E_PLAIN && M <= 2) ? 4
+                 : std::is_same<F, FmtP12G>::value ? 5 : 6;
     const int cap_waves = dev.cus * per_cu * 4;
     // ... and of the counts from there to two more, the one whose workgroups fill the CUs' turns most evenly (when it
     // gains a twentieth or more): a launch ends with its fullest CU, and the forms that widen are bound by what a CU
@@ -461,6 +468,9 @@ template <class F, int XMODE, int EPI>
 static int32_t launch_by_m(const typename F::Params& p, const XArgs& xa, void* y, int R, int C, int M, hipStream_t st) {
     switch (M) {
         case 1:
+            if constexpr (XMODE == X_ADDNORM) {
+                if (C > 3072 && C <= 4096) return launch_by_lanes<F, 1, X_ADDNORM_4, EPI>(p, xa, y, R, C, st);
+            }
             return launch_by_lanes<F, 1, XMODE, EPI>(p, xa, y, R, C, st);
         case 2:
             return launch_by_lanes<F, 2, XMODE, EPI>(p, xa, y, R, C, st);

@@ -697,3 +697,40 @@ def test_fp8_rows_past_10240_columns(card, R, C, block, M):
     card.gemv_fp8(w, x.cuda(), y)
     check(y, oracle.gemv_fp8(q.view(torch.uint8).numpy(), s.numpy(), x.float().numpy(), threads=0))
     assert bool((room[M * R:] == 7.0).all())
+
+
+@pytest.mark.parametrize("form,C", [("bf16", 3080), ("bf16", 4088), ("bf16", 4096), ("pack12", 3088), ("pack12", 4096),
+                                    ("fp8", 3200), ("fp8", 4096), ("fp8", 4224), ("bf16", 3072), ("bf16", 4104)])
+@pytest.mark.parametrize("glu,with_y", [(False, True), (True, True), (False, False)])
+def test_one_row_norm_over_four_words_a_thread(card, form, C, glu, with_y):
+    """One row of x of 3073 to 4096 columns, made in one round of four words a thread (and the lengths either side):
+    `gemv_norm` and `gemv_embed_norm` with the bits of add_rmsnorm, then the matvec (then silu_mul)."""
+    R = 640
+    wf = weights_bf16(R, C, seed=700 + C)
+    if form == "fp8":
+        q, s = fp8.quantize(wf.float(), (128, 128 if C % 128 == 0 else C))
+        w = fp8.F8Weight(q.view(torch.uint8).cuda(), s.cuda(), R, C)
+        op = card.gemv_fp8
+    elif form == "pack12":
+        w, op = P12Weight.pack(wf.cuda(), card), card.gemv_p12
+    else:
+        w, op = wf.cuda(), card.gemv
+    table = acts_bf16(3, C, seed=701).cuda()
+    h = table[2:3].contiguous()
+    y = acts_bf16(1, C, seed=702).cuda() if with_y else None
+    nw = (1.0 + 0.1 * torch.randn(C, generator=torch.Generator().manual_seed(703))).to(torch.bfloat16).cuda()
+    h1, x1 = h.clone(), torch.empty_like(h)
+    card.add_rmsnorm(h1, y, nw, 1e-6, x1)
+    want = op(w, x1)
+    if glu:
+        m = torch.empty(1, R // 2, dtype=torch.bfloat16, device="cuda")
+        card.silu_mul(want, m)
+        want = m
+    h2, out = torch.empty_like(h), torch.empty_like(want)
+    card.gemv_norm(w, h, y, nw, 1e-6, h2, out, glu=glu)
+    assert torch.equal(out.view(torch.int16), want.view(torch.int16))
+    assert torch.equal(h2.view(torch.int16), h1.view(torch.int16))
+    if not with_y:
+        card.gemv_embed_norm(w, table, torch.tensor([2], dtype=torch.int32, device="cuda"), nw, 1e-6, h2.zero_(), out.zero_())
+        assert torch.equal(out.view(torch.int16), want.view(torch.int16))
+        assert torch.equal(h2.view(torch.int16), h1.view(torch.int16))
