@@ -72,6 +72,7 @@ static Knob g_knobs[] = {
     {"mfma_tile_rows", {-1}},
     {"mfma_stream_x", {-1}},
     {"mfma_direct", {-1}},
+    {"mfma_split", {-1}},
     {"mfma_direct_grid", {-1}},
     {"p12_pair_table", {-1}},
     {"moe_grouped", {-1}},

@@ -521,6 +521,11 @@ int32_t gemv_mfma_lds_p12(const uint8_t* lo, const uint8_t* hi4, const uint8_t* 
                           const uint8_t* esc_val, const int32_t* row_ptr, const void* x, void* y, int R, int C, int M,
                           hipStream_t st);
 
+// the matrix-core matvec of more than sixteen rows with the columns split over workgroups (gemv_mfma_split.hip)
+size_t mfma_split_floats(size_t R, size_t M);
+bool mfma_split_fits(size_t R, size_t C);
+int32_t gemv_mfma_split_bf16(const void* w, const void* x, void* y, int R, int C, int M, float* ws, hipStream_t st);
+
 // the direct-to-LDS form of the matrix-core matvec for the long rows of the block-scaled forms (gemv_mfma_dl.hip)
 bool mfma_dl_fits(int R, int C, int M);
 bool mfma_dl_fits_fp8(int R, int C, int M, int bm, int bn);
@@ -589,6 +594,25 @@ static size_t mx4_matrix_from(size_t R, size_t C) {
 }
 // (FP8 likewise: [4096 x 12288] at 3 / 4 rows 15.9 / 24.8 us on the vector kernel, 28.8 / 29.0 here)
 static size_t fp8_matrix_from(size_t R, size_t C) { return R * C >= (1u << 25) && C <= 10240 ? 3 : 5; }
+
+// Where the columns split over workgroups pay (bf16; the bits are the staged kernel's, so the line moves none). The split
+// saves each CU most of x (64 C bytes at 32 rows) and fills the CUs where tiles are few; it costs a second launch and the
+// partial sums' way out and back, which grow with R. Measured on MI355X over 48 shapes of 256 to 19456 rows by 1536 to 10240
+// columns, us staged / split at 8, 16, 17, 32 rows of x:
+//   [2560 x 9728] 12.3 / 14.2, 16.9 / 14.3, 23.0 / 15.6, 29.4 / 16.1; [8192 x 5120] 18.4 / 18.8, 20.3 / 19.4, 27.2 / 21.4,
+//   36.6 / 22.5; [2560 x 4096] 7.7 / 8.3, 8.8 / 8.7, 10.0 / 9.1, 12.4 / 9.5; [4096 x 4096] 9.1 / 10.2, 10.2 / 10.7, 11.3 / 11.8,
+//   14.1 / 12.3; [8192 x 4096] 14.2 / 15.1, 15.7 / 16.0, 16.8 / 18.0, 19.2 / 19.1; [19456 x 2560] 19.7 / 22.2, 21.0 / 24.4,
+//   22.0 / 27.2, 24.8 / 28.1; [2560 x 2560] 6.2 / 7.3, 7.0 / 7.6, 7.7 / 8.2, 9.0 / 8.6; [1024 x 3072] 6.4 / 5.8, 7.5 / 6.0,
+//   8.4 / 6.4, 10.2 / 6.7; [1024 x 1536] 4.1 / 5.2, 4.5 / 5.3, 5.0 / 5.6, 5.9 / 6.0; [1536 x 3072] 6.4 / 6.3, 7.3 / 6.7, 8.3 / 7.0,
+//   9.8 / 7.4; [16384 x 7168] 40.8 / 43.3, 43.7 / 44.5, 60.9 / 46.7, 82.6 / 47.8
+static bool split_pays(size_t M, size_t R, size_t C) {
+    if (tuning("mfma_split") >= 0) return tuning("mfma_split") != 0;
+    if (M > 16) return C > 4096 || (C >= 2048 && M * C >= 25000 + 14 * R);
+    if (M < 8 || C < 2560) return false;
+    if (R <= 1024) return true;
+    if (R <= 2048) return M * C >= 30 * R;
+    return C > 7168 ? M >= 14 : C > 4096 && M >= 15 && R <= 12288;
+}
 
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 static bool aligned2(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 1u) == 0; }
@@ -689,6 +713,27 @@ int32_t btb_hip_gemv_bf16(const void* w, const void* x, void* y, size_t R, size_
     }
     FmtBf16::Params p{static_cast<const uint4*>(w)};
     return run_rows<FmtBf16, X_PLAIN, E_PLAIN>(p, plain_x(x), y, R, C, M, static_cast<hipStream_t>(stream));
+}
+
+size_t btb_hip_gemv_bf16_floats(size_t R, size_t C, size_t M) {
+    if (check_dims(R, C, M, FmtBf16::UW) != OK || !wide_pass(Form::BF16, M, R, C) || !mfma_split_fits(R, C) || !split_pays(M, R, C))
+        return 0;
+    return mfma_split_floats(R, M);
+}
+
+int32_t btb_hip_gemv_bf16_ws(const void* w, const void* x, void* y, size_t R, size_t C, size_t M, float* ws, void* stream) {
+    if (w == nullptr || x == nullptr || y == nullptr) return ERR_NULL;
+    if (!aligned16(ws)) return ERR_DOMAIN;
+    if (ws == nullptr || btb_hip_gemv_bf16_floats(R, C, M) == 0) return btb_hip_gemv_bf16(w, x, y, R, C, M, stream);
+    if (!aligned16(w) || !aligned16(x) || !aligned2(y)) return ERR_DOMAIN;
+    const uint16_t* xp = static_cast<const uint16_t*>(x);
+    uint16_t* yp = static_cast<uint16_t*>(y);
+    for (size_t m0 = 0; m0 < M; m0 += 32) {
+        const int32_t rc = gemv_mfma_split_bf16(w, xp + m0 * C, yp + m0 * R, (int)R, (int)C, (int)(M - m0 < 32 ? M - m0 : 32), ws,
+                                                static_cast<hipStream_t>(stream));
+        if (rc != OK) return rc;
+    }
+    return OK;
 }
 
 int32_t btb_hip_gemv_silu_bf16(const void* w, const void* gu, void* y, size_t R, size_t C, size_t M, void* stream) {

@@ -37,6 +37,8 @@ SIGNATURES: dict[str, tuple[Any, list[Any]]] = {
     "btb_hip_set_tuning": (_i32, [ctypes.c_char_p, _i32]),
     "btb_hip_stream_probe": (_i32, [_vp, _sz, _vp, _vp]),
     "btb_hip_gemv_bf16": (_i32, [_vp, _vp, _vp, _sz, _sz, _sz, _vp]),
+    "btb_hip_gemv_bf16_floats": (_sz, [_sz, _sz, _sz]),
+    "btb_hip_gemv_bf16_ws": (_i32, [_vp, _vp, _vp, _sz, _sz, _sz, _vp, _vp]),
     "btb_hip_gemv_silu_bf16": (_i32, [_vp, _vp, _vp, _sz, _sz, _sz, _vp]),
     "btb_hip_gemv_glu_silu_bf16": (_i32, [_vp, _vp, _vp, _sz, _sz, _sz, _vp]),
     "btb_hip_gemv_bf16_norm": (_i32, [_vp, _vp, _vp, _vp, ctypes.c_float, _i32, _vp, _vp, _sz, _sz, _sz, _i32, _vp]),
@@ -294,7 +296,13 @@ class HipCard(CardLaunch):
             self._need(y, torch.bfloat16, "y")
             if y.numel() != M * R:
                 raise ValueError(f"[hip] gemv: y holds {y.numel()} elements, the product has {M * R}")
-        self._call("btb_hip_gemv_bf16", _p(w), _p(x), _p(y), R, C, M, _stream())
+        # a wide pass over some shapes splits its columns over workgroups and takes a workspace (this call's own)
+        floats = self.lib.btb_hip_gemv_bf16_floats(R, C, M) if M >= 8 else 0
+        if floats:
+            ws = torch.empty(floats, dtype=torch.float32, device=w.device)
+            self._call("btb_hip_gemv_bf16_ws", _p(w), _p(x), _p(y), R, C, M, _p(ws), _stream())
+        else:
+            self._call("btb_hip_gemv_bf16", _p(w), _p(x), _p(y), R, C, M, _stream())
         return y
 
     def gemv_silu(self, w: torch.Tensor, gu: torch.Tensor, y: torch.Tensor | None = None) -> torch.Tensor:

@@ -299,3 +299,37 @@ def test_refusals_launch_nothing(card):
     assert L.btb_hip_gemv_bf16(None, card.ptr(ctypes.c_void_p, x), card.ptr(ctypes.c_void_p, y), 0, 64, 1, None) == -1  # null before domain
     torch.cuda.synchronize()
     assert torch.all(y == 7.0)
+
+
+@pytest.mark.parametrize("R,C", [(16, 1312), (17, 2592), (33, 2560), (100, 3008), (520, 9728), (1001, 4096), (2560, 9728),
+                                 (4112, 10240), (2064, 7168)])
+@pytest.mark.parametrize("M", [5, 8, 16, 17, 31, 32, 33, 50])
+def test_columns_split_over_workgroups_change_no_bit(card, R, C, M):
+    """The wide passes whose columns are split over workgroups (knob mfma_split = 1 wherever the shape fits) against the staged
+    kernel (0), bit for bit: tiles that overlap, slices of different lengths and without columns, passes of 32 rows and the
+    rest. `gemv` picks by shape; a workspace of NULL is the plain call."""
+    w, x = weights_bf16(R, C, seed=180).cuda(), acts_bf16(M, C, seed=181).cuda()
+    L, y = card.lib, torch.empty(M, R, dtype=torch.bfloat16, device="cuda")
+    try:
+        card.set_tuning("mfma_split", 0)
+        want = card.gemv(w, x)
+        assert L.btb_hip_gemv_bf16_floats(R, C, M) == 0
+        card.set_tuning("mfma_split", 1)
+        floats = L.btb_hip_gemv_bf16_floats(R, C, M)
+        if floats:  # the staged kernel's shapes only (M = 5 with few columns, ragged rows past 4096 columns: others')
+            ws = torch.full((floats + 64,), float("nan"), device="cuda")
+            p = lambda t: ctypes.c_void_p(t.data_ptr())
+            assert L.btb_hip_gemv_bf16_ws(p(w), p(x), p(y), R, C, M, p(ws), None) == 0
+            torch.cuda.synchronize()
+            assert torch.equal(y.view(torch.int16), want.view(torch.int16))
+            assert torch.isnan(ws[floats:]).all()
+            assert L.btb_hip_gemv_bf16_ws(p(w), p(x), p(y), R, C, M, ctypes.c_void_p(ws.data_ptr() + 4), None) == -6
+            assert L.btb_hip_gemv_bf16_ws(p(w), p(x), p(y.zero_()), R, C, M, None, None) == 0
+            torch.cuda.synchronize()
+            assert torch.equal(y.view(torch.int16), want.view(torch.int16))
+        else:
+            assert M < 8 or R % 16 != 0 or C > 10240
+    finally:
+        card.set_tuning("mfma_split", -1)
+    assert torch.equal(card.gemv(w, x).view(torch.int16), want.view(torch.int16))
+
