@@ -12,6 +12,8 @@
 //
 // Nothing goes back to the host between the steps, so the layer records into a hipGraph.
 
+#include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "btb_common.hpp"
@@ -587,12 +589,41 @@ static int lanes_for_mx4(int units) {
     return 16;
 }
 
+// The gate/up launch of `whole` workgroups an expert, each wave one tile, made smaller by a whole divisor where `wgs` of them
+// have work in all: what a workgroup does before its first product - its picks, then x, then weights that need the picks - then
+// costs more than the occupancy its successor brings. us a layer without the router, divisor 1 / 2 / 4 / 8:
+//   bf16: 128 experts of which 8, 2048 / 768, 8 rows (40 working workgroups a CU at 1) 95.4 / 87.3 / 85.8 / 88.0, 16 rows (61) 166 /
+//   148 / 143 / 146; 32 of which 4, 2048 / 1536, 8 rows (31) 98.4 / 89.9 / 85.8 / 89.4: nine a CU. Below eight rows, where a
+//   workgroup is a pair's: level or slower.
+//   MXFP4: gpt-oss (32 of 4, 2880 / 2880) 4 rows (11) 57.8 / 56.3 / 55.8 / 65.2, 8 rows (15) 108 / 100 / 100 / 107, 16 rows (20) 189
+//   / 176 / 173 / 181; 128 of 8, 2048 / 768, 8 rows (10) 44.9 / 41.3 / 41.3 / 47.2, 1 row (1.5) 11.9 / 12.7 / 15.1: four.
+static int gate_up_grid(int whole, double wgs, double per_cu) {
+    const int div = std::min((int)(wgs / (per_cu * device_info().cus) + 0.5), 4);
+    return div <= 1 ? whole : (whole + div - 1) / div;
+}
+// The down launch of `whole` workgroups a row of x. Two rows that picked an expert read the same rows of its matrix: with a
+// multiple of eight workgroups a row the same ones of every row are on one die, and with no more of them than are resident at
+// once they run side by side, so the second reads that die's L2. bf16, us a layer without the router, workgroups a CU as many
+// as tiles / here: 128 of 8, 8 rows 85.8 / 82.9, 16 rows 143 / 136, 32 rows 233 / 212; 32 of 4, 2048 / 1536, 4 / 8 / 16 rows 54.9 / 50.6,
+// 89.6 / 73.8, 142 / 102; 16 of 2, 1024 / 512, whose waves have 2 KB on their way each, 32 rows at two / four a CU 40.9 / 35.3 (56.7).
+// (A third of the workgroups instead of a quarter, no multiple of eight: 86.2 and 147 for the first two.) MXFP4's are bound by
+// the widening and keep a wave a tile.
+static int down_grid(int whole, int T, bool widens, size_t wave_bytes) {
+    if (T == 1) return whole;
+    const int eights = (whole + 7) / 8 * 8;
+    const int most = std::max(8, (wave_bytes >= 8192 ? 2 : 4) * device_info().cus / T / 8 * 8);
+    return widens || T < 4 ? eights : std::min(eights, most);
+}
+// the experts that T rows of k picks out of E name, were they drawn evenly
+static double distinct_experts(int E, int k, int T) { return E * (1.0 - std::pow(1.0 - (double)k / E, T)); }
+
 template <class F, bool OSS, int LPR>
 static int32_t launch_gate_up(Stack stack, const void* x, const int32_t* idx, void* gu, int R, int C, int k, int E,
                               int pairs, Glu glu, hipStream_t st) {
     constexpr int RPW = 2, U = 4, G = WAVE / LPR;
+    constexpr bool MX = std::is_same<F, FmtMx4>::value;
     const int ntiles = (R / 2 + G - 1) / G;
-    const int grid = (ntiles + 3) / 4;
+    const int whole = (ntiles + 3) / 4;
     // From eight rows on, the rows that share an expert go through it together. Fewer rows share few experts (4 rows of
     // top-8 over 128 experts: 30 distinct of 32 picks) and the wider pass costs more than the sharing saves: measured on
     // the Qwen3-30B-A3B shape, a layer takes 64 against 62 us at 4 rows, 88 against 86 at 6, 106 against 109 at 8, 180
@@ -611,10 +642,12 @@ static int32_t launch_gate_up(Stack stack, const void* x, const int32_t* idx, vo
                                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
             if (e != hipSuccess) return hip_status(e, "hipFuncSetAttribute");
         }
+        const int grid = gate_up_grid(whole, whole * distinct_experts(E, k, pairs / k), MX ? 4 : 9);
         hipLaunchKernelGGL(kern, dim3(grid, pairs), dim3(256), lds, st, stack, static_cast<const uint16_t*>(x), idx,
                            static_cast<uint16_t*>(gu), R, C, k, E, pairs, glu);
         return hip_status(hipGetLastError(), "moe gate_up launch");
     }
+    const int grid = MX ? gate_up_grid(whole, (double)whole * pairs, 4) : whole;
     hipLaunchKernelGGL((moe_gate_up_kernel<F, OSS, LPR, RPW, U>), dim3(grid, pairs), dim3(256), (size_t)C * 2, st, stack,
                        static_cast<const uint16_t*>(x), idx, static_cast<uint16_t*>(gu), R, C, k, E, glu);
     return hip_status(hipGetLastError(), "moe gate_up launch");
@@ -625,7 +658,8 @@ static int32_t launch_down(Stack stack, const void* gu, const int32_t* idx, cons
                            int E, int T, const void* bias, hipStream_t st) {
     constexpr int RPW = 1, G = WAVE / LPR;
     const int ntiles = (R + G * RPW - 1) / (G * RPW);
-    const int grid = (ntiles + 3) / 4;
+    const int whole = (ntiles + 3) / 4;
+    const int grid = down_grid(whole, T, std::is_same<F, FmtMx4>::value, (size_t)k * C * 2);
     const size_t lds = (size_t)k * C * 2;
     // a row of at most three units a lane (the 768-wide experts of the C4 shape: 96 bf16 units over 64 lanes, 24 MXFP4
     // units over 16): all eight picks' rows in one request

@@ -321,3 +321,29 @@ def test_mxfp4_experts_refusals(card):
     assert L.btb_hip_moe_experts_mxfp4(*a, p(y), None, p(x), p(idx), p(w), p(h), p(y), 2, 2, 4, 64, 64, 0, 0.0, 0.0,
                                        None) == -6          # a bias without the gpt-oss form
     assert bool((y == 0).all())
+
+
+@pytest.mark.parametrize("H_,I_,k", [(1480, 520, 3), (2048, 1536, 4), (264, 64, 2)])
+@pytest.mark.parametrize("T", [2, 4, 13, 33])
+@pytest.mark.parametrize("form", ["bf16", "mxfp4"])
+def test_how_the_experts_launches_are_cut_changes_no_bit(card, form, H_, I_, k, T):
+    """The grids of the experts' launches follow the rows of x (fewer workgroups than tiles, a multiple of eight a row): every
+    row of a pass has the bits of that row alone."""
+    from btb_amd.moe import MxExpertsLayer
+
+    E_ = 16
+    if form == "mxfp4":
+        H_, I_ = (H_ + 31) // 32 * 32, (I_ + 31) // 32 * 32
+        layer = MxExpertsLayer(card, to_gpu(mx_stacks(560, E_, I_, H_)), oss=False)
+    else:
+        g = gen(561)
+        layer = Experts(card, (torch.randn(E_, 2 * I_, H_, generator=g) * 0.02).to(torch.bfloat16).cuda(),
+                        (torch.randn(E_, H_, I_, generator=g) * 0.02).to(torch.bfloat16).cuda())
+    x = acts_bf16(T, H_, seed=562).cuda()
+    g = gen(563)
+    picks = torch.stack([torch.randperm(E_, generator=g)[:k] for _ in range(T)]).to(torch.int32).cuda()
+    w = torch.rand(T, k, generator=g).to(torch.bfloat16).cuda()
+    y = layer(x, picks, w).clone()
+    for t in range(T):
+        one = layer(x[t : t + 1].contiguous(), picks[t : t + 1].contiguous(), w[t : t + 1].contiguous())
+        assert torch.equal(y[t : t + 1].view(torch.int16), one.view(torch.int16)), t
