@@ -5,15 +5,16 @@
 //   2. p12_table_kernel   the table: the 15 most frequent high bytes, equal counts by ascending byte value; with it the
 //                         pair table, the byte -> code map and the number of escapes (n less what the table covers)
 //   3. p12_encode_kernel  low bytes and codes (2 B read, 1.5 B written a weight), escapes counted a chunk of 2048
-//   4. p12_emit_kernel    the escape list in ascending order out of the codes (0.5 B a weight read back), and every
-//                         row's first entry in it
+//                         and listed a workgroup of sixteen chunks as they are met
+//   4. p12_emit_kernel    the workgroups' lists end to end, and every row's first entry; a workgroup whose list was too
+//                         long to keep is read out of its codes (0.5 B a weight)
 //
 // The list's length has to be known on the host before the list can be allocated. It is known after the table's launch, so
 // the host waits for that one (an event) while the encoder is already queued behind it.
 //
-// Bound: HBM, 2 + 2 + 1.5 + 0.5 B a weight; the second read of a tensor that fits the 256 MB last-level cache comes out
-// of that. [19456 x 2560] packed, with its rows' words, and widened back: 1456 us with the packing in torch, 118 in these launches: 27 us for the
-// histogram, 4 for the table, 28 to encode (6.2 TB/s), 15 for the list.
+// Bound: HBM, 2 + 2 + 1.5 B a weight; the second read of a tensor that fits the 256 MB last-level cache comes out
+// of that. [19456 x 2560] packed, with its rows' words, and widened back: 1456 us with the packing in torch, 103 in these
+// launches with every list read out of the codes (15 us of it), 92 with the lists kept (4).
 
 #include "btb_common.hpp"
 #include "btb_formats.hpp"
@@ -25,8 +26,12 @@ namespace btb {
 
 constexpr int P12_CHUNK = 2048;          // weights a wave encodes at a time: four 16-byte loads a lane
 constexpr int P12_BLOCK = 16;            // chunks a workgroup: four waves, four chunks each
+constexpr int P12_WAVE_LIST = 64;        // escapes a wave of the encoder lists (its four chunks of a matrix of weights hold two)
+constexpr int P12_LIST = 4 * P12_WAVE_LIST;
+constexpr uint32_t P12_LISTED = 0x80000000u;  // of a workgroup's count: the list holds its escapes
 constexpr int P12_COPIES = 32;           // copies of each LDS counter, one a lane of a half wave: no two lanes meet
-// words of the workspace: the counters, the byte -> code map, then a count a workgroup of chunks and a count a chunk
+// words of the workspace: the counters, the byte -> code map, then a count a workgroup of chunks, a count a chunk and a
+// list a workgroup: low byte | high byte << 8 | place among the workgroup's weights << 16
 constexpr int P12_HIST = 0, P12_CODES = 256, P12_BLOCKS = 256 + 64;
 static size_t p12_chunks(size_t n) { return (n + P12_CHUNK - 1) / P12_CHUNK; }
 static size_t p12_blocks(size_t n) { return (p12_chunks(n) + P12_BLOCK - 1) / P12_BLOCK; }
@@ -124,9 +129,10 @@ __device__ __forceinline__ uint32_t escape_marks(uint32_t codes) {
 __global__ void __launch_bounds__(256) p12_encode_kernel(const uint4* __restrict__ t, size_t n,
                                                          const uint32_t* __restrict__ code_map, uint2* __restrict__ lo,
                                                          uint32_t* __restrict__ hi4, uint32_t* __restrict__ block_counts,
-                                                         uint32_t* __restrict__ counts) {
+                                                         uint32_t* __restrict__ counts, uint32_t* __restrict__ lists) {
     __shared__ uint32_t map32[64];
     __shared__ uint32_t sums[4];
+    __shared__ uint32_t found[4][P12_WAVE_LIST];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const size_t units = n / 8;
     if (tid < 64) map32[tid] = code_map[tid];
@@ -141,7 +147,11 @@ __global__ void __launch_bounds__(256) p12_encode_kernel(const uint4* __restrict
         uint4 v[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) v[j] = units > 0 ? t[min(u0 + 64 * j, units - 1)] : make_uint4(0, 0, 0, 0);
-        uint32_t esc = 0;
+        uint32_t total = 0;  // the chunk's escapes, the same in every lane
+        const uint32_t place0 = (uint32_t)(wave * (P12_BLOCK / 4) + k) * P12_CHUNK;  // the chunk among the workgroup's weights
+        auto list = [&](uint32_t at, uint32_t place, uint32_t weight) {
+            if (at < P12_WAVE_LIST) found[wave][at] = weight | (place << 16);
+        };
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const size_t u = u0 + 64 * j;
@@ -153,54 +163,111 @@ __global__ void __launch_bounds__(256) p12_encode_kernel(const uint4* __restrict
                 c |= (uint32_t)map[(h0 >> (8 * e)) & 255u] << (4 * e);
                 c |= (uint32_t)map[(h1 >> (8 * e)) & 255u] << (4 * e + 16);
             }
+            const uint32_t marks = u < units ? escape_marks(c) : 0u;
             if (u < units) {
                 lo[u] = make_uint2(__builtin_amdgcn_perm(v[j].y, v[j].x, 0x06040200u),
                                    __builtin_amdgcn_perm(v[j].w, v[j].z, 0x06040200u));
                 hi4[u] = c;
-                esc += __popc(escape_marks(c));
+            }
+            if (__ballot(marks != 0) != 0) {  // rare: the lanes' escapes in ascending order
+                const uint32_t m = (uint32_t)__popc(marks);  // 0 .. 8 a lane: four bits, a ballot each
+                uint32_t before = 0, all = 0;
+#pragma unroll
+                for (int b = 0; b < 4; ++b) {
+                    const uint64_t w = __ballot((m >> b) & 1u);
+                    before += (uint32_t)__popcll(w & ((1ull << lane) - 1)) << b;
+                    all += (uint32_t)__popcll(w) << b;
+                }
+                uint32_t at = wave_total + total + before;
+                for (uint32_t left = marks; left != 0; left &= left - 1, ++at) {
+                    const uint32_t e = (uint32_t)(__ffs((int)left) - 1) / 4;
+                    const uint32_t lo2 = e & 2 ? v[j].y : v[j].x, hi2 = e & 2 ? v[j].w : v[j].z;
+                    const uint32_t pair = e & 4 ? hi2 : lo2;
+                    list(at, place0 + (uint32_t)(64 * j + lane) * 8 + e, e & 1 ? pair >> 16 : pair & 0xFFFFu);
+                }
+                total += all;
             }
         }
         // the tail (n % 8 weights) belongs to the last chunk: its first lane takes it, a code byte a pair
-        if (chunk == chunks - 1 && lane == 0) {
-            const uint16_t* s = reinterpret_cast<const uint16_t*>(t);
-            uint8_t* lo8 = reinterpret_cast<uint8_t*>(lo);
-            uint8_t* hi8 = reinterpret_cast<uint8_t*>(hi4);
-            for (size_t i = units * 8; i < n; i += 2) {
-                uint32_t c = 0;
-                for (size_t e = i; e < min(i + 2, n); ++e) {
-                    lo8[e] = (uint8_t)s[e];
-                    const uint32_t m = map[s[e] >> 8];
-                    c |= m << (4 * (e - i));
-                    esc += m == 15u ? 1u : 0u;
+        if (chunk == chunks - 1 && units * 8 < n) {
+            uint32_t tail = 0;
+            if (lane == 0) {
+                const uint16_t* s = reinterpret_cast<const uint16_t*>(t);
+                uint8_t* lo8 = reinterpret_cast<uint8_t*>(lo);
+                uint8_t* hi8 = reinterpret_cast<uint8_t*>(hi4);
+                for (size_t i = units * 8; i < n; i += 2) {
+                    uint32_t c = 0;
+                    for (size_t e = i; e < min(i + 2, n); ++e) {
+                        lo8[e] = (uint8_t)s[e];
+                        const uint32_t m = map[s[e] >> 8];
+                        c |= m << (4 * (e - i));
+                        if (m == 15u) list(wave_total + total + tail++, place0 + (uint32_t)(e - chunk * P12_CHUNK), s[e]);
+                    }
+                    hi8[i / 2] = (uint8_t)c;
                 }
-                hi8[i / 2] = (uint8_t)c;
             }
-        }
-        uint32_t total = 0;
-        if (__ballot(esc != 0) != 0) {
-#pragma unroll
-            for (int b = 0; b < 6; ++b) total += (uint32_t)__popcll(__ballot((esc >> b) & 1u)) << b;  // at most 39 a lane
+            total += __builtin_amdgcn_readfirstlane(tail);
         }
         if (lane == 0) counts[chunk] = total;
         wave_total += total;
     }
     if (lane == 0) sums[wave] = wave_total;
     __syncthreads();
-    if (tid == 0) block_counts[blockIdx.x] = sums[0] + sums[1] + sums[2] + sums[3];
+    const bool listed = max(max(sums[0], sums[1]), max(sums[2], sums[3])) <= P12_WAVE_LIST;
+    uint32_t first = 0;
+    for (int w = 0; w < wave; ++w) first += sums[w];
+    if (listed && lane < (int)wave_total) lists[(size_t)blockIdx.x * P12_LIST + first + lane] = found[wave][lane];
+    if (tid == 0) block_counts[blockIdx.x] = (sums[0] + sums[1] + sums[2] + sums[3]) | (listed ? P12_LISTED : 0u);
 }
 
-// The escape list out of the codes. A workgroup takes the chunks one of the encoding workgroups took; where its part
-// of the list begins is the sum of those workgroups' counts before it (summing the chunks' own counts, sixteen times
-// as many: 20 us for [19456 x 2560]); 15 us: a chain of three trips to memory - codes, the escapes' weights, the stores.
-// Row r's first entry (row_ptr) is written by the chunk that holds the row's first weight.
+// The escape list. A workgroup takes the chunks one of the encoding workgroups took; where its part of the list begins is the
+// sum of those workgroups' counts before it. Where the encoder kept its escapes they are copied, and a row's first entry
+// (row_ptr, for the rows whose first weight lies here) is a search among them: [19456 x 2560] 15 us -> 4. Else they come
+// out of the codes, a chain of three trips to memory - codes, the escapes' weights, the stores.
 __global__ void __launch_bounds__(256) p12_emit_kernel(const uint16_t* __restrict__ t, const uint8_t* __restrict__ hi4,
                                                        size_t n, const uint32_t* __restrict__ block_counts,
-                                                       const uint32_t* __restrict__ counts, size_t n_esc,
+                                                       const uint32_t* __restrict__ counts,
+                                                       const uint32_t* __restrict__ lists, size_t n_esc,
                                                        int32_t* __restrict__ esc_idx, uint8_t* __restrict__ esc_val,
                                                        size_t cols, size_t rows, int32_t* __restrict__ row_ptr) {
     __shared__ uint32_t part[4];
+    __shared__ uint32_t kept[P12_LIST];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const size_t chunks = (n + P12_CHUNK - 1) / P12_CHUNK;
+    const uint32_t here_all = block_counts[blockIdx.x];
+    const uint32_t entry = lists[(size_t)blockIdx.x * P12_LIST + tid];  // past the count: whatever lies there, unused
+    uint32_t s = 0;
+#pragma unroll 4
+    for (size_t i = tid; i < blockIdx.x; i += 256) s += block_counts[i] & ~P12_LISTED;
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) s += __shfl_xor(s, d, WAVE);
+    if (lane == 0) part[wave] = s;
+    if (here_all & P12_LISTED) {  // uniform
+        const uint32_t count = here_all & ~P12_LISTED;
+        kept[tid] = entry >> 16;
+        __syncthreads();
+        const uint32_t base = part[0] + part[1] + part[2] + part[3];
+        const size_t b0 = (size_t)blockIdx.x * P12_BLOCK * P12_CHUNK, b1 = min(b0 + (size_t)P12_BLOCK * P12_CHUNK, n);
+        if (tid < (int)count && base + tid < n_esc) {
+            esc_idx[base + tid] = (int32_t)(b0 + (entry >> 16));
+            esc_val[base + tid] = (uint8_t)(entry >> 8);
+        }
+        const uint32_t r0 = ((uint32_t)b0 + (uint32_t)cols - 1) / (uint32_t)cols;  // below 2^32: n and cols are below 2^31
+        for (size_t r = r0 + (size_t)tid; r < rows && r * cols < b1; r += 256) {
+            const uint32_t o = (uint32_t)(r * cols - b0);  // the row's first weight among the workgroup's
+            uint32_t below = 0, above = count;
+            while (below < above) {
+                const uint32_t mid = (below + above) / 2;
+                if (kept[mid] < o)
+                    below = mid + 1;
+                else
+                    above = mid;
+            }
+            row_ptr[r] = (int32_t)(base + below);
+        }
+        if (rows != 0 && b1 == n && tid == 0) row_ptr[rows] = (int32_t)n_esc;
+        return;
+    }
     const size_t mine = (size_t)blockIdx.x * P12_BLOCK + (size_t)wave * (P12_BLOCK / 4);
     // everything that does not depend on anything is asked for first: the wave's codes, the counts
     uint32_t marks[P12_BLOCK / 4][4];
@@ -213,12 +280,6 @@ __global__ void __launch_bounds__(256) p12_emit_kernel(const uint16_t* __restric
         }
     const size_t c16 = (size_t)blockIdx.x * P12_BLOCK + (lane & (P12_BLOCK - 1));
     const uint32_t count16 = c16 < chunks ? counts[c16] : 0;  // lane l: the count of the workgroup's chunk l % 16
-    uint32_t s = 0;
-#pragma unroll 4
-    for (size_t i = tid; i < blockIdx.x; i += 256) s += block_counts[i];
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) s += __shfl_xor(s, d, WAVE);
-    if (lane == 0) part[wave] = s;
     __syncthreads();
     uint32_t base = part[0] + part[1] + part[2] + part[3];
     for (int c = 0; c < wave * (P12_BLOCK / 4); ++c) base += __builtin_amdgcn_readlane(count16, c);
@@ -287,7 +348,7 @@ using namespace btb;
 
 extern "C" {
 
-size_t btb_hip_p12_pack_words(size_t n) { return P12_BLOCKS + p12_blocks(n) + p12_chunks(n); }
+size_t btb_hip_p12_pack_words(size_t n) { return P12_BLOCKS + p12_blocks(n) * (1 + P12_LIST) + p12_chunks(n); }
 
 int32_t btb_hip_p12_pack(const void* t, size_t n, void* lo, void* hi4, void* table, void* pairs, void* work,
                          int32_t* host_total, void* stream) {
@@ -315,7 +376,7 @@ int32_t btb_hip_p12_pack(const void* t, size_t n, void* lo, void* hi4, void* tab
     const size_t blocks = p12_blocks(n);
     hipLaunchKernelGGL(p12_encode_kernel, dim3((unsigned)blocks), dim3(256), 0, st, static_cast<const uint4*>(t), n,
                        w + P12_CODES, static_cast<uint2*>(lo), static_cast<uint32_t*>(hi4),
-                       w + P12_BLOCKS, w + P12_BLOCKS + blocks);
+                       w + P12_BLOCKS, w + P12_BLOCKS + blocks, w + P12_BLOCKS + blocks + p12_chunks(n));
     if (e == hipSuccess) e = hipGetLastError();
     if (e == hipSuccess) e = hipEventSynchronize(ready);
     (void)hipEventDestroy(ready);
@@ -335,7 +396,9 @@ int32_t btb_hip_p12_emit(const void* t, const void* hi4, size_t n, const void* w
     hipLaunchKernelGGL(p12_emit_kernel, dim3((unsigned)blocks), dim3(256), 0, static_cast<hipStream_t>(stream),
                        static_cast<const uint16_t*>(t), static_cast<const uint8_t*>(hi4), n,
                        static_cast<const uint32_t*>(work) + P12_BLOCKS,
-                       static_cast<const uint32_t*>(work) + P12_BLOCKS + blocks, n_esc, static_cast<int32_t*>(esc_idx),
+                       static_cast<const uint32_t*>(work) + P12_BLOCKS + blocks,
+                       static_cast<const uint32_t*>(work) + P12_BLOCKS + blocks + p12_chunks(n), n_esc,
+                       static_cast<int32_t*>(esc_idx),
                        static_cast<uint8_t*>(esc_val), row_ptr != nullptr ? cols : 1, row_ptr != nullptr ? rows : 0,
                        static_cast<int32_t*>(row_ptr));
     return hip_status(hipGetLastError(), "p12_emit launch");

@@ -42,6 +42,27 @@ def test_packed_on_the_card(card, kind, rows, cols):
     assert np.array_equal(pw.row_ptr.cpu().numpy(), np.searchsorted(idx, np.arange(rows + 1) * cols))
 
 
+@pytest.mark.parametrize("crowd", [63, 64, 65, 300])
+@pytest.mark.parametrize("cols", [2560, 1000, 7, 40000])
+def test_escapes_in_crowds(card, crowd, cols):
+    """The encoder lists up to 64 escapes a wave (8192 weights); a workgroup (32768) where a wave has more is read out of its
+    codes: crowds of that many, as they begin and end a wave's and a workgroup's weights, beside workgroups that have few."""
+    rows = -(-5 * 32768 // cols)
+    i = torch.arange(rows * cols, dtype=torch.int32)
+    w = ((0x30 + i % 15) << 8) | (i % 251)  # fifteen high bytes fill the table, every other is an escape
+    for at in (8192 - 10, 32768 + 8192, 3 * 32768 - crowd, 4 * 32768 - 3):
+        w[at : at + crowd] = 0x7100 + torch.arange(crowd, dtype=torch.int32) % 256
+    w[5::20011] = 0x7201
+    w = w.to(torch.int16).view(torch.bfloat16)
+    w = w.reshape(rows, cols)
+    pw = P12Weight.pack(w.cuda(), card)
+    lo, hi4, table, idx, val = codecs.pack12_pack(bits16(w))
+    assert idx.size >= 4 * crowd and (np.bincount(idx // 8192) >= crowd).any()
+    for got, want in ((pw.lo, lo), (pw.hi4, hi4), (pw.table, table), (pw.esc_idx, idx), (pw.esc_val, val)):
+        assert np.array_equal(got.cpu().numpy(), want)
+    assert np.array_equal(pw.row_ptr.cpu().numpy(), np.searchsorted(idx, np.arange(rows + 1) * cols))
+
+
 def test_a_view_that_is_not_16_byte_aligned(card):
     w = values("normal", 4096 + 3)
     pw = P12Weight.pack(w.cuda()[3:].reshape(64, 64), card)
