@@ -73,6 +73,7 @@ static Knob g_knobs[] = {
     {"mfma_stream_x", {-1}},
     {"mfma_direct", {-1}},
     {"mfma_split", {-1}},
+    {"mfma_ahead", {-1}},
     {"mfma_direct_grid", {-1}},
     {"p12_pair_table", {-1}},
     {"moe_grouped", {-1}},

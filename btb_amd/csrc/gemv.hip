@@ -595,22 +595,22 @@ static size_t mx4_matrix_from(size_t R, size_t C) {
 // (FP8 likewise: [4096 x 12288] at 3 / 4 rows 15.9 / 24.8 us on the vector kernel, 28.8 / 29.0 here)
 static size_t fp8_matrix_from(size_t R, size_t C) { return R * C >= (1u << 25) && C <= 10240 ? 3 : 5; }
 
-// Where the columns split over workgroups pay (bf16; the bits are the staged kernel's, so the line moves none). The split
+// Where the columns split over workgroups pay (bf16; the bits are the other kernels', so the line moves none). The split
 // saves each CU most of x (64 C bytes at 32 rows) and fills the CUs where tiles are few; it costs a second launch and the
-// partial sums' way out and back, which grow with R. Measured on MI355X over 48 shapes of 256 to 19456 rows by 1536 to 10240
-// columns, us staged / split at 8, 16, 17, 32 rows of x:
+// partial sums' way out and back, which grow with R. Measured on MI355X over 80 shapes of 256 to 19456 rows by 1536 to 10240
+// columns, us without / split at 8, 16, 17, 32 rows of x:
 //   [2560 x 9728] 12.3 / 14.2, 16.9 / 14.3, 23.0 / 15.6, 29.4 / 16.1; [8192 x 5120] 18.4 / 18.8, 20.3 / 19.4, 27.2 / 21.4,
-//   36.6 / 22.5; [2560 x 4096] 7.7 / 8.3, 8.8 / 8.7, 10.0 / 9.1, 12.4 / 9.5; [4096 x 4096] 9.1 / 10.2, 10.2 / 10.7, 11.3 / 11.8,
-//   14.1 / 12.3; [8192 x 4096] 14.2 / 15.1, 15.7 / 16.0, 16.8 / 18.0, 19.2 / 19.1; [19456 x 2560] 19.7 / 22.2, 21.0 / 24.4,
-//   22.0 / 27.2, 24.8 / 28.1; [2560 x 2560] 6.2 / 7.3, 7.0 / 7.6, 7.7 / 8.2, 9.0 / 8.6; [1024 x 3072] 6.4 / 5.8, 7.5 / 6.0,
-//   8.4 / 6.4, 10.2 / 6.7; [1024 x 1536] 4.1 / 5.2, 4.5 / 5.3, 5.0 / 5.6, 5.9 / 6.0; [1536 x 3072] 6.4 / 6.3, 7.3 / 6.7, 8.3 / 7.0,
-//   9.8 / 7.4; [16384 x 7168] 40.8 / 43.3, 43.7 / 44.5, 60.9 / 46.7, 82.6 / 47.8
+//   36.6 / 22.5; [2560 x 4096] 7.1 / 8.5, 8.2 / 8.9, 10.2 / 9.5, 12.5 / 10.0; [4096 x 4096] 9.1 / 11.0, 10.3 / 11.3, 12.1 / 12.2,
+//   14.3 / 12.7; [8192 x 4096] 15.1 / 16.5, 16.5 / 17.3, 17.9 / 19.5, 20.0 / 20.3; [2560 x 2560] 5.5 / 7.3, 6.0 / 7.6, 6.7 / 8.3,
+//   8.0 / 8.6; [1536 x 2560] 5.2 / 6.4, 5.8 / 6.6, 6.4 / 6.9, 7.9 / 7.3; [1024 x 3072] 5.6 / 5.9, 6.6 / 6.2, 8.5 / 6.5, 10.4 / 6.9;
+//   [1536 x 3072] 5.6 / 6.5, 6.3 / 6.8, 8.4 / 7.1, 10.0 / 7.6; [4096 x 2624] 7.3 / 9.6, 8.0 / 9.8, 9.2 / 10.6, 10.7 / 11.1;
+//   [16384 x 7168] 40.8 / 43.3, 43.7 / 44.5, 60.9 / 46.7, 82.6 / 47.8
 static bool split_pays(size_t M, size_t R, size_t C) {
     if (tuning("mfma_split") >= 0) return tuning("mfma_split") != 0;
-    if (M > 16) return C > 4096 || (C >= 2048 && M * C >= 25000 + 14 * R);
+    if (M > 16) return C > 4096 || (C > 2560 ? M * C >= 27500 + 14 * R : C >= 2048 && M * C >= 20000 + 28 * R);
     if (M < 8 || C < 2560) return false;
-    if (R <= 1024) return true;
-    if (R <= 2048) return M * C >= 30 * R;
+    if (R <= 1024) return C > 3072 || M * C >= 20000 + 16 * R;
+    if (R <= 2048) return C > 3072 && M * C >= 30 * R;
     return C > 7168 ? M >= 14 : C > 4096 && M >= 15 && R <= 12288;
 }
 

@@ -1,0 +1,234 @@
+// bf16 verify widths (M = 5..32 rows of x) over rows of up to 4096 columns: two tiles of weights in flight a wave.
+//
+// The decomposition is gemv_mfma_lds's - KS waves a workgroup, a wave a fixed slice of the columns whose x fragments it holds
+// for the whole kernel, tiles of sixteen rows, the waves' partial tiles folded through LDS in wave order - and so are the
+// slices, the order of the products and the order of the sum: every output has that kernel's bits. What differs is how the
+// weights come in. There a wave has one sub-block of eight steps in flight, two trips to memory a tile for rows of 2560 columns,
+// the second a quarter full: 64 and then 16 KB a CU where the memory's latency under load asks for 160. Here a wave's whole
+// slice of a tile is one run of 16-byte pieces dealt out to the lanes (any slice length fills its load instructions), and
+// the next two tiles are always on their way.
+
+#include "btb_common.hpp"
+#include "btb_tuning.hpp"
+
+#include "../../include/btb_hip.h"
+
+namespace btb {
+
+// SPW: the steps (32 columns) a wave's slice holds at most. TR: the rows of a tile that are rows of the matrix; the others are
+// not read, and what the matrix cores make of them is not written. RAG: R is no multiple of TR (and at least that): the last
+// tile starts TR rows before the end and writes the rows no other tile has. GLU: W is I gate rows over I up rows, a tile
+// eight of each (the same outputs'), y their fold [M, I].
+template <int KS, int MT, int SPW, int TR, bool RAG, bool GLU>
+__global__ void __launch_bounds__(KS * 64) mfma_ahead_kernel(const uint8_t* __restrict__ w, const uint4* __restrict__ x,
+                                                             uint16_t* __restrict__ y, int R, int C, int M) {
+    constexpr int PIECES = SPW * 4;                      // 16-byte pieces a slice has of a row
+    constexpr int NLD = (TR * PIECES + WAVE - 1) / WAVE;  // load instructions a wave's share of a tile takes
+    constexpr int STRIDE = SPW * 64 + 16;                // a slab row: 4 banks past a multiple of 32
+    constexpr int SLAB = 16 * STRIDE;
+    static_assert(!GLU || (TR == 16 && !RAG), "a folded tile is eight gate rows over eight up rows");
+    extern __shared__ __align__(16) uint8_t lds[];  // KS slabs, then two sets of KS * MT partial tiles
+    const int lane = threadIdx.x & (WAVE - 1);
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    const int li = lane & 15, lg = lane >> 4;
+    uint8_t* slab = lds + wv * SLAB;
+    f32x4* part = reinterpret_cast<f32x4*>(lds + KS * SLAB);
+    const int nsteps = C / 32, spw = (nsteps + KS - 1) / KS, s0 = wv * spw;
+    const int n = max(min(s0 + spw, nsteps) - s0, 0);  // this wave's steps; none: it adds zeros
+    const uint32_t rowbytes = (uint32_t)C * 2;
+    const int ntiles = RAG ? (R + TR - 1) / TR : R / TR;
+    const int grid = (int)gridDim.x, first = (int)blockIdx.x;
+    const int turns = (ntiles - first + grid - 1) / grid;
+
+    const int sn = n > 0 ? s0 : 0, last = max(n, 1) - 1;  // a wave without steps reads (and leaves) the first slice's
+    uint4 xb[MT][SPW];
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+        const uint4* xr = x + (size_t)min(t * 16 + li, M - 1) * (C / 8) + lg + (size_t)sn * 4;
+#pragma unroll
+        for (int i = 0; i < SPW; ++i) xb[t][i] = xr[min(i, last) * 4];
+    }
+
+    // where the lane's pieces of a tile lie: in the matrix past the tile's first byte of the slice, and in the slab. Pieces
+    // past the tile are its last one again, bytes past the slice's end its last sixteen again (they meet no product)
+    const uint32_t valid = (uint32_t)max(n, 1) * 64;
+    constexpr bool WHOLE = WAVE % PIECES == 0;  // a load covers whole rows of the slice: one offset a lane for all of them
+    constexpr int NOFF = WHOLE ? 1 : NLD;
+    uint32_t goff[NOFF], loff[NOFF];
+#pragma unroll
+    for (int q = 0; q < NOFF; ++q) {
+        const int p = WHOLE ? lane : min(q * WAVE + lane, TR * PIECES - 1);
+        const uint32_t row = (uint32_t)p / PIECES, byte = (uint32_t)p % PIECES * 16;
+        goff[q] = (row + (GLU && !WHOLE && row >= 8 ? (uint32_t)R / 2 - 8 : 0)) * rowbytes + min(byte, valid - 16);
+        loff[q] = row * STRIDE + byte;
+    }
+    constexpr int RPL = WAVE / PIECES;  // WHOLE: rows a load covers
+    static_assert(!WHOLE || TR % RPL == 0, "a tile is whole loads");
+    auto row_of = [&](int tile) { return GLU ? tile * 8 : RAG ? min(tile * TR, R - TR) : tile * TR; };
+    uint4 raw[2][NLD];
+    // The loads of the workgroup's k-th tile. Past its last one they are issued all the same, of one piece a wave: loads under
+    // a condition are loads the compiler cannot count, and it then waits for every one in flight.
+    auto request = [&](int k, uint4 (&r)[NLD]) {
+        const bool live = k < turns;
+        const uint8_t* base = w + (size_t)row_of(live ? first + k * grid : first) * rowbytes + (size_t)sn * 64;
+#pragma unroll
+        for (int q = 0; q < NLD; ++q) {
+            const uint32_t rows = WHOLE ? (uint32_t)(q * RPL) + (GLU && q * RPL >= 8 ? (uint32_t)R / 2 - 8 : 0u) : 0u;
+            const uint8_t* at = base + (live ? (size_t)rows * rowbytes : 0);
+            r[q] = load_stream16(reinterpret_cast<const uint4*>(at + (live ? goff[WHOLE ? 0 : q] : 0u)));
+        }
+    };
+    __builtin_amdgcn_sched_barrier(0);  // x ahead of the weights: loads come back in order
+    request(0, raw[0]);
+    __builtin_amdgcn_sched_barrier(0);
+    request(1, raw[1]);
+    __builtin_amdgcn_sched_barrier(0);
+
+    auto turn = [&](int k, uint4 (&r)[NLD]) {
+        const int tile = first + k * grid;
+#pragma unroll
+        for (int q = 0; q < NLD; ++q) *reinterpret_cast<uint4*>(slab + (WHOLE ? loff[0] + q * RPL * STRIDE : loff[q])) = r[q];
+        __builtin_amdgcn_sched_barrier(0);
+        request(k + 2, r);
+        __builtin_amdgcn_sched_barrier(0);
+        f32x4 acc[MT];
+#pragma unroll
+        for (int t = 0; t < MT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        auto product = [&](int i) {
+            const bf16x8 a = *reinterpret_cast<const bf16x8*>(slab + li * STRIDE + i * 64 + lg * 16);
+#pragma unroll
+            for (int t = 0; t < MT; ++t)
+                acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, __builtin_bit_cast(bf16x8, xb[t][i]), acc[t], 0, 0, 0);
+        };
+        if (n == SPW) {
+#pragma unroll
+            for (int i = 0; i < SPW; ++i) product(i);
+        } else {
+#pragma unroll
+            for (int i = 0; i < SPW; ++i)
+                if (i < n) product(i);  // uniform
+        }
+        // the KS partial tiles, folded in wave order; two sets of partials alternate so one barrier a tile suffices
+        f32x4* mine = part + (size_t)(k & 1) * KS * MT * WAVE;
+#pragma unroll
+        for (int t = 0; t < MT; ++t) mine[(wv * MT + t) * WAVE + lane] = acc[t];
+        __syncthreads();
+        if (wv < MT) {
+            f32x4 s = mine[wv * WAVE + lane];
+#pragma unroll
+            for (int q = 1; q < KS; ++q) {
+                const f32x4 o = mine[(q * MT + wv) * WAVE + lane];
+                s.x += o.x;
+                s.y += o.y;
+                s.z += o.z;
+                s.w += o.w;
+            }
+            const int m = wv * 16 + li;
+            if constexpr (GLU) {
+                // lanes of row groups 0, 1 hold gate sums, the lanes 32 further on the up sums of the same outputs
+                const f32x4 up = f32x4{xor32(s.x), xor32(s.y), xor32(s.z), xor32(s.w)};
+                if (m < M && lg < 2) {
+                    // the arithmetic of the stand-alone fold over the two rounded outputs (silu_pair)
+                    auto fold = [](float g, float u) {
+                        const float gb = bfround(g), ub = bfround(u);
+                        return f32_bf16(bfround(gb / (1.f + expf(-gb))) * ub);
+                    };
+                    uint16_t* o = y + (size_t)m * (R / 2) + tile * 8 + lg * 4;
+                    o[0] = fold(s.x, up.x);
+                    o[1] = fold(s.y, up.y);
+                    o[2] = fold(s.z, up.z);
+                    o[3] = fold(s.w, up.w);
+                }
+            } else {
+                const int in_tile = lg * 4, row = row_of(tile) + in_tile;
+                const int own = RAG ? tile * TR : 0;  // the tile's own rows begin here
+                if (m < M) {
+                    uint16_t* o = y + (size_t)m * R + row;
+                    if (in_tile + 0 < TR && row + 0 >= own) o[0] = f32_bf16(s.x);
+                    if (in_tile + 1 < TR && row + 1 >= own) o[1] = f32_bf16(s.y);
+                    if (in_tile + 2 < TR && row + 2 >= own) o[2] = f32_bf16(s.z);
+                    if (in_tile + 3 < TR && row + 3 >= own) o[3] = f32_bf16(s.w);
+                }
+            }
+        }
+    };
+    // (the odd last turn stands alone: leaving from the middle of the loop is, to the compiler, a way round it on which the
+    // first buffer's loads are the newest, and it waits for everything)
+    int k = 0;
+    for (; k + 1 < turns; k += 2) {
+        turn(k, raw[0]);
+        turn(k + 1, raw[1]);
+    }
+    if (k < turns) turn(k, raw[0]);
+}
+
+template <int KS, int MT, int SPW, int TR, bool RAG, bool GLU>
+static int32_t launch_ahead(const void* w, const void* x, void* y, int R, int C, int M, int cap, hipStream_t st) {
+    constexpr int SLAB = 16 * (SPW * 64 + 16);
+    const size_t lds = (size_t)KS * SLAB + 2 * (size_t)KS * MT * WAVE * sizeof(f32x4);
+    auto kern = mfma_ahead_kernel<KS, MT, SPW, TR, RAG, GLU>;
+    if (lds > 64 * 1024) {
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return hip_status(e, "hipFuncSetAttribute");
+    }
+    const int ntiles = RAG ? (R + TR - 1) / TR : R / TR;
+    // whole turns of the grid over the tiles: the smallest grid that walks them in ceil(ntiles / cap) turns
+    const int turns = (ntiles + cap - 1) / cap, grid = (ntiles + turns - 1) / turns;
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(KS * 64), lds, st, static_cast<const uint8_t*>(w), static_cast<const uint4*>(x),
+                       static_cast<uint16_t*>(y), R, C, M);
+    return hip_status(hipGetLastError(), "gemv_mfma_ahead launch");
+}
+
+template <int KS, int MT, int SPW>
+static int32_t run_ahead(const void* w, const void* x, void* y, int R, int C, int M, bool glu, hipStream_t st) {
+    // eight waves a CU are what two tiles in flight leave registers for; a launch of one turn at twelve takes those (us at 8 rows,
+    // eight / twelve waves: [9728 x 1024] 7.4 / 6.3, [40000 x 1024] 15.9 / 17.5)
+    int per_cu = tuning("mfma_wgs_per_cu");
+    if (per_cu <= 0) per_cu = R <= 16 * (12 / KS) * device_info().cus ? 12 / KS : 8 / KS;
+    const int cap = device_info().cus * per_cu;
+    if (glu) return launch_ahead<KS, MT, SPW, 16, false, true>(w, x, y, R, C, M, cap, st);
+    if (R % 16 != 0 && R % 12 != 0 && R % 10 != 0) return launch_ahead<KS, MT, SPW, 16, true, false>(w, x, y, R, C, M, cap, st);
+    if constexpr (KS == 8) {
+        if (tuning("mfma_tile_rows") != 0) {
+            auto rows_of = [&](int t) { return (long)(((R + t - 1) / t + cap - 1) / cap) * t; };
+            int tr = 16;
+            if (R % 12 == 0 && rows_of(12) * 8 <= rows_of(16) * 7) tr = 12;
+            if (R % 10 == 0 && rows_of(10) * 8 <= rows_of(16) * 7 && rows_of(10) < rows_of(tr)) tr = 10;
+            if (tr == 12) return launch_ahead<KS, MT, SPW, 12, false, false>(w, x, y, R, C, M, cap, st);
+            if (tr == 10) return launch_ahead<KS, MT, SPW, 10, false, false>(w, x, y, R, C, M, cap, st);
+        }
+    }
+    if (R % 16 != 0) return launch_ahead<KS, MT, SPW, 16, true, false>(w, x, y, R, C, M, cap, st);
+    return launch_ahead<KS, MT, SPW, 16, false, false>(w, x, y, R, C, M, cap, st);
+}
+
+// Which shapes. Measured on MI355X, us a launch, gemv_mfma_lds / this at 8, 16, 17, 32 rows of x: [19456 x 2560] with the fold
+// 20.6 / 18.9, 21.7 / 19.7, 22.5 / 20.7, 24.4 / 22.1 (4.5 TB/s); [151936 x 2560] 131.8 / 125.5, 144.7 / 132.0, 148.5 / 135.0,
+// 163.9 / 144.2; [6144 x 2560] 9.2 / 8.9, 10.5 / 9.5, 10.9 / 10.2, 13.0 / 11.9; [1024 x 1280] 4.7 / 3.8, 4.9 / 4.0, 5.6 / 4.5,
+// 6.4 / 5.1; [40000 x 1024] 18.9 / 15.9, 20.0 / 16.5, 22.6 / 17.0, 25.3 / 19.4; [512 x 512] 3.3 / 2.7, 3.4 / 2.8, 3.8 / 3.0,
+// 3.9 / 3.2. Past 2560 columns that kernel has two full sub-blocks a tile and the x fragments of a second tile of x rows do not
+// fit beside two tiles of weights: up to 16 rows of x, and where the CUs go round once ([2560 x 4096] at 8 rows 7.9 / 7.2,
+// [2048 x 3072] 6.7 / 6.0; but [24576 x 4096] 35.8 / 36.5, [8192 x 3072] 12.1 / 12.4).
+bool mfma_ahead_fits(int R, int C, int M, bool glu) {
+    const int nsteps = C / 32;
+    if (tuning("mfma_ahead") == 0 || R < 16 || C % 32 != 0 || nsteps > 128 || (glu && R % 16 != 0)) return false;
+    if (glu && (uint64_t)R * C >= 1ull << 31) return false;  // a gate row's up row within 32 bits
+    return nsteps <= 80 ? M <= 32 : M <= 16 && R <= 16 * device_info().cus;
+}
+// the waves a tile by row length as gemv_mfma_lds has them (two, four or eight), the slice's size close above its steps
+int32_t gemv_mfma_ahead_bf16(const void* w, const void* x, void* y, int R, int C, int M, bool glu, hipStream_t st) {
+    const int nsteps = C / 32;
+#define BTB_AHEAD(KS_, SPW_) \
+    return M <= 16 ? run_ahead<KS_, 1, SPW_>(w, x, y, R, C, M, glu, st) : run_ahead<KS_, 2, SPW_>(w, x, y, R, C, M, glu, st)
+    if (nsteps <= 16) BTB_AHEAD(2, 8);
+    if (nsteps <= 20) BTB_AHEAD(2, 10);
+    if (nsteps <= 32) BTB_AHEAD(4, 8);
+    if (nsteps <= 40) BTB_AHEAD(4, 10);
+    if (nsteps <= 64) BTB_AHEAD(8, 8);
+    if (nsteps <= 80) BTB_AHEAD(8, 10);
+#undef BTB_AHEAD
+    if (nsteps <= 96) return run_ahead<8, 1, 12>(w, x, y, R, C, M, glu, st);
+    return run_ahead<8, 1, 16>(w, x, y, R, C, M, glu, st);
+}
+
+}  // namespace btb

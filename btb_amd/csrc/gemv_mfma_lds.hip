@@ -794,13 +794,19 @@ static int32_t run_lds(const typename MF::Mat& mat, const void* x, void* y, int 
     return OK;
 }
 
+// up to 4096 columns, two tiles of weights in flight a wave (gemv_mfma_ahead.hip): the same bits
+bool mfma_ahead_fits(int R, int C, int M, bool glu);
+int32_t gemv_mfma_ahead_bf16(const void* w, const void* x, void* y, int R, int C, int M, bool glu, hipStream_t st);
+
 // M = 5..32 and a shape the fits() above take (a whole tile of 16 rows at least): the callers (gemv.hip) check before
 // they come here
 int32_t gemv_mfma_lds_bf16(const void* w, const void* x, void* y, int R, int C, int M, hipStream_t st) {
+    if (mfma_ahead_fits(R, C, M, false)) return gemv_mfma_ahead_bf16(w, x, y, R, C, M, false, st);
     return run_lds<MfBf16>(MfBf16::Mat{static_cast<const uint8_t*>(w)}, x, y, R, C, M, st);
 }
 // W = [gate; up], 2I rows: y [M, I] = bf16(bf16(silu(g)) * u)
 int32_t gemv_mfma_lds_glu_bf16(const void* w, const void* x, void* y, int I, int C, int M, hipStream_t st) {
+    if (mfma_ahead_fits(2 * I, C, M, true)) return gemv_mfma_ahead_bf16(w, x, y, 2 * I, C, M, true, st);
     return run_lds<MfBf16>(MfBf16::Mat{static_cast<const uint8_t*>(w)}, x, y, 2 * I, C, M, st, I / 16);
 }
 // ... with x made by the residual add and RMSNorm (XArgs); I > 0: W = [gate; up] and y the fold, as above. Rows of

@@ -333,3 +333,24 @@ def test_columns_split_over_workgroups_change_no_bit(card, R, C, M):
         card.set_tuning("mfma_split", -1)
     assert torch.equal(card.gemv(w, x).view(torch.int16), want.view(torch.int16))
 
+
+
+@pytest.mark.parametrize("R,C", [(16, 32), (17, 544), (4128, 512), (16416, 640), (48, 672), (12336, 1024), (1001, 1280),
+                                 (6144, 1312), (32, 2048), (5003, 2080), (2560, 2560), (8224, 2528), (2560, 2592), (3008, 3136),
+                                 (4096, 3584), (1536, 4096), (32, 4000)])
+@pytest.mark.parametrize("M", [5, 8, 16, 17, 32, 40])
+def test_two_tiles_of_weights_in_flight_change_no_bit(card, R, C, M):
+    """The kernel with two tiles of weights in flight (knob mfma_ahead = 0: without) against the staged one, bit for bit, plain
+    and with the gate / up fold: one to many turns a workgroup, odd and even, tiles of 10, 12 and 16 rows and overlapping ones,
+    slices shorter than the kernel's and waves without a step, non-finite weights in rows of their own."""
+    w, x = weights_bf16(R, C, seed=190), acts_bf16(M, C, seed=191).cuda()
+    w[R // 2, C - 1], w[R - 1, 0] = float("nan"), float("inf")
+    w, got = w.cuda(), []
+    try:
+        for knob in (0, -1):
+            card.set_tuning("mfma_ahead", knob)
+            got.append([card.gemv(w, x)] + ([card.gemv_glu_silu(w, x)] if R % 32 == 0 else []))
+    finally:
+        card.set_tuning("mfma_ahead", -1)
+    for want, y in zip(*got):
+        assert torch.equal(y.view(torch.int16), want.view(torch.int16))
