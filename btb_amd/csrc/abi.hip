@@ -77,6 +77,7 @@ static Knob g_knobs[] = {
     {"mfma_direct_grid", {-1}},
     {"p12_pair_table", {-1}},
     {"moe_grouped", {-1}},
+    {"moe_units", {-1}},
     {"attn_heads_per_wg", {-1}},
     {"attn_merge_few", {-1}},
     {"attn_mfma", {-1}},

@@ -220,13 +220,20 @@ template <bool OSS>
 __device__ __forceinline__ int glu_row(int r, int j, int I) {
     return OSS ? 2 * r + j : r + j * I;
 }
+// the gate's and the up half's bias of output r, asked for beside the rows' weights (asked for with the sums in hand they were a
+// trip to memory at a tile's end); without biases, or in the other form, nothing is read
 template <bool OSS>
-__device__ __forceinline__ uint16_t glu_out(float g, float u, const Glu& a, int expert, int r, int I) {
+__device__ __forceinline__ ushort2 glu_bias(const Glu& a, int expert, int r, int I) {
+    if (!OSS || a.bias == nullptr) return make_ushort2(0, 0);
+    const uint16_t* b = a.bias + (size_t)expert * 2 * I + 2 * min(r, I - 1);
+    return make_ushort2(b[0], b[1]);
+}
+template <bool OSS>
+__device__ __forceinline__ uint16_t glu_out(float g, float u, const Glu& a, ushort2 bias) {
     if (!OSS) return f32_bf16(bfround(g / (1.f + expf(-g))) * u);
     if (a.bias != nullptr) {
-        const uint16_t* b = a.bias + (size_t)expert * 2 * I + 2 * r;
-        g = bfround(g + bf16_f32(b[0]));
-        u = bfround(u + bf16_f32(b[1]));
+        g = bfround(g + bf16_f32(bias.x));
+        u = bfround(u + bf16_f32(bias.y));
     }
     g = g > a.limit ? a.limit : g;  // a NaN stays a NaN, as in torch's clamp
     u = u > a.limit ? a.limit : (u < -a.limit ? -a.limit : u);
@@ -268,11 +275,13 @@ __global__ void __launch_bounds__(256) moe_gate_up_kernel(Stack stack, const uin
     // weights do not depend on x, and nothing about these loads is conditional (a wave past the last tile requests the
     // last tile's and drops them)
     typename F::Raw first[U][RPW] = {};
+    ushort2 first_bias;
     stage_x<X_PLAIN, 0, false, 256>(xs, XArgs{x + (size_t)token * C, nullptr, nullptr, nullptr, 0.f, 0}, 1, C, [&] {
         typename F::RowCtx c0[RPW];
 #pragma unroll
         for (int j = 0; j < RPW; ++j)
             c0[j] = F::row_ctx(p, (size_t)glu_row<OSS>(min(min(wave, ntiles - 1) * ROWS + lane / LPR, I - 1), j, I), units);
+        first_bias = glu_bias<OSS>(glu, expert, min(wave, ntiles - 1) * ROWS + lane / LPR, I);
         load_span_always<F, LPR, RPW, U>(first, c0, 0, sl, units);
     });
     const uint4* xs4 = reinterpret_cast<const uint4*>(xs);
@@ -284,6 +293,7 @@ __global__ void __launch_bounds__(256) moe_gate_up_kernel(Stack stack, const uin
             rows[j] = tile * ROWS + lane / LPR;
             ctx[j] = F::row_ctx(p, (size_t)glu_row<OSS>(min(rows[j], I - 1), j, I), units);
         }
+        const ushort2 bias = tile == wave ? first_bias : glu_bias<OSS>(glu, expert, rows[0], I);
         float acc[RPW][1];
 #pragma unroll
         for (int j = 0; j < RPW; ++j) acc[j][0] = 0.f;
@@ -304,7 +314,7 @@ __global__ void __launch_bounds__(256) moe_gate_up_kernel(Stack stack, const uin
         }
         const float g = bfround(group_sum_last<LPR>(acc[0][0]));  // in the group's last lane: the one that stores
         const float u = bfround(group_sum_last<LPR>(acc[1][0]));
-        if (sl == LPR - 1 && rows[0] < I) y[rows[0]] = glu_out<OSS>(g, u, glu, expert, rows[0], I);
+        if (sl == LPR - 1 && rows[0] < I) y[rows[0]] = glu_out<OSS>(g, u, glu, bias);
     }
 }
 
@@ -383,6 +393,7 @@ __global__ void __launch_bounds__(256) moe_gate_up_grouped_kernel(Stack stack, c
     auto pass = [&](auto mtag, int r0, int mc) {
         constexpr int M = decltype(mtag)::value;
         typename F::Raw first[U][RPW] = {};
+        const ushort2 first_bias = glu_bias<OSS>(glu, expert, min(wave, ntiles - 1) * ROWS + lane / LPR, I);
         {
             typename F::RowCtx c0[RPW];
 #pragma unroll
@@ -412,6 +423,7 @@ __global__ void __launch_bounds__(256) moe_gate_up_grouped_kernel(Stack stack, c
                 rows[j] = tile * ROWS + lane / LPR;
                 ctx[j] = F::row_ctx(p, (size_t)glu_row<OSS>(min(rows[j], I - 1), j, I), units);
             }
+            const ushort2 bias = tile == wave ? first_bias : glu_bias<OSS>(glu, expert, rows[0], I);
             float acc[RPW][M];
 #pragma unroll
             for (int j = 0; j < RPW; ++j)
@@ -437,7 +449,7 @@ __global__ void __launch_bounds__(256) moe_gate_up_grouped_kernel(Stack stack, c
                 const float g = bfround(group_sum_last<LPR>(acc[0][m]));
                 const float u = bfround(group_sum_last<LPR>(acc[1][m]));
                 if (sl == LPR - 1 && rows[0] < I && m < mc)
-                    h[(size_t)prs[m] * I + rows[0]] = glu_out<OSS>(g, u, glu, expert, rows[0], I);
+                    h[(size_t)prs[m] * I + rows[0]] = glu_out<OSS>(g, u, glu, bias);
             }
         }
     };
@@ -510,6 +522,10 @@ __global__ void __launch_bounds__(256) moe_down_kernel(Stack stack, const uint16
 
     typename F::RowCtx ctx[KB][RPW];
     typename F::Raw first[KB][U][RPW] = {};
+    // the biases come with the weights (behind the products they were a trip to memory a pick); without any, the picks' weights
+    // stand in for them, unused
+    constexpr bool BIAS = std::is_same<F, FmtMx4>::value;
+    [[maybe_unused]] uint16_t bv[KB][RPW];
     auto request = [&](int tile, int q0, auto always) {
 #pragma unroll
         for (int b = 0; b < KB; ++b) {
@@ -518,6 +534,11 @@ __global__ void __launch_bounds__(256) moe_down_kernel(Stack stack, const uint16
 #pragma unroll
             for (int j = 0; j < RPW; ++j)
                 ctx[b][j] = F::row_ctx(p, (size_t)min(tile * ROWS + j * G + lane / LPR, R - 1), units);
+            if constexpr (BIAS) {
+#pragma unroll
+                for (int j = 0; j < RPW; ++j)
+                    bv[b][j] = *(bias != nullptr ? bias + (size_t)expert * R + min(tile * ROWS + j * G + lane / LPR, R - 1) : wts);
+            }
             if constexpr (decltype(always)::value)
                 load_span_always<F, LPR, RPW, U>(first[b], ctx[b], 0, sl, units);  // past the k-th: the k-th again
             else if (q0 + b < k)
@@ -561,8 +582,8 @@ __global__ void __launch_bounds__(256) moe_down_kernel(Stack stack, const uint16
                     for (int j = 0; j < RPW; ++j) {
                         // the expert's down product, as the row's dtype (in the group's last lane, which stores)
                         float d = bfround(group_sum_last<LPR>(acc[j][0]));
-                        if (bias != nullptr)
-                            d = bfround(d + bf16_f32(bias[(size_t)(s_expert[q] & 0xFFFFF) * R + min(rows[j], R - 1)]));
+                        if constexpr (BIAS)
+                            if (bias != nullptr) d = bfround(d + bf16_f32(bv[b][j]));
                         out[j] = bfround(out[j] + bfround(d * wq));    // times its weight, added in bf16
                     }
                 }
@@ -648,7 +669,19 @@ static int32_t launch_gate_up(Stack stack, const void* x, const int32_t* idx, vo
         return hip_status(hipGetLastError(), "moe gate_up launch");
     }
     const int grid = MX ? gate_up_grid(whole, (double)whole * pairs, 4) : whole;
-    hipLaunchKernelGGL((moe_gate_up_kernel<F, OSS, LPR, RPW, U>), dim3(grid, pairs), dim3(256), (size_t)C * 2, st, stack,
+    auto kern = moe_gate_up_kernel<F, OSS, LPR, RPW, U>;
+    // MXFP4 rows of five to seven units a lane in one trip to memory instead of two, where the waves are few. us a layer without
+    // the router, two trips / one: gpt-oss (six units) one row (11 waves a CU) 22.6 / 21.4, two rows 32.9 / 31.8, four (45) 57.5 /
+    // 59.8; 32 experts of 4, 3584 / 2560 (seven) 20.8 / 19.5, 29.6 / 28.9, 57.8 / 59.5. bf16's rows and the grouped kernel lose by
+    // it at any width (gpt-oss 8 rows 98.6 / 133).
+    if constexpr (MX) {
+        const int upl = (C / F::UW + LPR - 1) / LPR;
+        if ((double)ntiles * pairs <= 24.0 * device_info().cus && upl > 4 && upl < 8 && tuning("moe_units") != 0)
+            kern = upl == 5   ? moe_gate_up_kernel<F, OSS, LPR, RPW, 5>
+                   : upl == 6 ? moe_gate_up_kernel<F, OSS, LPR, RPW, 6>
+                              : moe_gate_up_kernel<F, OSS, LPR, RPW, 7>;
+    }
+    hipLaunchKernelGGL(kern, dim3(grid, pairs), dim3(256), (size_t)C * 2, st, stack,
                        static_cast<const uint16_t*>(x), idx, static_cast<uint16_t*>(gu), R, C, k, E, glu);
     return hip_status(hipGetLastError(), "moe gate_up launch");
 }
@@ -667,6 +700,14 @@ static int32_t launch_down(Stack stack, const void* gu, const int32_t* idx, cons
     auto kern = upl <= 2   ? moe_down_kernel<F, LPR, RPW, 2, 8>
                 : upl <= 3 ? moe_down_kernel<F, LPR, RPW, 3, 8>
                            : moe_down_kernel<F, LPR, RPW, 4, 4>;
+    // MXFP4 rows of five to seven: four picks' rows whole in one request. In spans of four a row's second span was a trip to
+    // memory a pick: us a layer at 1 / 2 / 8 / 32 rows, gpt-oss (six units) 22.5 / 33.0 / 98.2 / 284 -> 20.7 / 31.7 / 89.8 / 262,
+    // 64 experts of 8, 2592 / 2336 (five) 34.0 / 48.7 / 144 / 437 -> 30.8 / 47.1 / 140 / 417. Eight are two whole spans (in one: 16
+    // of 4, 1696 / 4064, 8 rows 80.7 -> 91.3); bf16 loses (64 of 4, 1600 / 2016, 8 rows 89.7 -> 95.8).
+    if constexpr (std::is_same<F, FmtMx4>::value) {
+        if (upl > 4 && upl < 8 && tuning("moe_units") != 0)
+            kern = upl <= 6 ? moe_down_kernel<F, LPR, RPW, 6, 4> : moe_down_kernel<F, LPR, RPW, 7, 4>;
+    }
     if (lds > 64 * 1024) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);

@@ -347,3 +347,32 @@ def test_how_the_experts_launches_are_cut_changes_no_bit(card, form, H_, I_, k, 
     for t in range(T):
         one = layer(x[t : t + 1].contiguous(), picks[t : t + 1].contiguous(), w[t : t + 1].contiguous())
         assert torch.equal(y[t : t + 1].view(torch.int16), one.view(torch.int16)), t
+
+
+@pytest.mark.parametrize("oss", [True, False])
+@pytest.mark.parametrize("H_,I_", [(2592, 2336), (2080, 3072), (3584, 2080), (4064, 3552), (4608, 64), (64, 6144), (2048, 4064)])
+@pytest.mark.parametrize("T,k", [(1, 4), (2, 7), (9, 3)])
+def test_mxfp4_rows_whole_in_one_trip_change_no_bit(card, oss, H_, I_, T, k):
+    """MXFP4 rows of five to seven units a lane, of 16 and of 32 lanes, asked for in one trip (knob moe_units = 0: in spans of
+    four), against the spans, bit for bit, with the gpt-oss form's biases and without; and the biases count."""
+    from btb_amd.load import MxExperts
+    from btb_amd.moe import MxExpertsLayer
+
+    E_, g = 8, gen(591)
+    ex = mx_stacks(590, E_, I_, H_)
+    biases = [(torch.randn(E_, n, generator=g) * 0.5).to(torch.bfloat16) for n in (2 * I_, H_)] if oss else [None, None]
+    layer = MxExpertsLayer(card, to_gpu(MxExperts(ex.gate_up_blocks, ex.gate_up_scales, ex.down_blocks, ex.down_scales, *biases)), oss=oss)
+    x = acts_bf16(T, H_, seed=592).cuda()
+    picks = torch.stack([torch.randperm(E_, generator=g)[:k] for _ in range(T)]).to(torch.int32).cuda()
+    w = torch.rand(T, k, generator=g).to(torch.bfloat16).cuda()
+    got = []
+    try:
+        for knob in (0, -1):
+            card.set_tuning("moe_units", knob)
+            got.append(layer(x, picks, w).clone())
+    finally:
+        card.set_tuning("moe_units", -1)
+    assert torch.equal(got[0].view(torch.int16), got[1].view(torch.int16))
+    if oss:
+        bare = MxExpertsLayer(card, to_gpu(ex), oss=True)(x, picks, w)
+        assert not torch.equal(bare.view(torch.int16), got[0].view(torch.int16))
