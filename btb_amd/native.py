@@ -111,6 +111,9 @@ SIGNATURES: dict[str, tuple[Any, list[Any]]] = {
     "btb_hip_silu_mul": (_i32, [_vp, _vp, _sz, _sz, _vp]),
     "btb_hip_argmax": (_i32, [_vp, _vp, _sz, _sz, _vp]),
     "btb_hip_publish": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "btb_hip_argmax_floats": (_sz, [_sz, _sz]),
+    "btb_hip_argmax_ws": (_i32, [_vp, _vp, _sz, _sz, _vp, _vp]),
+    "btb_hip_argmax_publish_ws": (_i32, [_vp, _sz, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "btb_hip_argmax_publish": (_i32, [_vp, _sz, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
 }
 
@@ -1026,7 +1029,10 @@ class HipCard(CardLaunch):
         self._need(logits, torch.bfloat16, "logits")
         self._need(out, torch.int32, "out")
         V = int(logits.shape[-1])
-        self._call("btb_hip_argmax", _p(logits), _p(out), int(logits.numel()) // V, V, _stream())
+        T = int(logits.numel()) // V
+        floats = self.lib.btb_hip_argmax_floats(T, V)  # long rows go over many workgroups and take a workspace (this call's own)
+        ws = torch.empty(floats, dtype=torch.float32, device=logits.device) if floats else None
+        self._call("btb_hip_argmax_ws", _p(logits), _p(out), T, V, None if ws is None else _p(ws), _stream())
         return out
 
     def publish(self, n0: torch.Tensor, picked: torch.Tensor, next_ids: torch.Tensor | None = None,
@@ -1046,7 +1052,7 @@ class HipCard(CardLaunch):
     def argmax_publish(self, logits: torch.Tensor, picked: torch.Tensor, n0: torch.Tensor,
                        next_ids: torch.Tensor | None = None, out_tok: torch.Tensor | None = None,
                        out_n0: torch.Tensor | None = None, out_ts: torch.Tensor | None = None) -> None:
-        """`argmax` over one row and `publish` in one launch"""
+        """`argmax` over one row and `publish`, in its last launch"""
         self._need(logits, torch.bfloat16, "logits")
         self._need(picked, torch.int32, "picked")
         self._need(n0, torch.int32, "n0")
@@ -1054,8 +1060,10 @@ class HipCard(CardLaunch):
         if logits.numel() != V:
             raise ValueError("[hip] argmax_publish: one row of logits")
         p = lambda t: None if t is None else _p(t)
-        self._call("btb_hip_argmax_publish", _p(logits), V, _p(picked), _p(n0), p(next_ids),
-                   p(out_tok), p(out_n0), p(out_ts), _stream())
+        floats = self.lib.btb_hip_argmax_floats(1, V)
+        ws = torch.empty(floats, dtype=torch.float32, device=logits.device) if floats else None
+        self._call("btb_hip_argmax_publish_ws", _p(logits), V, _p(picked), _p(n0), p(next_ids),
+                   p(out_tok), p(out_n0), p(out_ts), p(ws), _stream())
 
 
 class Native:

@@ -466,6 +466,14 @@ int32_t btb_hip_argmax(const void* logits, int32_t* out, size_t T, size_t V, voi
 int32_t btb_hip_argmax_publish(const void* logits, size_t V, int32_t* picked, int32_t* n0, int32_t* next_ids,
                                int32_t* out_tok, int32_t* out_n0, int64_t* out_ts, void* stream);
 
+/* Both with a workspace: long rows (65536 logits and more) over many workgroups, whose picks meet in `ws`
+ * (btb_hip_argmax_floats of them, 8-byte aligned; nothing in it need be cleared, nothing is kept; calls that overlap take one
+ * each). The same pick. 0 floats, ws NULL, logits not 16-byte aligned: the functions above are called. */
+size_t btb_hip_argmax_floats(size_t T, size_t V);
+int32_t btb_hip_argmax_ws(const void* logits, int32_t* out, size_t T, size_t V, float* ws, void* stream);
+int32_t btb_hip_argmax_publish_ws(const void* logits, size_t V, int32_t* picked, int32_t* n0, int32_t* next_ids,
+                                  int32_t* out_tok, int32_t* out_n0, int64_t* out_ts, float* ws, void* stream);
+
 /* The step's end, one thread: *next_ids = *picked (the next step's input, when not NULL), *n0 += 1, and with
  * out_tok not NULL (pinned host memory) the token and the GPU's clock, then - after a system fence - the new
  * length, so a host that sees the length sees the token. Replaces btb_publish (native/cuda/btb_kernels.cu:448-465). */

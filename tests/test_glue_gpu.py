@@ -646,3 +646,34 @@ def test_attn_span_count_limit(card):
                          card.attn_scratch(1, Hq, Hk, D, S + 1))
     torch.cuda.synchronize()
     assert bool((att == 3.0).all())
+
+
+@pytest.mark.parametrize("V", [65536, 65544, 69632, 151936, 300008])
+@pytest.mark.parametrize("T", [1, 3, 32])
+def test_argmax_of_long_rows_over_many_workgroups(card, T, V):
+    """Rows whose pick comes from many workgroups: ties within and across them (the lowest index wins), NaN, rows with nothing
+    above -inf (index 0), the last logit - and the publishing form - against one workgroup a row."""
+    x = acts_bf16(T, V, seed=640)
+    x[0, V - 1] = x[0, 4096 * 3 + 5] = x[0, V - 9] = 40.0
+    if T > 1:
+        x[1, :] = float("nan")
+        x[2, :] = float("-inf")
+        x[2, V - 1] = -3e38
+    if T > 3:
+        x[3, 0], x[3, 5000], x[4, :] = float("nan"), 50.0, float("-inf")
+        x[5, V - 1] = 60.0
+    x = x.cuda()
+    L, p = card.lib, lambda t: t.data_ptr()
+    want, got, one = (torch.full((n,), -1, dtype=torch.int32, device="cuda") for n in (T, T, 1))
+    assert L.btb_hip_argmax_floats(T, V) > 0
+    assert L.btb_hip_argmax(p(x), p(want), T, V, None) == 0
+    card.argmax(x, got)
+    assert torch.equal(got, want) and got[0] == 4096 * 3 + 5
+    n0 = torch.full((1,), 7, dtype=torch.int32, device="cuda")
+    ids, tok, ln = torch.zeros_like(n0), torch.zeros(1, dtype=torch.int32).pin_memory(), torch.zeros(1, dtype=torch.int32).pin_memory()
+    card.argmax_publish(x[:1], one, n0, ids, tok, ln)
+    torch.cuda.synchronize()
+    assert one.item() == ids.item() == tok.item() == want[0].item() and n0.item() == ln.item() == 8
+    odd = x.view(-1)[1 : V - 7].contiguous()  # no multiple of eight from an aligned place: one workgroup
+    card.argmax(odd, one)
+    assert one.item() == (4096 * 3 + 4 if x.view(-1)[4096 * 3 + 5] == 40.0 else -1)
