@@ -521,6 +521,10 @@ int32_t gemv_mfma_lds_p12(const uint8_t* lo, const uint8_t* hi4, const uint8_t* 
                           const uint8_t* esc_val, const int32_t* row_ptr, const void* x, void* y, int R, int C, int M,
                           hipStream_t st);
 
+// two tiles of weights in flight (gemv_mfma_ahead.hip): also the rows whose columns are no multiple of 32
+bool mfma_ahead_ragged_fits(int R, int C);
+int32_t gemv_mfma_ahead_bf16(const void* w, const void* x, void* y, int R, int C, int M, bool glu, hipStream_t st);
+
 // the matrix-core matvec of more than sixteen rows with the columns split over workgroups (gemv_mfma_split.hip)
 size_t mfma_split_floats(size_t R, size_t M);
 bool mfma_split_fits(size_t R, size_t C);
@@ -707,6 +711,15 @@ int32_t btb_hip_gemv_bf16(const void* w, const void* x, void* y, size_t R, size_
                                                       static_cast<hipStream_t>(stream))
                                  : gemv_mfma_bf16(w, xp + m0 * C, yp + m0 * R, (int)R, (int)C, mm,
                                                   static_cast<hipStream_t>(stream));
+            if (rc != OK) return rc;
+        }
+        return OK;
+    }
+    if (M >= 5 && tuning("gemv_no_mfma") <= 0 && mfma_ahead_ragged_fits((int)R, (int)C)) {
+        const size_t step = C <= 2560 ? 32 : 16;
+        for (size_t m0 = 0; m0 < M; m0 += step) {
+            rc = gemv_mfma_ahead_bf16(w, static_cast<const uint16_t*>(x) + m0 * C, static_cast<uint16_t*>(y) + m0 * R, (int)R, (int)C,
+                                      (int)(M - m0 < step ? M - m0 : step), false, static_cast<hipStream_t>(stream));
             if (rc != OK) return rc;
         }
         return OK;

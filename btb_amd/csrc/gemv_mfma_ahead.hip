@@ -1,4 +1,5 @@
-// bf16 verify widths (M = 5..32 rows of x) over rows of up to 4096 columns: two tiles of weights in flight a wave.
+// bf16 verify widths (M = 5..32 rows of x) over rows of up to 4096 columns, any multiple of 8: two tiles of weights in flight a
+// wave.
 //
 // The decomposition is gemv_mfma_lds's - KS waves a workgroup, a wave a fixed slice of the columns whose x fragments it holds
 // for the whole kernel, tiles of sixteen rows, the waves' partial tiles folded through LDS in wave order - and so are the
@@ -33,7 +34,7 @@ __global__ void __launch_bounds__(KS * 64) mfma_ahead_kernel(const uint8_t* __re
     const int li = lane & 15, lg = lane >> 4;
     uint8_t* slab = lds + wv * SLAB;
     f32x4* part = reinterpret_cast<f32x4*>(lds + KS * SLAB);
-    const int nsteps = C / 32, spw = (nsteps + KS - 1) / KS, s0 = wv * spw;
+    const int nsteps = (C + 31) / 32, spw = (nsteps + KS - 1) / KS, s0 = wv * spw;
     const int n = max(min(s0 + spw, nsteps) - s0, 0);  // this wave's steps; none: it adds zeros
     const uint32_t rowbytes = (uint32_t)C * 2;
     const int ntiles = RAG ? (R + TR - 1) / TR : R / TR;
@@ -41,17 +42,19 @@ __global__ void __launch_bounds__(KS * 64) mfma_ahead_kernel(const uint8_t* __re
     const int turns = (ntiles - first + grid - 1) / grid;
 
     const int sn = n > 0 ? s0 : 0, last = max(n, 1) - 1;  // a wave without steps reads (and leaves) the first slice's
+    // the slice's bytes of a row; C no multiple of 32: the last step is short, x and the weights past its end are zeros
+    const uint32_t valid = min((uint32_t)(last + 1) * 64, rowbytes - (uint32_t)sn * 64);
+    const bool ragged = valid % 64 != 0;  // uniform
     uint4 xb[MT][SPW];
 #pragma unroll
     for (int t = 0; t < MT; ++t) {
-        const uint4* xr = x + (size_t)min(t * 16 + li, M - 1) * (C / 8) + lg + (size_t)sn * 4;
+        const uint4* xr = x + (size_t)min(t * 16 + li, M - 1) * (C / 8) + (size_t)sn * 4;
 #pragma unroll
-        for (int i = 0; i < SPW; ++i) xb[t][i] = xr[min(i, last) * 4];
+        for (int i = 0; i < SPW; ++i) xb[t][i] = xr[min(min(i, last) * 4 + lg, (int)valid / 16 - 1)];
     }
 
     // where the lane's pieces of a tile lie: in the matrix past the tile's first byte of the slice, and in the slab. Pieces
     // past the tile are its last one again, bytes past the slice's end its last sixteen again (they meet no product)
-    const uint32_t valid = (uint32_t)max(n, 1) * 64;
     constexpr bool WHOLE = WAVE % PIECES == 0;  // a load covers whole rows of the slice: one offset a lane for all of them
     constexpr int NOFF = WHOLE ? 1 : NLD;
     uint32_t goff[NOFF], loff[NOFF];
@@ -65,6 +68,17 @@ __global__ void __launch_bounds__(KS * 64) mfma_ahead_kernel(const uint8_t* __re
     constexpr int RPL = WAVE / PIECES;  // WHOLE: rows a load covers
     static_assert(!WHOLE || TR % RPL == 0, "a tile is whole loads");
     auto row_of = [&](int tile) { return GLU ? tile * 8 : RAG ? min(tile * TR, R - TR) : tile * TR; };
+    uint32_t past = 0;  // the loads whose piece lies past a short last step's end
+    if (ragged) {
+#pragma unroll
+        for (int q = 0; q < NLD; ++q)
+            if ((uint32_t)min(q * WAVE + lane, TR * PIECES - 1) % PIECES * 16 >= valid) past |= 1u << q;
+#pragma unroll
+        for (int t = 0; t < MT; ++t)
+#pragma unroll
+            for (int i = 0; i < SPW; ++i)
+                if (i * 64 + lg * 16 >= (int)valid) xb[t][i] = make_uint4(0, 0, 0, 0);
+    }
     uint4 raw[2][NLD];
     // The loads of the workgroup's k-th tile. Past its last one they are issued all the same, of one piece a wave: loads under
     // a condition are loads the compiler cannot count, and it then waits for every one in flight.
@@ -86,6 +100,11 @@ __global__ void __launch_bounds__(KS * 64) mfma_ahead_kernel(const uint8_t* __re
 
     auto turn = [&](int k, uint4 (&r)[NLD]) {
         const int tile = first + k * grid;
+        if (ragged) {
+#pragma unroll
+            for (int q = 0; q < NLD; ++q)
+                if (past >> q & 1) r[q] = make_uint4(0, 0, 0, 0);
+        }
 #pragma unroll
         for (int q = 0; q < NLD; ++q) *reinterpret_cast<uint4*>(slab + (WHOLE ? loff[0] + q * RPL * STRIDE : loff[q])) = r[q];
         __builtin_amdgcn_sched_barrier(0);
@@ -215,9 +234,17 @@ bool mfma_ahead_fits(int R, int C, int M, bool glu) {
     if (glu && (uint64_t)R * C >= 1ull << 31) return false;  // a gate row's up row within 32 bits
     return nsteps <= 80 ? M <= 32 : M <= 16 && R <= 16 * device_info().cus;
 }
+// Rows of a multiple of 8 columns but not of 32, which the other matrix-core kernels do not take and which went through passes
+// of four rows on the vector units: from five rows of x on, in passes of 32 rows, or of 16 past 2560 columns. us at 5 / 8 / 16 / 32
+// rows, those passes / here: [512 x 520] 4.5 / 3.2, 5.2 / 3.3, 10.0 / 3.4, 19.5 / 3.9; [2560 x 2056] 9.0 / 5.4, 9.8 / 5.5, 18.8 / 5.9,
+// 37.7 / 7.5; [5003 x 3000] 16.1 / 11.3, 17.3 / 11.5, 32.3 / 11.7, 63.8 / 23.0; [40000 x 3000] 84 / 43, 85 / 44, 168 / 45, 318 / 87
+// (5.5 TB/s); [512 x 4088] 7.1 / 6.5, 8.6 / 6.7, 16.6 / 7.7, 32.8 / 14.8.
+bool mfma_ahead_ragged_fits(int R, int C) {
+    return tuning("mfma_ahead") != 0 && tuning("mfma_lds") != 0 && R >= 16 && C % 32 != 0 && C % 8 == 0 && C >= 64 && C <= 4096;
+}
 // the waves a tile by row length as gemv_mfma_lds has them (two, four or eight), the slice's size close above its steps
 int32_t gemv_mfma_ahead_bf16(const void* w, const void* x, void* y, int R, int C, int M, bool glu, hipStream_t st) {
-    const int nsteps = C / 32;
+    const int nsteps = (C + 31) / 32;
 #define BTB_AHEAD(KS_, SPW_) \
     return M <= 16 ? run_ahead<KS_, 1, SPW_>(w, x, y, R, C, M, glu, st) : run_ahead<KS_, 2, SPW_>(w, x, y, R, C, M, glu, st)
     if (nsteps <= 16) BTB_AHEAD(2, 8);

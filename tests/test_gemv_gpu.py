@@ -354,3 +354,23 @@ def test_two_tiles_of_weights_in_flight_change_no_bit(card, R, C, M):
         card.set_tuning("mfma_ahead", -1)
     for want, y in zip(*got):
         assert torch.equal(y.view(torch.int16), want.view(torch.int16))
+
+
+@pytest.mark.parametrize("R,C", [(16, 72), (17, 520), (512, 536), (100, 648), (4097, 1016), (1001, 1288), (2560, 2056), (5003, 2552),
+                                 (2560, 2568), (300, 3000), (9000, 3000), (1536, 3592), (33, 4088)])
+@pytest.mark.parametrize("M", [5, 8, 16, 17, 33])
+def test_rows_of_no_multiple_of_32_columns_on_the_matrix_cores(card, R, C, M):
+    """Rows whose last step of 32 columns is short, against 64 bits: the output's rounding (bf16 has eight significant bits: half
+    a step is at most 2^-8 of the value) and C roundings of 2^-24 of the sum of magnitudes, twice over for the accumulator's own;
+    a non-finite weight at a row's end stays in its row, non-finite x in its own."""
+    w, x = weights_bf16(R, C, seed=200), acts_bf16(M, C, seed=201)
+    w[1, C - 1], w[3, C - 8], w[R - 1, 0] = float("nan"), float("inf"), float("-inf")
+    x[M - 1, C - 1] = float("nan")
+    y = card.gemv(w.cuda(), x.cuda()).float().cpu().double()
+    ref = x.double() @ w.double().T
+    assert bool(y[: M - 1, 1].isnan().all()) and bool(y[M - 1].isnan().all())
+    assert not bool(y[: M - 1, [r for r in (3, R - 1) if r != 1]].isfinite().any())
+    keep = [r for r in range(R) if r not in (1, 3, R - 1)]
+    y, ref = y[: M - 1, keep], ref[: M - 1, keep]
+    bound = 2.0**-8 * ref.abs() * 1.01 + 2 * C * 2.0**-24 * (x[: M - 1].double().abs() @ w[keep].double().abs().T)
+    assert bool(((y - ref).abs() <= bound).all())
