@@ -58,18 +58,15 @@ class Experts:
         self.gate_up = gate_up.contiguous()
         self.down = down.contiguous()
         self.num_experts, self.hidden_dim, self.intermediate_dim = E, H, I2 // 2
-        self._gu: torch.Tensor | None = None
 
     def __call__(self, hidden_states: torch.Tensor, top_k_index: torch.Tensor, top_k_weights: torch.Tensor,
                  out: torch.Tensor | None = None) -> torch.Tensor:
         x = hidden_states.reshape(-1, self.hidden_dim)
         if x.dtype != torch.bfloat16:
             raise ValueError("[moe] the card's experts take bf16 rows")
-        T, k = top_k_index.shape
-        if self._gu is None or self._gu.shape[0] < T or self._gu.shape[1] != k:
-            self._gu = torch.empty(T, k, 2 * self.intermediate_dim, dtype=torch.bfloat16, device=x.device)
+        # (what passes between the two launches is the call's own, on its stream or in its capture's pool)
         return self.card.moe_experts(self.gate_up, self.down, x.contiguous(), top_k_index.to(torch.int32).contiguous(),
-                                     top_k_weights.to(torch.bfloat16).contiguous(), out, self._gu[:T])
+                                     top_k_weights.to(torch.bfloat16).contiguous(), out)
 
 
 class MxExpertsLayer:
@@ -84,16 +81,12 @@ class MxExpertsLayer:
             raise ValueError("[moe] expert biases belong to the gpt-oss form")
         self.card, self.stacks, self.oss, self.alpha, self.limit = card, stacks, bool(oss), float(alpha), float(limit)
         self.num_experts, self.hidden_dim, self.intermediate_dim = stacks.experts, stacks.hidden, stacks.intermediate
-        self._h: torch.Tensor | None = None
 
     def __call__(self, hidden_states: torch.Tensor, top_k_index: torch.Tensor, top_k_weights: torch.Tensor,
                  out: torch.Tensor | None = None) -> torch.Tensor:
         x = hidden_states.reshape(-1, self.hidden_dim)
         if x.dtype != torch.bfloat16:
             raise ValueError("[moe] the card's experts take bf16 rows")
-        T, k = top_k_index.shape
-        if self._h is None or self._h.shape[0] < T or self._h.shape[1] != k:
-            self._h = torch.empty(T, k, self.intermediate_dim, dtype=torch.bfloat16, device=x.device)
         return self.card.moe_experts_mx4(self.stacks, x.contiguous(), top_k_index.to(torch.int32).contiguous(),
-                                         top_k_weights.to(torch.bfloat16).contiguous(), out, self._h[:T], oss=self.oss,
-                                         alpha=self.alpha, limit=self.limit)
+                                         top_k_weights.to(torch.bfloat16).contiguous(), out, oss=self.oss, alpha=self.alpha,
+                                         limit=self.limit)
