@@ -524,6 +524,7 @@ int32_t gemv_mfma_lds_p12(const uint8_t* lo, const uint8_t* hi4, const uint8_t* 
 // two tiles of weights in flight (gemv_mfma_ahead.hip): also the rows whose columns are no multiple of 32
 bool mfma_ahead_ragged_fits(int R, int C);
 int32_t gemv_mfma_ahead_bf16(const void* w, const void* x, void* y, int R, int C, int M, bool glu, hipStream_t st);
+int32_t gemv_mfma_ahead_norm_bf16(const void* w, const XArgs& xa, void* y, int R, int C, int M, bool glu, hipStream_t st);
 
 // the matrix-core matvec of more than sixteen rows with the columns split over workgroups (gemv_mfma_split.hip)
 size_t mfma_split_floats(size_t R, size_t M);
@@ -582,6 +583,35 @@ static bool wide_pass(Form f, size_t M, size_t R, size_t C, size_t from = 5) {
     return M >= from && (set || staged_pays(f, M, R, C)) &&
            (f == Form::BF16 ? mfma_lds_fits_bf16((int)R, (int)C) : mfma_lds_fits_packed((int)R, (int)C)) &&
            tuning("gemv_no_mfma") <= 0 && tuning("mfma_lds") != 0;
+}
+
+// Whether a bf16 pass of M rows over rows of C % 32 != 0 columns goes to the matrix cores: the plain matvec's, the gate / up fold's
+// and the add + norm's alike, so that the three keep to one order of the sums.
+static bool ragged_pass(size_t M, size_t R, size_t C) {
+    return M >= 5 && tuning("gemv_no_mfma") <= 0 && mfma_ahead_ragged_fits((int)R, (int)C);
+}
+static int32_t run_ragged(const void* w, const void* x, void* y, size_t R, size_t C, size_t M, bool glu, hipStream_t st) {
+    const size_t step = C <= 2560 ? 32 : 16, outs = glu ? R / 2 : R;
+    for (size_t m0 = 0; m0 < M; m0 += step) {
+        const int32_t rc = gemv_mfma_ahead_bf16(w, static_cast<const uint16_t*>(x) + m0 * C, static_cast<uint16_t*>(y) + m0 * outs,
+                                                (int)R, (int)C, (int)(M - m0 < step ? M - m0 : step), glu, st);
+        if (rc != OK) return rc;
+    }
+    return OK;
+}
+static int32_t run_ragged_norm(const void* w, XArgs xa, void* y, size_t R, size_t C, size_t M, bool glu, hipStream_t st) {
+    for (size_t m0 = 0; m0 < M; m0 += 16) {
+        const int32_t rc = gemv_mfma_ahead_norm_bf16(w, xa, static_cast<uint16_t*>(y) + m0 * (glu ? R / 2 : R), (int)R, (int)C,
+                                                     (int)(M - m0 < 16 ? M - m0 : 16), glu, st);
+        if (rc != OK) return rc;
+        if (xa.ids != nullptr)
+            xa.ids += 16;
+        else
+            xa.x += 16 * C;
+        if (xa.y != nullptr) xa.y += 16 * C;
+        if (xa.h_out != nullptr) xa.h_out += 16 * C;
+    }
+    return OK;
 }
 
 // the block-scaled forms' vector kernels pay for every further row of x in LDS reads and in widening, the matrix-core
@@ -715,15 +745,7 @@ int32_t btb_hip_gemv_bf16(const void* w, const void* x, void* y, size_t R, size_
         }
         return OK;
     }
-    if (M >= 5 && tuning("gemv_no_mfma") <= 0 && mfma_ahead_ragged_fits((int)R, (int)C)) {
-        const size_t step = C <= 2560 ? 32 : 16;
-        for (size_t m0 = 0; m0 < M; m0 += step) {
-            rc = gemv_mfma_ahead_bf16(w, static_cast<const uint16_t*>(x) + m0 * C, static_cast<uint16_t*>(y) + m0 * R, (int)R, (int)C,
-                                      (int)(M - m0 < step ? M - m0 : step), false, static_cast<hipStream_t>(stream));
-            if (rc != OK) return rc;
-        }
-        return OK;
-    }
+    if (ragged_pass(M, R, C)) return run_ragged(w, x, y, R, C, M, false, static_cast<hipStream_t>(stream));
     FmtBf16::Params p{static_cast<const uint4*>(w)};
     return run_rows<FmtBf16, X_PLAIN, E_PLAIN>(p, plain_x(x), y, R, C, M, static_cast<hipStream_t>(stream));
 }
@@ -773,6 +795,7 @@ int32_t btb_hip_gemv_glu_silu_bf16(const void* w, const void* x, void* m, size_t
         }
         return OK;
     }
+    if (ragged_pass(M, 2 * I, C)) return run_ragged(w, x, m, 2 * I, C, M, true, static_cast<hipStream_t>(stream));
     FmtBf16::Params p{static_cast<const uint4*>(w)};
     return run_rows<FmtBf16, X_PLAIN, E_GLU>(p, plain_x(x), m, 2 * I, C, M, static_cast<hipStream_t>(stream));
 }
@@ -792,6 +815,7 @@ int32_t btb_hip_gemv_bf16_norm(const void* w, const void* h_in, const void* y, c
     // the verify widths: the matrix cores, the rows made by each workgroup ahead of its first tile
     if (norm_on_mfma(xa, R, C, M, glu != 0))
         return gemv_mfma_lds_norm_bf16(w, xa, out, (int)R, (int)C, (int)M, glu ? (int)(R / 2) : 0, st);
+    if (ragged_pass(M, R, C) && tuning("mfma_lds_norm") != 0) return run_ragged_norm(w, xa, out, R, C, M, glu != 0, st);
     return glu ? run_rows<FmtBf16, X_ADDNORM, E_GLU>(p, xa, out, R, C, M, st)
                : run_rows<FmtBf16, X_ADDNORM, E_PLAIN>(p, xa, out, R, C, M, st);
 }
@@ -809,6 +833,8 @@ int32_t btb_hip_gemv_bf16_embed_norm(const void* w, const void* table, const int
     FmtBf16::Params p{static_cast<const uint4*>(w)};
     if (norm_on_mfma(xa, R, C, M, false))
         return gemv_mfma_lds_norm_bf16(w, xa, out, (int)R, (int)C, (int)M, 0, static_cast<hipStream_t>(stream));
+    if (ragged_pass(M, R, C) && tuning("mfma_lds_norm") != 0)
+        return run_ragged_norm(w, xa, out, R, C, M, false, static_cast<hipStream_t>(stream));
     return run_rows<FmtBf16, X_ADDNORM, E_PLAIN>(p, xa, out, R, C, M, static_cast<hipStream_t>(stream));
 }
 

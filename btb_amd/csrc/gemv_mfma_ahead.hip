@@ -10,6 +10,8 @@
 // the next two tiles are always on their way.
 
 #include "btb_common.hpp"
+#include "btb_formats.hpp"
+#include "btb_stream.hpp"
 #include "btb_tuning.hpp"
 
 #include "../../include/btb_hip.h"
@@ -19,16 +21,17 @@ namespace btb {
 // SPW: the steps (32 columns) a wave's slice holds at most. TR: the rows of a tile that are rows of the matrix; the others are
 // not read, and what the matrix cores make of them is not written. RAG: R is no multiple of TR (and at least that): the last
 // tile starts TR rows before the end and writes the rows no other tile has. GLU: W is I gate rows over I up rows, a tile
-// eight of each (the same outputs'), y their fold [M, I].
-template <int KS, int MT, int SPW, int TR, bool RAG, bool GLU>
+// eight of each (the same outputs'), y their fold [M, I]; RAG there: I is no multiple of eight. XN: x is not given but made, the
+// residual add and RMSNorm of xa (every workgroup makes the pass's rows, add_rmsnorm_kernel's bits).
+template <int KS, int MT, int SPW, int TR, bool RAG, bool GLU, bool XN>
 __global__ void __launch_bounds__(KS * 64) mfma_ahead_kernel(const uint8_t* __restrict__ w, const uint4* __restrict__ x,
-                                                             uint16_t* __restrict__ y, int R, int C, int M) {
+                                                             uint16_t* __restrict__ y, int R, int C, int M, XArgs xa) {
     constexpr int PIECES = SPW * 4;                      // 16-byte pieces a slice has of a row
     constexpr int NLD = (TR * PIECES + WAVE - 1) / WAVE;  // load instructions a wave's share of a tile takes
     constexpr int STRIDE = SPW * 64 + 16;                // a slab row: 4 banks past a multiple of 32
     constexpr int SLAB = 16 * STRIDE;
-    static_assert(!GLU || (TR == 16 && !RAG), "a folded tile is eight gate rows over eight up rows");
-    extern __shared__ __align__(16) uint8_t lds[];  // KS slabs, then two sets of KS * MT partial tiles
+    static_assert(!GLU || TR == 16, "a folded tile is eight gate rows over eight up rows");
+    extern __shared__ __align__(16) uint8_t lds[];  // KS slabs, then two sets of KS * MT partial tiles; XN: the made rows first
     const int lane = threadIdx.x & (WAVE - 1);
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
     const int li = lane & 15, lg = lane >> 4;
@@ -46,8 +49,88 @@ __global__ void __launch_bounds__(KS * 64) mfma_ahead_kernel(const uint8_t* __re
     const uint32_t valid = min((uint32_t)(last + 1) * 64, rowbytes - (uint32_t)sn * 64);
     const bool ragged = valid % 64 != 0;  // uniform
     uint4 xb[MT][SPW];
+    if constexpr (XN) {
+        static_assert(MT == 1, "sixteen rows in the making");
+        const int stride = C * 2 + 16;
+        // A wave makes a row by itself: four sums a lane, each that of a lane of one of the four waves that add_rmsnorm_kernel
+        // gives a row, over the same words in the same order. (Rows and weights at any 2-byte place, as in stage_x.)
+        // Several rows' words are asked for at once where the rows are short: two waves that made eight rows of 520 values one
+        // after the other took 6 us of a launch of 13.
+        constexpr int WORDS = (KS * SPW * 32 + 1023) / 1024;  // 4-element words a lane has of each of the four
+        constexpr int ROWS = WORDS == 1 ? 4 : WORDS == 2 ? 2 : 1;
+        const int n4 = C / 4;
+        const bool has_y = xa.y != nullptr, writer = first == 0 && xa.h_out != nullptr;
+        const uint2* ws = reinterpret_cast<const uint2*>(xa.norm_w);
+        auto word = [&](int v, int q) { return q * 256 + v * 64 + lane; };
+        for (int m0 = wv; m0 < M; m0 += KS * ROWS) {
+            uint2 hv[ROWS][4][WORDS], yv[ROWS][4][WORDS];
 #pragma unroll
-    for (int t = 0; t < MT; ++t) {
+            for (int r = 0; r < ROWS; ++r) {  // past the pass's rows its last again, made and left like the first time
+                const int m = min(m0 + r * KS, M - 1);
+                size_t hrow = (size_t)m;
+                if (xa.ids != nullptr) hrow = (size_t)min(max(xa.ids[m], 0), xa.vocab - 1);
+                const uint2* hs = reinterpret_cast<const uint2*>(xa.x + hrow * C);
+                const uint2* ys = has_y ? reinterpret_cast<const uint2*>(xa.y + (size_t)m * C) : hs;
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+#pragma unroll
+                    for (int q = 0; q < WORDS; ++q) {
+                        hv[r][v][q] = hs[min(word(v, q), n4 - 1)];
+                        yv[r][v][q] = ys[min(word(v, q), n4 - 1)];
+                    }
+            }
+#pragma unroll
+            for (int r = 0; r < ROWS; ++r) {
+                const int m = min(m0 + r * KS, M - 1);
+                float sums[4];
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    float ss = 0.f;
+#pragma unroll
+                    for (int q = 0; q < WORDS; ++q) {
+                        const int i = word(v, q);
+                        const uint2 hw = hv[r][v][q], yw = yv[r][v][q];
+                        float f[4] = {bf16lo_f32(hw.x), bf16hi_f32(hw.x), bf16lo_f32(hw.y), bf16hi_f32(hw.y)};
+                        const float g[4] = {bf16lo_f32(yw.x), bf16hi_f32(yw.x), bf16lo_f32(yw.y), bf16hi_f32(yw.y)};
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const float sum = bfround(f[e] + g[e]);
+                            f[e] = has_y ? sum : f[e];
+                            const float sq = fmaf(f[e], f[e], ss);
+                            ss = i < n4 ? sq : ss;
+                        }
+                        hv[r][v][q] = make_uint2(f32x2_bf16(f[0], f[1]), f32x2_bf16(f[2], f[3]));  // exact: bf16 values
+                        if (writer && i < n4) reinterpret_cast<uint2*>(xa.h_out + (size_t)m * C)[i] = hv[r][v][q];
+                    }
+                    sums[v] = wave_sum(ss);
+                }
+                const float rstd = rsqrtf((((sums[0] + sums[1]) + sums[2]) + sums[3]) / (float)C + xa.eps);
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+#pragma unroll
+                    for (int q = 0; q < WORDS; ++q) {
+                        const int i = word(v, q);
+                        const uint2 hw = hv[r][v][q], nw = ws[min(i, n4 - 1)];
+                        const float f[4] = {bf16lo_f32(hw.x), bf16hi_f32(hw.x), bf16lo_f32(hw.y), bf16hi_f32(hw.y)};
+                        const float g[4] = {bf16lo_f32(nw.x), bf16hi_f32(nw.x), bf16lo_f32(nw.y), bf16hi_f32(nw.y)};
+                        float o[4];
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) o[e] = f[e] * rstd * (xa.centered ? 1.f + g[e] : g[e]);
+                        if (i < n4)
+                            *reinterpret_cast<uint2*>(lds + (size_t)m * stride + (size_t)i * 8) =
+                                make_uint2(f32x2_bf16(o[0], o[1]), f32x2_bf16(o[2], o[3]));
+                    }
+            }
+        }
+        __syncthreads();
+        const uint8_t* xr = lds + (size_t)min(li, M - 1) * stride + (size_t)sn * 64;
+#pragma unroll
+        for (int i = 0; i < SPW; ++i)
+            xb[0][i] = *reinterpret_cast<const uint4*>(xr + min(min(i, last) * 4 + lg, (int)valid / 16 - 1) * 16);
+        __syncthreads();  // the rows have been read: the slabs may take their place
+    }
+#pragma unroll
+    for (int t = 0; t < (XN ? 0 : MT); ++t) {
         const uint4* xr = x + (size_t)min(t * 16 + li, M - 1) * (C / 8) + (size_t)sn * 4;
 #pragma unroll
         for (int i = 0; i < SPW; ++i) xb[t][i] = xr[min(min(i, last) * 4 + lg, (int)valid / 16 - 1)];
@@ -67,7 +150,9 @@ __global__ void __launch_bounds__(KS * 64) mfma_ahead_kernel(const uint8_t* __re
     }
     constexpr int RPL = WAVE / PIECES;  // WHOLE: rows a load covers
     static_assert(!WHOLE || TR % RPL == 0, "a tile is whole loads");
-    auto row_of = [&](int tile) { return GLU ? tile * 8 : RAG ? min(tile * TR, R - TR) : tile * TR; };
+    constexpr int OUT = GLU ? 8 : TR;  // outputs a tile
+    const int outs = GLU ? R / 2 : R;
+    auto row_of = [&](int tile) { return RAG ? min(tile * OUT, outs - OUT) : tile * OUT; };
     uint32_t past = 0;  // the loads whose piece lies past a short last step's end
     if (ragged) {
 #pragma unroll
@@ -152,11 +237,12 @@ __global__ void __launch_bounds__(KS * 64) mfma_ahead_kernel(const uint8_t* __re
                         const float gb = bfround(g), ub = bfround(u);
                         return f32_bf16(bfround(gb / (1.f + expf(-gb))) * ub);
                     };
-                    uint16_t* o = y + (size_t)m * (R / 2) + tile * 8 + lg * 4;
-                    o[0] = fold(s.x, up.x);
-                    o[1] = fold(s.y, up.y);
-                    o[2] = fold(s.z, up.z);
-                    o[3] = fold(s.w, up.w);
+                    const int row = row_of(tile) + lg * 4, own = RAG ? tile * OUT : 0;
+                    uint16_t* o = y + (size_t)m * outs + row;
+                    if (row + 0 >= own) o[0] = fold(s.x, up.x);
+                    if (row + 1 >= own) o[1] = fold(s.y, up.y);
+                    if (row + 2 >= own) o[2] = fold(s.z, up.z);
+                    if (row + 3 >= own) o[3] = fold(s.w, up.w);
                 }
             } else {
                 const int in_tile = lg * 4, row = row_of(tile) + in_tile;
@@ -181,11 +267,13 @@ __global__ void __launch_bounds__(KS * 64) mfma_ahead_kernel(const uint8_t* __re
     if (k < turns) turn(k, raw[0]);
 }
 
-template <int KS, int MT, int SPW, int TR, bool RAG, bool GLU>
-static int32_t launch_ahead(const void* w, const void* x, void* y, int R, int C, int M, int cap, hipStream_t st) {
+template <int KS, int MT, int SPW, int TR, bool RAG, bool GLU, bool XN = false>
+static int32_t launch_ahead(const void* w, const void* x, void* y, int R, int C, int M, int cap, hipStream_t st,
+                            const XArgs& xa = XArgs{}) {
     constexpr int SLAB = 16 * (SPW * 64 + 16);
-    const size_t lds = (size_t)KS * SLAB + 2 * (size_t)KS * MT * WAVE * sizeof(f32x4);
-    auto kern = mfma_ahead_kernel<KS, MT, SPW, TR, RAG, GLU>;
+    size_t lds = (size_t)KS * SLAB + 2 * (size_t)KS * MT * WAVE * sizeof(f32x4);
+    if (XN && 16 * ((size_t)C * 2 + 16) > lds) lds = 16 * ((size_t)C * 2 + 16);  // the made rows, before the slabs
+    auto kern = mfma_ahead_kernel<KS, MT, SPW, TR, RAG, GLU, XN>;
     if (lds > 64 * 1024) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return hip_status(e, "hipFuncSetAttribute");
@@ -194,7 +282,7 @@ static int32_t launch_ahead(const void* w, const void* x, void* y, int R, int C,
     // whole turns of the grid over the tiles: the smallest grid that walks them in ceil(ntiles / cap) turns
     const int turns = (ntiles + cap - 1) / cap, grid = (ntiles + turns - 1) / turns;
     hipLaunchKernelGGL(kern, dim3(grid), dim3(KS * 64), lds, st, static_cast<const uint8_t*>(w), static_cast<const uint4*>(x),
-                       static_cast<uint16_t*>(y), R, C, M);
+                       static_cast<uint16_t*>(y), R, C, M, xa);
     return hip_status(hipGetLastError(), "gemv_mfma_ahead launch");
 }
 
@@ -205,7 +293,10 @@ static int32_t run_ahead(const void* w, const void* x, void* y, int R, int C, in
     int per_cu = tuning("mfma_wgs_per_cu");
     if (per_cu <= 0) per_cu = R <= 16 * (12 / KS) * device_info().cus ? 12 / KS : 8 / KS;
     const int cap = device_info().cus * per_cu;
-    if (glu) return launch_ahead<KS, MT, SPW, 16, false, true>(w, x, y, R, C, M, cap, st);
+    if (glu) {
+        if (R % 16 != 0) return launch_ahead<KS, MT, SPW, 16, true, true>(w, x, y, R, C, M, cap, st);
+        return launch_ahead<KS, MT, SPW, 16, false, true>(w, x, y, R, C, M, cap, st);
+    }
     if (R % 16 != 0 && R % 12 != 0 && R % 10 != 0) return launch_ahead<KS, MT, SPW, 16, true, false>(w, x, y, R, C, M, cap, st);
     if constexpr (KS == 8) {
         if (tuning("mfma_tile_rows") != 0) {
@@ -238,9 +329,13 @@ bool mfma_ahead_fits(int R, int C, int M, bool glu) {
 // of four rows on the vector units: from five rows of x on, in passes of 32 rows, or of 16 past 2560 columns. us at 5 / 8 / 16 / 32
 // rows, those passes / here: [512 x 520] 4.5 / 3.2, 5.2 / 3.3, 10.0 / 3.4, 19.5 / 3.9; [2560 x 2056] 9.0 / 5.4, 9.8 / 5.5, 18.8 / 5.9,
 // 37.7 / 7.5; [5003 x 3000] 16.1 / 11.3, 17.3 / 11.5, 32.3 / 11.7, 63.8 / 23.0; [40000 x 3000] 84 / 43, 85 / 44, 168 / 45, 318 / 87
-// (5.5 TB/s); [512 x 4088] 7.1 / 6.5, 8.6 / 6.7, 16.6 / 7.7, 32.8 / 14.8.
+// (5.5 TB/s); [512 x 4088] 7.1 / 6.5, 8.6 / 6.7, 16.6 / 7.7, 32.8 / 14.8. The gate / up fold and the add + norm go with it, or their
+// sums would be in another order than the matvec's: at 5 / 8 / 16 rows the fold [2560 x 520] 7.4 / 4.5, 8.7 / 4.5, 16.6 / 4.5,
+// [8192 x 2056] 17.7 / 11.3, 19.1 / 11.3, 37.8 / 12.0; the norm [2560 x 520] 8.9 / 8.2, 11.4 / 8.2, 22.3 / 12.1, [1000 x 1016] 8.7 /
+// 9.0, 11.3 / 9.0, 21.9 / 9.2, [8192 x 2056] 22.0 / 14.4, 28.5 / 14.8, 55.3 / 18.9, [512 x 4088] 14.6 / 12.8, 22.6 / 13.1, 44.8 / 19.8.
 bool mfma_ahead_ragged_fits(int R, int C) {
-    return tuning("mfma_ahead") != 0 && tuning("mfma_lds") != 0 && R >= 16 && C % 32 != 0 && C % 8 == 0 && C >= 64 && C <= 4096;
+    return tuning("mfma_ahead") != 0 && tuning("mfma_lds") != 0 && R >= 16 && C % 32 != 0 && C % 8 == 0 && C >= 64 && C <= 4096 &&
+           (uint64_t)R * C < 1ull << 31;  // a gate row's up row within 32 bits
 }
 // the waves a tile by row length as gemv_mfma_lds has them (two, four or eight), the slice's size close above its steps
 int32_t gemv_mfma_ahead_bf16(const void* w, const void* x, void* y, int R, int C, int M, bool glu, hipStream_t st) {
@@ -256,6 +351,26 @@ int32_t gemv_mfma_ahead_bf16(const void* w, const void* x, void* y, int R, int C
 #undef BTB_AHEAD
     if (nsteps <= 96) return run_ahead<8, 1, 12>(w, x, y, R, C, M, glu, st);
     return run_ahead<8, 1, 16>(w, x, y, R, C, M, glu, st);
+}
+
+// ... with x made by the residual add and RMSNorm, for the ragged rows (mfma_ahead_ragged_fits): up to sixteen rows of the
+// residual stream
+template <int KS, int SPW>
+static int32_t run_ahead_norm(const void* w, const XArgs& xa, void* y, int R, int C, int M, bool glu, hipStream_t st) {
+    const int cap = device_info().cus * (8 / KS);
+    if (glu) return launch_ahead<KS, 1, SPW, 16, true, true, true>(w, nullptr, y, R, C, M, cap, st, xa);
+    return launch_ahead<KS, 1, SPW, 16, true, false, true>(w, nullptr, y, R, C, M, cap, st, xa);
+}
+int32_t gemv_mfma_ahead_norm_bf16(const void* w, const XArgs& xa, void* y, int R, int C, int M, bool glu, hipStream_t st) {
+    const int nsteps = (C + 31) / 32;
+    if (nsteps <= 16) return run_ahead_norm<2, 8>(w, xa, y, R, C, M, glu, st);
+    if (nsteps <= 20) return run_ahead_norm<2, 10>(w, xa, y, R, C, M, glu, st);
+    if (nsteps <= 32) return run_ahead_norm<4, 8>(w, xa, y, R, C, M, glu, st);
+    if (nsteps <= 40) return run_ahead_norm<4, 10>(w, xa, y, R, C, M, glu, st);
+    if (nsteps <= 64) return run_ahead_norm<8, 8>(w, xa, y, R, C, M, glu, st);
+    if (nsteps <= 80) return run_ahead_norm<8, 10>(w, xa, y, R, C, M, glu, st);
+    if (nsteps <= 96) return run_ahead_norm<8, 12>(w, xa, y, R, C, M, glu, st);
+    return run_ahead_norm<8, 16>(w, xa, y, R, C, M, glu, st);
 }
 
 }  // namespace btb

@@ -84,14 +84,18 @@ int32_t btb_hip_gemv_silu_bf16(const void* w, const void* gu, void* y, size_t R,
 
 /* Gate, up and the activation in one kernel: w [2I, C] bf16 (gate rows, then up rows), x [M, C], m [M, I] =
  * bf16(bf16(silu(g)) * u) with g = bf16(w[i] . x), u = bf16(w[I + i] . x): the bits of btb_hip_gemv_bf16 followed by
- * btb_hip_silu_mul. Replaces btb_gemv_mma_glu_silu (native/cuda/btb_gemv_mma.cuh:216-315). */
+ * btb_hip_silu_mul (from five rows of x on with C a multiple of 32: where I is a multiple of 16 and C at most 10240; the
+ * matvec's other matrix-core kernel has no fold, and this entry's sums are then in the vector kernels' order). Replaces
+ * btb_gemv_mma_glu_silu (native/cuda/btb_gemv_mma.cuh:216-315). */
 int32_t btb_hip_gemv_glu_silu_bf16(const void* w, const void* x, void* m, size_t I, size_t C, size_t M, void* stream);
 
 /* The matvec with the residual add and the RMSNorm folded into its x load: h' = bf16(h_in + y) (y NULL: h' = h_in),
  * x = bf16(h' * rsqrt(mean(h'^2) + eps) * norm_w) (or * (1 + norm_w) when centered), out = W x; h' is written to
  * h_out (NULL: not kept; never h_in itself). With glu != 0, W is [R = 2I, C] and out is the gate/up fold m [M, I] of
- * btb_hip_gemv_glu_silu_bf16. The bits are those of btb_hip_add_rmsnorm followed by the matvec; it replaces that
- * pair of launches of the reference's step (btb/engine/cuda.py:1730-1733, 1770-1793). */
+ * btb_hip_gemv_glu_silu_bf16. The bits are those of btb_hip_add_rmsnorm followed by the matvec (from five rows of x on
+ * with C a multiple of 32: where C is 1312 .. 2560, R - with glu R / 2 - a multiple of 16 and the rows 8-byte aligned; elsewhere
+ * the sums are in the vector kernels' order); it replaces that pair of launches of the reference's step
+ * (btb/engine/cuda.py:1730-1733, 1770-1793). */
 int32_t btb_hip_gemv_bf16_norm(const void* w, const void* h_in, const void* y, const void* norm_w, float eps,
                                int32_t centered, void* h_out, void* out, size_t R, size_t C, size_t M, int32_t glu,
                                void* stream);

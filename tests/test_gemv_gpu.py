@@ -374,3 +374,35 @@ def test_rows_of_no_multiple_of_32_columns_on_the_matrix_cores(card, R, C, M):
     y, ref = y[: M - 1, keep], ref[: M - 1, keep]
     bound = 2.0**-8 * ref.abs() * 1.01 + 2 * C * 2.0**-24 * (x[: M - 1].double().abs() @ w[keep].double().abs().T)
     assert bool(((y - ref).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("R,C,M", [(16, 72, 5), (34, 520, 8), (512, 648, 17), (1008, 1016, 33), (130, 1288, 6), (2576, 2056, 12),
+                                   (5006, 2552, 16), (2560, 2568, 20), (300, 3000, 5), (1536, 3592, 16), (16, 4088, 8)])
+def test_the_forms_of_rows_of_no_multiple_of_32_columns_agree(card, R, C, M):
+    """From five rows of x on, over rows whose last step of 32 columns is short: the gate / up fold has the bits of the matvec and
+    silu_mul, the add + norm forms those of add_rmsnorm and the matvec, a row those it has in a narrower pass."""
+    bits = lambda t: t.view(torch.int16)
+    empty = lambda rows, cols: torch.empty(rows, cols, dtype=torch.bfloat16, device="cuda")
+    w, x, d = weights_bf16(R, C, seed=210).cuda(), acts_bf16(M, C, seed=211).cuda(), acts_bf16(M, C, seed=212).cuda()
+    nw = (1.0 + 0.1 * torch.randn(C, generator=torch.Generator().manual_seed(213))).to(torch.bfloat16).cuda()
+    y = card.gemv(w, x)
+    m = empty(M, R // 2)
+    card.silu_mul(y, m)
+    assert torch.equal(bits(card.gemv_glu_silu(w, x)), bits(m))
+    assert torch.equal(bits(card.gemv(w, x[:5].contiguous())), bits(y[:5]))
+    for add in (d, None):
+        h, xn, h2 = x.clone(), empty(M, C), empty(M, C)
+        card.add_rmsnorm(h, add, nw, 1e-6, xn)
+        want = card.gemv(w, xn)
+        got = card.gemv_norm(w, x, add, nw, 1e-6, h2, empty(M, R))
+        assert torch.equal(bits(got), bits(want)) and torch.equal(bits(h2), bits(h))
+        card.silu_mul(want, m)
+        got = card.gemv_norm(w, x, add, nw, 1e-6, h2.zero_(), empty(M, R // 2), glu=True)
+        assert torch.equal(bits(got), bits(m)) and torch.equal(bits(h2), bits(h))
+        got = card.gemv_norm(w, x, add, nw, 1e-6, None, empty(M, R), centered=True)
+        card.add_rmsnorm(x.clone(), add, nw, 1e-6, xn, centered=True)
+        assert torch.equal(bits(got), bits(card.gemv(w, xn)))
+    ids = torch.arange(M - 1, -1, -1, dtype=torch.int32, device="cuda")
+    card.add_rmsnorm(x.flip(0).contiguous(), None, nw, 1e-6, xn)
+    got = card.gemv_embed_norm(w, x, ids, nw, 1e-6, h2, empty(M, R))
+    assert torch.equal(bits(got), bits(card.gemv(w, xn))) and torch.equal(bits(h2), bits(x.flip(0)))
