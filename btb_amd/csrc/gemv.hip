@@ -586,9 +586,11 @@ static bool wide_pass(Form f, size_t M, size_t R, size_t C, size_t from = 5) {
 }
 
 // Whether a bf16 pass of M rows over rows of C % 32 != 0 columns goes to the matrix cores: the plain matvec's, the gate / up fold's
-// and the add + norm's alike, so that the three keep to one order of the sums.
+// and the add + norm's alike, so that the three keep to one order of the sums. The family has no other kernel for such rows, so
+// only the knobs that choose the family move them.
 static bool ragged_pass(size_t M, size_t R, size_t C) {
-    return M >= 5 && tuning("gemv_no_mfma") <= 0 && mfma_ahead_ragged_fits((int)R, (int)C);
+    const size_t from = tuning("gemv_mfma_from") > 0 ? (size_t)tuning("gemv_mfma_from") : 5;
+    return M >= from && tuning("gemv_no_mfma") <= 0 && mfma_ahead_ragged_fits((int)R, (int)C);
 }
 static int32_t run_ragged(const void* w, const void* x, void* y, size_t R, size_t C, size_t M, bool glu, hipStream_t st) {
     const size_t step = C <= 2560 ? 32 : 16, outs = glu ? R / 2 : R;

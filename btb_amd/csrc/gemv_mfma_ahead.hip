@@ -334,7 +334,7 @@ bool mfma_ahead_fits(int R, int C, int M, bool glu) {
 // [8192 x 2056] 17.7 / 11.3, 19.1 / 11.3, 37.8 / 12.0; the norm [2560 x 520] 8.9 / 8.2, 11.4 / 8.2, 22.3 / 12.1, [1000 x 1016] 8.7 /
 // 9.0, 11.3 / 9.0, 21.9 / 9.2, [8192 x 2056] 22.0 / 14.4, 28.5 / 14.8, 55.3 / 18.9, [512 x 4088] 14.6 / 12.8, 22.6 / 13.1, 44.8 / 19.8.
 bool mfma_ahead_ragged_fits(int R, int C) {
-    return tuning("mfma_ahead") != 0 && tuning("mfma_lds") != 0 && R >= 16 && C % 32 != 0 && C % 8 == 0 && C >= 64 && C <= 4096 &&
+    return R >= 16 && C % 32 != 0 && C % 8 == 0 && C >= 64 && C <= 4096 &&
            (uint64_t)R * C < 1ull << 31;  // a gate row's up row within 32 bits
 }
 // the waves a tile by row length as gemv_mfma_lds has them (two, four or eight), the slice's size close above its steps

@@ -406,3 +406,27 @@ def test_the_forms_of_rows_of_no_multiple_of_32_columns_agree(card, R, C, M):
     card.add_rmsnorm(x.flip(0).contiguous(), None, nw, 1e-6, xn)
     got = card.gemv_embed_norm(w, x, ids, nw, 1e-6, h2, empty(M, R))
     assert torch.equal(bits(got), bits(card.gemv(w, xn))) and torch.equal(bits(h2), bits(x.flip(0)))
+
+
+@pytest.mark.parametrize("R,C,M", [(34, 520, 8), (1008, 1016, 33), (2576, 2056, 12), (300, 3000, 5)])
+def test_knobs_over_rows_of_no_multiple_of_32_columns(card, R, C, M):
+    """The knobs that choose a kernel within the matrix-core family move no bit of such rows, `gemv_no_mfma` and `gemv_mfma_from`
+    choose the family as they do for other rows."""
+    bits = lambda t: t.view(torch.int16)
+    w, x = weights_bf16(R, C, seed=214).cuda(), acts_bf16(M, C, seed=215).cuda()
+    y = card.gemv(w, x)
+    try:
+        for knob in ("mfma_ahead", "mfma_lds", "mfma_tile_rows"):
+            card.set_tuning(knob, 0)
+            assert torch.equal(bits(card.gemv(w, x)), bits(y)), knob
+            card.set_tuning(knob, -1)
+        card.set_tuning("gemv_no_mfma", 1)
+        vector = card.gemv(w, x)
+        card.set_tuning("gemv_no_mfma", -1)
+        card.set_tuning("gemv_mfma_from", M + 1)
+        assert torch.equal(bits(card.gemv(w, x)), bits(vector))
+        card.set_tuning("gemv_mfma_from", 2)
+        assert torch.equal(bits(card.gemv(w, x[:3].contiguous())), bits(y[:3]))
+    finally:
+        for knob in ("mfma_ahead", "mfma_lds", "mfma_tile_rows", "gemv_no_mfma", "gemv_mfma_from"):
+            card.set_tuning(knob, -1)
