@@ -137,9 +137,10 @@ __global__ void __launch_bounds__(256) lane16_kernel(W w, const XT* __restrict__
 // chain of fused multiply-adds in the same column order. Writes and reads of a slab are one wave's, which LDS serves in
 // program order: no barrier between them. TAIL: the row ends inside its last step (a multiple of 8 columns, so that rows
 // and pieces stay 16-byte aligned): the pieces past its end are the row's last piece again and their products are
-// dropped (x's place there holds whatever LDS held). Bound by the chain of a lane's fused multiply-adds and the two LDS
+// dropped (x's place there holds whatever LDS held); only that step looks (with every step looking, us: 128 rows of 4104, four
+// rows of x 27.9, now 15.6). Bound by the chain of a lane's fused multiply-adds and the two LDS
 // reads each takes, so few waves a CU are best: a router's workgroup is eight rows (128 threads). Measured with the
-// routing behind it, us: [32 x 2880] one row 22.3 (lane16_kernel) -> 9.6, 32 rows 43.9 (passes of four) -> 10.1;
+// routing behind it, us: [32 x 2880] one row 22.3 (lane16_kernel) -> 8.2, 32 rows 43.9 (passes of four) -> 8.5;
 // [128 x 2048] 7.1 -> 6.4 (sixteen rows a workgroup -> eight), [128 x 4096] 9.5 -> 8.6.
 template <int B, int NB, class XT, bool TAIL, int NT>
 __global__ void __launch_bounds__(NT) lane16_bf16_wide_kernel(const uint16_t* __restrict__ w, const XT* __restrict__ x,
@@ -147,7 +148,7 @@ __global__ void __launch_bounds__(NT) lane16_bf16_wide_kernel(const uint16_t* __
                                                               size_t btotal) {
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr int BP = B == 3 ? 4 : B;  // a column's B values of x side by side, one LDS read
-    const int nchunks = (int)((cols + 127) / 128);
+    const int nchunks = (int)((cols + 127) / 128), whole = (int)(cols / 128);
     float* xs = reinterpret_cast<float*>(smem);                           // [nchunks * 128][BP]
     unsigned char* slabs = smem + (size_t)BP * (size_t)nchunks * 128 * 4;  // [NT / 16 groups][NB][256]
     b0 += (size_t)blockIdx.y * B;
@@ -201,21 +202,22 @@ __global__ void __launch_bounds__(NT) lane16_bf16_wide_kernel(const uint16_t* __
 #pragma unroll
         for (int n = 0; n < NB; ++n) *reinterpret_cast<u32x4*>(mine + n * 256 + 16 * j) = raw[n];
         if (n0 + NB < nchunks) request(n0 + NB);
+        auto step = [&](int n, auto part) {  // part: the row ends inside it
 #pragma unroll
-        for (int n = 0; n < NB; ++n) {
-            if (n0 + n < nchunks) {
+            for (int u = 0; u < 8; ++u) {
+                const float wv = bf16_f32(*reinterpret_cast<const uint16_t*>(mine + n * 256 + 2 * (j + 16 * u)));
+                const size_t c = (size_t)(n0 + n) * 128 + j + 16 * u;
 #pragma unroll
-                for (int u = 0; u < 8; ++u) {
-                    const float wv = bf16_f32(*reinterpret_cast<const uint16_t*>(mine + n * 256 + 2 * (j + 16 * u)));
-                    const size_t c = (size_t)(n0 + n) * 128 + j + 16 * u;
-#pragma unroll
-                    for (int i = 0; i < B; ++i) {
-                        const float sum = fmaf(wv, xs[c * BP + i], acc[i]);
-                        acc[i] = !TAIL || c < cols ? sum : acc[i];
-                    }
+                for (int i = 0; i < B; ++i) {
+                    const float sum = fmaf(wv, xs[c * BP + i], acc[i]);
+                    acc[i] = !decltype(part)::value || c < cols ? sum : acc[i];
                 }
             }
-        }
+        };
+#pragma unroll
+        for (int n = 0; n < NB; ++n)
+            if (n0 + n < whole) step(n, std::false_type{});
+        if (TAIL && n0 + NB > whole) step(whole - n0, std::true_type{});  // the last batch: whole < nchunks
     }
 #pragma unroll
     for (int i = 0; i < B; ++i) {
@@ -246,17 +248,50 @@ static bool launch_wide_as(const uint16_t* w, const XT* x, float* y, size_t rows
 // a matrix small enough that what bounds a pass is a row's chain, not its bytes
 static bool router_sized(size_t rows, size_t cols) { return rows * cols <= (1u << 20); }
 
-template <int B, int NB, class XT>
+// A pass a row of x, all of them in one launch: the matrix is re-read once a row out of L2, but every row's sums start at once,
+// where passes of four rows take four times the arithmetic each behind a fourfold staging. It pays while the launch's rows are
+// few, us passes of four / this: [128 x 2048] 32 rows of x 7.6 / 4.9, 64 7.8 / 6.8; [512 x 1024] 16 5.4 / 5.2, 32 5.6 / 8.5; [1024 x
+// 1024] with the routing 8 19.4 / 18.1, 16 19.6 / 21.4; [2048 x 520] 2 4.7 / 4.7, 4 4.9 / 5.7; [5697 x 128] 64 13.6 / 78.
+static bool pass_a_row(size_t rows, size_t cols, size_t b) {
+    // (b no multiple of four: the passes of four leave a launch of one to three rows behind them, [512 x 1024] 17 rows 8.7 / 6.2)
+    const bool whole = b % 4 == 0;
+    const size_t most = rows <= 1024 ? (whole ? 8192 : 16384) : (!whole && b > 4 && b < 8 ? 12288 : 4096);
+    return b > 1 && b <= 64 && router_sized(rows, cols) && rows * b <= most;
+}
+
+// Whether the wide kernel takes n rows of x (four and more: in passes of four) over f32 x and rows that end inside a step, which
+// lane16_kernel takes 512 columns at a time (128 from two rows on) and what is left sixteen by sixteen. us lane16_kernel / wide: one
+// row of x [128 x 520] 2.6 / 3.6, [128 x 2056] 4.8 / 6.2, [14615 x 544] 6.2 / 10.2, [170 x 6424] 13.8 / 15.3, but [276 x 240] 5.0 /
+// 4.3, [2048 x 264] 6.2 / 3.3, [512 x 2880] 9.3 / 7.8; two rows [2048 x 520] 5.3 / 4.7, [2048 x 136] 2.9 / 3.2, [793 x 208] 5.1 / 4.3,
+// [8192 x 520] 5.7 / 6.3, [8192 x 2056] 18.7 / 14.1, [32768 x 520] 13.0 / 17.3; four [8192 x 136] 4.0 / 4.3, [10746 x 504] 10.8 / 8.5, [32768 x
+// 264] 9.7 / 11.4; eight [32768 x 136] 13.0 / 13.0. (A bf16 x is 2 bytes a request there: [128 x 520] one row 7.6 / 5.5.)
+static bool wide_pays(size_t rows, size_t cols, size_t n, bool f32) {
+    if (!f32 || cols % 128 == 0 || n >= 8) return true;
+    if (n == 1) return cols % 512 > 176 + cols / 64;
+    if (n < 4) return rows <= (cols < 1024 ? 4096u : 8192u) && (cols >= 256 || cols % 128 >= 64);
+    return cols >= rows / 32;
+}
+
+// SMALL: workgroups of eight rows
+template <int B, int NB, bool SMALL = false, class XT>
 static bool launch_wide(const uint16_t* w, const XT* x, float* y, size_t rows, size_t cols, size_t b0, size_t b,
                         unsigned passes, hipStream_t st) {
-    if constexpr (B == 1) {
-        if (router_sized(rows, cols)) {
-            if (cols % 128 == 0) return launch_wide_as<B, NB, false, 128>(w, x, y, rows, cols, b0, b, passes, st);
-            return launch_wide_as<B, NB, true, 128>(w, x, y, rows, cols, b0, b, passes, st);
-        }
+    if constexpr (SMALL) {
+        if (cols % 128 == 0) return launch_wide_as<B, NB, false, 128>(w, x, y, rows, cols, b0, b, passes, st);
+        return launch_wide_as<B, NB, true, 128>(w, x, y, rows, cols, b0, b, passes, st);
     }
     if (cols % 128 == 0) return launch_wide_as<B, NB, false, 256>(w, x, y, rows, cols, b0, b, passes, st);
     return launch_wide_as<B, NB, true, 256>(w, x, y, rows, cols, b0, b, passes, st);
+}
+// one row of x a pass. Eight rows of the matrix a workgroup where the launch's arithmetic is small, else its x is staged too often:
+// us at eight / sixteen, [128 x 2048] 32 rows of x 4.9 / 5.2, [128 x 4096] 32 8.2 / 8.2, 64 15.8 / 12.2, [128 x 2880] 64 16.8 / 11.7;
+// past 4096 columns a CU holds one workgroup of sixteen: [136 x 4992] 40 13.7 / 18.9
+template <class XT>
+static bool launch_wide_rows(const uint16_t* w, const XT* x, float* y, size_t rows, size_t cols, size_t b0, size_t b,
+                             unsigned passes, hipStream_t st) {
+    if (router_sized(rows, cols) && (cols > 4096 || rows * passes * cols <= (1u << 24)))
+        return launch_wide<1, 16, true>(w, x, y, rows, cols, b0, b, passes, st);
+    return launch_wide<1, 16>(w, x, y, rows, cols, b0, b, passes, st);
 }
 
 template <class W, class XT>
@@ -265,18 +300,15 @@ static int32_t launch_lane16(const W& w, const XT* x, float* y, size_t rows, siz
     size_t b0 = 0;
     if constexpr (std::is_same<W, W16Bf16>::value) {
         if (cols % 8 == 0 && ((reinterpret_cast<uintptr_t>(w.w) | reinterpret_cast<uintptr_t>(x)) & 15) == 0) {
-            // every pass of four rows of x in one launch (the pass is the grid's second dimension), then the rest
-            bool done = true;
-            // Rows of x against a small matrix (a router at the verify widths): a pass a row, all in one launch. The
-            // matrix is re-read once a row out of L2, but every row's sums start at once, where passes of four rows
-            // take four times the arithmetic each behind a fourfold staging (32 / 64 rows, with the routing: [32 x 2880]
-            // 25.2 / 25.4 -> 10.1 / 10.3 us, [128 x 2048] 12.3 / 12.4 -> 7.9 / 9.7, [128 x 4096] 19.6 / 19.7 -> 10.8 /
-            // 17.3). A (row, vector) sum is the same chain of operations in every form.
-            if (b > 1 && b <= 64 && router_sized(rows, cols)) {
-                done = launch_wide<1, 16>(w.w, x, y, rows, cols, 0, b, (unsigned)b, st);
+            // every pass of four rows of x in one launch (the pass is the grid's second dimension), then the rest; a (row,
+            // vector) sum is the same chain of operations in every form
+            constexpr bool F32 = sizeof(XT) == 4;
+            bool done = wide_pays(rows, cols, b, F32);
+            if (done && pass_a_row(rows, cols, b)) {
+                done = launch_wide_rows(w.w, x, y, rows, cols, 0, b, (unsigned)b, st);
                 if (done) b0 = b;
             }
-            const size_t fours = b0 < b ? std::min<size_t>(b / 4, 65535) : 0;
+            const size_t fours = done && b0 < b ? std::min<size_t>(b / 4, 65535) : 0;
             if (fours > 0) {
                 // few rows of weights (a router): every step of a row asked for at once, as the one-row pass does
                 done = rows <= 1024 && launch_wide<4, 16>(w.w, x, y, rows, cols, 0, b, (unsigned)fours, st);
@@ -289,8 +321,9 @@ static int32_t launch_lane16(const W& w, const XT* x, float* y, size_t rows, siz
                     done = launch_wide<4, 4>(w.w, x, y, rows, cols, b0, b, 1, st);
                     if (done) b0 += 4;
                 } else {
-                    done = left >= 2 ? launch_wide<3, 4>(w.w, x, y, rows, cols, b0, b, 1, st)
-                                     : launch_wide<1, 16>(w.w, x, y, rows, cols, b0, b, 1, st);
+                    done = wide_pays(rows, cols, left, F32) &&
+                           (left >= 2 ? launch_wide<3, 4>(w.w, x, y, rows, cols, b0, b, 1, st)
+                                      : launch_wide_rows(w.w, x, y, rows, cols, b0, b, 1, st));
                     if (done) b0 = b;
                 }
             }

@@ -51,6 +51,17 @@ def test_bf16_rows_that_end_inside_a_step(card, rows, cols, b):
     assert np.array_equal(f32_bits(picks), f32_bits(oracle.gemv_bf16(bits16(w), xb.float().numpy(), threads=0)))
 
 
+@pytest.mark.parametrize("rows,cols,b", [(1025, 200, 5), (9000, 136, 2), (9000, 136, 4), (5000, 248, 7), (136, 4992, 40), (512, 2056, 16),
+                                         (1024, 1024, 8), (1024, 1024, 9), (2000, 128, 6), (4100, 1032, 3), (170, 6424, 1), (600, 720, 1),
+                                         (8200, 520, 13)])
+def test_bf16_rows_at_the_lines_between_the_kernels(card, rows, cols, b):
+    """shapes either side of where a pass goes row by row, in fours, or to the kernel that looks at one column a load: the
+    host's bits from all of them"""
+    w, x = weights_bf16(rows, cols, seed=404, std=1.0), xs(b, cols, 405)
+    got = card.gemv_lane16(w.cuda(), x.cuda()).cpu().numpy()
+    assert np.array_equal(f32_bits(got), f32_bits(oracle.gemv_bf16(bits16(w), x.numpy(), threads=0)))
+
+
 @pytest.mark.parametrize("rows,cols", [(64, 512), (9, 1040), (3, 16)])
 def test_p12_rows_bits(card, rows, cols):
     w = weights_bf16(rows, cols, seed=410)
