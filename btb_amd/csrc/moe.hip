@@ -323,11 +323,18 @@ __global__ void __launch_bounds__(256) moe_gate_up_kernel(Stack stack, const uin
 // gathered rows of x a pass, where the kernel above streams them once a pair. The workgroups of the later pairs leave
 // before asking memory for anything. A product is a row of x against a row of weights in the lane order above, so
 // each h row has the bits the kernel above gives it. n = T k <= GROUP_MAX_PAIRS.
+// SPREAD (a launch cut for fewer workgroups, gate_up_grid): every share-th pair of an expert has work, the rows from it on, share (a
+// multiple of MC) what an expert has where rows pick for themselves. The cut counts on that; where they pick the same experts - a
+// tree's rows often do - few experts have all the work, and a workgroup that made all their passes left most of the chip idle.
+// us a layer without the router, every row the same picks, one workgroup for all passes / spread (uncut): MXFP4 128 of 8, 2048 /
+// 768, 16 rows 87.7 / 55.1 (61.5), 32 rows 169.6 / 102.5 (115); bf16 128 of 2, 1536 / 640, 20 rows 45.2 / 30.6 (39.9); rows that pick for
+// themselves level (120.7 / 121.1). Uncut launches lose by it: MXFP4 16 of 8, 960 / 416, 29 rows 48.1 / 53.4.
 constexpr int GROUP_MAX_PAIRS = 256;
-template <class F, bool OSS, int LPR, int RPW, int U, int MC>
+template <class F, bool OSS, int LPR, int RPW, int U, int MC, bool SPREAD>
 __global__ void __launch_bounds__(256) moe_gate_up_grouped_kernel(Stack stack, const uint16_t* __restrict__ x,
                                                                   const int32_t* __restrict__ idx, uint16_t* __restrict__ h,
-                                                                  int R, int C, int k, int E, int n, Glu glu) {
+                                                                  int R, int C, int k, int E, int n, Glu glu,
+                                                                  int share) {
     static_assert(RPW == 2, "gate and up");
     extern __shared__ __align__(16) uint32_t xs[];  // [MC][C / 2]
     constexpr int G = WAVE / LPR, ROWS = G;
@@ -347,18 +354,19 @@ __global__ void __launch_bounds__(256) moe_gate_up_grouped_kernel(Stack stack, c
 #pragma unroll
     for (int i = 0; i < NM; ++i)
         mask[i] = i * WAVE < n ? __ballot(i * WAVE + lane < n && clamp(picks[i]) == expert) : 0ull;
-    // an earlier pair of the same expert does the work
+    // how many earlier pairs picked the expert: its first pair does the work (SPREAD: see above)
+    int earlier = 0;
     {
-        unsigned long long earlier = 0ull;
 #pragma unroll
         for (int i = 0; i < NM; ++i) {
             unsigned long long m = mask[i];
             if (i == pair / WAVE) m &= (1ull << (pair % WAVE)) - 1ull;
             if (i > pair / WAVE) m = 0ull;
-            earlier |= m;
+            earlier += __builtin_popcountll(m);
         }
-        if (earlier != 0ull) return;  // uniform
+        if (SPREAD ? earlier % share != 0 : earlier != 0) return;  // uniform
     }
+    const int r_first = SPREAD ? earlier : 0;
     int rows_n = 0;
 #pragma unroll
     for (int i = 0; i < NM; ++i) rows_n += __builtin_popcountll(mask[i]);
@@ -402,7 +410,7 @@ __global__ void __launch_bounds__(256) moe_gate_up_grouped_kernel(Stack stack, c
                                    units);
             load_span_always<F, LPR, RPW, U>(first, c0, 0, sl, units);
         }
-        if (r0 != 0) __syncthreads();  // the previous pass has read its rows
+        if (r0 != r_first) __syncthreads();  // the previous pass has read its rows
         // the pass's rows of x, a row past the last being the last again (its sums are dropped)
         int prs[M];
 #pragma unroll
@@ -453,7 +461,8 @@ __global__ void __launch_bounds__(256) moe_gate_up_grouped_kernel(Stack stack, c
             }
         }
     };
-    for (int r0 = 0; r0 < rows_n; r0 += MC) {
+    const int r_end = SPREAD ? min(r_first + share, rows_n) : rows_n;
+    for (int r0 = r_first; r0 < r_end; r0 += MC) {
         const int mc = min(MC, rows_n - r0);
         if (mc == 1)
             pass(std::integral_constant<int, 1>{}, r0, mc);
@@ -616,8 +625,9 @@ static int lanes_for_mx4(int units) {
 //   bf16: 128 experts of which 8, 2048 / 768, 8 rows (40 working workgroups a CU at 1) 95.4 / 87.3 / 85.8 / 88.0, 16 rows (61) 166 /
 //   148 / 143 / 146; 32 of which 4, 2048 / 1536, 8 rows (31) 98.4 / 89.9 / 85.8 / 89.4: nine a CU. Below eight rows, where a
 //   workgroup is a pair's: level or slower.
-//   MXFP4: gpt-oss (32 of 4, 2880 / 2880) 4 rows (11) 57.8 / 56.3 / 55.8 / 65.2, 8 rows (15) 108 / 100 / 100 / 107, 16 rows (20) 189
-//   / 176 / 173 / 181; 128 of 8, 2048 / 768, 8 rows (10) 44.9 / 41.3 / 41.3 / 47.2, 1 row (1.5) 11.9 / 12.7 / 15.1: four.
+//   MXFP4: gpt-oss (32 of 4, 2880 / 2880) 8 rows (15 a CU) 108 / 100 / 100 / 107, 16 rows (20) 189 / 176 / 173 / 181; 128 of 8, 2048 /
+//   768, 8 rows (10) 44.9 / 41.3 / 41.3 / 47.2: four. Below eight rows level (gpt-oss 4 rows 53.3 / 52.9, at 3 55.3) or slower (32 of 8,
+//   1632 / 448, 7 rows 22.5 / 24.6).
 static int gate_up_grid(int whole, double wgs, double per_cu) {
     const int div = std::min((int)(wgs / (per_cu * device_info().cus) + 0.5), 4);
     return div <= 1 ? whole : (whole + div - 1) / div;
@@ -627,13 +637,20 @@ static int gate_up_grid(int whole, double wgs, double per_cu) {
 // once they run side by side, so the second reads that die's L2. bf16, us a layer without the router, workgroups a CU as many
 // as tiles / here: 128 of 8, 8 rows 85.8 / 82.9, 16 rows 143 / 136, 32 rows 233 / 212; 32 of 4, 2048 / 1536, 4 / 8 / 16 rows 54.9 / 50.6,
 // 89.6 / 73.8, 142 / 102; 16 of 2, 1024 / 512, whose waves have 2 KB on their way each, 32 rows at two / four a CU 40.9 / 35.3 (56.7).
-// (A third of the workgroups instead of a quarter, no multiple of eight: 86.2 and 147 for the first two.) MXFP4's are bound by
-// the widening and keep a wave a tile.
-static int down_grid(int whole, int T, bool widens, size_t wave_bytes) {
+// (A third of the workgroups instead of a quarter, no multiple of eight: 86.2 and 147 for the first two.) Rows of more than four units
+// a lane take two trips to memory a pick: waves of one or two tiles more than others cost that much more, and small launches
+// lose by the cut (64 of 4, 1056 / 1216, 132 workgroups a row, 8 rows 47.7 -> 51.2, 23 rows 94.7 -> 106; 32 of 4, 768 / 1728, 96, 6 rows 31.0 ->
+// 34.3; but 64 of 2, 3712 / 1056, 464, 13 rows 111 -> 102, 128 of 6, 960 / 2816, 240, 31 rows 347 -> 332). MXFP4's are bound by the widening and keep a wave a tile. The
+// multiple of eight is left where it would begin another turn of the CUs: MXFP4 32 of 4, 1632 / 832, 5 rows, 510 workgroups or 520,
+// 17.6 / 19.9; 16 of 8, 2720 / 928, 3 rows 27.4 / 30.5.
+static int down_grid(int whole, int T, bool widens, size_t wave_bytes, int units_a_lane) {
     if (T == 1) return whole;
-    const int eights = (whole + 7) / 8 * 8;
-    const int most = std::max(8, (wave_bytes >= 8192 ? 2 : 4) * device_info().cus / T / 8 * 8);
-    return widens || T < 4 ? eights : std::min(eights, most);
+    const int cus = device_info().cus, eights = (whole + 7) / 8 * 8;
+    auto turns = [&](int n) { return ((long)n * T + cus - 1) / cus; };
+    const int full = turns(eights) > turns(whole) ? whole : eights;
+    if (widens || T < 4 || (units_a_lane > 4 && whole <= 192)) return full;
+    const int most = std::max(8, (wave_bytes > 8192 ? 2 : 4) * cus / T / 8 * 8);
+    return std::min(full, most);
 }
 // the experts that T rows of k picks out of E name, were they drawn evenly
 static double distinct_experts(int E, int k, int T) { return E * (1.0 - std::pow(1.0 - (double)k / E, T)); }
@@ -656,19 +673,21 @@ static int32_t launch_gate_up(Stack stack, const void* x, const int32_t* idx, vo
     const int grouped = tuning("moe_grouped");
     const bool wanted = grouped >= 0 ? grouped != 0 && pairs > k : pairs >= 8 * k;
     if (wanted && pairs <= GROUP_MAX_PAIRS && (size_t)MC * C * 2 <= (size_t)device_info().lds_bytes - 16 * 1024) {
-        auto kern = moe_gate_up_grouped_kernel<F, OSS, LPR, RPW, U, MC>;
+        const double distinct = distinct_experts(E, k, pairs / k);
+        const int grid = gate_up_grid(whole, whole * distinct, MX ? 4 : 9);
+        const int share = (int)std::ceil(pairs / (distinct * MC)) * MC;  // at most pairs' next multiple of MC
+        auto kern = grid < whole ? moe_gate_up_grouped_kernel<F, OSS, LPR, RPW, U, MC, true>
+                                 : moe_gate_up_grouped_kernel<F, OSS, LPR, RPW, U, MC, false>;
         const size_t lds = (size_t)MC * C * 2;
         if (lds > 48 * 1024) {
             hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
             if (e != hipSuccess) return hip_status(e, "hipFuncSetAttribute");
         }
-        const int grid = gate_up_grid(whole, whole * distinct_experts(E, k, pairs / k), MX ? 4 : 9);
         hipLaunchKernelGGL(kern, dim3(grid, pairs), dim3(256), lds, st, stack, static_cast<const uint16_t*>(x), idx,
-                           static_cast<uint16_t*>(gu), R, C, k, E, pairs, glu);
+                           static_cast<uint16_t*>(gu), R, C, k, E, pairs, glu, share);
         return hip_status(hipGetLastError(), "moe gate_up launch");
     }
-    const int grid = MX ? gate_up_grid(whole, (double)whole * pairs, 4) : whole;
     auto kern = moe_gate_up_kernel<F, OSS, LPR, RPW, U>;
     // MXFP4 rows of five to seven units a lane in one trip to memory instead of two, where the waves are few. us a layer without
     // the router, two trips / one: gpt-oss (six units) one row (11 waves a CU) 22.6 / 21.4, two rows 32.9 / 31.8, four (45) 57.5 /
@@ -681,7 +700,7 @@ static int32_t launch_gate_up(Stack stack, const void* x, const int32_t* idx, vo
                    : upl == 6 ? moe_gate_up_kernel<F, OSS, LPR, RPW, 6>
                               : moe_gate_up_kernel<F, OSS, LPR, RPW, 7>;
     }
-    hipLaunchKernelGGL(kern, dim3(grid, pairs), dim3(256), (size_t)C * 2, st, stack,
+    hipLaunchKernelGGL(kern, dim3(whole, pairs), dim3(256), (size_t)C * 2, st, stack,
                        static_cast<const uint16_t*>(x), idx, static_cast<uint16_t*>(gu), R, C, k, E, glu);
     return hip_status(hipGetLastError(), "moe gate_up launch");
 }
@@ -692,11 +711,11 @@ static int32_t launch_down(Stack stack, const void* gu, const int32_t* idx, cons
     constexpr int RPW = 1, G = WAVE / LPR;
     const int ntiles = (R + G * RPW - 1) / (G * RPW);
     const int whole = (ntiles + 3) / 4;
-    const int grid = down_grid(whole, T, std::is_same<F, FmtMx4>::value, (size_t)k * C * 2);
     const size_t lds = (size_t)k * C * 2;
     // a row of at most three units a lane (the 768-wide experts of the C4 shape: 96 bf16 units over 64 lanes, 24 MXFP4
     // units over 16): all eight picks' rows in one request
     const int upl = (C / F::UW + LPR - 1) / LPR;
+    const int grid = down_grid(whole, T, std::is_same<F, FmtMx4>::value, (size_t)k * C * 2, upl);
     auto kern = upl <= 2   ? moe_down_kernel<F, LPR, RPW, 2, 8>
                 : upl <= 3 ? moe_down_kernel<F, LPR, RPW, 3, 8>
                            : moe_down_kernel<F, LPR, RPW, 4, 4>;

@@ -376,3 +376,28 @@ def test_mxfp4_rows_whole_in_one_trip_change_no_bit(card, oss, H_, I_, T, k):
     if oss:
         bare = MxExpertsLayer(card, to_gpu(ex), oss=True)(x, picks, w)
         assert not torch.equal(bare.view(torch.int16), got[0].view(torch.int16))
+
+
+@pytest.mark.parametrize("form", ["bf16", "mxfp4"])
+@pytest.mark.parametrize("T", [8, 9, 21, 32])
+def test_rows_that_pick_the_same_experts_change_no_bit(card, form, T):
+    """A launch cut for rows that pick for themselves, given rows that do not: all the same picks, every other row's, one expert
+    that all have; each row with the bits it has alone."""
+    from btb_amd.moe import MxExpertsLayer
+
+    E_, H_, I_, k, g = 32, 256, 1536, 4, gen(595)
+    if form == "mxfp4":
+        layer = MxExpertsLayer(card, to_gpu(mx_stacks(596, E_, I_, H_)), oss=False)
+    else:
+        layer = Experts(card, (torch.randn(E_, 2 * I_, H_, generator=g) * 0.02).to(torch.bfloat16).cuda(),
+                        (torch.randn(E_, H_, I_, generator=g) * 0.02).to(torch.bfloat16).cuda())
+    x = acts_bf16(T, H_, seed=597).cuda()
+    w = torch.rand(T, k, generator=g).to(torch.bfloat16).cuda()
+    own, base = torch.stack([torch.randperm(E_, generator=g)[:k] for _ in range(T)]), torch.randperm(E_, generator=g)[:k]
+    one_shared = torch.stack([torch.cat([base[:1], torch.tensor([e for e in r.tolist() if e != base[0]])[: k - 1]]) for r in own])
+    for picks in (base.repeat(T, 1), torch.where(torch.arange(T)[:, None] % 2 == 0, base, own), one_shared):
+        picks = picks.to(torch.int32).cuda()
+        y = layer(x, picks, w)
+        for t in range(T):
+            one = layer(x[t : t + 1].contiguous(), picks[t : t + 1].contiguous(), w[t : t + 1].contiguous())
+            assert torch.equal(y[t : t + 1].view(torch.int16), one.view(torch.int16)), t
