@@ -170,10 +170,12 @@ __global__ void __launch_bounds__(KS * 64) mfma_ahead_kernel(const uint8_t* __re
     auto request = [&](int k, uint4 (&r)[NLD]) {
         const bool live = k < turns;
         const uint8_t* base = w + (size_t)row_of(live ? first + k * grid : first) * rowbytes + (size_t)sn * 64;
+        // (a row is no bytes past the last tile, not a choice a load: of those the compiler made a branch each in the fold)
+        const uint32_t pitch = live ? rowbytes : 0;
 #pragma unroll
         for (int q = 0; q < NLD; ++q) {
             const uint32_t rows = WHOLE ? (uint32_t)(q * RPL) + (GLU && q * RPL >= 8 ? (uint32_t)R / 2 - 8 : 0u) : 0u;
-            const uint8_t* at = base + (live ? (size_t)rows * rowbytes : 0);
+            const uint8_t* at = base + (size_t)rows * pitch;
             r[q] = load_stream16(reinterpret_cast<const uint4*>(at + (live ? goff[WHOLE ? 0 : q] : 0u)));
         }
     };
