@@ -290,10 +290,14 @@ static int32_t launch_ahead(const void* w, const void* x, void* y, int R, int C,
 
 template <int KS, int MT, int SPW>
 static int32_t run_ahead(const void* w, const void* x, void* y, int R, int C, int M, bool glu, hipStream_t st) {
-    // eight waves a CU are what two tiles in flight leave registers for; a launch of one turn at twelve takes those (us at 8 rows,
-    // eight / twelve waves: [9728 x 1024] 7.4 / 6.3, [40000 x 1024] 15.9 / 17.5)
+    // Eight waves a CU are what two tiles in flight leave registers for; a launch of one turn at twelve takes those (us at 8 rows,
+    // eight / twelve waves: [9728 x 1024] 7.4 / 6.3, [40000 x 1024] 15.9 / 17.5). Not workgroups of two waves that hold more than
+    // one short slice of x: the registers or the LDS of six of them a CU are not there, and the last ones begin when others end
+    // (1000 shapes of 256 to 640 columns whose tiles are four to six a CU, twelve / eight, medians: slices of eight steps and one tile
+    // of x rows 1 / 1.07, two 1 / 0.88; of ten steps 1 / 0.99 and 1 / 0.89). Four waves of any slice: 1 / 1.03 to 1 / 1.18.
+    constexpr bool TWELVE = KS == 4 || (KS == 2 && MT == 1 && SPW == 8);
     int per_cu = tuning("mfma_wgs_per_cu");
-    if (per_cu <= 0) per_cu = R <= 16 * (12 / KS) * device_info().cus ? 12 / KS : 8 / KS;
+    if (per_cu <= 0) per_cu = TWELVE && R <= 16 * (12 / KS) * device_info().cus ? 12 / KS : 8 / KS;
     const int cap = device_info().cus * per_cu;
     if (glu) {
         if (R % 16 != 0) return launch_ahead<KS, MT, SPW, 16, true, true>(w, x, y, R, C, M, cap, st);
