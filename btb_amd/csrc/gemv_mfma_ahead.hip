@@ -324,12 +324,28 @@ static int32_t run_ahead(const void* w, const void* x, void* y, int R, int C, in
 // 6.4 / 5.1; [40000 x 1024] 18.9 / 15.9, 20.0 / 16.5, 22.6 / 17.0, 25.3 / 19.4; [512 x 512] 3.3 / 2.7, 3.4 / 2.8, 3.8 / 3.0,
 // 3.9 / 3.2. Past 2560 columns that kernel has two full sub-blocks a tile and the x fragments of a second tile of x rows do not
 // fit beside two tiles of weights: up to 16 rows of x, and where the CUs go round once ([2560 x 4096] at 8 rows 7.9 / 7.2,
-// [2048 x 3072] 6.7 / 6.0; but [24576 x 4096] 35.8 / 36.5, [8192 x 3072] 12.1 / 12.4).
+// [2048 x 3072] 6.7 / 6.0; but [24576 x 4096] 35.8 / 36.5, [8192 x 3072] 12.1 / 12.4), with slices of twelve steps or all of sixteen
+// ([4096 x 3584], fourteen, at 5 / 8 / 16 rows 8.45 / 8.56, 8.73 / 8.85, 9.55 / 9.79).
 bool mfma_ahead_fits(int R, int C, int M, bool glu) {
-    const int nsteps = C / 32;
+    const int nsteps = C / 32, cus = device_info().cus;
     if (tuning("mfma_ahead") == 0 || R < 16 || C % 32 != 0 || nsteps > 128 || (glu && R % 16 != 0)) return false;
     if (glu && (uint64_t)R * C >= 1ull << 31) return false;  // a gate row's up row within 32 bits
-    return nsteps <= 80 ? M <= 32 : M <= 16 && R <= 16 * device_info().cus;
+    if (tuning("mfma_ahead") > 0) return nsteps <= 80 ? M <= 32 : M <= 16;
+    if (nsteps > 80) return M <= 16 && R <= 16 * cus && (nsteps <= 96 || nsteps > 120);
+    // Slices of the kernel's eight steps or fewer. What it gains by two tiles in flight it gains in long launches and, with two or
+    // four waves a workgroup, in those of at most half a turn of eight waves a CU. In between nothing of the second tile is
+    // ahead, and a slice of four to seven steps still loads and stores all eight. 6600 shapes, medians of the time against
+    // gemv_mfma_lds's by turns (to half a turn, to two, more), one tile of x rows / two: short slices of two waves 0.92 / 0.89, 1.03 /
+    // 1.03, 1.00 / 0.86, of four 0.98 / 0.98, 1.04 / 1.05, 0.95 / 0.85, of eight 1.03 / 1.06, 1.04 / 1.06, 0.88 / 0.91; whole ones 0.97 /
+    // 0.95, 0.99 / 0.97, 0.92 / 0.86 (nine and ten steps 0.90 / 0.95, 0.94 / 0.95, 0.89 / 0.82). With the fold 0.03 to 0.06 more: two waves' short slices
+    // then pay to a quarter of a turn, and slices of nine steps not between one turn and two ([18816 x 544] 5 rows 7.4 / 8.2).
+    const int ks = nsteps <= 20 ? 2 : nsteps <= 40 ? 4 : 8, steps = (nsteps + ks - 1) / ks;
+    const int64_t waves = (int64_t)((R + 15) / 16) * ks;
+    if (M > 32) return false;
+    if (steps > 8) return !(glu && steps == 9 && M <= 16 && waves > 8 * cus && waves <= 16 * cus);
+    if (waves > 16 * cus) return M > 16 || ks != 2 || steps == 8;
+    if (steps == 8) return !glu || ks == 2;
+    return glu ? ks == 2 && waves <= 2 * cus : ks < 8 && waves <= 4 * cus;
 }
 // Rows of a multiple of 8 columns but not of 32, which the other matrix-core kernels do not take and which went through passes
 // of four rows on the vector units: from five rows of x on, in passes of 32 rows, or of 16 past 2560 columns. us at 5 / 8 / 16 / 32

@@ -340,20 +340,24 @@ def test_columns_split_over_workgroups_change_no_bit(card, R, C, M):
                                  (4096, 3584), (1536, 4096), (32, 4000)])
 @pytest.mark.parametrize("M", [5, 8, 16, 17, 32, 40])
 def test_two_tiles_of_weights_in_flight_change_no_bit(card, R, C, M):
-    """The kernel with two tiles of weights in flight (knob mfma_ahead = 0: without) against the staged one, bit for bit, plain
-    and with the gate / up fold: one to many turns a workgroup, odd and even, tiles of 10, 12 and 16 rows and overlapping ones,
-    slices shorter than the kernel's and waves without a step, non-finite weights in rows of their own."""
+    """The kernel with two tiles of weights in flight (knob mfma_ahead = 1: wherever the shape fits, 0: nowhere, -1: by the rule)
+    against the staged one, bit for bit, plain and with the gate / up fold: one to many turns a workgroup, odd and even, tiles of
+    10, 12 and 16 rows and overlapping ones, slices shorter than the kernel's and waves without a step, non-finite weights in rows
+    of their own. From five rows on whatever the shape, so that the small ragged matrices reach both kernels."""
     w, x = weights_bf16(R, C, seed=190), acts_bf16(M, C, seed=191).cuda()
     w[R // 2, C - 1], w[R - 1, 0] = float("nan"), float("inf")
     w, got = w.cuda(), []
     try:
-        for knob in (0, -1):
+        card.set_tuning("gemv_mfma_from", 5)
+        for knob in (0, 1, -1):
             card.set_tuning("mfma_ahead", knob)
             got.append([card.gemv(w, x)] + ([card.gemv_glu_silu(w, x)] if R % 32 == 0 else []))
     finally:
         card.set_tuning("mfma_ahead", -1)
-    for want, y in zip(*got):
-        assert torch.equal(y.view(torch.int16), want.view(torch.int16))
+        card.set_tuning("gemv_mfma_from", -1)
+    for want, *others in zip(*got):
+        for y in others:
+            assert torch.equal(y.view(torch.int16), want.view(torch.int16))
 
 
 @pytest.mark.parametrize("R,C", [(16, 72), (17, 520), (512, 536), (100, 648), (4097, 1016), (1001, 1288), (2560, 2056), (5003, 2552),
