@@ -151,6 +151,24 @@ def _p(t: torch.Tensor) -> int:
 _Tensor = torch.Tensor
 
 
+# A second launch and the workspace's allocation are 3.8 us of the host's, which a recorded call does not pay: there the faster kernels
+# are taken wherever the library offers a workspace, in an eager call only where they save more than that. us a call, one launch / with
+# the workspace, calls one after the other: gemv [512 x 3584] 8 rows 7.8 / 11.4, 32 rows 11.5 / 11.5, [1024 x 3072] 16 rows 8.0 / 11.5,
+# [1536 x 5120] 12 / 16 / 17 rows 9.8 / 11.5, 10.9 / 11.5, 13.3 / 11.5, [1024 x 7168] 8 / 12 rows 11.7 / 11.6, 13.2 / 11.6, [4096 x 5120]
+# 16 rows 13.1 / 12.8, [2560 x 9728] 32 rows 29.0 / 16.1; argmax of 65536 logits 5.8 / 9.7, 151936 9.3 / 9.7, 200064 11.0 / 9.7.
+def _recording() -> bool:
+    """whether the current stream's calls are being captured"""
+    return torch._C._cuda_isCurrentStreamCapturing()
+
+
+def _split_pays(R: int, C: int, M: int) -> bool:
+    """whether an eager matvec gains by the columns split over workgroups where the library would split them"""
+    return M * C >= (122880 if C <= 4096 else 86016) or (M > 16 and C > 4096) or R * C >= 1 << 24
+
+
+_ARGMAX_EAGER = 163840  # logits a row from which an eager argmax gains by the many workgroups
+
+
 def _rows(x: torch.Tensor, C: int) -> int:
     """how many rows of C values the contiguous x holds"""
     if x.dim() == 2 and x.shape[1] == C:
@@ -288,7 +306,8 @@ class HipCard(CardLaunch):
     # -- bf16 matvec ------------------------------------------------------------------------------------------
 
     def gemv(self, w: torch.Tensor, x: torch.Tensor, y: torch.Tensor | None = None) -> torch.Tensor:
-        """y [M, R] = x [M, C] @ w [R, C]^T, bf16 in and out, f32 accumulate (`btb_gemv_bf16_m{M}`)"""
+        """y [M, R] = x [M, C] @ w [R, C]^T, bf16 in and out, f32 accumulate (`btb_gemv_bf16_m{M}`). Some passes of eight rows and
+        more allocate a workspace besides y: 512 bytes a row of w to sixteen rows, 1024 beyond."""
         self._need(w, torch.bfloat16, "w")
         self._need(x, torch.bfloat16, "x")
         R, C = w.shape
@@ -300,7 +319,7 @@ class HipCard(CardLaunch):
             if y.numel() != M * R:
                 raise ValueError(f"[hip] gemv: y holds {y.numel()} elements, the product has {M * R}")
         # a wide pass over some shapes splits its columns over workgroups and takes a workspace (this call's own)
-        floats = self.lib.btb_hip_gemv_bf16_floats(R, C, M) if M >= 8 else 0
+        floats = self.lib.btb_hip_gemv_bf16_floats(R, C, M) if M >= 8 and (_split_pays(R, C, M) or _recording()) else 0
         if floats:
             ws = torch.empty(floats, dtype=torch.float32, device=w.device)
             self._call("btb_hip_gemv_bf16_ws", _p(w), _p(x), _p(y), R, C, M, _p(ws), _stream())
@@ -1025,13 +1044,18 @@ class HipCard(CardLaunch):
         self._call("btb_hip_silu_mul", _p(gu), _p(m), int(gu.numel()) // (2 * I), I, _stream())
         return m
 
+    def _argmax_ws(self, logits: torch.Tensor, T: int, V: int) -> torch.Tensor | None:
+        """the workspace with which long rows go over many workgroups (the call's own), or None"""
+        floats = self.lib.btb_hip_argmax_floats(T, V) if V >= _ARGMAX_EAGER or _recording() else 0
+        return torch.empty(floats, dtype=torch.float32, device=logits.device) if floats else None
+
     def argmax(self, logits: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
+        """out [T] = the first largest of each row of logits [T, V]. Long rows allocate a workspace: 8 bytes for 4096 logits."""
         self._need(logits, torch.bfloat16, "logits")
         self._need(out, torch.int32, "out")
         V = int(logits.shape[-1])
         T = int(logits.numel()) // V
-        floats = self.lib.btb_hip_argmax_floats(T, V)  # long rows go over many workgroups and take a workspace (this call's own)
-        ws = torch.empty(floats, dtype=torch.float32, device=logits.device) if floats else None
+        ws = self._argmax_ws(logits, T, V)
         self._call("btb_hip_argmax_ws", _p(logits), _p(out), T, V, None if ws is None else _p(ws), _stream())
         return out
 
@@ -1052,7 +1076,7 @@ class HipCard(CardLaunch):
     def argmax_publish(self, logits: torch.Tensor, picked: torch.Tensor, n0: torch.Tensor,
                        next_ids: torch.Tensor | None = None, out_tok: torch.Tensor | None = None,
                        out_n0: torch.Tensor | None = None, out_ts: torch.Tensor | None = None) -> None:
-        """`argmax` over one row and `publish`, in its last launch"""
+        """`argmax` over one row (with its workspace) and `publish`, in its last launch"""
         self._need(logits, torch.bfloat16, "logits")
         self._need(picked, torch.int32, "picked")
         self._need(n0, torch.int32, "n0")
@@ -1060,8 +1084,7 @@ class HipCard(CardLaunch):
         if logits.numel() != V:
             raise ValueError("[hip] argmax_publish: one row of logits")
         p = lambda t: None if t is None else _p(t)
-        floats = self.lib.btb_hip_argmax_floats(1, V)
-        ws = torch.empty(floats, dtype=torch.float32, device=logits.device) if floats else None
+        ws = self._argmax_ws(logits, 1, V)
         self._call("btb_hip_argmax_publish_ws", _p(logits), V, _p(picked), _p(n0), p(next_ids),
                    p(out_tok), p(out_n0), p(out_ts), p(ws), _stream())
 

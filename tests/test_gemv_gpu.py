@@ -310,15 +310,18 @@ def test_columns_split_over_workgroups_change_no_bit(card, R, C, M):
     rest. `gemv` picks by shape; a workspace of NULL is the plain call."""
     w, x = weights_bf16(R, C, seed=180).cuda(), acts_bf16(M, C, seed=181).cuda()
     L, y = card.lib, torch.empty(M, R, dtype=torch.bfloat16, device="cuda")
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
     try:
+        card.set_tuning("gemv_mfma_from", 5)  # the staged kernel's shapes whatever their size, small ragged ones too
         card.set_tuning("mfma_split", 0)
         want = card.gemv(w, x)
         assert L.btb_hip_gemv_bf16_floats(R, C, M) == 0
         card.set_tuning("mfma_split", 1)
         floats = L.btb_hip_gemv_bf16_floats(R, C, M)
-        if floats:  # the staged kernel's shapes only (M = 5 with few columns, ragged rows past 4096 columns: others')
+        # (more than sixteen rows of x over long rows of a ragged matrix are the column-interleaved kernel's)
+        assert (floats > 0) == (M <= 16 or R % 16 == 0 or C <= 4096)
+        if floats:
             ws = torch.full((floats + 64,), float("nan"), device="cuda")
-            p = lambda t: ctypes.c_void_p(t.data_ptr())
             assert L.btb_hip_gemv_bf16_ws(p(w), p(x), p(y), R, C, M, p(ws), None) == 0
             torch.cuda.synchronize()
             assert torch.equal(y.view(torch.int16), want.view(torch.int16))
@@ -327,12 +330,32 @@ def test_columns_split_over_workgroups_change_no_bit(card, R, C, M):
             assert L.btb_hip_gemv_bf16_ws(p(w), p(x), p(y.zero_()), R, C, M, None, None) == 0
             torch.cuda.synchronize()
             assert torch.equal(y.view(torch.int16), want.view(torch.int16))
-        else:
-            assert M < 8 or R % 16 != 0 or C > 10240
+        card.set_tuning("mfma_split", -1)
+        assert torch.equal(card.gemv(w, x).view(torch.int16), want.view(torch.int16))
     finally:
         card.set_tuning("mfma_split", -1)
-    assert torch.equal(card.gemv(w, x).view(torch.int16), want.view(torch.int16))
+        card.set_tuning("gemv_mfma_from", -1)
 
+
+@pytest.mark.parametrize("R,C,M,eager", [(1024, 3072, 16, False), (512, 3584, 32, False), (1536, 5120, 16, False), (1024, 7168, 12, True),
+                                         (1536, 5120, 17, True), (2560, 9728, 32, True), (4096, 5120, 16, True)])
+def test_an_eager_call_takes_a_second_launch_only_where_it_gains(card, monkeypatch, R, C, M, eager):
+    """The columns split over workgroups take two launches and an allocation: a recorded call takes them wherever the library offers,
+    an eager one where the kernels save more than the host pays; the bits are the same."""
+    w, x, called = weights_bf16(R, C, seed=182).cuda(), acts_bf16(M, C, seed=183).cuda(), []
+    assert card.lib.btb_hip_gemv_bf16_floats(R, C, M) > 0
+    inner = type(card)._call
+    monkeypatch.setattr(type(card), "_call", lambda self, name, *args: (called.append(name), inner(self, name, *args))[1])
+    want, y = card.gemv(w, x), torch.empty(M, R, dtype=torch.bfloat16, device="cuda")
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        card.gemv(w, x, y)
+    assert called == ["btb_hip_gemv_bf16_ws" if eager else "btb_hip_gemv_bf16", "btb_hip_gemv_bf16_ws"]
+    for _ in range(3):
+        y.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y.view(torch.int16), want.view(torch.int16))
 
 
 @pytest.mark.parametrize("R,C", [(16, 32), (17, 544), (4128, 512), (16416, 640), (48, 672), (12336, 1024), (1001, 1280),

@@ -650,9 +650,10 @@ def test_attn_span_count_limit(card):
 
 @pytest.mark.parametrize("V", [65536, 65544, 69632, 151936, 300008])
 @pytest.mark.parametrize("T", [1, 3, 32])
-def test_argmax_of_long_rows_over_many_workgroups(card, T, V):
+def test_argmax_of_long_rows_over_many_workgroups(card, monkeypatch, T, V):
     """Rows whose pick comes from many workgroups: ties within and across them (the lowest index wins), NaN, rows with nothing
     above -inf (index 0), the last logit - and the publishing form - against one workgroup a row."""
+    monkeypatch.setattr("btb_amd.native._ARGMAX_EAGER", 65536)  # eager calls over many workgroups from the first length on
     x = acts_bf16(T, V, seed=640)
     x[0, V - 1] = x[0, 4096 * 3 + 5] = x[0, V - 9] = 40.0
     if T > 1:
@@ -677,3 +678,22 @@ def test_argmax_of_long_rows_over_many_workgroups(card, T, V):
     odd = x.view(-1)[1 : V - 7].contiguous()  # no multiple of eight from an aligned place: one workgroup
     card.argmax(odd, one)
     assert one.item() == (4096 * 3 + 4 if x.view(-1)[4096 * 3 + 5] == 40.0 else -1)
+
+
+@pytest.mark.parametrize("V,eager", [(65536, False), (151936, False), (163840, True), (262144, True)])
+def test_an_eager_argmax_takes_many_workgroups_only_where_it_gains(card, monkeypatch, V, eager):
+    """the second launch and the workspace: always in a recorded call, in an eager one from the length on that pays for them"""
+    x, out = acts_bf16(1, V, seed=641).cuda(), torch.zeros(1, dtype=torch.int32, device="cuda")
+    given, inner = [], type(card)._call
+    monkeypatch.setattr(type(card), "_call", lambda self, name, *args: (given.append(args[-2] is not None), inner(self, name, *args))[1])
+    card.argmax(x, out)
+    want = out.clone()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        card.argmax(x, out)
+    assert given == [eager, True]
+    for _ in range(3):
+        out.fill_(-1)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
