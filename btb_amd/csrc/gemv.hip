@@ -526,7 +526,7 @@ bool mfma_ahead_ragged_fits(int R, int C);
 int32_t gemv_mfma_ahead_bf16(const void* w, const void* x, void* y, int R, int C, int M, bool glu, hipStream_t st);
 int32_t gemv_mfma_ahead_norm_bf16(const void* w, const XArgs& xa, void* y, int R, int C, int M, bool glu, hipStream_t st);
 
-// the matrix-core matvec of more than sixteen rows with the columns split over workgroups (gemv_mfma_split.hip)
+// the matrix-core matvec with the columns split over workgroups, for many rows of x or few of the matrix (gemv_mfma_split.hip)
 size_t mfma_split_floats(size_t R, size_t M);
 bool mfma_split_fits(size_t R, size_t C);
 int32_t gemv_mfma_split_bf16(const void* w, const void* x, void* y, int R, int C, int M, float* ws, hipStream_t st);
@@ -647,6 +647,10 @@ static bool split_pays(size_t M, size_t R, size_t C) {
     if (M < 8 || C < 2560) return false;
     if (R <= 1024) return C > 3072 || M * C >= 20000 + 16 * R;
     if (R <= 2048) return C > 3072 && M * C >= 30 * R;
+    // (the other kernel's tiles are one a CU and nearly all CUs have one: [4096 x 8192] at 14 / 16 rows 16.1 / 18.1, 16.7 / 18.4,
+    // [4096 x 9728] 19.3 / 20.4, 20.2 / 20.4, [4048 x 6176] at 15 15.6 / 16.5)
+    const size_t cus = (size_t)device_info().cus;
+    if (R > 14 * cus && R <= 16 * cus) return false;
     return C > 7168 ? M >= 14 : C > 4096 && M >= 15 && R <= 12288;
 }
 

@@ -1,4 +1,4 @@
-// More than sixteen rows of x against a bf16 matrix, the columns split over workgroups.
+// Eight to thirty-two rows of x against a bf16 matrix, the columns split over workgroups.
 //
 // gemv_mfma_lds gives a workgroup whole rows of the matrix, so every workgroup reads all of x: 32 rows of 9728 values are
 // 622 KB a CU where the CU's share of a [2560 x 9728] matrix is 195 KB, and a CU takes in 25 to 30 bytes a nanosecond

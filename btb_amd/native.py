@@ -154,8 +154,8 @@ _Tensor = torch.Tensor
 # A second launch and the workspace's allocation are 3.8 us of the host's, which a recorded call does not pay: there the faster kernels
 # are taken wherever the library offers a workspace, in an eager call only where they save more than that. us a call, one launch / with
 # the workspace, calls one after the other: gemv [512 x 3584] 8 rows 7.8 / 11.4, 32 rows 11.5 / 11.5, [1024 x 3072] 16 rows 8.0 / 11.5,
-# [1536 x 5120] 12 / 16 / 17 rows 9.8 / 11.5, 10.9 / 11.5, 13.3 / 11.5, [1024 x 7168] 8 / 12 rows 11.7 / 11.6, 13.2 / 11.6, [4096 x 5120]
-# 16 rows 13.1 / 12.8, [2560 x 9728] 32 rows 29.0 / 16.1; argmax of 65536 logits 5.8 / 9.7, 151936 9.3 / 9.7, 200064 11.0 / 9.7.
+# [1536 x 5120] 12 / 16 / 17 rows 9.8 / 11.5, 10.9 / 11.5, 13.3 / 11.5, [1024 x 7168] 8 / 12 rows 11.7 / 11.6, 13.2 / 11.6, [8192 x 5120]
+# 16 rows 19.8 / 19.1, [2560 x 9728] 32 rows 29.0 / 16.1; argmax of 65536 logits 5.8 / 9.7, 151936 9.3 / 9.7, 200064 11.0 / 9.7.
 def _recording() -> bool:
     """whether the current stream's calls are being captured"""
     return torch._C._cuda_isCurrentStreamCapturing()

@@ -71,10 +71,11 @@ int32_t btb_hip_stream_probe(const void* a, size_t rows, uint32_t* sink, void* s
  * argument, any value from 1 to 1024. */
 int32_t btb_hip_gemv_bf16(const void* w, const void* x, void* y, size_t R, size_t C, size_t M, void* stream);
 
-/* The same for wide passes with a workspace: more than sixteen rows of x over some shapes are fastest with the columns split
- * over workgroups, whose f32 sums meet in `ws` (btb_hip_gemv_bf16_floats of them, 16-byte aligned; nothing in it need be
- * cleared, nothing is kept; calls that overlap take one each). The bits are btb_hip_gemv_bf16's. 0 floats, or ws NULL: that
- * function is called. */
+/* The same for wide passes with a workspace: from eight rows of x on some shapes are fastest with the columns split over
+ * workgroups, whose f32 sums meet in `ws`. btb_hip_gemv_bf16_floats says how many it takes, 0 where the split does not pay
+ * (16-byte aligned; nothing in it need be cleared, nothing is kept; calls that overlap take one each). It is two launches: an
+ * eager caller gains less by it than a recorded one. The bits are btb_hip_gemv_bf16's. 0 floats, or ws NULL: that function is
+ * called. */
 size_t btb_hip_gemv_bf16_floats(size_t R, size_t C, size_t M);
 int32_t btb_hip_gemv_bf16_ws(const void* w, const void* x, void* y, size_t R, size_t C, size_t M, float* ws, void* stream);
 

@@ -338,7 +338,7 @@ def test_columns_split_over_workgroups_change_no_bit(card, R, C, M):
 
 
 @pytest.mark.parametrize("R,C,M,eager", [(1024, 3072, 16, False), (512, 3584, 32, False), (1536, 5120, 16, False), (1024, 7168, 12, True),
-                                         (1536, 5120, 17, True), (2560, 9728, 32, True), (4096, 5120, 16, True)])
+                                         (1536, 5120, 17, True), (2560, 9728, 32, True), (6144, 5120, 16, True)])
 def test_an_eager_call_takes_a_second_launch_only_where_it_gains(card, monkeypatch, R, C, M, eager):
     """The columns split over workgroups take two launches and an allocation: a recorded call takes them wherever the library offers,
     an eager one where the kernels save more than the host pays; the bits are the same."""
