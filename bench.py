@@ -574,6 +574,21 @@ def other_configs(args: argparse.Namespace) -> list[dict]:
     return out
 
 
+def second_launches(step, card) -> int:
+    """the launches of a recorded pass beyond one an operator: the greedy pick over long rows, and the fold of every bf16 matvec
+    whose columns are split over workgroups"""
+    import torch
+
+    alone = {"o", "down"} if step.fused else {"qkv", "o", "gu", "down", "head"}  # launched as plain matvecs
+    if not step.fused:
+        alone -= {"gu"} if step.glu_fold else {"down"} if step.fold_silu else set()
+    more = int(card.lib.btb_hip_argmax_floats(step.T, step.cfg.vocab) > 0)
+    for name, lin in step.w.items():
+        if name.split(".")[-1] in alone and isinstance(lin.w, torch.Tensor):
+            more += int(card.lib.btb_hip_gemv_bf16_floats(*lin.shape, step.T) > 0)
+    return more
+
+
 def decode_workload(args: argparse.Namespace) -> dict:
     """the decode step (configs[1]; `decode_p12`: configs[2]) as one replayed hipGraph: the line's dict"""
     import torch
@@ -679,8 +694,10 @@ def decode_workload(args: argparse.Namespace) -> dict:
             "head_dim": cfg.head_dim, "intermediate": cfg.intermediate, "vocab": cfg.vocab, "context": CTX,
             "weight_bytes_per_step": wbytes, "kv_bytes_per_step": kvbytes,
             "kernels_per_step": (2 + 6 * cfg.layers if args.rows == 1 else
-                                 3 + (7 - step.rows_attn_fused) * cfg.layers if step.fused else
-                                 5 + (10 - step.rows_attn_fused - (step.glu_fold and not packed)) * cfg.layers),
+                                 3 + (7 - (step.rows_attn_fused or step.span_fused)) * cfg.layers if step.fused else
+                                 5 + (10 - (step.rows_attn_fused or step.span_fused)
+                                      - (step.glu_fold and not packed)) * cfg.layers)
+                                + second_launches(step, card),
             "host_wall_ms_per_step": round(wall * 1e3 / args.steps, 4),
             **({"tuning": tuned} if tuned else {}),
         },
