@@ -239,12 +239,13 @@ __global__ void __launch_bounds__(KS * 64) mfma_ahead_kernel(const uint8_t* __re
                         const float gb = bfround(g), ub = bfround(u);
                         return f32_bf16(bfround(gb / (1.f + expf(-gb))) * ub);
                     };
-                    const int row = row_of(tile) + lg * 4, own = RAG ? tile * OUT : 0;
+                    // (the four outputs under one condition where no tiles overlap: one store)
+                    const int row = row_of(tile) + lg * 4, own = tile * OUT;
                     uint16_t* o = y + (size_t)m * outs + row;
-                    if (row + 0 >= own) o[0] = fold(s.x, up.x);
-                    if (row + 1 >= own) o[1] = fold(s.y, up.y);
-                    if (row + 2 >= own) o[2] = fold(s.z, up.z);
-                    if (row + 3 >= own) o[3] = fold(s.w, up.w);
+                    if (!RAG || row + 0 >= own) o[0] = fold(s.x, up.x);
+                    if (!RAG || row + 1 >= own) o[1] = fold(s.y, up.y);
+                    if (!RAG || row + 2 >= own) o[2] = fold(s.z, up.z);
+                    if (!RAG || row + 3 >= own) o[3] = fold(s.w, up.w);
                 }
             } else {
                 const int in_tile = lg * 4, row = row_of(tile) + in_tile;
