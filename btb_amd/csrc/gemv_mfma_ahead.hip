@@ -302,7 +302,8 @@ static int32_t launch_ahead(const void* w, const void* x, void* y, int R, int C,
     // whole turns of the grid over the tiles: the smallest grid that walks them in ceil(ntiles / cap) turns
     const int turns = (ntiles + cap - 1) / cap, grid = (ntiles + turns - 1) / turns;
     if constexpr (XN)
-        hipLaunchKernelGGL(kern, dim3(grid), dim3(KS * 64), lds, st, static_cast<const uint8_t*>(w), static_cast<uint16_t*>(y), R, C, M, xa);
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(KS * 64), lds, st, static_cast<const uint8_t*>(w), static_cast<uint16_t*>(y), R, C, M,
+                           xa);
     else
         hipLaunchKernelGGL(kern, dim3(grid), dim3(KS * 64), lds, st, static_cast<const uint8_t*>(w), static_cast<const uint4*>(x),
                            static_cast<uint16_t*>(y), R, C, M);
@@ -358,8 +359,9 @@ bool mfma_ahead_fits(int R, int C, int M, bool glu) {
     // ahead, and a slice of four to seven steps still loads and stores all eight. 6600 shapes, medians of the time against
     // gemv_mfma_lds's by turns (to half a turn, to two, more), one tile of x rows / two: short slices of two waves 0.92 / 0.89, 1.03 /
     // 1.03, 1.00 / 0.86, of four 0.98 / 0.98, 1.04 / 1.05, 0.95 / 0.85, of eight 1.03 / 1.06, 1.04 / 1.06, 0.88 / 0.91; whole ones 0.97 /
-    // 0.95, 0.99 / 0.97, 0.92 / 0.86 (nine and ten steps 0.90 / 0.95, 0.94 / 0.95, 0.89 / 0.82). With the fold 0.03 to 0.06 more: two waves' short slices
-    // then pay to a quarter of a turn, and slices of nine steps not between one turn and two ([18816 x 544] 5 rows 7.4 / 8.2).
+    // 0.95, 0.99 / 0.97, 0.92 / 0.86 (nine and ten steps 0.90 / 0.95, 0.94 / 0.95, 0.89 / 0.82). With the fold 0.03 to 0.06
+    // more: two waves' short slices then pay to a quarter of a turn, and slices of nine steps not between one turn and two ([18816 x
+    // 544] 5 rows 7.4 / 8.2).
     const int ks = nsteps <= 20 ? 2 : nsteps <= 40 ? 4 : 8, steps = (nsteps + ks - 1) / ks;
     const int64_t waves = (int64_t)((R + 15) / 16) * ks;
     if (M > 32) return false;

@@ -263,8 +263,8 @@ static bool pass_a_row(size_t rows, size_t cols, size_t b) {
 // lane16_kernel takes 512 columns at a time (128 from two rows on) and what is left sixteen by sixteen. us lane16_kernel / wide: one
 // row of x [128 x 520] 2.6 / 3.6, [128 x 2056] 4.8 / 6.2, [14615 x 544] 6.2 / 10.2, [170 x 6424] 13.8 / 15.3, but [276 x 240] 5.0 /
 // 4.3, [2048 x 264] 6.2 / 3.3, [512 x 2880] 9.3 / 7.8; two rows [2048 x 520] 5.3 / 4.7, [2048 x 136] 2.9 / 3.2, [793 x 208] 5.1 / 4.3,
-// [8192 x 520] 5.7 / 6.3, [8192 x 2056] 18.7 / 14.1, [32768 x 520] 13.0 / 17.3; four [8192 x 136] 4.0 / 4.3, [10746 x 504] 10.8 / 8.5, [32768 x
-// 264] 9.7 / 11.4; eight [32768 x 136] 13.0 / 13.0. (A bf16 x is 2 bytes a request there: [128 x 520] one row 7.6 / 5.5.)
+// [8192 x 520] 5.7 / 6.3, [8192 x 2056] 18.7 / 14.1, [32768 x 520] 13.0 / 17.3; four [8192 x 136] 4.0 / 4.3, [10746 x 504] 10.8 / 8.5,
+// [32768 x 264] 9.7 / 11.4; eight [32768 x 136] 13.0 / 13.0. (A bf16 x is 2 bytes a request there: [128 x 520] one row 7.6 / 5.5.)
 static bool wide_pays(size_t rows, size_t cols, size_t n, bool f32) {
     if (!f32 || cols % 128 == 0 || n >= 8) return true;
     if (n == 1) return cols % 512 > 176 + cols / 64;

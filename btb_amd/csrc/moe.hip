@@ -639,10 +639,10 @@ static int gate_up_grid(int whole, double wgs, double per_cu) {
 // 89.6 / 73.8, 142 / 102; 16 of 2, 1024 / 512, whose waves have 2 KB on their way each, 32 rows at two / four a CU 40.9 / 35.3 (56.7).
 // (A third of the workgroups instead of a quarter, no multiple of eight: 86.2 and 147 for the first two.) Rows of more than four units
 // a lane take two trips to memory a pick: waves of one or two tiles more than others cost that much more, and small launches
-// lose by the cut (64 of 4, 1056 / 1216, 132 workgroups a row, 8 rows 47.7 -> 51.2, 23 rows 94.7 -> 106; 32 of 4, 768 / 1728, 96, 6 rows 31.0 ->
-// 34.3; but 64 of 2, 3712 / 1056, 464, 13 rows 111 -> 102, 128 of 6, 960 / 2816, 240, 31 rows 347 -> 332). MXFP4's are bound by the widening and keep a wave a tile. The
-// multiple of eight is left where it would begin another turn of the CUs: MXFP4 32 of 4, 1632 / 832, 5 rows, 510 workgroups or 520,
-// 17.6 / 19.9; 16 of 8, 2720 / 928, 3 rows 27.4 / 30.5.
+// lose by the cut (64 of 4, 1056 / 1216, 132 workgroups a row, 8 rows 47.7 -> 51.2, 23 rows 94.7 -> 106; 32 of 4, 768 / 1728, 96, 6
+// rows 31.0 -> 34.3; but 64 of 2, 3712 / 1056, 464, 13 rows 111 -> 102, 128 of 6, 960 / 2816, 240, 31 rows 347 -> 332). MXFP4's are
+// bound by the widening and keep a wave a tile. The multiple of eight is left where it would begin another turn of the CUs: MXFP4 32
+// of 4, 1632 / 832, 5 rows, 510 workgroups or 520, 17.6 / 19.9; 16 of 8, 2720 / 928, 3 rows 27.4 / 30.5.
 static int down_grid(int whole, int T, bool widens, size_t wave_bytes, int units_a_lane) {
     if (T == 1) return whole;
     const int cus = device_info().cus, eights = (whole + 7) / 8 * 8;
