@@ -313,8 +313,9 @@ static int32_t launch_variant(const typename F::Params& p, const XArgs& xa, void
     constexpr bool BF16_NORM_ROW =
         std::is_same<F, FmtBf16>::value && M == 1 && (XMODE == X_ADDNORM || XMODE == X_ADDNORM_4) && EPI == E_PLAIN;
     // FP8's gate / up rows at one row of x: five. At four the even cut below could leave two workgroups a CU, whose waves
-    // are too few to hide the widening: [19456 x 2560] 15.4 -> 12.5 us, [28672 x 3584] 21.8 -> 20.7, [25600 x 3328] 20.9 ->
-    // 19.6, [24576 x 4096] 20.0 -> 19.6; at six [24576 x 4096] takes 20.7, [24576 x 3200] 19.4 (17.3 at five).
+    // are too few to hide the widening: with the add + norm, us in turn at four / five / six, [19456 x 2560] 16.9 / 13.2 / 13.3,
+    // [25600 x 3328] 21.8 / 20.0 / 19.9, [28672 x 3584] 22.6 / 21.2 / 21.1, [24576 x 4096] 20.1 / 19.9 / 21.7, [24576 x 3200] 18.0 /
+    // 17.9 / 19.6.
     constexpr bool FP8_GLU_ROW = std::is_same<F, FmtF8>::value && M == 1 && EPI != E_PLAIN;
     if (per_cu <= 0)
         per_cu = BF16_NORM_ROW ? 2
