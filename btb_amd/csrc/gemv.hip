@@ -315,8 +315,11 @@ static int32_t launch_variant(const typename F::Params& p, const XArgs& xa, void
     // FP8's gate / up rows at one row of x: five. At four the even cut below could leave two workgroups a CU, whose waves
     // are too few to hide the widening: with the add + norm, us in turn at four / five / six, [19456 x 2560] 16.9 / 13.2 / 13.3,
     // [25600 x 3328] 21.8 / 20.0 / 19.9, [28672 x 3584] 22.6 / 21.2 / 21.1, [24576 x 4096] 20.1 / 19.9 / 21.7, [24576 x 3200] 18.0 /
-    // 17.9 / 19.6.
-    constexpr bool FP8_GLU_ROW = std::is_same<F, FmtF8>::value && M == 1 && EPI != E_PLAIN;
+    // 17.9 / 19.6. Not rows of which a CU's LDS holds four or three workgroups, and still not two (9217 to 13312 columns): the fifth
+    // waits for one of them to end. us at four / five, [10240 x 9984] 25.3 / 26.8, [10240 x 11008] 26.9 / 29.9, [10240 x 13184] 30.5 / 32.8,
+    // but [20480 x 7168] 33.4 / 28.1, [8704 x 14720] 44.2 / 41.2; 10000 shapes past 8192 columns, five against four by length: 1.00 to
+    // 9216 columns, 1.003 to 1.008 to 13312 (a tenth of them 1.03 and more), 0.986 to 0.992 beyond.
+    const bool FP8_GLU_ROW = std::is_same<F, FmtF8>::value && M == 1 && EPI != E_PLAIN && (C <= 9216 || C > 13312);
     if (per_cu <= 0)
         per_cu = BF16_NORM_ROW ? 2
                  : FP8_GLU_ROW ? 5

@@ -683,6 +683,27 @@ def test_fp8_one_row_over_long_rows(card, R, C, block):
     assert torch.equal(out.view(torch.int16), card.gemv_fp8(w, x1).view(torch.int16)) and torch.equal(h2, h1)
 
 
+@pytest.mark.parametrize("C", [9216, 9344, 13312, 13440])
+def test_fp8_gate_up_at_the_lines_of_its_grid(card, C):
+    """one row's gate / up fold either side of the lengths at which its launch is cut otherwise: the bits of the matvec and
+    silu_mul, by the rule and at any count of workgroups"""
+    R, g = 10240, gen(97 + C)
+    raw = torch.randint(0, 256, (R * C,), generator=g, dtype=torch.uint8)
+    raw[raw & 0x7F == 0x7F] = 0  # no NaN
+    w = fp8.F8Weight(raw.cuda(), torch.full((R // 128, C // 128), 1e-4).cuda(), R, C)
+    h, nw = acts_bf16(1, C, seed=98).cuda(), torch.ones(C, dtype=torch.bfloat16, device="cuda")
+    h1, x1, m = h.clone(), torch.empty_like(h), torch.empty(1, R // 2, dtype=torch.bfloat16, device="cuda")
+    card.add_rmsnorm(h1, None, nw, 1e-6, x1)
+    card.silu_mul(card.gemv_fp8(w, x1), m)
+    try:
+        for per_cu in (-1, 2, 4, 5):
+            card.set_tuning("gemv_wgs_per_cu", per_cu)
+            out = card.gemv_norm(w, h, None, nw, 1e-6, torch.empty_like(h), torch.empty_like(m), glu=True)
+            assert torch.equal(out.view(torch.int16), m.view(torch.int16)), per_cu
+    finally:
+        card.set_tuning("gemv_wgs_per_cu", -1)
+
+
 # FP8 rows past 10240 columns, x streamed beside the weights: one tile of x rows and two; matrices the vector kernel keeps
 # (fewer than 2048 rows) beside those the staged kernel takes, a last tile that starts inside the one before it
 @pytest.mark.parametrize("R,C,block", [(2048, 12288, (128, 128)), (2064, 16384, (16, 128)), (144, 12288, (16, 32)),
