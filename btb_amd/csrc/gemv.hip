@@ -290,7 +290,9 @@ static int32_t launch_variant(const typename F::Params& p, const XArgs& xa, void
     constexpr int ROWS = tile_outputs<LPR, RPW, EPI>();
     const DeviceInfo& dev = device_info();
     const size_t lds = stage_lds_bytes(XMODE, M, C);
-    if (lds > (size_t)dev.lds_bytes) {
+    // what the kernel holds besides: the norm's four partial sums, the pair table
+    constexpr size_t FIXED = (XMODE == X_ADDNORM || XMODE == X_ADDNORM_4 ? 16 : 0) + (std::is_same<F, FmtP12G>::value ? 512 : 0);
+    if (lds + FIXED > (size_t)dev.lds_bytes) {
         set_error("gemv: the x rows do not fit LDS");
         return ERR_DOMAIN;
     }

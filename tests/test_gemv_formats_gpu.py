@@ -15,6 +15,7 @@ import torch
 
 import oracle
 from btb_amd import fp8, mxfp4, pack12
+from btb_amd.native import HipError
 from btb_amd.pack12 import P12Weight
 from oracle import codecs
 
@@ -681,6 +682,27 @@ def test_fp8_one_row_over_long_rows(card, R, C, block):
     card.add_rmsnorm(h1, None, nw, 1e-6, x1)
     card.gemv_embed_norm(w, h, torch.zeros(1, dtype=torch.int32, device="cuda"), nw, 1e-6, h2, out)
     assert torch.equal(out.view(torch.int16), card.gemv_fp8(w, x1).view(torch.int16)) and torch.equal(h2, h1)
+
+
+@pytest.mark.parametrize("form", ["bf16", "pack12", "fp8"])
+def test_rows_that_fill_the_lds_are_refused_on_the_host(card, form):
+    """four rows of 16384 values and a raw one are all of a CU's LDS, with nothing left for the norm's own sums: refused before
+    any launch, with the code other rows too long get and no error left for the next call; three rows are taken"""
+    R, C = 32, 16384
+    wf = weights_bf16(R, C, seed=99)
+    if form == "fp8":
+        q, s = fp8.quantize(wf.float(), (32, 128))
+        w, op = fp8.F8Weight(q.view(torch.uint8).cuda(), s.cuda(), R, C), card.gemv_fp8
+    else:
+        w, op = (P12Weight.pack(wf.cuda(), card), card.gemv_p12) if form == "pack12" else (wf.cuda(), card.gemv)
+    h, nw = acts_bf16(4, C, seed=100).cuda(), torch.ones(C, dtype=torch.bfloat16, device="cuda")
+    with pytest.raises(HipError, match="fit LDS"):
+        card.gemv_norm(w, h, None, nw, 1e-6, torch.empty_like(h), torch.empty(4, R, dtype=torch.bfloat16, device="cuda"))
+    assert float(torch.ones(8, device="cuda").sum()) == 8.0
+    h1, x1 = h[:3].clone(), torch.empty_like(h[:3])
+    card.add_rmsnorm(h1, None, nw, 1e-6, x1)
+    out = card.gemv_norm(w, h[:3], None, nw, 1e-6, torch.empty_like(h1), torch.empty(3, R, dtype=torch.bfloat16, device="cuda"))
+    assert torch.equal(out.view(torch.int16), op(w, x1).view(torch.int16))
 
 
 @pytest.mark.parametrize("C", [9216, 9344, 13312, 13440])
