@@ -267,7 +267,17 @@ static bool pass_a_row(size_t rows, size_t cols, size_t b) {
 // [32768 x 264] 9.7 / 11.4; eight [32768 x 136] 13.0 / 13.0. (A bf16 x is 2 bytes a request there: [128 x 520] one row 7.6 / 5.5.)
 static bool wide_pays(size_t rows, size_t cols, size_t n, bool f32) {
     if (!f32 || cols % 128 == 0 || n >= 8) return true;
-    if (n == 1) return cols % 512 > 176 + cols / 64;
+    if (n == 1) {  // more rows of the matrix: what a leftover column costs the narrow kernel overlaps, staging x in every workgroup
+                   // does not. Medians of wide / narrow over 6200 shapes by what is left of 512 columns (180 .. 300 / .. 400 / .. 511): up to 4096
+                   // rows 0.98 / 0.77 / 0.70; fewer than 512 columns 1.10 / 0.92 / 0.82 to 8192 rows, 1.5 / 1.25 / 1.1 to 20000, 1.8 / 1.2 /
+                   // 0.85 beyond; to 2048 columns past 8192 rows 1.15 / 0.95 / 0.85; to 4096 columns 1.12 / 1.03 / 0.97 to 12288 rows, 1.25 / 1.17
+                   // / 1.08 beyond; longer past 4096 rows 1.2. [17646 x 264] 4.6 / 8.8 us, [6324 x 5624] 18.5 / 25.3.
+        const size_t left = cols % 512;
+        if (left <= 176 + cols / 64) return false;
+        if (rows <= 4096 || (rows <= 8192 && cols >= 512 && cols < 4096)) return true;
+        if (cols < 512) return rows <= 8192 ? left > 288 : rows > 20000 && left > 448;
+        return cols < 2048 ? left > 352 : cols < 4096 && rows <= 12288 && left > 400;
+    }
     if (n < 4) return rows <= (cols < 1024 ? 4096u : 8192u) && (cols >= 256 || cols % 128 >= 64);
     return cols >= rows / 32;
 }

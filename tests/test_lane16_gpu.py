@@ -53,7 +53,8 @@ def test_bf16_rows_that_end_inside_a_step(card, rows, cols, b):
 
 @pytest.mark.parametrize("rows,cols,b", [(1025, 200, 5), (9000, 136, 2), (9000, 136, 4), (5000, 248, 7), (136, 4992, 40), (512, 2056, 16),
                                          (1024, 1024, 8), (1024, 1024, 9), (2000, 128, 6), (4100, 1032, 3), (170, 6424, 1), (600, 720, 1),
-                                         (8200, 520, 13)])
+                                         (8200, 520, 13), (4096, 184, 1), (4097, 184, 1), (8193, 480, 1), (20001, 480, 1), (8193, 960, 1),
+                                         (4097, 4600, 1)])
 def test_bf16_rows_at_the_lines_between_the_kernels(card, rows, cols, b):
     """shapes either side of where a pass goes row by row, in fours, or to the kernel that looks at one column a load: the
     host's bits from all of them"""
